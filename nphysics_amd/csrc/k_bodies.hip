@@ -19,7 +19,8 @@
 // body's dynamics update (the reference updates the dynamics after the position solve from that
 // velocity, mechanical_world.rs:343-346; k_apply_force needs it between steps).
 // k_apply_force restates Body::apply_force (rigid_body.rs:771-822) between steps.
-// All are HBM bound: 112 B read + 160 B written per body for k_prestep, 96 B + 48 B for
+// k_state_out / k_state_in move the bodies' state to and from the caller's packed rows (see there).
+// The others are HBM bound: 112 B read + 160 B written per body for k_prestep, 96 B + 48 B for
 // k_integrate (plus the optional attribute arrays when some body uses them).
 #include <hip/hip_runtime.h>
 
@@ -215,6 +216,83 @@ __global__ void __launch_bounds__(256) k_clear_dyn_marks(DevBodies b) {
 void launch_clear_dyn_marks(const DevBodies& b, hipStream_t s) {
   if (b.n == 0) return;
   hipLaunchKernelGGL(k_clear_dyn_marks, dim3((b.n + 255) / 256), dim3(256), 0, s, b);
+}
+
+// State transfer. The caller's rows are packed (3, 4, 3 and 3 floats per body), the device's are
+// float4s, poses interleaved; both sides of the copy are pinned host memory that the kernels address
+// directly. A workgroup moves the rows of 256 bodies through LDS, so that the host side of every
+// access is a contiguous run of 16-byte words (a lane's own row is 12 or 16 bytes: written lane by
+// lane it crosses the host link in 4-byte pieces). Bound by the host link: 52 B per body. Measured
+// through nphys_get_state: 13.6 ms -> 24 us for 1,001 bodies and 1.52 s -> 0.39 ms for 99,996, most
+// of it now the host's own copy into the caller's arrays; before, the interleaved poses went by
+// hipMemcpy2D into pageable memory, one 16-byte row at a time (about 7 us a row).
+constexpr int kIoBlock = 256;
+
+// The first `count` floats of the workgroup's packed rows, 16 bytes per lane and access.
+template <bool kOut>
+__device__ __forceinline__ void io_rows(float* host, float* rows, int count) {
+  float4* h4 = reinterpret_cast<float4*>(host);
+  float4* r4 = reinterpret_cast<float4*>(rows);
+  for (int k = threadIdx.x; k < count / 4; k += kIoBlock) {
+    if (kOut) h4[k] = r4[k];
+    else r4[k] = h4[k];
+  }
+  for (int k = (count & ~3) + int(threadIdx.x); k < count; k += kIoBlock) {
+    if (kOut) host[k] = rows[k];
+    else rows[k] = host[k];
+  }
+}
+
+__global__ void __launch_bounds__(kIoBlock) k_state_out(DevBodies b, StateRows o) {
+  __shared__ __align__(16) float s_rows[4 * kIoBlock];
+  const int i0 = blockIdx.x * kIoBlock, i = i0 + threadIdx.x, t = threadIdx.x;
+  const int m = b.n - i0 < kIoBlock ? b.n - i0 : kIoBlock;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    if (!o.row[a]) continue;
+    const int w = a == 1 ? 4 : 3;
+    if (i < b.n) {
+      const float4 v = a == 0 ? b.pos(i) : (a == 1 ? b.rot(i) : (a == 2 ? b.linvel[i] : b.angvel[i]));
+      s_rows[w * t] = v.x;
+      s_rows[w * t + 1] = v.y;
+      s_rows[w * t + 2] = v.z;
+      if (w == 4) s_rows[w * t + 3] = v.w;
+    }
+    __syncthreads();
+    io_rows<true>(o.row[a] + long(i0) * w, s_rows, w * m);
+    __syncthreads();
+  }
+  __threadfence_system();
+}
+
+__global__ void __launch_bounds__(kIoBlock) k_state_in(DevBodies b, StateRows o) {
+  __shared__ __align__(16) float s_rows[4 * kIoBlock];
+  const int i0 = blockIdx.x * kIoBlock, i = i0 + threadIdx.x, t = threadIdx.x;
+  const int m = b.n - i0 < kIoBlock ? b.n - i0 : kIoBlock;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    if (!o.row[a]) continue;
+    const int w = a == 1 ? 4 : 3;
+    io_rows<false>(o.row[a] + long(i0) * w, s_rows, w * m);
+    __syncthreads();
+    if (i < b.n) {
+      const float4 v = make_float4(s_rows[w * t], s_rows[w * t + 1], s_rows[w * t + 2], w == 4 ? s_rows[w * t + 3] : 0.0f);
+      if (a == 0) b.pos(i) = v;
+      else if (a == 1) b.rot(i) = v;
+      else if (b.status[i] == STATUS_DYNAMIC) (a == 2 ? b.linvel : b.angvel)[i] = v;
+    }
+    __syncthreads();
+  }
+}
+
+void launch_state_out(const DevBodies& b, const StateRows& o, hipStream_t s) {
+  if (b.n == 0) return;
+  hipLaunchKernelGGL(k_state_out, dim3((b.n + kIoBlock - 1) / kIoBlock), dim3(kIoBlock), 0, s, b, o);
+}
+
+void launch_state_in(const DevBodies& b, const StateRows& o, hipStream_t s) {
+  if (b.n == 0) return;
+  hipLaunchKernelGGL(k_state_in, dim3((b.n + kIoBlock - 1) / kIoBlock), dim3(kIoBlock), 0, s, b, o);
 }
 
 void launch_apply_force(const DevBodies& b, const SimParams& p, int nu, const int* ubody, const int* off,

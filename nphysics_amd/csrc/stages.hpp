@@ -11,6 +11,15 @@ void launch_prestep(const DevBodies& b, const SimParams& p, hipStream_t s);
 // only: when given, the bodies with only[i] != 0 (a CCD substep's island)
 void launch_integrate(const DevBodies& b, const SimParams& p, hipStream_t s, const uint32_t* only = nullptr);
 void launch_clear_dyn_marks(const DevBodies& b, hipStream_t s);
+// Packed rows of the bodies' state in pinned host memory as the device addresses it: positions (3
+// floats per body), rotations (4), linear and angular velocities (3 each), each 16-byte aligned; null:
+// not moved. Velocities are set for dynamic bodies only.
+struct StateRows {
+  float* row[4];
+};
+void launch_state_out(const DevBodies& b, const StateRows& o, hipStream_t s);
+void launch_state_in(const DevBodies& b, const StateRows& o, hipStream_t s);
+
 void launch_save_rot_dyn(const DevBodies& b, float4* out, hipStream_t s);
 void launch_apply_force(const DevBodies& b, const SimParams& p, int nu, const int* ubody, const int* off,
                         const int* order, const float* forces, const float* points, int type, int wake,

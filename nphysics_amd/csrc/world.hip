@@ -243,6 +243,9 @@ struct World {
   uint32_t* rb_host = nullptr;
   uint32_t* rb_dev = nullptr;
   uint32_t rb_seq = 0, class_seq = 0;
+  // Staging of set_state and get_state (pinned, device-mapped): 52 B per body, grown on first use.
+  float *io_host = nullptr, *io_dev = nullptr;
+  size_t io_cap = 0;
   struct RbSeg {
     const uint32_t* src;
     int n;
@@ -258,6 +261,7 @@ struct World {
     if (h_visit) (void)hipHostFree(h_visit);
     if (red_pinned) (void)hipHostFree(red_pinned);
     if (rb_host) (void)hipHostFree(rb_host);
+    if (io_host) (void)hipHostFree(io_host);
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     for (auto& e : kt_ev)
@@ -535,7 +539,7 @@ struct World {
     if (first) *first = n;
     if (d.n == 0) return NPHYS_OK;
     const int n0 = n, n1 = n + d.n;
-    std::vector<float4> hp(d.n), hr(d.n), hv(d.n), hw(d.n), hmn(d.n), hmx(d.n);
+    std::vector<float4> hp(size_t(d.n) * kPoseBlock), hv(d.n), hw(d.n), hmn(d.n), hmx(d.n);
     std::vector<float2> ha(d.n);
     bool any_sleeper = false;
     int64_t new_dynamic = 0;
@@ -636,8 +640,9 @@ struct World {
       h_ccd_key.push_back(ckey);
       const float* p = d.pos + 3 * k;
       const float* q = d.rot + 4 * k;
-      hp[k] = make_float4(p[0], p[1], p[2], 0.0f);
-      hr[k] = make_float4(q[0], q[1], q[2], q[3]);
+      const float4 hpos = make_float4(p[0], p[1], p[2], 0.0f), hrot = make_float4(q[0], q[1], q[2], q[3]);
+      hp[size_t(k) * kPoseBlock] = hpos;
+      hp[size_t(k) * kPoseBlock + 1] = hrot;
       const bool dyn = st == NPHYS_STATUS_DYNAMIC;
       // ActivationStatus::new_active (body.rs:77-82): energy 4 x the default threshold 0.01
       const float thr = d.sleep_threshold ? d.sleep_threshold[k] : -1.0f;
@@ -649,7 +654,7 @@ struct World {
       hw[k] = (dyn && d.angvel) ? make_float4(d.angvel[3 * k], d.angvel[3 * k + 1], d.angvel[3 * k + 2], 0.0f)
                                 : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       // proxy creation: loose = aabb(pos) loosened by the query limit, then by 0.01
-      const aabb a = shape_aabb(sh, xyz(he), xyz(hp[k]), toq(hr[k]));
+      const aabb a = shape_aabb(sh, xyz(he), xyz(hpos), toq(hrot));
       const aabb lo = loosened(loosened(a, h_qlim.back()), 0.01f);
       hmn[k] = f4(lo.mn, 0.0f);
       hmx[k] = f4(lo.mx, 0.0f);
@@ -702,8 +707,7 @@ struct World {
     HIPCK(hipMemsetAsync(sol.as<float4>() + size_t(n0) * kSolverBlock, 0, size_t(d.n) * kSolverBlock * f4b, stream));
     HIPCK(hipMemcpyAsync(act.as<float2>() + n0, ha.data(), size_t(d.n) * sizeof(float2), hipMemcpyHostToDevice,
                          stream));
-    HIPCK(pose_copy(0, hp.data(), n0, d.n, hipMemcpyHostToDevice));
-    HIPCK(pose_copy(1, hr.data(), n0, d.n, hipMemcpyHostToDevice));
+    HIPCK(up(pose, hp.data(), size_t(d.n) * kPoseBlock * f4b, size_t(n0) * kPoseBlock * f4b));
     HIPCK(up(linvel, hv.data(), size_t(d.n) * f4b, size_t(n0) * f4b));
     HIPCK(up(angvel, hw.data(), size_t(d.n) * f4b, size_t(n0) * f4b));
     HIPCK(up(loose_mn, hmn.data(), size_t(d.n) * f4b, size_t(n0) * f4b));
@@ -760,15 +764,25 @@ struct World {
     return NPHYS_OK;
   }
 
-  // Copies the positions (slot 0) or rotations (slot 1) of `count` pose blocks from body `first`
-  // on, to or from a packed host array of float4.
-  hipError_t pose_copy(int slot, float4* host, int first, int count, hipMemcpyKind kind) {
-    if (count <= 0) return hipSuccess;
-    const size_t pitch = kPoseBlock * sizeof(float4), w = sizeof(float4);
-    float4* dev = pose.as<float4>() + size_t(first) * kPoseBlock + slot;
-    if (kind == hipMemcpyHostToDevice)
-      return hipMemcpy2DAsync(dev, pitch, host, w, w, size_t(count), kind, stream);
-    return hipMemcpy2DAsync(host, w, dev, pitch, w, size_t(count), kind, stream);
+  // Where the four packed state arrays stand in the pinned staging buffer (grown to fit, at 16-byte
+  // aligned starts): as the host and as the device address them.
+  int state_rows(const bool (&want)[4], StateRows& host, StateRows& dev) {
+    const size_t pad = (size_t(n) + 3) & ~size_t(3), need = pad * 13 * sizeof(float);
+    if (need > io_cap) {
+      HIPCK(hipStreamSynchronize(stream));
+      if (io_host) (void)hipHostFree(io_host);
+      io_host = nullptr;
+      io_cap = 0;
+      HIPCK(hipHostMalloc(reinterpret_cast<void**>(&io_host), need, hipHostMallocMapped | hipHostMallocCoherent));
+      io_cap = need;
+      HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&io_dev), io_host, 0));
+    }
+    const size_t off[4] = {0, pad * 3, pad * 7, pad * 10};
+    for (int a = 0; a < 4; ++a) {
+      host.row[a] = want[a] ? io_host + off[a] : nullptr;
+      dev.row[a] = want[a] ? io_dev + off[a] : nullptr;
+    }
+    return NPHYS_OK;
   }
 
   int set_state(const float* p, const float* r, const float* lv, const float* av) {
@@ -776,35 +790,18 @@ struct World {
     if (r && !rot_dyn_saved) {
       // impulses applied before the next step use the augmented mass of the rotation the last
       // dynamics update saw (the reference recomputes it only in the next step)
-      if (any_ccd) {
-        launch_save_rot_dyn(bodies(), rot_dyn.as<float4>(), stream);
-      } else {
-        HIPCK(hipMemcpy2DAsync(rot_dyn.p, sizeof(float4), pose.as<float4>() + 1, kPoseBlock * sizeof(float4),
-                               sizeof(float4), size_t(n), hipMemcpyDeviceToDevice, stream));
-      }
+      launch_save_rot_dyn(bodies(), rot_dyn.as<float4>(), stream);
       rot_dyn_saved = true;
     }
-    std::vector<float4> hp(n), hr(n), hv(n), hw(n);
-    const size_t f4b = sizeof(float4);
-    HIPCK(pose_copy(0, hp.data(), 0, n, hipMemcpyDeviceToHost));
-    HIPCK(pose_copy(1, hr.data(), 0, n, hipMemcpyDeviceToHost));
-    HIPCK(hipMemcpyAsync(hv.data(), linvel.p, n * f4b, hipMemcpyDeviceToHost, stream));
-    HIPCK(hipMemcpyAsync(hw.data(), angvel.p, n * f4b, hipMemcpyDeviceToHost, stream));
-    HIPCK(hipStreamSynchronize(stream));
-    for (int i = 0; i < n; ++i) {
-      if (p) hp[i] = make_float4(p[3 * i], p[3 * i + 1], p[3 * i + 2], 0.0f);
-      if (r) hr[i] = make_float4(r[4 * i], r[4 * i + 1], r[4 * i + 2], r[4 * i + 3]);
-      if (h_status[i] == NPHYS_STATUS_DYNAMIC) {
-        if (lv) hv[i] = make_float4(lv[3 * i], lv[3 * i + 1], lv[3 * i + 2], 0.0f);
-        if (av) hw[i] = make_float4(av[3 * i], av[3 * i + 1], av[3 * i + 2], 0.0f);
-      }
-    }
-    HIPCK(pose_copy(0, hp.data(), 0, n, hipMemcpyHostToDevice));
-    HIPCK(pose_copy(1, hr.data(), 0, n, hipMemcpyHostToDevice));
-    HIPCK(hipMemcpyAsync(linvel.p, hv.data(), n * f4b, hipMemcpyHostToDevice, stream));
-    HIPCK(hipMemcpyAsync(angvel.p, hw.data(), n * f4b, hipMemcpyHostToDevice, stream));
+    const float* in[4] = {p, r, lv, av};
+    StateRows host, dev;
+    int rc = state_rows({p != nullptr, r != nullptr, lv != nullptr, av != nullptr}, host, dev);
+    if (rc) return rc;
+    for (int a = 0; a < 4; ++a)
+      if (in[a]) std::memcpy(host.row[a], in[a], size_t(n) * (a == 1 ? 4 : 3) * sizeof(float));
+    launch_state_in(bodies(), dev, stream);
     if (sleeping || any_ccd) launch_clear_dyn_marks(bodies(), stream);
-    HIPCK(hipStreamSynchronize(stream));
+    if ((rc = readback({}))) return rc;  // the staging buffer has been read
     moved = true;
     wake_pending = sleeping;
     return NPHYS_OK;
@@ -839,24 +836,14 @@ struct World {
 
   int get_state(float* p, float* r, float* lv, float* av) {
     if (n == 0) return NPHYS_OK;
-    std::vector<float4> h(n);
-    const size_t f4b = sizeof(float4);
-    struct Item { DBuf* b; int slot; float* out; int w; };
-    const Item items[4] = {{nullptr, 0, p, 3}, {nullptr, 1, r, 4}, {&linvel, 0, lv, 3}, {&angvel, 0, av, 3}};
-    for (const Item& it : items) {
-      if (!it.out) continue;
-      if (it.b)
-        HIPCK(hipMemcpyAsync(h.data(), it.b->p, n * f4b, hipMemcpyDeviceToHost, stream));
-      else
-        HIPCK(pose_copy(it.slot, h.data(), 0, n, hipMemcpyDeviceToHost));
-      HIPCK(hipStreamSynchronize(stream));
-      for (int i = 0; i < n; ++i) {
-        it.out[it.w * i + 0] = h[i].x;
-        it.out[it.w * i + 1] = h[i].y;
-        it.out[it.w * i + 2] = h[i].z;
-        if (it.w == 4) it.out[4 * i + 3] = h[i].w;
-      }
-    }
+    float* out[4] = {p, r, lv, av};
+    StateRows host, dev;
+    int rc = state_rows({p != nullptr, r != nullptr, lv != nullptr, av != nullptr}, host, dev);
+    if (rc) return rc;
+    launch_state_out(bodies(), dev, stream);
+    if ((rc = readback({}))) return rc;
+    for (int a = 0; a < 4; ++a)
+      if (out[a]) std::memcpy(out[a], host.row[a], size_t(n) * (a == 1 ? 4 : 3) * sizeof(float));
     return NPHYS_OK;
   }
 
