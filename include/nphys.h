@@ -212,12 +212,12 @@ typedef struct nphys_counters {
   int64_t sweep_variant;  /* solve of the last step: 0 per-colour launches, 256/512/1024 scene-blocked */
   int64_t loose_changes;  /* accumulated loose AABBs replaced by the end-of-step syncs */
   int64_t pair_rebuilds;  /* accumulated end-of-step broad-phase pair rebuilds */
-  /* accumulated pair rebuilds done incrementally (only the bodies whose loose AABB was replaced
-   * re-traversed, the tree refitted by expansion) instead of by a full tree build */
+  /* accumulated pair rebuilds done incrementally: only the bodies whose loose AABB was replaced, and
+   * those they touch or touched, search anew */
   int64_t incremental_pair_updates;
   int64_t active_bodies;  /* awake dynamic bodies after the last step's activation update */
-  /* accumulated incremental pair updates that overflowed a clean body's candidate segment and
-   * fell back to a full build with larger segments */
+  /* accumulated incremental pair updates that overflowed a body's segment of partners: all bodies
+   * then search anew, with larger segments */
   int64_t incremental_overflows;
   /* learned warm start, while counters are enabled: device time of the network's inference
    * kernel (HIP events around its launch on the world's stream) and the rows it evaluated */
@@ -386,11 +386,10 @@ int nphys_set_residual_target(nphys_world* w, double target, int32_t max_sweeps,
 int nphys_set_sweep_variant(nphys_world* w, int32_t variant);
 
 /* How the pair set follows replaced loose AABBs. 1 (default): when only dynamic bodies' loose
- * AABBs were replaced since the last pair build (at most n/8 of them, and a full build at least
- * every 32 updates), only those bodies are re-traversed in the previous tree refitted by
- * expansion; 0: the tree is rebuilt and every body traversed. The pair set is identical either
- * way. Replaces ncollide's incremental DBVT update (geometrical_world.rs:285-312; the DBVT itself
- * is not in the reference tree). */
+ * AABBs were replaced since the last pair search (at most n/8 of them, and at most 1,024), only those bodies search
+ * for their pairs anew, and the ones that they touch or touched; 0: every body searches. The pair
+ * set is identical either way. Replaces ncollide's incremental DBVT update
+ * (geometrical_world.rs:285-312; the DBVT itself is not in the reference tree). */
 int nphys_set_incremental_pairs(nphys_world* w, int32_t on);
 
 /* Activation energy of every body (ActivationStatus::energy, body.rs:65-125): 0 for a sleeping

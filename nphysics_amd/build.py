@@ -23,6 +23,7 @@ FLAGS = [
     "-fno-gpu-flush-denormals-to-zero",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument",
+    "-Wno-bitwise-instead-of-logical",
 ]
 
 

@@ -62,7 +62,7 @@ struct DevBodies {
   float4* angvel;
   float4* ext_lin;
   float4* ext_ang;
-  float4* loose_mn;
+  float4* loose_mn;      // w: 1 dynamic, 0 static
   float4* loose_mx;
   float2* act;           // (activation energy, sleep threshold); null when no body can sleep
   // Optional per-body attributes, null when every body has the default:

@@ -244,7 +244,7 @@ void launch_activation(const DevBodies& b, const DevContacts& c, int M, const Ac
   }
   if (M > 0) {
     hipLaunchKernelGGL(k_act_manifolds, dim3(nb(M)), dim3(256), 0, s, b, c, M, a.mflag);
-    scan_exclusive_u32(a.mflag, a.pos, M, a.tmp, s);
+    scan_exclusive_u32(a.mflag, a.pos, M, *a.scan, s);
   }
 }
 

@@ -10,26 +10,24 @@
 //   * pairs = every two bodies whose loose AABBs overlap (closed intervals), not the same body and
 //     not both static; stored as (first, second) with first dynamic and second static or larger,
 //     sorted.
-// The pair set is found with a linear BVH rebuilt whenever a loose AABB changed: Morton codes of
-// the loose-AABB centroids, stable LDS radix sort, Karras (HPG 2012) radix-tree construction, an
-// atomic min/max refit with early termination, then one thread per dynamic body (in Morton order, so
-// a wavefront walks neighbouring subtrees) traverses the tree and writes its partners into its
-// own fixed-capacity segment; segments are sorted and compacted with a scan. The result is
-// deterministic and independent of thread timing. Algorithmic bytes: 124 per body + 8 per pair.
-// When only a few dynamic bodies' loose AABBs were replaced since the last pair build (the common
-// case of a resting pile), the segments are updated instead (see the incremental kernels below):
-// a few thousand traversals and one pass over the segments in place of a tree build and n
-// traversals; the pair list is the same.
+// A world of one small scene is searched directly (k_direct). Others go by a tree 64 wide over the
+// colliders in Morton order: boxes of 64 consecutive colliders and boxes of 64 of those (k_boxes, k_top),
+// made anew at every search, while the order itself is sorted every kOrderAge-th time only: any order gives the same pairs,
+// an old one slightly larger boxes. A wave
+// searches for one body (k_search).
+// Every body's partners go to its own fixed-capacity segment; a scan compacts the segments
+// (k_compact). The result is deterministic and independent of thread timing. Algorithmic bytes: 124
+// per body + 8 per pair. When only a few bodies' loose AABBs were replaced since the last search,
+// the other bodies' segments are kept; the pair list is the same.
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "scan.hpp"
 #include "stages.hpp"
 
 namespace nph {
 
 namespace {
-
-constexpr int kStack = 64;
 
 __device__ __forceinline__ uint32_t f2ord(float f) {
   const uint32_t u = __float_as_uint(f);
@@ -39,29 +37,67 @@ __device__ __forceinline__ float ord2f(uint32_t u) {
   return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
 }
 
-__global__ void __launch_bounds__(256) k_loose_update(DevBodies b, int mode, uint32_t* changed,
-                                                     uint32_t* dirty) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= b.n) return;
-  if (mode != 0 && b.status[i] != STATUS_DYNAMIC) return;
-  const int kind = b.shape[i];
-  const f3 he = xyz(b.dims[i]);
-  aabb a = shape_aabb(kind, he, xyz(b.pos(i)), toq(b.rot(i)));
-  if (mode == 2) {  // safe_position (rigid_body.rs:904-910): position0, with linear motion interpolation
-                   // the current rotation
-    const q4 r0 = (b.ccd && (b.ccd[i] & 2)) ? toq(b.rot(i)) : toq(b.rot0[i]);
-    a = merged(shape_aabb(kind, he, xyz(b.pos0[i]), r0), a);
-  }
-  else a = merged(a, a);
+// Replaces body i's loose AABB when it no longer contains `a` loosened by the query limit.
+__device__ __forceinline__ bool loose_one(const DevBodies& b, int i, const aabb& a, aabb& loose) {
   const aabb tight = loosened(a, b.qlim[i]);
-  const aabb loose{xyz(b.loose_mn[i]), xyz(b.loose_mx[i])};
-  if (!contains(loose, tight)) {
-    const aabb nl = loosened(tight, 0.01f);
-    b.loose_mn[i] = f4(nl.mn, 0.0f);
-    b.loose_mx[i] = f4(nl.mx, 0.0f);
+  if (contains(loose, tight)) return false;
+  loose = loosened(tight, 0.01f);
+  return true;
+}
+
+// One thread per body. passes: bit 0 the current pose of every body (of dynamic ones alone with
+// bit 2 clear), bit 1 first the AABB swept from pos0/rot0 to the current pose (dynamic bodies; the
+// CCD phase's sync, geometrical_world.rs:250-261). Both in one launch: a body's second pass reads
+// nothing that another body's first one writes. changed[0..1]: the swept pass's counts, [2..3] the
+// other's. Bodies replaced for the first time since the last pair build go to the dirty list.
+__global__ void __launch_bounds__(256) k_loose_update(DevBodies b, int passes, uint32_t* changed, uint32_t* dirty,
+                                                     int* list, uint32_t* list_count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool in = i < b.n;
+  const bool dynamic = in && b.status[i] == STATUS_DYNAMIC;
+  const bool work = in && (dynamic || (passes & 4));
+  bool swept = false, final = false;
+  if (work) {
+    const int kind = b.shape[i];
+    const f3 he = xyz(b.dims[i]);
+    const q4 rot = toq(b.rot(i));
+    const aabb a = shape_aabb(kind, he, xyz(b.pos(i)), rot);
+    aabb loose{xyz(b.loose_mn[i]), xyz(b.loose_mx[i])};
+    if ((passes & 2) && dynamic) {  // safe_position (rigid_body.rs:904-910): position0, with linear motion
+                                    // interpolation the current rotation
+      const q4 r0 = (b.ccd && (b.ccd[i] & 2)) ? rot : toq(b.rot0[i]);
+      swept = loose_one(b, i, merged(shape_aabb(kind, he, xyz(b.pos0[i]), r0), a), loose);
+    }
+    if (passes & 1) final = loose_one(b, i, merged(a, a), loose);
+    if (swept || final) {
+      b.loose_mn[i] = f4(loose.mn, dynamic ? 1.0f : 0.0f);
+      b.loose_mx[i] = f4(loose.mx, 0.0f);
+    }
+  }
+  // counts and places in the dirty list, one atomic of each per workgroup: changed[0] every AABB the
+  // swept pass replaced, [1] those of non-dynamic bodies, [2] and [3] the other pass's
+  __shared__ uint32_t s_count[5][4];
+  __shared__ uint32_t s_base;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool add = (swept || final) && dirty[i] == 0u;
+  const uint64_t m[5] = {__ballot(swept), __ballot(swept && !dynamic), __ballot(final), __ballot(final && !dynamic),
+                         __ballot(add)};
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) s_count[k][wave] = uint32_t(__popcll(m[k]));
+  }
+  __syncthreads();
+  if (threadIdx.x < 5) {
+    const uint32_t c = s_count[threadIdx.x][0] + s_count[threadIdx.x][1] + s_count[threadIdx.x][2] + s_count[threadIdx.x][3];
+    if (threadIdx.x == 4) s_base = c ? atomicAdd(list_count, c) : 0u;
+    else if (c) atomicAdd(&changed[threadIdx.x], c);
+  }
+  __syncthreads();
+  if (add) {
+    uint32_t at = s_base + uint32_t(__popcll(m[4] & ((1ull << lane) - 1ull)));
+    for (int w = 0; w < wave; ++w) at += s_count[4][w];
     dirty[i] = 1u;
-    atomicAdd(&changed[0], 1u);
-    if (b.status[i] != STATUS_DYNAMIC) atomicAdd(&changed[1], 1u);
+    list[at] = i;
   }
 }
 
@@ -132,399 +168,405 @@ __global__ void __launch_bounds__(256) k_morton(DevBodies b, const uint32_t* bou
   vals[i] = uint32_t(i);
 }
 
-__device__ __forceinline__ int delta(const uint32_t* __restrict__ keys, int n, int i, int j) {
-  if (j < 0 || j >= n) return -1;
-  const uint32_t a = keys[i], c = keys[j];
-  if (a == c) return 32 + __clz(uint32_t(i ^ j));
-  return __clz(a ^ c);
-}
-
-// Karras 2012: internal node i spans a key range with one split; children < n-1 are internal,
-// children >= n-1 are leaves (leaf t is node n-1+t).
-__global__ void __launch_bounds__(256) k_lbvh(const uint32_t* __restrict__ keys, int n, int scene_shift,
-                                             int* child, int* parent, int2* node_scene) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n - 1) return;
-  const int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
-  const int dmin = delta(keys, n, i, i - d);
-  int lmax = 2;
-  while (delta(keys, n, i, i + lmax * d) > dmin) lmax <<= 1;
-  int l = 0;
-  for (int t = lmax >> 1; t >= 1; t >>= 1)
-    if (delta(keys, n, i, i + (l + t) * d) > dmin) l += t;
-  const int j = i + l * d;
-  const int dnode = delta(keys, n, i, j);
-  int s = 0;
-  int t = l;
-  do {
-    t = (t + 1) >> 1;
-    if (delta(keys, n, i, i + (s + t) * d) > dnode) s += t;
-  } while (t > 1);
-  const int gamma = i + s * d + (d < 0 ? d : 0);
-  const int lo = i < j ? i : j, hi = i < j ? j : i;
-  const int left = lo == gamma ? (n - 1 + gamma) : gamma;
-  const int right = hi == gamma + 1 ? (n - 1 + gamma + 1) : gamma + 1;
-  child[2 * i] = left;
-  child[2 * i + 1] = right;
-  node_scene[i] = make_int2(int(keys[lo] >> scene_shift), int(keys[hi] >> scene_shift));
-  parent[left] = i;
-  parent[right] = i;
-  if (i == 0) parent[0] = -1;
-}
-
-// Leaf nodes hold the loose AABBs in Morton order.
-__global__ void __launch_bounds__(256) k_leaf_nodes(DevBodies b, const uint32_t* __restrict__ vals, int n,
-                                                   float4* node_mn, float4* node_mx, int* leaf_of) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int body = int(vals[t]);
-  node_mn[n - 1 + t] = b.loose_mn[body];
-  node_mx[n - 1 + t] = b.loose_mx[body];
-  leaf_of[body] = t;
-}
-
-// Internal-node bounds by atomic min/max on order-preserving integer encodings: every leaf climbs
-// towards the root and stops at the first ancestor none of whose six bounds it changes (a value
-// that does not change a node is dominated by one whose writer keeps climbing). No arrival
-// counters or fences are needed and the bounds are exact (min/max of the leaves below).
-__global__ void __launch_bounds__(256) k_refit_atomic(DevBodies b, const uint32_t* __restrict__ vals, int n,
-                                                     const int* __restrict__ parent, uint32_t* inode) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int body = int(vals[t]);
-  const float4 mn = b.loose_mn[body], mx = b.loose_mx[body];
-  const uint32_t e[6] = {f2ord(mn.x), f2ord(mn.y), f2ord(mn.z), f2ord(mx.x), f2ord(mx.y), f2ord(mx.z)};
-  int p = parent[n - 1 + t];
-  while (p >= 0) {
-    uint32_t* q = inode + 8 * long(p);
-    bool changed = false;
+// Box of 64 consecutive colliders of the order, or of 64 such boxes: bounds, the scenes of its
+// colliders and the largest index a partner can have in it (no limit with a non-dynamic collider).
+__device__ __forceinline__ void wave_box(aabb& a, int& smin, int& smax, int& top) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      if (atomicMin(&q[k], e[k]) > e[k]) changed = true;
-      if (atomicMax(&q[4 + k], e[3 + k]) < e[3 + k]) changed = true;
-    }
-    if (!changed) break;
-    p = parent[p];
+  for (int off = 32; off > 0; off >>= 1) {
+    a.mn.x = fminf(a.mn.x, __shfl_xor(a.mn.x, off));
+    a.mn.y = fminf(a.mn.y, __shfl_xor(a.mn.y, off));
+    a.mn.z = fminf(a.mn.z, __shfl_xor(a.mn.z, off));
+    a.mx.x = fmaxf(a.mx.x, __shfl_xor(a.mx.x, off));
+    a.mx.y = fmaxf(a.mx.y, __shfl_xor(a.mx.y, off));
+    a.mx.z = fmaxf(a.mx.z, __shfl_xor(a.mx.z, off));
+    smin = min(smin, __shfl_xor(smin, off));
+    smax = max(smax, __shfl_xor(smax, off));
+    top = max(top, __shfl_xor(top, off));
   }
 }
 
-__global__ void __launch_bounds__(256) k_decode_nodes(int n, const uint32_t* __restrict__ inode, float4* node_mn,
-                                                     float4* node_mx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n - 1) return;
-  const uint32_t* q = inode + 8 * long(i);
-  node_mn[i] = make_float4(ord2f(q[0]), ord2f(q[1]), ord2f(q[2]), 0.0f);
-  node_mx[i] = make_float4(ord2f(q[4]), ord2f(q[5]), ord2f(q[6]), 0.0f);
+constexpr float kInf = __builtin_huge_valf();
+constexpr int kDynBit = 1 << 30;
+
+// One wave per box: the colliders' loose AABBs in the order (mn.w: index and dynamic flag, mx.w: scene)
+// and their box.
+__global__ void __launch_bounds__(256) k_boxes(DevBodies b, BroadPhaseBufs bp) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63;
+  const bool in = p < b.n;
+  if ((p & ~63) >= b.n) return;
+  aabb a{{kInf, kInf, kInf}, {-kInf, -kInf, -kInf}};
+  int smin = 0x7fffffff, smax = -1, top = -1;
+  if (in) {
+    const int o = int(bp.vals[p]);
+    const float4 mn = b.loose_mn[o], mx = b.loose_mx[o];
+    const bool dyn = mn.w != 0.0f;
+    const int sc = b.scene[o];
+    bp.leaf_mn[p] = f4(xyz(mn), __int_as_float(o | (dyn ? kDynBit : 0)));
+    bp.leaf_mx[p] = f4(xyz(mx), __int_as_float(sc));
+    a = aabb{xyz(mn), xyz(mx)};
+    smin = smax = sc;
+    top = dyn ? o : 0x7fffffff;
+  }
+  wave_box(a, smin, smax, top);
+  if (lane == 0) {
+    bp.box_mn[p >> 6] = f4(a.mn, __int_as_float(smin));
+    bp.box_mx[p >> 6] = f4(a.mx, __int_as_float(smax));
+    bp.box_top[p >> 6] = top;
+  }
 }
 
-__global__ void __launch_bounds__(256) k_init_inodes(int n, uint32_t* inode) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n - 1) return;
-  uint4* q = reinterpret_cast<uint4*>(inode + 8 * long(i));
-  q[0] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0u);
-  q[1] = make_uint4(0u, 0u, 0u, 0u);
+// One wave per box of boxes, stored after the nbox boxes.
+__global__ void __launch_bounds__(64) k_top(BroadPhaseBufs bp, int nbox) {
+  const int k = blockIdx.x * 64 + threadIdx.x;
+  aabb a{{kInf, kInf, kInf}, {-kInf, -kInf, -kInf}};
+  int smin = 0x7fffffff, smax = -1, top = -1;
+  if (k < nbox) {
+    const float4 mn = bp.box_mn[k], mx = bp.box_mx[k];
+    a = aabb{xyz(mn), xyz(mx)};
+    smin = __float_as_int(mn.w);
+    smax = __float_as_int(mx.w);
+    top = bp.box_top[k];
+  }
+  wave_box(a, smin, smax, top);
+  if (threadIdx.x == 0) {
+    bp.box_mn[nbox + blockIdx.x] = f4(a.mn, __int_as_float(smin));
+    bp.box_mx[nbox + blockIdx.x] = f4(a.mx, __int_as_float(smax));
+    bp.box_top[nbox + blockIdx.x] = top;
+  }
 }
 
-// Packed internal nodes for the traversals: one 64-byte record per internal node with both
-// children's bounds and references, so descending one level is a single 64-byte load:
-//   [0] (child0 min, ref0)  [1] (child0 max, ref1)  [2] (child1 min, first scene)
-//   [3] (child1 max, last scene)
-// ref = internal node index, or kLeafRef | dynamic << 30 | body for a leaf; the scene range is
-// that of the node's own leaves.
-constexpr uint32_t kLeafRef = 0x80000000u;
-
-__device__ __forceinline__ uint32_t child_ref(DevBodies b, const uint32_t* __restrict__ vals, int n, int c) {
-  if (c < n - 1) return uint32_t(c);
-  const int o = int(vals[c - (n - 1)]);
-  return kLeafRef | (b.status[o] == STATUS_DYNAMIC ? 1u << 30 : 0u) | uint32_t(o);
+// All six comparisons evaluated (intersects() stops at the first that fails: a branch each).
+__device__ __forceinline__ bool overlap(const aabb& a, const aabb& c) {
+  return (a.mn.x <= c.mx.x) & (c.mn.x <= a.mx.x) & (a.mn.y <= c.mx.y) & (c.mn.y <= a.mx.y) & (a.mn.z <= c.mx.z) &
+         (c.mn.z <= a.mx.z);
 }
 
-__global__ void __launch_bounds__(256) k_pack_nodes(DevBodies b, const uint32_t* __restrict__ vals, int n,
-                                                   const int* __restrict__ child,
-                                                   const float4* __restrict__ node_mn,
-                                                   const float4* __restrict__ node_mx,
-                                                   const int2* __restrict__ node_scene, float4* pnode) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n - 1) return;
-  const int c0 = child[2 * i], c1 = child[2 * i + 1];
-  const int2 sr = node_scene[i];
-  float4* r = pnode + 4 * long(i);
-  r[0] = f4(xyz(node_mn[c0]), __uint_as_float(child_ref(b, vals, n, c0)));
-  r[1] = f4(xyz(node_mx[c0]), __uint_as_float(child_ref(b, vals, n, c1)));
-  r[2] = f4(xyz(node_mn[c1]), __int_as_float(sr.x));
-  r[3] = f4(xyz(node_mx[c1]), __int_as_float(sr.y));
+// Whether the segments of bodies that nothing happened to are kept: the counts of this step's
+// loose-AABB passes are on the device, so no readback stands between the passes and the search.
+__device__ __forceinline__ bool search_incremental(const BroadPhaseBufs& bp, const SearchRun& r, int n) {
+  const uint32_t all = bp.changed[0] + bp.changed[2], fixed = bp.changed[1] + bp.changed[3];
+  return r.may_increment && fixed == 0u && r.dirty_before + long(all) <= long(kept_limit(n));
 }
 
-// Walks the packed tree for the loose AABB of body q and calls leaf(o, dynamic) for every other
-// body of q's scene whose loose AABB overlaps it and whose collision groups can interact with q's.
-// Returns false on a stack overflow.
-// The traversal stack lives in LDS, interleaved across the workgroup's lanes (entry k of lane t at
-// stack[k * kTraverseBlock + t]): a stack in private memory would be scratch, one memory round trip
-// per push and pop on the traversal's dependent chain.
-constexpr int kTraverseBlock = 64;
-
-template <bool kScenes, class F>
-__device__ __forceinline__ bool walk_tree(const DevBodies& b, const float4* __restrict__ pnode, int q,
-                                          int* __restrict__ stack, F&& leaf) {
-  const aabb Q{xyz(b.loose_mn[q]), xyz(b.loose_mx[q])};
-  const int qs = kScenes ? b.scene[q] : 0;
+// ---- search by boxes -----------------------------------------------------------------------------
+// A wave searches for one body, its bounds in scalar registers: it tests 64 upper boxes at a time, then the 64 boxes
+// of each that overlaps, then the 64 colliders of each of those (its lanes the boxes or colliders), and a ballot tells each
+// hit its place in the segment. The loads of the next box are in flight while one is tested. A body meets three to
+// five boxes, so about eight tests of some forty instructions, however many colliders there are. (One wave for the 64
+// bodies of a box, descending by their common bounds, has fewer tests but the slowest wave of a launch, one whose
+// bodies straddle a jump of the Morton curve, held it up: 370 us at 8,001 bodies and 1.75 ms at 99,996.)
+// Measured: 14 us at 8,001 bodies, 29 us at 21,004 and 121 us at 99,996 in piles. With k_boxes, k_top and the
+// compaction the whole phase takes 58, 76 and 190 us there; the binary tree it replaces (topology, atomic
+// refit, packing and a stack per lane, on a sort at every build) took 268, 337 and 526 us.
+//
+// Incremental form: a body searches anew if its loose AABB was replaced (dirty), if it held a dirty
+// partner, or if a dirty body with a larger index now overlaps it; the others keep their segments.
+template <bool kScenes>
+__global__ void __launch_bounds__(256) k_search(DevBodies b, BroadPhaseBufs bp, SearchRun r) {
+  const int lane = threadIdx.x & 63, n = b.n;
+  const uint64_t below = (1ull << lane) - 1ull;
+  const int p = __builtin_amdgcn_readfirstlane(int((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+  if (p >= n) return;
+  const float4 mn = bp.leaf_mn[p], mx = bp.leaf_mx[p];
+  const int code = __float_as_int(mn.w), q = code & (kDynBit - 1), sc = __float_as_int(mx.w);
+  if ((code & kDynBit) == 0) {
+    if (lane == 0) bp.cand_count[q] = 0u;
+    return;
+  }
+  const aabb Q{xyz(mn), xyz(mx)};
   const uint4 qg = b.groups ? b.groups[q] : uint4{};
-  int sp = 0;
-  int node = 0;
-  bool ok = true;
-  while (true) {
-    const float4* r = pnode + 4 * long(node);
-    const float4 a0 = r[0], a1 = r[1], a2 = r[2], a3 = r[3];
-    if (!kScenes || (qs >= __float_as_int(a2.w) && qs <= __float_as_int(a3.w))) {
-      const uint32_t ref[2] = {__float_as_uint(a0.w), __float_as_uint(a1.w)};
-      const aabb B[2] = {{xyz(a0), xyz(a1)}, {xyz(a2), xyz(a3)}};
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        if (!intersects(Q, B[k])) continue;
-        const uint32_t c = ref[k];
-        if (c & kLeafRef) {
-          const int o = int(c & 0x3fffffffu);
-          if (o != q && (!kScenes || b.scene[o] == qs) && (!b.groups || groups_interact(qg, b.groups[o])))
-            leaf(o, ((c >> 30) & 1u) != 0);
-        } else if (sp < kStack) {
-          stack[(sp++) * kTraverseBlock] = int(c);
-        } else {
-          ok = false;
-        }
+  int* seg = bp.cand + long(q) * r.cap;
+  auto partner = [&](int o, bool dyn, int osc, const aabb& B) {
+    bool hit = overlap(Q, B) & (o != q) & (!dyn | (o > q));
+    if (kScenes) hit = hit & (osc == sc);
+    if (b.groups) hit = hit && groups_interact(qg, b.groups[o]);
+    return hit;
+  };
+  if (search_incremental(bp, r, n) && bp.dirty[q] == 0u) {
+    bool again = false;
+    const int c = min(int(bp.cand_count[q]), r.cap), nd = int(*bp.list_count);
+    for (int k = lane; k < c; k += 64) again = again || bp.dirty[seg[k]] != 0u;
+    for (int k = lane; k < nd; k += 64) {  // the dirty bodies are all dynamic here
+      const int o = bp.list[k];
+      again = again || partner(o, true, kScenes ? b.scene[o] : 0, aabb{xyz(b.loose_mn[o]), xyz(b.loose_mx[o])});
+    }
+    if (!__any(again)) return;
+  }
+  auto enter = [&](int k) {
+    const float4 cmn = bp.box_mn[k], cmx = bp.box_mx[k];
+    bool ok = overlap(Q, aabb{xyz(cmn), xyz(cmx)}) & (bp.box_top[k] > q);
+    if (kScenes) ok = ok & (__float_as_int(cmn.w) <= sc) & (__float_as_int(cmx.w) >= sc);
+    return ok;
+  };
+  uint32_t cnt = 0;
+  const int nbox = (n + 63) >> 6, ntop = (nbox + 63) >> 6;
+  for (int t0 = 0; t0 < ntop; t0 += 64) {
+    uint64_t mt = 1ull;
+    if (ntop > 1) {
+      const int t = t0 + lane;
+      mt = __ballot((t < ntop) & enter(nbox + (t < ntop ? t : t0)));
+    }
+    while (mt) {
+      const int t = t0 + __ffsll(static_cast<long long>(mt)) - 1;
+      mt &= mt - 1;
+      const int c = t * 64 + lane;
+      uint64_t mb = __ballot((c < nbox) & enter(c < nbox ? c : nbox - 1));
+      float4 nmn{}, nmx{};
+      auto load = [&](int box) {
+        const int k = box * 64 + lane < n ? box * 64 + lane : n - 1;
+        nmn = bp.leaf_mn[k];
+        nmx = bp.leaf_mx[k];
+      };
+      int next = mb ? t * 64 + __ffsll(static_cast<long long>(mb)) - 1 : -1;
+      if (next >= 0) load(next);
+      while (next >= 0) {
+        const int box = next;
+        const float4 omn = nmn, omx = nmx;
+        mb &= mb - 1;
+        next = mb ? t * 64 + __ffsll(static_cast<long long>(mb)) - 1 : -1;
+        if (next >= 0) load(next);
+        const int ocode = __float_as_int(omn.w), o = ocode & (kDynBit - 1);
+        const bool hit = (box * 64 + lane < n) & partner(o, (ocode & kDynBit) != 0, __float_as_int(omx.w),
+                                                        aabb{xyz(omn), xyz(omx)});
+        const uint64_t m = __ballot(hit);
+        const uint32_t at = cnt + uint32_t(__popcll(m & below));
+        if (hit && at < uint32_t(r.cap)) seg[at] = o;
+        cnt += uint32_t(__popcll(m));
       }
     }
-    if (sp == 0) break;
-    node = stack[(--sp) * kTraverseBlock];
   }
-  return ok;
+  if (lane == 0) {
+    bp.cand_count[q] = cnt;
+    if (cnt > uint32_t(r.cap)) atomicMax(&bp.stats[0], cnt);
+  }
 }
 
-template <bool kScenes>
-__global__ void __launch_bounds__(kTraverseBlock) k_traverse(DevBodies b, const uint32_t* __restrict__ vals, int n,
-                                                 const float4* __restrict__ pnode, int* cand,
-                                                 uint32_t* cand_count, int cap, uint32_t* stats) {
-  __shared__ int s_stack[kStack * kTraverseBlock];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int q = int(vals[t]);
-  if (b.status[q] != STATUS_DYNAMIC || n < 2) {
-    cand_count[q] = 0;
-    return;
-  }
-  const long base = long(q) * cap;
-  uint32_t cnt = 0;
-  const bool ok = walk_tree<kScenes>(b, pnode, q, s_stack + threadIdx.x, [&](int o, bool dyn) {
-    if (!dyn || o > q) {
-      if (cnt < uint32_t(cap)) cand[base + cnt] = o;
-      ++cnt;
-    }
-  });
-  cand_count[q] = cnt;
-  atomicMax(&stats[0], cnt);
-  if (!ok) atomicOr(&stats[1], 1u);
-}
+// ---- direct pair search ------------------------------------------------------------------------
+// A world of one scene with at most kDirectBodies colliders: a wave takes kDirectGroup bodies and tests
+// them against all colliders, 64 at a time in ascending order, and a ballot per body and 64 tells
+// each hit its place, so that the segments come out sorted. There the time is the few launches and
+// the loads' latency (kDirectAhead of them in flight), which boxes would only add to; above, the
+// tests do, growing with the square: 13 us at 1,001 bodies, where the boxes and their search take 12 us
+// and ordering and sorting as much again, and 98 us at 8,001, where they take 22 us.
+constexpr int kDirectGroup = 4;
+constexpr int kDirectAhead = 4;
 
-// ---- incremental pair update -------------------------------------------------------------------
-// Used when only dynamic bodies' loose AABBs were replaced since the last pair build (dirty[i]).
-// Pairs of two clean bodies cannot have changed, so: (1) every clean body's segment drops its
-// dirty partners (order kept: segments are sorted); (2) the dirty leaves get their new bounds and
-// expand their ancestors by atomic min/max (node bounds stay a superset of the leaves below, which
-// is all a traversal needs; a full build restores tight bounds); (3) each dirty body traverses the
-// tree: a partner that is static or has a larger index goes into its own segment, a clean dynamic
-// partner with a smaller index gets the dirty body appended to its segment (atomic count), a dirty
-// one finds it itself. The segments then hold exactly what a full traversal would write, up to
-// order, and are sorted by the compaction as before.
-
-__global__ void __launch_bounds__(256) k_seg_filter(DevBodies b, const uint32_t* __restrict__ dirty, int* cand,
-                                                   uint32_t* cand_count, int cap) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= b.n) return;
-  if (b.status[q] != STATUS_DYNAMIC) return;
-  if (dirty[q]) {
-    cand_count[q] = 0;
-    return;
-  }
-  const int c = int(cand_count[q]);
-  int* seg = cand + long(q) * cap;
-  int k = 0;
-  for (int i = 0; i < c; ++i) {
-    const int o = seg[i];
-    if (!dirty[o]) seg[k++] = o;
-  }
-  if (k != c) cand_count[q] = uint32_t(k);
-}
-
-// Dirty dynamic bodies (in arbitrary order: the segments are sorted afterwards).
-__global__ void __launch_bounds__(256) k_dirty_list(DevBodies b, const uint32_t* __restrict__ vals, int n,
-                                                   const uint32_t* __restrict__ dirty, int* list,
-                                                   uint32_t* list_count) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int q = int(vals[t]);
-  if (dirty[q] && b.status[q] == STATUS_DYNAMIC) list[atomicAdd(list_count, 1u)] = q;
-}
-
-__global__ void __launch_bounds__(256) k_refit_dirty(DevBodies b, const int* __restrict__ list,
-                                                    const uint32_t* __restrict__ list_count, int n,
-                                                    const int* __restrict__ leaf_of, const int* __restrict__ parent,
-                                                    float4* node_mn, float4* node_mx, uint32_t* inode) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= int(*list_count)) return;
-  const int body = list[t];
-  const int leaf = n - 1 + leaf_of[body];
-  const float4 mn = b.loose_mn[body], mx = b.loose_mx[body];
-  node_mn[leaf] = mn;
-  node_mx[leaf] = mx;
-  const uint32_t e[6] = {f2ord(mn.x), f2ord(mn.y), f2ord(mn.z), f2ord(mx.x), f2ord(mx.y), f2ord(mx.z)};
-  int p = parent[leaf];
-  while (p >= 0) {
-    uint32_t* q = inode + 8 * long(p);
-    bool changed = false;
+__global__ void __launch_bounds__(256) k_direct(DevBodies b, BroadPhaseBufs bp, SearchRun r) {
+  constexpr int G = kDirectGroup;
+  const int lane = threadIdx.x & 63, n = b.n;
+  const uint64_t below = (1ull << lane) - 1ull;
+  const int first = __builtin_amdgcn_readfirstlane(int((blockIdx.x * blockDim.x + threadIdx.x) >> 6)) * G;
+  if (first >= n) return;
+  int q[G];
+  uint32_t cnt[G];
+  bool todo[G];
+  aabb Q[G];
+  uint4 qg[G];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      if (atomicMin(&q[k], e[k]) > e[k]) changed = true;
-      if (atomicMax(&q[4 + k], e[3 + k]) < e[3 + k]) changed = true;
+  for (int g = 0; g < G; ++g) {
+    cnt[g] = 0;
+    q[g] = first + g < n ? first + g : n - 1;
+    const float4 mn = b.loose_mn[q[g]], mx = b.loose_mx[q[g]];
+    todo[g] = first + g < n && mn.w != 0.0f;  // dynamic
+    if (first + g < n && !todo[g] && lane == 0) bp.cand_count[q[g]] = 0;
+    Q[g] = aabb{xyz(mn), xyz(mx)};
+    qg[g] = b.groups ? b.groups[q[g]] : uint4{};
+  }
+  auto hits = [&](int g, int o, bool dyn, const aabb& B) {
+    const bool hit = overlap(Q[g], B) & (o != q[g]) & (!dyn | (o > q[g]));
+    return b.groups ? hit && groups_interact(qg[g], b.groups[o]) : hit;
+  };
+  if (search_incremental(bp, r, n)) {
+    const int nd = int(*bp.list_count);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (!todo[g] || bp.dirty[q[g]] != 0u) continue;
+      bool again = false;
+      const int c = min(int(bp.cand_count[q[g]]), r.cap);
+      for (int k = lane; k < c; k += 64) again = again || bp.dirty[bp.cand[long(q[g]) * r.cap + k]] != 0u;
+      for (int k = lane; k < nd; k += 64) {  // the dirty bodies are all dynamic here
+        const int o = bp.list[k];
+        again = again || hits(g, o, true, aabb{xyz(b.loose_mn[o]), xyz(b.loose_mx[o])});
+      }
+      todo[g] = __any(again);
     }
-    if (!changed) break;
-    p = parent[p];
+  }
+  if (!(todo[0] || todo[1] || todo[2] || todo[3])) return;
+  // colliders [0, fixed_end) hold the last non-dynamic one; the dynamic ones before the first body have
+  // smaller indices
+  for (int c = 0; c < n; c += 64 * kDirectAhead) {
+    if (c >= r.fixed_end && c + 63 < first) c = first & ~63;
+    float4 mn[kDirectAhead], mx[kDirectAhead];
+#pragma unroll
+    for (int u = 0; u < kDirectAhead; ++u) {
+      const int o = c + 64 * u + lane;
+      mn[u] = b.loose_mn[o < n ? o : n - 1];
+      mx[u] = b.loose_mx[o < n ? o : n - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kDirectAhead; ++u) {
+      if (c + 64 * u >= n) break;
+      const int o = c + 64 * u + lane;
+      const bool dyn = mn[u].w != 0.0f;
+      const aabb B{xyz(mn[u]), xyz(mx[u])};
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (!todo[g]) continue;
+        const bool hit = (o < n) & hits(g, o < n ? o : n - 1, dyn, B);
+        const uint64_t m = __ballot(hit);
+        if (!m) continue;
+        const uint32_t k = cnt[g] + uint32_t(__popcll(m & below));
+        if (hit && k < uint32_t(r.cap)) bp.cand[long(q[g]) * r.cap + k] = o;
+        cnt[g] += uint32_t(__popcll(m));
+      }
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (!todo[g]) continue;
+      bp.cand_count[q[g]] = cnt[g];
+      if (cnt[g] > uint32_t(r.cap)) atomicMax(&bp.stats[0], cnt[g]);
+    }
   }
 }
 
-template <bool kScenes>
-__global__ void __launch_bounds__(kTraverseBlock) k_traverse_dirty(DevBodies b, const int* __restrict__ list,
-                                                       const uint32_t* __restrict__ list_count,
-                                                       const float4* __restrict__ pnode,
-                                                       const uint32_t* __restrict__ dirty, int* cand,
-                                                       uint32_t* cand_count, int cap, uint32_t* stats) {
-  __shared__ int s_stack[kStack * kTraverseBlock];
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= int(*list_count)) return;
-  const int q = list[t];
-  const long base = long(q) * cap;
-  uint32_t cnt = 0, most = 0;
-  const bool ok = walk_tree<kScenes>(b, pnode, q, s_stack + threadIdx.x, [&](int o, bool dyn) {
-    if (!dyn || o > q) {
-      if (cnt < uint32_t(cap)) cand[base + cnt] = o;
-      ++cnt;
-    } else if (!dirty[o]) {
-      const uint32_t pos = atomicAdd(&cand_count[o], 1u);
-      if (pos < uint32_t(cap)) cand[long(o) * cap + pos] = q;
-      most = pos + 1 > most ? pos + 1 : most;
-    }
-  });
-  cand_count[q] = cnt;
-  atomicMax(&stats[0], cnt > most ? cnt : most);
-  if (!ok) atomicOr(&stats[1], 1u);
-}
+// ---- compaction ----------------------------------------------------------------------------------
+// The segments, one after another in body order, into the pair list, and every pair into the narrow
+// phase's list of its kind. One launch: a tile of kCompactBodies bodies looks back for the pairs
+// before it (scan.hpp). The pairs of a tile are written by consecutive lanes, each finding its body
+// in the tile's prefix sums in LDS (one lane per body wrote 8-byte pieces and waited for its own
+// reads: 52 us at 100,000 bodies beside the offsets' four launches; now 11 us at
+// 1,001 bodies and 38 us at 99,996). With kSort the
+// segments are in any order, and a pair's place is the number of smaller partners in its segment
+// (the direct search leaves them sorted). It also clears what
+// the next loose-AABB pass and this step's narrow phase start from: the dirty flags and the manifold
+// index. No pair at or above pair_cap is written: the caller sees the count and runs it again.
+constexpr int kCompactBodies = 256;
 
-__global__ void __launch_bounds__(256) k_clamp_counts(const uint32_t* cnt, uint32_t* out, int n, int cap) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t c = cnt[i];
-  out[i] = c < uint32_t(cap) ? c : uint32_t(cap);
-}
-
-__global__ void __launch_bounds__(256) k_sort_compact(int n, int* cand, const uint32_t* __restrict__ cnt,
-                                                     const uint32_t* __restrict__ off, int cap,
-                                                     int2* pairs) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const uint32_t c0 = cnt[q];
-  const int c = int(c0 < uint32_t(cap) ? c0 : uint32_t(cap));
-  if (c == 0) return;
-  int* seg = cand + long(q) * cap;
-  for (int i = 1; i < c; ++i) {
-    const int v = seg[i];
-    int j = i - 1;
-    while (j >= 0 && seg[j] > v) {
-      seg[j + 1] = seg[j];
-      --j;
-    }
-    seg[j + 1] = v;
+template <bool kSort>
+__global__ void __launch_bounds__(kScanThreads) k_compact(DevBodies b, BroadPhaseBufs bp, int cap, ScanRun run,
+                                                          PairOut o) {
+  __shared__ uint32_t s_wave[kScanWaves];
+  __shared__ uint32_t s_tile, s_before, s_box, s_ball;
+  __shared__ uint32_t s_off[kCompactBodies];
+  const uint32_t tile = scan_tile(run, &s_tile);
+  if (tile >= gridDim.x) return;  // only after a launch that failed: its tickets were never taken
+  const int t = threadIdx.x;
+  const int q = int(tile) * kCompactBodies + t;
+  uint32_t c = 0;
+  if (q < b.n) {
+    c = bp.cand_count[q];
+    c = c < uint32_t(cap) ? c : uint32_t(cap);
+    bp.dirty[q] = 0u;
+    if (o.bfirst) o.bfirst[q] = -1;
   }
-  const uint32_t o = off[q];
-  for (int i = 0; i < c; ++i) pairs[o + i] = make_int2(q, seg[i]);
+  uint32_t total;
+  s_off[t] = block_exclusive(c, s_wave, total);
+  if (t < 64) {
+    const uint32_t before = scan_look_back(run, tile, total);
+    if (t == 0) {
+      s_before = before;
+      if (tile == gridDim.x - 1) *o.npairs = before + total;
+    }
+  }
+  __syncthreads();
+  const uint32_t before = s_before;
+  // kGo pairs per lane in one go, so that the places in the two lists take one atomic of each per go
+  constexpr int kGo = 8;
+  for (uint32_t k0 = 0; k0 < total; k0 += kGo * kScanThreads) {
+    uint32_t at[kGo];
+    bool live[kGo], box[kGo];
+    uint32_t boxes = 0, balls = 0;
+#pragma unroll
+    for (int u = 0; u < kGo; ++u) {
+      const uint32_t k = k0 + uint32_t(u * kScanThreads + t);
+      live[u] = box[u] = false;
+      if (k >= total) continue;
+      int lo = 0, hi = kCompactBodies - 1;  // the last body whose offset is <= k: it has pairs
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s_off[mid] <= k) lo = mid;
+        else hi = mid - 1;
+      }
+      const int x = int(tile) * kCompactBodies + lo;
+      const int* seg = bp.cand + long(x) * cap;
+      const int y = seg[k - s_off[lo]];
+      at[u] = before + k;
+      if (kSort) {
+        const uint32_t c = (lo + 1 < kCompactBodies ? s_off[lo + 1] : total) - s_off[lo];
+        at[u] = before + s_off[lo];
+        for (uint32_t j = 0; j < c; ++j) at[u] += seg[j] < y ? 1u : 0u;
+      }
+      if (at[u] >= uint32_t(o.pair_cap)) continue;
+      bp.pairs[at[u]] = make_int2(x, y);
+      live[u] = true;
+      box[u] = b.shape[x] == SHAPE_CUBOID && b.shape[y] == SHAPE_CUBOID;
+      if (box[u]) ++boxes;
+      else ++balls;
+    }
+    uint32_t nbox, nball;
+    uint32_t ab = block_exclusive(boxes, s_wave, nbox);
+    uint32_t aa = block_exclusive(balls, s_wave, nball);
+    if (t == 0 && nbox) s_box = atomicAdd(o.nbox, nbox);
+    if (t == 64 && nball) s_ball = atomicAdd(o.nball, nball);
+    __syncthreads();
+    ab += s_box;
+    aa += s_ball;
+#pragma unroll
+    for (int u = 0; u < kGo; ++u) {
+      if (!live[u]) continue;
+      if (box[u]) o.perm[ab++] = at[u];
+      else o.perm[uint32_t(o.pair_cap) - 1u - aa++] = at[u];
+    }
+    __syncthreads();
+  }
 }
 
 inline unsigned nb(long n) { return unsigned((n + 255) / 256); }
 
 }  // namespace
 
-void launch_loose_update(const DevBodies& b, int mode, uint32_t* changed, uint32_t* dirty, hipStream_t s) {
+void launch_loose_update(const DevBodies& b, int passes, BroadPhaseBufs& bp, hipStream_t s) {
   if (b.n == 0) return;
-  hipLaunchKernelGGL(k_loose_update, dim3(nb(b.n)), dim3(256), 0, s, b, mode, changed, dirty);
+  hipLaunchKernelGGL(k_loose_update, dim3(nb(b.n)), dim3(256), 0, s, b, passes, bp.changed, bp.dirty, bp.list,
+                     bp.list_count);
 }
 
-void launch_build_lbvh(const DevBodies& b, BroadPhaseBufs& bp, hipStream_t s) {
+void launch_order(const DevBodies& b, BroadPhaseBufs& bp, hipStream_t s) {
   const int n = b.n;
-  if (n < 2) return;
-  const uint32_t init[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
-  (void)hipMemcpyAsync(bp.bounds, init, sizeof(init), hipMemcpyHostToDevice, s);
+  if (n == 0) return;
+  fill_u32(bp.bounds, 0xffffffffu, 3, s);
+  fill_u32(bp.bounds + 3, 0u, 3, s);
   hipLaunchKernelGGL(k_bounds, dim3(nb(n)), dim3(256), 0, s, b, bp.bounds);
   hipLaunchKernelGGL(k_morton, dim3(nb(n)), dim3(256), 0, s, b, bp.bounds, bp.scene_bits, bp.keys, bp.vals);
-  radix_sort_pairs(bp.keys, bp.vals, bp.keys_alt, bp.vals_alt, n, 30, bp.tmp, s);
-  const int scene_shift = 3 * ((30 - bp.scene_bits) / 3);
-  hipLaunchKernelGGL(k_lbvh, dim3(nb(n - 1)), dim3(256), 0, s, bp.keys, n, scene_shift, bp.child, bp.parent,
-                     bp.node_scene);
-  hipLaunchKernelGGL(k_init_inodes, dim3(nb(n - 1)), dim3(256), 0, s, n, bp.visit);
-  hipLaunchKernelGGL(k_leaf_nodes, dim3(nb(n)), dim3(256), 0, s, b, bp.vals, n, bp.node_mn, bp.node_mx,
-                     bp.leaf_of);
-  hipLaunchKernelGGL(k_refit_atomic, dim3(nb(n)), dim3(256), 0, s, b, bp.vals, n, bp.parent, bp.visit);
-  hipLaunchKernelGGL(k_decode_nodes, dim3(nb(n - 1)), dim3(256), 0, s, n, bp.visit, bp.node_mn, bp.node_mx);
-  hipLaunchKernelGGL(k_pack_nodes, dim3(nb(n - 1)), dim3(256), 0, s, b, bp.vals, n, bp.child, bp.node_mn,
-                     bp.node_mx, bp.node_scene, bp.pnode);
+  radix_sort_pairs(bp.keys, bp.vals, bp.keys_alt, bp.vals_alt, n, 30, bp.tmp, *bp.scan, s);
 }
 
-void launch_traverse(const DevBodies& b, BroadPhaseBufs& bp, int cap, hipStream_t s) {
+void launch_search(const DevBodies& b, BroadPhaseBufs& bp, const SearchRun& r, hipStream_t s) {
   const int n = b.n;
   if (n == 0) return;
-  fill_u32(bp.stats, 0u, 4, s);
-  if (n < 2) {
-    fill_u32(bp.cand_count, 0u, size_t(n), s);
+  if (r.direct) {
+    // four waves per workgroup
+    hipLaunchKernelGGL(k_direct, dim3(unsigned((n + 4 * kDirectGroup - 1) / (4 * kDirectGroup))), dim3(256), 0, s, b, bp, r);
     return;
   }
-  if (bp.scene_bits)
-    hipLaunchKernelGGL(k_traverse<true>, dim3(unsigned((n + kTraverseBlock - 1) / kTraverseBlock)), dim3(kTraverseBlock), 0, s, b, bp.vals, n, bp.pnode, bp.cand,
-                       bp.cand_count, cap, bp.stats);
-  else
-    hipLaunchKernelGGL(k_traverse<false>, dim3(unsigned((n + kTraverseBlock - 1) / kTraverseBlock)), dim3(kTraverseBlock), 0, s, b, bp.vals, n, bp.pnode, bp.cand,
-                       bp.cand_count, cap, bp.stats);
+  const int nbox = (n + 63) / 64, ntop = (nbox + 63) / 64;
+  hipLaunchKernelGGL(k_boxes, dim3(nb(n)), dim3(256), 0, s, b, bp);
+  if (ntop > 1) hipLaunchKernelGGL(k_top, dim3(unsigned(ntop)), dim3(64), 0, s, bp, nbox);
+  const dim3 grid(unsigned((n + 3) / 4));  // four waves per workgroup
+  if (bp.scene_bits) hipLaunchKernelGGL(k_search<true>, grid, dim3(256), 0, s, b, bp, r);
+  else hipLaunchKernelGGL(k_search<false>, grid, dim3(256), 0, s, b, bp, r);
 }
 
-void launch_incremental_pairs(const DevBodies& b, BroadPhaseBufs& bp, int cap, int max_dirty, hipStream_t s) {
-  const int n = b.n;
-  if (n < 2) return;
-  fill_u32(bp.stats, 0u, 4, s);
-  fill_u32(bp.list_count, 0u, 1, s);
-  hipLaunchKernelGGL(k_seg_filter, dim3(nb(n)), dim3(256), 0, s, b, bp.dirty, bp.cand, bp.cand_count, cap);
-  hipLaunchKernelGGL(k_dirty_list, dim3(nb(n)), dim3(256), 0, s, b, bp.vals, n, bp.dirty, bp.list, bp.list_count);
-  if (max_dirty <= 0) return;
-  hipLaunchKernelGGL(k_refit_dirty, dim3(nb(max_dirty)), dim3(256), 0, s, b, bp.list, bp.list_count, n,
-                     bp.leaf_of, bp.parent, bp.node_mn, bp.node_mx, bp.visit);
-  hipLaunchKernelGGL(k_decode_nodes, dim3(nb(n - 1)), dim3(256), 0, s, n, bp.visit, bp.node_mn, bp.node_mx);
-  hipLaunchKernelGGL(k_pack_nodes, dim3(nb(n - 1)), dim3(256), 0, s, b, bp.vals, n, bp.child, bp.node_mn,
-                     bp.node_mx, bp.node_scene, bp.pnode);
-  if (bp.scene_bits)
-    hipLaunchKernelGGL(k_traverse_dirty<true>, dim3(unsigned((max_dirty + kTraverseBlock - 1) / kTraverseBlock)), dim3(kTraverseBlock), 0, s, b, bp.list, bp.list_count,
-                       bp.pnode, bp.dirty, bp.cand, bp.cand_count, cap, bp.stats);
-  else
-    hipLaunchKernelGGL(k_traverse_dirty<false>, dim3(unsigned((max_dirty + kTraverseBlock - 1) / kTraverseBlock)), dim3(kTraverseBlock), 0, s, b, bp.list, bp.list_count,
-                       bp.pnode, bp.dirty, bp.cand, bp.cand_count, cap, bp.stats);
-}
+size_t compact_tiles(int n) { return (size_t(n) + kCompactBodies - 1) / kCompactBodies; }
 
-void launch_compact_pairs(const DevBodies& b, BroadPhaseBufs& bp, int cap, hipStream_t s) {
-  const int n = b.n;
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_sort_compact, dim3(nb(n)), dim3(256), 0, s, n, bp.cand, bp.cand_count, bp.cand_off,
-                     cap, bp.pairs);
-}
-
-// Exclusive scan of min(count, cap) into cand_off; the clamped counts reuse keys_alt.
-void launch_pair_offsets(const DevBodies& b, BroadPhaseBufs& bp, int cap, hipStream_t s) {
-  const int n = b.n;
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_clamp_counts, dim3(nb(n)), dim3(256), 0, s, bp.cand_count, bp.keys_alt, n, cap);
-  scan_exclusive_u32(bp.keys_alt, bp.cand_off, n, bp.tmp, s);
+void launch_compact_pairs(const DevBodies& b, BroadPhaseBufs& bp, int cap, bool sorted, const PairOut& o, hipStream_t s) {
+  if (b.n == 0) return;
+  const uint32_t tiles = uint32_t(compact_tiles(b.n));
+  const ScanRun run = bp.scan->next(tiles, s);
+  if (sorted) hipLaunchKernelGGL(k_compact<false>, dim3(tiles), dim3(kScanThreads), 0, s, b, bp, cap, run, o);
+  else hipLaunchKernelGGL(k_compact<true>, dim3(tiles), dim3(kScanThreads), 0, s, b, bp, cap, run, o);
 }
 
 }  // namespace nph

@@ -547,7 +547,7 @@ void launch_ccd_predict(const DevBodies& b, const int2* pairs, int npairs, CcdBu
     hipLaunchKernelGGL(k_ccd_first_pass, dim3(blocks_of(npairs, 128)), dim3(128), 0, s, b, pairs, npairs, c,
                        end_time, dt0, target, on_penetration);
     hipLaunchKernelGGL(k_ccd_degree, dim3(blocks_of(npairs, 256)), dim3(256), 0, s, npairs, c);
-    scan_exclusive_u32(c.deg, c.off, b.n, c.tmp, s);
+    scan_exclusive_u32(c.deg, c.off, b.n, *c.scan, s);
     hipLaunchKernelGGL(k_ccd_fill, dim3(blocks_of(npairs, 256)), dim3(256), 0, s, npairs, c);
   }
   if (b.n <= kFzCap)
@@ -578,7 +578,7 @@ void launch_ccd_compact(const int2* pairs, int npairs, const uint32_t* flag, Ccd
     fill_u32(c.ctl + kCcdList, 0u, 1, s);
     return;
   }
-  scan_exclusive_u32(flag, c.cpos, npairs, c.tmp, s);
+  scan_exclusive_u32(flag, c.cpos, npairs, *c.scan, s);
   hipLaunchKernelGGL(k_ccd_scatter, dim3(blocks_of(npairs, 256)), dim3(256), 0, s, pairs, npairs, flag, c);
 }
 

@@ -12,33 +12,39 @@
 
 #include "kernels.hpp"
 #include "np_geometry.hpp"
+#include "scan.hpp"
 #include "stages.hpp"
 
 namespace nph {
 
 namespace {
 
-// Lanes are binned by pair kind: cuboid-cuboid pairs (SAT + clipping, the expensive one) first,
-// run by k_np_boxes with their clip polygons in LDS, all other pairs after, run by k_np_balls.
-// Only the lane -> pair mapping changes; every pair still writes its own slots, so the output is
-// the unbinned one.
-__global__ void __launch_bounds__(256) k_np_flag(DevBodies b, const int2* __restrict__ pairs, int npairs,
-                                                uint32_t* flag) {
+// Lanes are binned by pair kind: cuboid-cuboid pairs (SAT + clipping, the expensive one) are run by
+// k_np_boxes with their clip polygons in LDS, all other pairs by k_np_balls. The compaction of the
+// broad phase fills the two lists as it writes the pairs; k_np_bin does it for lists of pairs from
+// elsewhere. The order within a list is arbitrary: every pair writes its own slots.
+__global__ void __launch_bounds__(256) k_np_bin(DevBodies b, const int2* __restrict__ pairs, NarrowPhaseBufs np,
+                                               DevContacts out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npairs) return;
-  const int2 pr = pairs[i];
-  flag[i] = (b.shape[pr.x] == SHAPE_CUBOID && b.shape[pr.y] == SHAPE_CUBOID) ? 1u : 0u;
-}
-
-__global__ void __launch_bounds__(256) k_np_perm(int npairs, const uint32_t* __restrict__ flag,
-                                                const uint32_t* __restrict__ before, uint32_t* perm,
-                                                uint32_t* nbox) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npairs) return;
-  const uint32_t nbb = before[npairs - 1] + flag[npairs - 1];
-  if (i == 0) *nbox = nbb;
-  const uint32_t b = before[i];
-  perm[flag[i] ? b : nbb + (uint32_t(i) - b)] = uint32_t(i);
+  if (out.bfirst && i < out.bcount) out.bfirst[i] = -1;
+  const bool in = i < int(*np.npairs);
+  bool box = false;
+  if (in) {
+    const int2 pr = pairs[i];
+    box = b.shape[pr.x] == SHAPE_CUBOID && b.shape[pr.y] == SHAPE_CUBOID;
+  }
+  const uint64_t mb = __ballot(in && box), ma = __ballot(in && !box);
+  const int lane = threadIdx.x & 63;
+  uint32_t wb = 0, wa = 0;
+  if (lane == 0) {
+    if (mb) wb = atomicAdd(np.nbox, uint32_t(__popcll(mb)));
+    if (ma) wa = atomicAdd(np.nball, uint32_t(__popcll(ma)));
+  }
+  wb = __shfl(wb, 0);
+  wa = __shfl(wa, 0);
+  const uint64_t below = (1ull << lane) - 1ull;
+  if (in && box) np.perm[wb + uint32_t(__popcll(mb & below))] = uint32_t(i);
+  if (in && !box) np.perm[uint32_t(np.pair_cap) - 1u - (wa + uint32_t(__popcll(ma & below)))] = uint32_t(i);
 }
 
 // Writes contact k of pair i as a 96-byte record into the pair's slots.
@@ -52,18 +58,16 @@ __device__ __forceinline__ void put_contact(const DevContacts& out_c, int i, int
   r[5] = f4(ct.ln, 0.0f);
 }
 
-// Cuboid-cuboid pairs (lanes [0, nbox) of the binned order): SAT + clipping, the clip polygons
+// Cuboid-cuboid pairs: SAT + clipping, the clip polygons
 // and separations of each lane interleaved in LDS.
 constexpr int kBoxBlock = 64;
-__global__ void __launch_bounds__(kBoxBlock) k_np_boxes(DevBodies b, const int2* __restrict__ pairs, int npairs,
-                                                       const uint32_t* __restrict__ perm,
-                                                       const uint32_t* __restrict__ nbox, NarrowPhaseBufs np,
-                                                       DevContacts out_c) {
+__global__ void __launch_bounds__(kBoxBlock) k_np_boxes(DevBodies b, const int2* __restrict__ pairs,
+                                                       NarrowPhaseBufs np, DevContacts out_c) {
   __shared__ ClipVert s_poly[2 * 8 * kBoxBlock];
   __shared__ float s_sep[8 * kBoxBlock];
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= int(*nbox)) return;
-  const int i = int(perm[j]);
+  if (j >= int(*np.nbox)) return;
+  const int i = int(np.perm[j]);
   const int2 pr = pairs[i];
   const int a = pr.x, c = pr.y;
   const float prediction = b.qlim[a] + b.qlim[c];
@@ -73,17 +77,14 @@ __global__ void __launch_bounds__(kBoxBlock) k_np_boxes(DevBodies b, const int2*
                                  xyz(b.dims[c]), prediction, p0, p1, sep,
                                  [&](int k, const Contact& ct) { put_contact(out_c, i, k, ct); });
   np.count[i] = uint32_t(nc);
-  np.has[i] = nc > 0 ? 1u : 0u;
 }
 
-// Pairs with a ball (lanes [nbox, npairs)).
-__global__ void __launch_bounds__(256) k_np_balls(DevBodies b, const int2* __restrict__ pairs, int npairs,
-                                                 const uint32_t* __restrict__ perm,
-                                                 const uint32_t* __restrict__ nbox, NarrowPhaseBufs np,
+// Pairs with a ball.
+__global__ void __launch_bounds__(256) k_np_balls(DevBodies b, const int2* __restrict__ pairs, NarrowPhaseBufs np,
                                                  DevContacts out_c) {
-  const int j = int(*nbox) + blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= npairs) return;
-  const int i = int(perm[j]);
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= int(*np.nball)) return;
+  const int i = int(np.perm[np.pair_cap - 1 - j]);
   const int2 pr = pairs[i];
   const int a = pr.x, c = pr.y;
   const float prediction = b.qlim[a] + b.qlim[c];
@@ -91,33 +92,57 @@ __global__ void __launch_bounds__(256) k_np_balls(DevBodies b, const int2* __res
                                    xyz(b.dims[c]), xyz(b.pos(c)), toq(b.rot(c)), prediction,
                                    [&](int k, const Contact& ct) { put_contact(out_c, i, k, ct); });
   np.count[i] = uint32_t(nc);
-  np.has[i] = nc > 0 ? 1u : 0u;
 }
 
-// The manifold list: one entry per pair with contacts, in pair order; its contacts stay in the
-// pair's slots.
-__global__ void __launch_bounds__(256) k_np_manifolds(const int2* __restrict__ pairs, int npairs,
-                                                     NarrowPhaseBufs np, DevContacts out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npairs) return;
-  const uint32_t nc = np.count[i];
-  if (i == npairs - 1) {
-    np.totals[0] = np.coff[i] + nc;
-    np.totals[1] = np.moff[i] + (nc > 0 ? 1u : 0u);
+// The manifold list: one entry per pair with contacts, in pair order (its contacts stay in the pair's
+// slots), and per body the first manifold it is body 1 of. One launch: each workgroup's tile of
+// pairs looks back for the manifolds before it (scan.hpp). The scans of flags and counts, the list
+// and the index were eight launches of 2.5-4 us: 30 us and more together, now
+// 4.7 us at 3,566 pairs and 13 us at 533,260.
+constexpr int kManifoldItems = 8;
+constexpr int kManifoldTile = kScanThreads * kManifoldItems;
+
+__global__ void __launch_bounds__(kScanThreads) k_np_manifolds(const int2* __restrict__ pairs, NarrowPhaseBufs np,
+                                                              DevContacts out, ScanRun run) {
+  __shared__ uint32_t s_wave[kScanWaves];
+  __shared__ uint32_t s_tile, s_before;
+  const uint32_t tile = scan_tile(run, &s_tile);
+  if (tile >= gridDim.x) return;  // only after a launch that failed: its tickets were never taken
+  const int npairs = int(*np.npairs) < np.pair_cap ? int(*np.npairs) : np.pair_cap;
+  const int base = int(tile) * kManifoldTile + int(threadIdx.x) * kManifoldItems;
+  uint32_t cnt[kManifoldItems];
+  uint32_t both = 0;  // manifolds, and their contacts (at most 4 x 2,048 in a tile) from bit 16 up
+  int2 pr[kManifoldItems];
+#pragma unroll
+  for (int k = 0; k < kManifoldItems; ++k) {
+    cnt[k] = base + k < npairs ? np.count[base + k] : 0u;
+    pr[k] = base + k < npairs ? pairs[base + k] : int2{-1, -1};
+    both += cnt[k] ? 1u + (cnt[k] << 16) : 0u;
   }
-  if (nc == 0) return;
-  const uint32_t m = np.moff[i];
-  out.mbody[m] = pairs[i];
-  out.mfirst[m] = i * kPairSlots;
-  out.mcount[m] = int(nc);
-}
-
-// Per-body index of the manifold list (sorted by body pair): the first manifold of each body 1.
-__global__ void __launch_bounds__(256) k_np_index(int npairs, const uint32_t* __restrict__ totals, DevContacts out) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= npairs || m >= int(totals[1])) return;
-  const int b = out.mbody[m].x;
-  if (m == 0 || out.mbody[m - 1].x != b) out.bfirst[b] = m;
+  uint32_t total;
+  uint32_t m = block_exclusive(both, s_wave, total) & 0xffffu;
+  if (threadIdx.x < 64) {
+    const uint32_t before = scan_look_back(run, tile, total & 0xffffu);
+    if (threadIdx.x == 0) {
+      s_before = before;
+      if (total) atomicAdd(&np.totals[0], total >> 16);
+      if (tile == gridDim.x - 1) np.totals[1] = before + (total & 0xffffu);
+    }
+  }
+  __syncthreads();
+  m += s_before;
+  int body = -1;  // body 1 of this lane's previous manifold
+#pragma unroll
+  for (int k = 0; k < kManifoldItems; ++k) {
+    if (cnt[k] == 0u) continue;
+    out.mbody[m] = pr[k];
+    out.mfirst[m] = (base + k) * kPairSlots;
+    out.mcount[m] = int(cnt[k]);
+    // the body's first manifold: the smallest of what the lanes that hold some of its pairs offer
+    if (out.bfirst && pr[k].x != body) atomicMin(reinterpret_cast<uint32_t*>(out.bfirst) + pr[k].x, m);
+    body = pr[k].x;
+    ++m;
+  }
 }
 
 __global__ void __launch_bounds__(256) k_gather_contacts(DevContacts c, int M, const uint32_t* __restrict__ moff,
@@ -136,26 +161,21 @@ __global__ void __launch_bounds__(256) k_gather_contacts(DevContacts c, int M, c
 
 }  // namespace
 
-void launch_narrow_phase(const DevBodies& b, const int2* pairs, int npairs, NarrowPhaseBufs& np,
-                         DevContacts out, hipStream_t s) {
-  if (out.bfirst) fill_u32(reinterpret_cast<uint32_t*>(out.bfirst), 0xffffffffu, size_t(out.bcount), s);
-  if (npairs <= 0) {
-    fill_u32(np.totals, 0u, 2, s);
-    return;
-  }
-  const unsigned g = unsigned((npairs + 255) / 256);
-  // binning by kind: flags in np.has, their exclusive scan in np.moff (both rewritten below)
-  hipLaunchKernelGGL(k_np_flag, dim3(g), dim3(256), 0, s, b, pairs, npairs, np.has);
-  scan_exclusive_u32(np.has, np.moff, npairs, np.tmp, s);
-  uint32_t* nbox = np.totals + 2;
-  hipLaunchKernelGGL(k_np_perm, dim3(g), dim3(256), 0, s, npairs, np.has, np.moff, np.perm, nbox);
-  hipLaunchKernelGGL(k_np_boxes, dim3(unsigned((npairs + kBoxBlock - 1) / kBoxBlock)), dim3(kBoxBlock), 0, s, b,
-                     pairs, npairs, np.perm, nbox, np, out);
-  hipLaunchKernelGGL(k_np_balls, dim3(g), dim3(256), 0, s, b, pairs, npairs, np.perm, nbox, np, out);
-  scan_exclusive_u32(np.count, np.coff, npairs, np.tmp, s);
-  scan_exclusive_u32(np.has, np.moff, npairs, np.tmp, s);
-  hipLaunchKernelGGL(k_np_manifolds, dim3(g), dim3(256), 0, s, pairs, npairs, np, out);
-  if (out.bfirst) hipLaunchKernelGGL(k_np_index, dim3(g), dim3(256), 0, s, npairs, np.totals, out);
+size_t manifold_tiles(int npairs) { return (size_t(npairs) + kManifoldTile - 1) / kManifoldTile; }
+
+void launch_narrow_bins(const DevBodies& b, const int2* pairs, NarrowPhaseBufs& np, DevContacts out, hipStream_t s) {
+  const int lanes = out.bfirst && out.bcount > np.pair_cap ? out.bcount : np.pair_cap;
+  hipLaunchKernelGGL(k_np_bin, dim3(unsigned((lanes + 255) / 256)), dim3(256), 0, s, b, pairs, np, out);
+}
+
+// Grids for pair_cap pairs of either kind: what the lists hold is known on the device.
+void launch_narrow_phase(const DevBodies& b, const int2* pairs, NarrowPhaseBufs& np, DevContacts out, hipStream_t s) {
+  const unsigned P = unsigned(np.pair_cap);
+  if (np.boxes)
+    hipLaunchKernelGGL(k_np_boxes, dim3((P + kBoxBlock - 1) / kBoxBlock), dim3(kBoxBlock), 0, s, b, pairs, np, out);
+  if (np.balls) hipLaunchKernelGGL(k_np_balls, dim3((P + 255) / 256), dim3(256), 0, s, b, pairs, np, out);
+  const uint32_t tiles = uint32_t(manifold_tiles(np.pair_cap));
+  hipLaunchKernelGGL(k_np_manifolds, dim3(tiles), dim3(kScanThreads), 0, s, pairs, np, out, np.scan->next(tiles, s));
 }
 
 void launch_gather_contacts(const DevContacts& c, int M, const uint32_t* moff, float4* dense,

@@ -1078,7 +1078,7 @@ void launch_colour_prepare(const DevBodies& b, const DevContacts& c, int M, cons
   if (M == 0) return;
   hipLaunchKernelGGL(k_inherit, dim3(nb(M)), dim3(256), 0, s, c, M, prev, prevM, prev_state, sb.state);
   hipLaunchKernelGGL(k_degree, dim3(nb(M)), dim3(256), 0, s, b, c, M, sb.deg);
-  scan_exclusive_u32(sb.deg, sb.adj_off, b.n, sb.tmp, s);
+  scan_exclusive_u32(sb.deg, sb.adj_off, b.n, *sb.scan, s);
   hipLaunchKernelGGL(k_adjacency, dim3(nb(M)), dim3(256), 0, s, b, c, M, sb.adj_off, sb.adj_fill, sb.adj);
 }
 
@@ -1100,11 +1100,11 @@ void launch_colour_order(const DevBodies& b_view_for_slots, const DevContacts& c
                          SolverBufs& sb, hipStream_t s) {
   if (M == 0) return;
   const int bits = ncolours <= 256 ? 8 : 16;
-  radix_sort_pairs(sb.ckeys, sb.order, sb.ckeys_alt, sb.order_alt, M, bits, sb.tmp, s);
+  radix_sort_pairs(sb.ckeys, sb.order, sb.ckeys_alt, sb.order_alt, M, bits, sb.tmp, *sb.scan, s);
   fill_u32(sb.col_start, 0xffffffffu, size_t(ncolours) + 1, s);
   hipLaunchKernelGGL(k_colour_starts, dim3(nb(M)), dim3(256), 0, s, c, M, sb.ckeys, sb.order, sb.col_start,
                      sb.mcount_ord);
-  scan_exclusive_u32(sb.mcount_ord, sb.soff, M, sb.tmp, s);
+  scan_exclusive_u32(sb.mcount_ord, sb.soff, M, *sb.scan, s);
   hipLaunchKernelGGL(k_slot_info, dim3(nb(M)), dim3(256), 0, s, b_view_for_slots, c, M, sb.order, sb.soff, sb.sinfo,
                      sb.slot_of);
 }
@@ -1199,7 +1199,7 @@ void launch_scene_order(const DevBodies& b, int M, int nscenes, int ncolours, So
                         hipStream_t s) {
   if (M == 0) return;
   hipLaunchKernelGGL(k_scene_keys, dim3(nb(M)), dim3(256), 0, s, b, M, sb, sc.keys, sc.slot);
-  radix_sort_pairs(sc.keys, sc.slot, sc.keys_alt, sc.slot_alt, M, 28, sb.tmp, s);
+  radix_sort_pairs(sc.keys, sc.slot, sc.keys_alt, sc.slot_alt, M, 28, sb.tmp, *sb.scan, s);
   const long total = long(nscenes) * (ncolours + 1);
   hipLaunchKernelGGL(k_scene_starts, dim3(nb(total)), dim3(256), 0, s, sc.keys, M, nscenes, ncolours, sc.start);
 }

@@ -1,63 +1,57 @@
 // nphysics_amd/csrc/k_util.hip -- device-wide exclusive scan and stable LDS radix sort.
 //
-// Scan: 256-thread blocks each own a tile of 2048 words (8 per thread); block totals are scanned
-// recursively and added back. Radix sort: 8-bit digits; per pass a histogram kernel (LDS
+// Scan: one launch, 256-thread blocks each own a tile of 2048 words (8 per thread) and look back for
+// the sum before it (scan.hpp). A launch per level (tiles, tile sums, add back) took 9-11 us above one
+// tile, three dependent launches of 2.5-4 us each; now
+// 3.4-5.8 us. Radix sort: 8-bit digits; per pass a histogram kernel (LDS
 // atomics, one 256-bin row per tile, digit-major so that one exclusive scan yields every tile's
 // output base) and a scatter kernel that ranks keys stably inside a tile with 64-lane wavefront
 // ballots (eight ballots give each lane the set of lanes holding the same digit).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels.hpp"
+#include "scan.hpp"
 
 namespace nph {
 
 namespace {
 
-constexpr int kScanThreads = 256;
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kScanThreads * kScanItems;
+constexpr int kScanItems = kScanTile / kScanThreads;
 
 constexpr int kRadixThreads = 256;
 constexpr int kRadixItems = 8;
 constexpr int kRadixTile = kRadixThreads * kRadixItems;
 constexpr int kRadixBins = 256;
 
-__global__ void __launch_bounds__(kScanThreads) k_scan_tiles(const uint32_t* __restrict__ in,
-                                                            uint32_t* __restrict__ out, int n,
-                                                            uint32_t* __restrict__ tile_sums) {
-  __shared__ uint32_t s_part[kScanThreads];
-  const int tid = threadIdx.x;
-  const long base = long(blockIdx.x) * kScanTile + long(tid) * kScanItems;
+__global__ void __launch_bounds__(kScanThreads) k_scan(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                      int n, ScanRun run) {
+  __shared__ uint32_t s_wave[kScanWaves];
+  __shared__ uint32_t s_tile, s_before;
+  const uint32_t tile = scan_tile(run, &s_tile);
+  if (tile >= gridDim.x) return;  // only after a launch that failed: its tickets were never taken
+  const long base = long(tile) * kScanTile + long(threadIdx.x) * kScanItems;
   uint32_t v[kScanItems];
   uint32_t acc = 0;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
-    const long i = base + k;
-    v[k] = i < n ? in[i] : 0u;
+    v[k] = base + k < n ? in[base + k] : 0u;
     acc += v[k];
   }
-  s_part[tid] = acc;
-  __syncthreads();
-  // Hillis-Steele inclusive scan of the per-thread sums.
-  for (int off = 1; off < kScanThreads; off <<= 1) {
-    const uint32_t x = tid >= off ? s_part[tid - off] : 0u;
-    __syncthreads();
-    s_part[tid] += x;
-    __syncthreads();
+  uint32_t total;
+  uint32_t at = block_exclusive(acc, s_wave, total);
+  if (threadIdx.x < 64) {
+    const uint32_t before = scan_look_back(run, tile, total);
+    if (threadIdx.x == 0) s_before = before;
   }
-  uint32_t run = tid > 0 ? s_part[tid - 1] : 0u;
+  __syncthreads();
+  at += s_before;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
-    const long i = base + k;
-    if (i < n) out[i] = run;
-    run += v[k];
+    if (base + k < n) out[base + k] = at;
+    at += v[k];
   }
-  if (tid == kScanThreads - 1 && tile_sums) tile_sums[blockIdx.x] = s_part[tid];
-}
-
-__global__ void k_scan_add(uint32_t* __restrict__ out, int n, const uint32_t* __restrict__ tile_offs) {
-  const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) out[i] += tile_offs[i / kScanTile];
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n) {
@@ -131,45 +125,60 @@ int div_up(long a, long b) { return int((a + b - 1) / b); }
 
 }  // namespace
 
-size_t scan_temp_words(int n) {
-  size_t words = 0;
-  long m = n;
-  while (m > kScanTile) {
-    const long t = (m + kScanTile - 1) / kScanTile;
-    words += 2 * size_t(t);
-    m = t;
-  }
-  return words + 16;
+ScanState::~ScanState() {
+  if (mem) (void)hipFree(mem);
 }
 
-void scan_exclusive_u32(const uint32_t* in, uint32_t* out, int n, uint32_t* tmp, hipStream_t s) {
-  if (n <= 0) return;
-  const int tiles = div_up(n, kScanTile);
-  if (tiles == 1) {
-    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanThreads), 0, s, in, out, n, nullptr);
-    return;
+hipError_t ScanState::ensure(size_t need, hipStream_t s) {
+  if (need <= tiles) return hipSuccess;
+  const size_t grown = std::max(need + need / 2, size_t(1024));
+  hipError_t e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return e;
+  void* q = nullptr;
+  if ((e = hipMalloc(&q, 64 + grown * sizeof(unsigned long long))) != hipSuccess) return e;
+  if (mem) (void)hipFree(mem);
+  mem = q;
+  tiles = grown;
+  base = epoch = 0;
+  fill_u32(static_cast<uint32_t*>(mem), 0u, 16 + 2 * tiles, s);
+  return hipSuccess;
+}
+
+ScanRun ScanState::next(uint32_t ntiles, hipStream_t s) {
+  if (++epoch >= (1u << 30)) {  // the epochs start over on cleared words
+    fill_u32(static_cast<uint32_t*>(mem) + 16, 0u, 2 * tiles, s);
+    epoch = 1;
   }
-  uint32_t* sums = tmp;
-  uint32_t* offs = tmp + tiles;
-  hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(kScanThreads), 0, s, in, out, n, sums);
-  scan_exclusive_u32(sums, offs, tiles, tmp + 2 * size_t(tiles), s);
-  hipLaunchKernelGGL(k_scan_add, dim3(div_up(n, 256)), dim3(256), 0, s, out, n, offs);
+  ScanRun r;
+  r.ticket = static_cast<uint32_t*>(mem);
+  r.word = reinterpret_cast<unsigned long long*>(static_cast<char*>(mem) + 64);
+  r.base = base;
+  r.epoch = epoch;
+  base += ntiles;
+  return r;
+}
+
+void scan_exclusive_u32(const uint32_t* in, uint32_t* out, int n, ScanState& st, hipStream_t s) {
+  if (n <= 0) return;
+  const uint32_t tiles = uint32_t(scan_tiles(size_t(n)));
+  hipLaunchKernelGGL(k_scan, dim3(tiles), dim3(kScanThreads), 0, s, in, out, n, st.next(tiles, s));
 }
 
 size_t radix_temp_words(int n) {
   const int ntiles = div_up(n > 0 ? n : 1, kRadixTile);
   const size_t h = size_t(kRadixBins) * ntiles;
-  return 2 * h + scan_temp_words(int(h)) + 16;
+  return 2 * h;
 }
 
+size_t radix_scan_tiles(int n) { return scan_tiles(size_t(kRadixBins) * div_up(n > 0 ? n : 1, kRadixTile)); }
+
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
-                      int n, int bits, uint32_t* tmp, hipStream_t s) {
+                      int n, int bits, uint32_t* tmp, ScanState& st, hipStream_t s) {
   if (n <= 1) return;
   const int ntiles = div_up(n, kRadixTile);
   const size_t h = size_t(kRadixBins) * ntiles;
   uint32_t* hist = tmp;
   uint32_t* offs = tmp + h;
-  uint32_t* stmp = tmp + 2 * h;
   uint32_t* kin = keys;
   uint32_t* vin = vals;
   uint32_t* kout = keys_alt;
@@ -177,7 +186,7 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32
   int passes = 0;
   for (int shift = 0; shift < bits; shift += 8, ++passes) {
     hipLaunchKernelGGL(k_radix_hist, dim3(ntiles), dim3(kRadixThreads), 0, s, kin, n, shift, ntiles, hist);
-    scan_exclusive_u32(hist, offs, int(h), stmp, s);
+    scan_exclusive_u32(hist, offs, int(h), st, s);
     hipLaunchKernelGGL(k_radix_scatter, dim3(ntiles), dim3(kRadixThreads), 0, s, kin, vin, kout, vout, n,
                        shift, ntiles, offs);
     uint32_t* t = kin; kin = kout; kout = t;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include "devworld.hpp"
+#include "kernels.hpp"
 
 namespace nph {
 
@@ -32,7 +33,7 @@ struct ActivationBufs {
   uint32_t* touch;   // [n] body that could sleep touches one that keeps its island awake
   uint32_t* mflag;   // [M] manifold handed to the solver
   uint32_t* pos;     // [M] its index in the solved list
-  uint32_t* tmp;     // scan temporary
+  ScanState* scan;
   uint32_t* totals;  // [3] solved manifolds, their contacts, awake dynamic bodies (zeroed by the caller)
 };
 void launch_wake(const DevBodies& b, hipStream_t s);
@@ -45,56 +46,85 @@ void launch_solve_list(const DevContacts& c, int M, const ActivationBufs& a, con
 
 // k_broadphase.hip ------------------------------------------------------------------------
 struct BroadPhaseBufs {
-  uint32_t* changed;      // [2] number of loose AABBs replaced: all, of non-dynamic bodies
+  uint32_t* changed;      // [4] number of loose AABBs replaced (all, of non-dynamic bodies) by the
+                          // swept pass and by the other
   uint32_t* bounds;       // [6] ordered-int encoded centroid bounds
   uint32_t* keys;         // [n] Morton codes
-  uint32_t* vals;         // [n] body indices
+  uint32_t* vals;         // [n] the order: body indices
   uint32_t* keys_alt;
   uint32_t* vals_alt;
-  int* child;             // [2(n-1)] children of internal nodes (>= n-1: leaf)
-  int* parent;            // [2n-1]
-  uint32_t* visit;        // [8(n-1)] internal-node bounds, order-preserving integer encoding
-  float4* node_mn;        // [2n-1]
-  float4* node_mx;
-  int2* node_scene;       // [n-1] scene range (first, last) of every internal node's leaves
-  float4* pnode;          // [4(n-1)] packed internal nodes for the traversals (k_broadphase.hip)
+  float4* leaf_mn;        // [n] loose AABBs in the order, with index and dynamic flag
+  float4* leaf_mx;        //     and scene
+  float4* box_mn;         // [search_boxes(n)] boxes of 64 of them, then boxes of 64 boxes, with first
+  float4* box_mx;         //     and last scene
+  int* box_top;           // and the largest index of a partner in them
   int scene_bits;         // Morton keys carry the scene in their top scene_bits bits
   int* cand;              // [n * cap] candidate partners per body
   uint32_t* cand_count;   // [n] partner count (may exceed cap)
-  uint32_t* cand_off;     // [n] exclusive scan of min(count, cap)
-  uint32_t* stats;        // [4] 0: max count, 1: traversal stack overflow
+  uint32_t* stats;        // [1] largest partner count above the capacity (else 0)
   int2* pairs;            // [pair capacity]
-  uint32_t* tmp;          // scan / radix scratch
+  uint32_t* tmp;          // radix scratch
+  ScanState* scan;
   uint32_t* dirty;        // [n] 1 where the loose AABB was replaced since the last pair build
-  int* leaf_of;           // [n] leaf of each body in the current tree
-  int* list;              // [n] dirty dynamic bodies (incremental update)
+  int* list;              // [n] dirty bodies
   uint32_t* list_count;   // [1]
 };
 
-// mode 0: current pose of every body (static ones included); mode 1: dynamic bodies, current
-// pose; mode 2: dynamic bodies, AABB swept from pos0/rot0 to pos/rot.
-void launch_loose_update(const DevBodies& b, int mode, uint32_t* changed, uint32_t* dirty, hipStream_t s);
-void launch_build_lbvh(const DevBodies& b, BroadPhaseBufs& bp, hipStream_t s);
-void launch_traverse(const DevBodies& b, BroadPhaseBufs& bp, int cap, hipStream_t s);
-void launch_pair_offsets(const DevBodies& b, BroadPhaseBufs& bp, int cap, hipStream_t s);
-void launch_compact_pairs(const DevBodies& b, BroadPhaseBufs& bp, int cap, hipStream_t s);
-// Pair segments updated for the dirty bodies only (the tree of the last full build refitted by
-// expansion); max_dirty bounds the number of dirty bodies. stats[0] > cap or stats[1] means the
-// caller must fall back to a full build.
-void launch_incremental_pairs(const DevBodies& b, BroadPhaseBufs& bp, int cap, int max_dirty, hipStream_t s);
+// Loose-AABB passes, as bits: the current pose of the dynamic bodies (1), first the AABB swept from
+// pos0/rot0 to pos/rot (2), the static bodies' current pose too (4).
+enum : int { LOOSE_FINAL = 1, LOOSE_SWEPT = 2, LOOSE_STATIC = 4 };
+void launch_loose_update(const DevBodies& b, int passes, BroadPhaseBufs& bp, hipStream_t s);
+// Boxes of n colliders and boxes of those.
+inline size_t search_boxes(size_t n) { return (n + 63) / 64 + (n + 4095) / 4096; }
+// The order of the colliders (by scene and Morton code), sorted anew.
+void launch_order(const DevBodies& b, BroadPhaseBufs& bp, hipStream_t s);
+// A pair search: directly, with the end of the last non-dynamic collider, or by boxes over the order;
+// the segment capacity, and whether segments may be kept (loose AABBs replaced before this step's
+// passes since the last search: dirty_before).
+// Segments are kept while at most this many of n bodies are dirty: every clean body tests them all,
+// which at 1,024 costs as much as a search of its own.
+__host__ __device__ inline int kept_limit(int n) { return n / 8 < 1024 ? n / 8 : 1024; }
+constexpr int kDirectBodies = 2048;  // colliders of the largest world searched directly
+struct SearchRun {
+  int direct;
+  int fixed_end;
+  int cap;
+  int may_increment;
+  long dirty_before;
+};
+void launch_search(const DevBodies& b, BroadPhaseBufs& bp, const SearchRun& r, hipStream_t s);
+// Where the compaction leaves the pairs: their number, the narrow phase's lists (cuboid-cuboid pairs
+// from perm[0] up, the others from perm[pair_cap - 1] down) and their lengths (zeroed by the caller),
+// and the manifold index to clear (may be null).
+struct PairOut {
+  uint32_t* npairs;
+  uint32_t* nbox;
+  uint32_t* nball;
+  uint32_t* perm;
+  int* bfirst;
+  int pair_cap;
+};
+size_t compact_tiles(int n);  // tiles of the scan state that the compaction of n bodies takes
+// sorted: the segments are in ascending order already
+void launch_compact_pairs(const DevBodies& b, BroadPhaseBufs& bp, int cap, bool sorted, const PairOut& o, hipStream_t s);
 
 // k_narrowphase.hip -------------------------------------------------------------------------
 struct NarrowPhaseBufs {
   uint32_t* count;        // [P] contacts per pair
-  uint32_t* coff;         // [P] exclusive scan of count
-  uint32_t* has;          // [P] count > 0
-  uint32_t* moff;         // [P] exclusive scan of has
-  uint32_t* perm;         // [P] pairs binned by kind (lane -> pair)
-  uint32_t* totals;       // [3] contacts, manifolds, cuboid-cuboid pairs
-  uint32_t* tmp;
+  uint32_t* perm;         // [pair_cap] pairs by kind: cuboid-cuboid from the front, the others from the back
+  uint32_t* npairs;       // on the device: pairs, cuboid-cuboid pairs, the others
+  uint32_t* nbox;
+  uint32_t* nball;
+  uint32_t* totals;       // [2] contacts (zeroed by the caller), manifolds
+  int pair_cap;           // pairs above it are left out (and the caller's to see)
+  bool boxes, balls;      // pairs of the kind can occur
+  ScanState* scan;
 };
-void launch_narrow_phase(const DevBodies& b, const int2* pairs, int npairs, NarrowPhaseBufs& np,
-                         DevContacts out, hipStream_t s);
+// Sorts the first *np.npairs pairs by kind (lists of pairs that did not come from the compaction) and
+// clears `out`'s manifold index; nbox and nball are zeroed by the caller.
+void launch_narrow_bins(const DevBodies& b, const int2* pairs, NarrowPhaseBufs& np, DevContacts out, hipStream_t s);
+size_t manifold_tiles(int npairs);  // tiles of the scan state that the narrow phase takes
+void launch_narrow_phase(const DevBodies& b, const int2* pairs, NarrowPhaseBufs& np, DevContacts out, hipStream_t s);
 // Contacts of all manifolds in manifold order, gathered from their slots into dense records
 // (kContactFields float4 each) and impulses (dense_imp may be null); moff = exclusive scan of the
 // manifolds' counts.
@@ -127,7 +157,8 @@ struct SolverBufs {
   int* visit;             // [max colours] colour classes in visiting order
   int2* vrange;           // [max colours] (first slot, slots) of the class visited k-th
   double* red;            // residual partials
-  uint32_t* tmp;
+  uint32_t* tmp;          // radix scratch
+  ScanState* scan;
 };
 constexpr int kMaxColours = 4096;
 constexpr int kRecFields = 4;  // float4 per contact row record
@@ -266,7 +297,7 @@ struct CcdBufs {
   uint32_t* cpos;          // [P] exclusive scan of a flag array
   int2* list;              // [P] compacted pairs, pair order
   int* list_pair;          // [P] their pair indices
-  uint32_t* tmp;           // scan scratch
+  ScanState* scan;
   uint32_t* deg;           // [n] CCD slots of each dynamic body
   uint32_t* off;           // [n] exclusive scan of deg
   uint32_t* fill;          // [n]

@@ -133,20 +133,22 @@ struct World {
   // due at the next step after the caller set the bodies' state.
   bool sleeping = false, wake_pending = false;
   int64_t n_dynamic = 0, active_bodies = 0;
-  DBuf act_parent, act_can, act_touch, act_pos, act_tmp, act_mflag[2], sl_mbody[2], sl_mfirst[2], sl_mcount[2];
+  DBuf act_parent, act_can, act_touch, act_pos, act_mflag[2], sl_mbody[2], sl_mfirst[2], sl_mcount[2];
+
+  ScanState scan;  // prefix sums on `stream`
 
   // broad phase
-  DBuf bp_dirty, bp_leaf_of, bp_list, bp_pnode;
-  // Incremental pair updates: the tree and segments of the last pair build are valid, how many
-  // incremental updates followed the last full build, and the loose-AABB replacements (all, of
-  // non-dynamic bodies) since the last pair build.
-  bool tree_valid = false;
+  DBuf bp_dirty, bp_list;
+  // The segments of the last search stand; searches by the present order (sorted anew every
+  // kOrderAge-th, and when the bodies were added or moved by the caller); the loose-AABB replacements (all,
+  // of non-dynamic bodies) since the last search.
+  bool segments_valid = false;
   bool incremental_bp = true;
-  int inc_since_full = 0;
+  static constexpr int kOrderAge = 16;
+  int order_age = kOrderAge;
   int64_t dirty_pending = 0, dirty_static_pending = 0;
-  static constexpr int kMaxIncremental = 32;
-  DBuf bp_small, keys, vals, keys_alt, vals_alt, child, parent, visit, node_mn, node_mx, node_scene, cand,
-      cand_count, cand_off, pairs, bp_tmp;
+  DBuf bp_small, keys, vals, keys_alt, vals_alt, leaf_mn, leaf_mx, box_mn, box_mx, box_top, cand, cand_count, pairs,
+      bp_tmp;
   int cap = 32;
   int npairs = 0;
   bool pairs_dirty = true;
@@ -154,7 +156,7 @@ struct World {
   bool recollide = false;  // collision groups changed: the next step starts with collision detection
 
   // narrow phase
-  DBuf np_count, np_coff, np_has, np_moff, np_perm, np_tmp;
+  DBuf np_count, np_perm;
   DBuf rd_moff, rd_rec, rd_imp;  // contact readback staging
   ContactBufs cb[2];
   int cur = 0;      // index of the manifolds produced by the last collision detection
@@ -194,6 +196,10 @@ struct World {
   // scene-major slot order, and the variant chosen by the autotuner (0 per-colour launches,
   // 256/512/1024 the blocked kernels' workgroup size for the scenes of more than 256 dynamic bodies)
   int nscenes = 1, max_scene_dyn = 0;
+  // end of the last non-dynamic body, and which kinds of pairs can occur (a cuboid-cuboid pair has a
+  // dynamic cuboid)
+  int fixed_end = 0;
+  bool any_cuboid = false, any_ball = false;
   DBuf sc_dyn_start, sc_dyn_list, sc_local, sc_keys, sc_slot, sc_keys_alt, sc_slot_alt, sc_start, sc_small, sc_large;
   int n_small_scenes = 0, n_large_scenes = 0;
   int variant_request = -1;  // -1: autotune; else forced
@@ -229,7 +235,7 @@ struct World {
   std::vector<int> h_ccd, h_ccd_key;
   std::map<std::pair<int, int>, int> static_owner;  // (scene, static body index) -> first collider
   DBuf ccd_flags, ccd_keys, ccd_rot, ccd_time, ccd_frozen, ccd_slot, ccd_heap, ccd_stage, ccd_imp, ccd_ctl,
-      ccd_in, ccd_new, ccd_prep, ccd_prepared, ccd_eval, ccd_kept, ccd_cand, ccd_cpos, ccd_list, ccd_lpair, ccd_tmp,
+      ccd_in, ccd_new, ccd_prep, ccd_prepared, ccd_eval, ccd_kept, ccd_cand, ccd_cpos, ccd_list, ccd_lpair,
       ccd_deg, ccd_off, ccd_fill, ccd_adj, ccd_pos, ccd_sbodies;
   ContactBufs ccd_cb;
   int ccd_cap = 0, ccd_nimp = 0;
@@ -656,7 +662,7 @@ struct World {
       // proxy creation: loose = aabb(pos) loosened by the query limit, then by 0.01
       const aabb a = shape_aabb(sh, xyz(he), xyz(hpos), toq(hrot));
       const aabb lo = loosened(loosened(a, h_qlim.back()), 0.01f);
-      hmn[k] = f4(lo.mn, 0.0f);
+      hmn[k] = f4(lo.mn, dyn ? 1.0f : 0.0f);
       hmx[k] = f4(lo.mx, 0.0f);
     }
     const size_t f4b = sizeof(float4);
@@ -752,6 +758,14 @@ struct World {
       HIPCK(sc_large.ensure(std::max<size_t>(large.size(), 1) * 4));
       if (!small.empty()) HIPCK(up(sc_small, small.data(), small.size() * 4, 0));
       if (!large.empty()) HIPCK(up(sc_large, large.data(), large.size() * 4, 0));
+    }
+    fixed_end = 0;
+    for (int i = 0; i < n1; ++i)
+      if (h_status[size_t(i)] != NPHYS_STATUS_DYNAMIC) fixed_end = i + 1;
+    any_cuboid = any_ball = false;
+    for (int i = 0; i < n1; ++i) {
+      any_cuboid = any_cuboid || (h_shape[size_t(i)] == NPHYS_SHAPE_CUBOID && h_status[size_t(i)] == NPHYS_STATUS_DYNAMIC);
+      any_ball = any_ball || h_shape[size_t(i)] == NPHYS_SHAPE_BALL;
     }
     tune_cands.clear();
     tuned = false;
@@ -850,27 +864,29 @@ struct World {
   // ------------------------------------------------------------------ broad phase
   int ensure_bp() {
     const size_t nn = size_t(std::max(n, 2));
-    for (DBuf* b : {&keys, &vals, &keys_alt, &vals_alt, &cand_count, &cand_off})
-      HIPCK(b->ensure(nn * 4));
-    HIPCK(visit.ensure(8 * nn * 4));
-    HIPCK(child.ensure(2 * nn * 4));
-    HIPCK(parent.ensure(2 * nn * 4));
-    HIPCK(node_mn.ensure(2 * nn * sizeof(float4)));
-    HIPCK(node_mx.ensure(2 * nn * sizeof(float4)));
-    HIPCK(node_scene.ensure(nn * sizeof(int2)));
-    HIPCK(bp_pnode.ensure(4 * nn * sizeof(float4)));
-    if (cand.bytes < nn * size_t(cap) * 4) tree_valid = false;  // segments are lost on growth
+    if (!direct_pairs()) {
+      for (DBuf* b : {&keys, &vals, &keys_alt, &vals_alt}) HIPCK(b->ensure(nn * 4));
+      for (DBuf* b : {&leaf_mn, &leaf_mx}) HIPCK(b->ensure(nn * sizeof(float4)));
+      for (DBuf* b : {&box_mn, &box_mx}) HIPCK(b->ensure(search_boxes(nn) * sizeof(float4)));
+      HIPCK(box_top.ensure(search_boxes(nn) * 4));
+      HIPCK(bp_tmp.ensure(radix_temp_words(int(nn)) * 4));
+      HIPCK(scan.ensure(radix_scan_tiles(int(nn)), stream));
+    }
+    HIPCK(cand_count.ensure(nn * 4));
+    if (cand.bytes < nn * size_t(cap) * 4) segments_valid = false;  // segments are lost on growth
     HIPCK(cand.ensure(nn * size_t(cap) * 4));
-    for (DBuf* b : {&bp_leaf_of, &bp_list}) HIPCK(b->ensure(nn * 4));
+    HIPCK(bp_list.ensure(nn * 4));
     if (bp_dirty.bytes < nn * 4) {
-      tree_valid = false;
+      segments_valid = false;
       HIPCK(bp_dirty.ensure(nn * 4));
       fill_u32(bp_dirty.as<uint32_t>(), 0u, nn, stream);
     }
-    const size_t tw = std::max(radix_temp_words(int(nn)), scan_temp_words(int(nn)));
-    HIPCK(bp_tmp.ensure(tw * 4));
+    HIPCK(scan.ensure(compact_tiles(int(nn)), stream));
     return NPHYS_OK;
   }
+
+  // Whether the pair search does without the order and its boxes (k_broadphase.hip).
+  bool direct_pairs() const { return nscenes == 1 && n <= kDirectBodies; }
 
   BroadPhaseBufs bp_view() {
     BroadPhaseBufs v;
@@ -882,23 +898,20 @@ struct World {
     v.vals = vals.as<uint32_t>();
     v.keys_alt = keys_alt.as<uint32_t>();
     v.vals_alt = vals_alt.as<uint32_t>();
-    v.child = child.as<int>();
-    v.parent = parent.as<int>();
-    v.visit = visit.as<uint32_t>();
-    v.node_mn = node_mn.as<float4>();
-    v.node_mx = node_mx.as<float4>();
-    v.node_scene = node_scene.as<int2>();
-    v.pnode = bp_pnode.as<float4>();
+    v.leaf_mn = leaf_mn.as<float4>();
+    v.leaf_mx = leaf_mx.as<float4>();
+    v.box_mn = box_mn.as<float4>();
+    v.box_mx = box_mx.as<float4>();
+    v.box_top = box_top.as<int>();
     v.scene_bits = scene_bits;
     v.cand = cand.as<int>();
     v.cand_count = cand_count.as<uint32_t>();
-    v.cand_off = cand_off.as<uint32_t>();
     v.pairs = pairs.as<int2>();
     v.tmp = bp_tmp.as<uint32_t>();
+    v.scan = &scan;
     v.dirty = bp_dirty.as<uint32_t>();
-    v.leaf_of = bp_leaf_of.as<int>();
     v.list = bp_list.as<int>();
-    v.list_count = sm + 28;
+    v.list_count = sm + kSmListCount;
     return v;
   }
 
@@ -935,103 +948,95 @@ struct World {
 
   int readback(std::initializer_list<RbSeg> segs) { return rb_wait(rb_post(segs)); }
 
-  // Loose-AABB pass; returns the number of replaced loose AABBs through *changed.
-  int loose_pass(int mode, uint32_t* changed) {
-    int rc = ensure_bp();  // the dirty flags
-    if (rc) return rc;
-    BroadPhaseBufs v = bp_view();
-    fill_u32(v.changed, 0u, 2, stream);
-    launch_loose_update(bodies(), mode, v.changed, v.dirty, stream);
-    if ((rc = readback({{v.changed, 2, 0}}))) return rc;
-    *changed = rb_host[0];
-    dirty_pending += rb_host[0];
-    dirty_static_pending += rb_host[1];
-    return NPHYS_OK;
-  }
+  // Words of bp_small that a detection starts from zeroed and reads back in one piece: the loose
+  // passes' counts (0-3), the search's largest segment (16), the narrow phase's contacts, manifolds and list lengths (24-27), the dirty list's length (28); and the pairs (29).
+  static constexpr int kSmStats = 16, kSmTotals = 24, kSmBoxes = 26, kSmBalls = 27, kSmListCount = 28, kSmPairs = 29;
 
-  // The end-of-step syncs (CCD-phase swept AABBs, then the final poses) with one readback.
-  // The swept pass is the first of solve_ccd's loop, which returns before it when dt or
-  // max_ccd_substeps is zero (mechanical_world.rs:578-581).
-  int loose_passes_end_of_step(uint32_t* ch_swept, uint32_t* ch_final) {
+  // GeometricalWorld::sync_colliders (the loose-AABB passes of `passes`), perform_broad_phase and,
+  // when `narrow`, perform_narrow_phase into cb[cur]. Everything is enqueued with room for an eighth
+  // more pairs than last time and read back once at the end; if the pairs or a body's segment did not
+  // fit, buffers grow and the launches after the loose passes run again. *changed: loose AABBs replaced.
+  // bp_done and np_done, when given, are recorded after the two phases.
+  int detect(int passes, bool narrow, int64_t* changed, hipEvent_t bp_done = nullptr, hipEvent_t np_done = nullptr) {
     int rc = ensure_bp();
     if (rc) return rc;
+    const DevBodies b = bodies();
     BroadPhaseBufs v = bp_view();
-    fill_u32(v.changed, 0u, 4, stream);
-    if (sp.dt != 0.0f && prm.max_ccd_substeps != 0) launch_loose_update(bodies(), 2, v.changed, v.dirty, stream);
-    launch_loose_update(bodies(), 1, v.changed + 2, v.dirty, stream);
-    if ((rc = readback({{v.changed, 4, 0}}))) return rc;
-    *ch_swept = rb_host[0];
-    *ch_final = rb_host[2];
-    dirty_pending += int64_t(rb_host[0]) + rb_host[2];
-    dirty_static_pending += int64_t(rb_host[1]) + rb_host[3];
-    return NPHYS_OK;
-  }
-
-  int rebuild_pairs() {
-    if (n < 2) {
-      npairs = 0;
+    uint32_t* sm = bp_small.as<uint32_t>();
+    const uint32_t* h = rb_host;
+    fill_u32(sm, 0u, kSmPairs + 1, stream);
+    launch_loose_update(b, passes, v, stream);
+    const bool direct = direct_pairs();
+    if (!direct && (pairs_dirty || (passes & LOOSE_STATIC) || ++order_age > kOrderAge)) {
+      launch_order(b, v, stream);
+      order_age = 0;
+    }
+    bool may = segments_valid && incremental_bp && !pairs_dirty && dirty_static_pending == 0;
+    const long dirty_before = long(dirty_pending);
+    bool first = true;
+    for (int room = npairs + npairs / 8 + 1024;;) {
+      // a manifold's first slot is packed in 28 bits of the solver's slot record
+      constexpr int kMostPairs = ((1 << 28) / kPairSlots) - 1;
+      if (npairs > kMostPairs) return set_err(NPHYS_ERR_CAPACITY, "too many broad-phase pairs");
+      room = std::min(room, kMostPairs);
+      ContactBufs& out = cb[cur];
+      NarrowPhaseBufs np{};
+      if ((rc = ensure_narrow(room, narrow ? &out : nullptr, np))) return rc;
+      HIPCK(pairs.ensure(size_t(room) * sizeof(int2)));
+      v = bp_view();
+      SearchRun r{};
+      r.direct = direct ? 1 : 0;
+      r.fixed_end = fixed_end;
+      r.cap = cap;
+      r.may_increment = may ? 1 : 0;
+      r.dirty_before = dirty_before;
+      launch_search(b, v, r, stream);
+      PairOut po;
+      po.npairs = sm + kSmPairs;
+      po.nbox = np.nbox;
+      po.nball = np.nball;
+      po.perm = np.perm;
+      po.bfirst = narrow ? out.bfirst.as<int>() : nullptr;
+      po.pair_cap = room;
+      launch_compact_pairs(b, v, cap, direct, po, stream);
+      if (bp_done) HIPCK(hipEventRecord(bp_done, stream));
+      if (narrow) launch_narrow_phase(b, pairs.as<int2>(), np, out.view(), stream);
+      if (np_done) HIPCK(hipEventRecord(np_done, stream));
+      if ((rc = readback({{sm, kSmPairs + 1, 0}}))) return rc;
+      if (first) {
+        dirty_pending += int64_t(h[0]) + h[2];
+        dirty_static_pending += int64_t(h[1]) + h[3];
+        *changed = int64_t(h[0]) + h[2];
+        first = false;
+      }
+      // the device's rule (search_incremental), for the counters
+      const bool incremental = may && dirty_static_pending == 0 && dirty_pending <= kept_limit(n);
+      if (int(h[kSmStats]) > cap) {
+        // a segment took more partners than it has room for: all search again, with larger segments
+        if (incremental) ++counters.incremental_overflows;
+        cap = int(h[kSmStats]) + 8;
+        if ((rc = ensure_bp())) return rc;
+        may = false;
+        fill_u32(sm + kSmStats, 0u, kSmListCount - kSmStats, stream);
+        continue;
+      }
+      npairs = int(h[kSmPairs]);
+      if (npairs > room) {
+        room = npairs + npairs / 8;
+        // the segments stand, and as the dirty flags are cleared an incremental search keeps them
+        fill_u32(sm + kSmStats, 0u, kSmListCount - kSmStats, stream);
+        continue;
+      }
+      if (incremental && *changed != 0) ++counters.incremental_pair_updates;
+      dirty_pending = dirty_static_pending = 0;
+      segments_valid = true;
       pairs_dirty = false;
+      if (narrow) {
+        out.C = int(h[kSmTotals]);
+        out.M = int(h[kSmTotals + 1]);
+      }
       return NPHYS_OK;
     }
-    int rc = ensure_bp();
-    if (rc) return rc;
-    DevBodies b = bodies();
-    BroadPhaseBufs v = bp_view();
-    bool done = false;
-    if (tree_valid && incremental_bp && !pairs_dirty && dirty_static_pending == 0 &&
-        inc_since_full < kMaxIncremental && dirty_pending <= n / 8) {
-      // the pair offsets are computed right away and read back with the overflow check; they are
-      // discarded if the update overflowed
-      launch_incremental_pairs(b, v, cap, int(dirty_pending), stream);
-      launch_pair_offsets(b, v, cap, stream);
-      if ((rc = readback({{v.stats, 2, 0}, {v.cand_off + (n - 1), 1, 2}, {v.keys_alt + (n - 1), 1, 3}}))) return rc;
-      done = rb_host[1] == 0 && int(rb_host[0]) <= cap;  // else the full build below
-      if (done) {
-        ++inc_since_full;
-        ++counters.incremental_pair_updates;
-        npairs = int(rb_host[2] + rb_host[3]);
-      } else if (rb_host[1] == 0) {
-        // a clean body's segment took more appended partners than it has room for: the full build
-        // below gets segments that large, so the following incremental updates fit
-        ++counters.incremental_overflows;
-        cap = int(rb_host[0]) + 8;
-        if ((rc = ensure_bp())) return rc;
-        v = bp_view();
-      }
-    }
-    if (!done) {
-      if ((rc = full_traversal(b, v))) return rc;
-      inc_since_full = 0;
-      launch_pair_offsets(b, v, cap, stream);
-      // total = off[n-1] + min(count[n-1], cap)
-      if ((rc = readback({{v.cand_off + (n - 1), 1, 0}, {v.keys_alt + (n - 1), 1, 1}}))) return rc;
-      npairs = int(rb_host[0] + rb_host[1]);
-    }
-    HIPCK(pairs.ensure(size_t(std::max(npairs, 1)) * sizeof(int2)));
-    v = bp_view();
-    launch_compact_pairs(b, v, cap, stream);
-    fill_u32(v.dirty, 0u, size_t(n), stream);
-    dirty_pending = dirty_static_pending = 0;
-    tree_valid = true;
-    pairs_dirty = false;
-    return NPHYS_OK;
-  }
-
-  // Full build: the tree from scratch and every dynamic body traversed, the segment capacity grown
-  // until no body overflows it.
-  int full_traversal(DevBodies& b, BroadPhaseBufs& v) {
-    int rc;
-    launch_build_lbvh(b, v, stream);
-    for (;;) {
-      launch_traverse(b, v, cap, stream);
-      if ((rc = readback({{v.stats, 2, 0}}))) return rc;
-      if (rb_host[1]) return set_err(NPHYS_ERR_STATE, "BVH traversal stack overflow");
-      if (int(rb_host[0]) <= cap) break;
-      cap = int(rb_host[0]) + 8;
-      if ((rc = ensure_bp())) return rc;
-      v = bp_view();
-    }
-    return NPHYS_OK;
   }
 
   // The contacts of `c` in manifold order (dense records and, when imp is given, impulses), with
@@ -1068,30 +1073,39 @@ struct World {
   }
 
   // ------------------------------------------------------------------ narrow phase
-  // `done`, when given, is recorded after the narrow phase and before its readback (the step's last
-  // stage event, complete once the readback is).
-  int narrow_phase(hipEvent_t done = nullptr) { return narrow_phase_of(pairs.as<int2>(), npairs, cb[cur], done); }
-
-  // The narrow phase of `np` pairs (in pair order) into `out`.
-  int narrow_phase_of(const int2* list, int np, ContactBufs& out, hipEvent_t done = nullptr) {
-    const size_t P = size_t(std::max(np, 1));
-    // a manifold's first slot is packed in 28 bits of the solver's slot record
-    if (kPairSlots * P >= (size_t(1) << 28)) return set_err(NPHYS_ERR_CAPACITY, "too many broad-phase pairs");
-    for (DBuf* b : {&np_count, &np_coff, &np_has, &np_moff, &np_perm}) HIPCK(b->ensure(P * 4));
-    HIPCK(np_tmp.ensure(scan_temp_words(int(P)) * 4 + 64));
-    HIPCK(out.ensure(P, kPairSlots * P));
-    HIPCK(out.bfirst.ensure(size_t(std::max(n, 1)) * 4));
-    out.nb = n;
-    NarrowPhaseBufs v;
+  // Buffers of a narrow phase over `room` pairs (and its output's, when given); `v` describes them.
+  int ensure_narrow(int room, ContactBufs* out, NarrowPhaseBufs& v) {
+    const size_t P = size_t(std::max(room, 1));
+    for (DBuf* b : {&np_count, &np_perm}) HIPCK(b->ensure(P * 4));
+    HIPCK(scan.ensure(manifold_tiles(int(P)), stream));
+    if (out) {
+      HIPCK(out->ensure(P, kPairSlots * P));
+      HIPCK(out->bfirst.ensure(size_t(std::max(n, 1)) * 4));
+      out->nb = n;
+    }
+    uint32_t* sm = bp_small.as<uint32_t>();
     v.count = np_count.as<uint32_t>();
-    v.coff = np_coff.as<uint32_t>();
-    v.has = np_has.as<uint32_t>();
     v.perm = np_perm.as<uint32_t>();
-    v.moff = np_moff.as<uint32_t>();
-    v.totals = bp_small.as<uint32_t>() + 24;
-    v.tmp = np_tmp.as<uint32_t>();
-    launch_narrow_phase(bodies(), list, np, v, out.view(), stream);
-    if (done) HIPCK(hipEventRecord(done, stream));
+    v.npairs = sm + kSmPairs;
+    v.nbox = sm + kSmBoxes;
+    v.nball = sm + kSmBalls;
+    v.totals = sm + kSmTotals;
+    v.pair_cap = int(P);
+    v.boxes = any_cuboid;
+    v.balls = any_ball;
+    v.scan = &scan;
+    return NPHYS_OK;
+  }
+
+  // The narrow phase of `np` pairs (in pair order; their number also at *count_dev) into `out`.
+  int narrow_phase_of(const int2* list, int np, uint32_t* count_dev, ContactBufs& out) {
+    NarrowPhaseBufs v{};
+    const int rc0 = ensure_narrow(np, &out, v);
+    if (rc0) return rc0;
+    v.npairs = count_dev;
+    fill_u32(v.totals, 0u, 4, stream);
+    launch_narrow_bins(bodies(), list, v, out.view(), stream);
+    launch_narrow_phase(bodies(), list, v, out.view(), stream);
     const int rc = readback({{v.totals, 2, 0}});
     if (rc) return rc;
     out.C = int(rb_host[0]);
@@ -1099,15 +1113,10 @@ struct World {
     return NPHYS_OK;
   }
 
-  // sync_colliders + perform_broad_phase + perform_narrow_phase on the current poses.
-  int collide_now(int mode) {
-    uint32_t changed = 0;
-    int rc = loose_pass(mode, &changed);
-    if (rc) return rc;
-    if (changed || pairs_dirty) {
-      if ((rc = rebuild_pairs())) return rc;
-    }
-    return narrow_phase();
+  // Collision detection on the current poses of every body, static ones included.
+  int collide_now() {
+    int64_t changed = 0;
+    return detect(LOOSE_FINAL | LOOSE_STATIC, true, &changed);
   }
 
   // ------------------------------------------------------------------ solver
@@ -1130,8 +1139,8 @@ struct World {
     rec_stride = long(std::min({sv_rec.bytes / (kRecFields * sizeof(float4)), sv_lam.bytes / sizeof(float4),
                                 sv_prec.bytes / (3 * sizeof(float4))}));
     HIPCK(sv_red.ensure((size_t(residual_blocks(M)) * 2 + 4) * sizeof(double)));  // + the joints' partial
-    const size_t tw = std::max({radix_temp_words(int(m)), scan_temp_words(int(m)), scan_temp_words(int(nn))});
-    HIPCK(sv_tmp.ensure(tw * 4 + 64));
+    HIPCK(sv_tmp.ensure(radix_temp_words(int(m)) * 4));
+    HIPCK(scan.ensure(std::max({radix_scan_tiles(int(m)), scan_tiles(m), scan_tiles(nn)}), stream));
     return NPHYS_OK;
   }
 
@@ -1162,6 +1171,7 @@ struct World {
     v.pgeo = sv_pgeo.as<float4>();
     v.red = sv_red.as<double>();
     v.tmp = sv_tmp.as<uint32_t>();
+    v.scan = &scan;
     return v;
   }
 
@@ -1528,7 +1538,7 @@ struct World {
     HIPCK(act_touch.ensure(nn * 4));
     HIPCK(act_mflag[cur].ensure(m * 4));
     HIPCK(act_pos.ensure(m * 4));
-    HIPCK(act_tmp.ensure(scan_temp_words(int(m)) * 4 + 64));
+    HIPCK(scan.ensure(scan_tiles(m), stream));
     HIPCK(sl_mbody[cur].ensure(m * sizeof(int2)));
     HIPCK(sl_mfirst[cur].ensure(m * 4));
     HIPCK(sl_mcount[cur].ensure(m * 4));
@@ -1538,7 +1548,7 @@ struct World {
     a.touch = act_touch.as<uint32_t>();
     a.mflag = act_mflag[cur].as<uint32_t>();
     a.pos = act_pos.as<uint32_t>();
-    a.tmp = act_tmp.as<uint32_t>();
+    a.scan = &scan;
     a.totals = bp_small.as<uint32_t>() + 48;
     fill_u32(a.totals, 0u, 3, stream);
     const DevContacts full = cc.view();
@@ -1748,7 +1758,7 @@ struct World {
     HIPCK(ccd_imp.ensure(cap * sizeof(unsigned long long)));
     ccd_cap = int(std::min<size_t>(ccd_heap.bytes / sizeof(ToiEntry), ccd_imp.bytes / sizeof(unsigned long long)));
     HIPCK(ccd_ctl.ensure(kCcdWords * 4));
-    HIPCK(ccd_tmp.ensure(std::max(scan_temp_words(int(P)), scan_temp_words(int(nn))) * 4 + 64));
+    HIPCK(scan.ensure(std::max(scan_tiles(P), scan_tiles(nn)), stream));
     return NPHYS_OK;
   }
 
@@ -1774,7 +1784,7 @@ struct World {
     c.cpos = ccd_cpos.as<uint32_t>();
     c.list = ccd_list.as<int2>();
     c.list_pair = ccd_lpair.as<int>();
-    c.tmp = ccd_tmp.as<uint32_t>();
+    c.scan = &scan;
     c.deg = ccd_deg.as<uint32_t>();
     c.off = ccd_off.as<uint32_t>();
     c.fill = ccd_fill.as<uint32_t>();
@@ -1782,17 +1792,21 @@ struct World {
     return c;
   }
 
+  // detect() within a step, with its counters.
+  int detect_counting(int passes, bool narrow, hipEvent_t bp_done = nullptr, hipEvent_t np_done = nullptr) {
+    int64_t changed = 0;
+    const bool stale = pairs_dirty;
+    const int rc = detect(passes, narrow, &changed, bp_done, np_done);
+    if (rc) return rc;
+    counters.loose_changes += changed;
+    if (changed || stale) ++counters.pair_rebuilds;
+    return NPHYS_OK;
+  }
+
   // The CCD phase's sync and broad phase with swept AABBs (position0 -> position).
   int ccd_broad_phase() {
-    uint32_t ch = 0;
-    int rc = loose_pass(2, &ch);
-    if (rc) return rc;
-    counters.loose_changes += int64_t(ch);
-    if (ch || pairs_dirty) {
-      if ((rc = rebuild_pairs())) return rc;
-      ++counters.pair_rebuilds;
-    }
-    return ensure_ccd();
+    const int rc = detect_counting(LOOSE_SWEPT, false);
+    return rc ? rc : ensure_ccd();
   }
 
   // predict_next_impacts up to end_time: sets *kind (PREDICT_*), the impact count, the last
@@ -1836,7 +1850,7 @@ struct World {
       if ((rc = readback({{c.ctl + kCcdList, 1, 0}}))) return rc;
       const int nl = int(rb_host[0]);
       if (nl == 0) break;
-      if ((rc = narrow_phase_of(c.list, nl, ccd_cb))) return rc;
+      if ((rc = narrow_phase_of(c.list, nl, c.ctl + kCcdList, ccd_cb))) return rc;
       launch_ccd_grow(b, c, nl, np_count.as<uint32_t>(), stream);
       launch_ccd_merge(n, c, stream);
     }
@@ -1845,7 +1859,7 @@ struct World {
     if ((rc = readback({{c.ctl + kCcdList, 1, 0}}))) return rc;
     const int nk = int(rb_host[0]);
     ContactBufs& cc = cb[cur];
-    if ((rc = narrow_phase_of(c.list, nk, cc))) return rc;
+    if ((rc = narrow_phase_of(c.list, nk, c.ctl + kCcdList, cc))) return rc;
     const int M = cc.M, C = cc.C;
     SimParams ss = sp;
     ss.dt = dt_sub;
@@ -1923,7 +1937,7 @@ struct World {
     spp.dyn_dt = moved ? sp.dt : dyn_dt_next;
     dyn_dt_next = sp.dt;
     if (moved || recollide) {
-      if ((rc = collide_now(0))) return rc;
+      if ((rc = collide_now())) return rc;
       moved = false;
       recollide = false;
     }
@@ -1946,26 +1960,16 @@ struct World {
       // the CCD phase (its swept syncs and broad phases, impacts and substeps), then the final sync
       if ((rc = solve_ccd())) return rc;
       HIPCK(hipEventRecord(ev[EV_CCD], stream));
-      uint32_t ch = 0;
-      if ((rc = loose_pass(1, &ch))) return rc;
-      counters.loose_changes += int64_t(ch);
-      if (ch || pairs_dirty) {
-        if ((rc = rebuild_pairs())) return rc;
-        ++counters.pair_rebuilds;
-      }
+      rc = detect_counting(LOOSE_FINAL, true, ev[EV_BP], ev[EV_NP]);
     } else {
+      // the CCD phase's swept sync, which solve_ccd's loop returns before when dt or max_ccd_substeps
+      // is zero (mechanical_world.rs:578-581), then the final one
       HIPCK(hipEventRecord(ev[EV_CCD], stream));
-      uint32_t ch1 = 0, ch2 = 0;
-      if ((rc = loose_passes_end_of_step(&ch1, &ch2))) return rc;  // CCD-phase sync, then the final one
-      counters.loose_changes += int64_t(ch1) + int64_t(ch2);
-      if (ch1 || ch2 || pairs_dirty) {
-        if ((rc = rebuild_pairs())) return rc;
-        ++counters.pair_rebuilds;
-      }
+      const bool swept = sp.dt != 0.0f && prm.max_ccd_substeps != 0;
+      rc = detect_counting(LOOSE_FINAL | (swept ? LOOSE_SWEPT : 0), true, ev[EV_BP], ev[EV_NP]);
     }
-    HIPCK(hipEventRecord(ev[EV_BP], stream));
-    // the narrow phase's readback completes the step: every earlier event and copy is done after it
-    if ((rc = narrow_phase(ev[EV_NP]))) return rc;
+    // the detection's readback completes the step: every earlier event and copy is done after it
+    if (rc) return rc;
     finish_residual();
     auto el = [&](int a, int c) {
       float ms = 0.0f;
@@ -2250,7 +2254,7 @@ int nphys_step(nphys_world* w, int32_t nsteps) {
 
 int nphys_collide(nphys_world* w) {
   if (!w) return set_err(NPHYS_ERR_INVALID, "null world");
-  const int rc = w->w.collide_now(0);
+  const int rc = w->w.collide_now();
   if (rc) return rc;
   w->w.moved = false;
   w->w.recollide = false;
