@@ -156,10 +156,10 @@ __global__ void __launch_bounds__(64) k_position(DevBodies b, SimParams p, Solve
 // Consecutive small classes of the visiting order in one workgroup, a barrier between classes
 // (the same corrections in the same order per body as one launch per class).
 template <bool kMask>
-__global__ void __launch_bounds__(kRunBlock) k_position_run(DevBodies b, SimParams p, SolverBufs sb, int kv0, int nk) {
+__global__ void __launch_bounds__(kRunBlock) k_position_run(DevBodies b, SimParams p, SolverBufs sb, ClassRun run) {
   const GlobalPose acc{b};
-  for (int kv = kv0; kv < kv0 + nk; ++kv) {
-    const int2 range = sb.vrange[kv];
+  for (int k = 0; k < run.n; ++k) {
+    const int2 range = run.r[k];
     for (int t = threadIdx.x; t < range.y; t += kRunBlock) position_one<kMask>(acc, b, p, sb, range.x + t);
     __syncthreads();
   }
@@ -169,8 +169,8 @@ __global__ void __launch_bounds__(kRunBlock) k_position_run(DevBodies b, SimPara
 // `iterations` passes over the colours in the visiting order with a barrier between colours.
 template <int kBlock, int kCap, bool kMask>
 __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimParams p, SolverBufs sb, SceneBlocks sc,
-                                                           const int* __restrict__ scene_list, int ncolours,
-                                                           int iterations) {
+                                                           const int* __restrict__ scene_list,
+                                                           VisitOrder visit, int iterations) {
   __shared__ float4 s_pos[kCap];
   __shared__ float4 s_rot[kCap];
   const int s = scene_list[blockIdx.x];
@@ -182,12 +182,12 @@ __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimPar
   }
   __syncthreads();
   const LdsPose acc{b, s_pos, s_rot, sc.local};
-  const uint32_t* st = sc.start + long(s) * (ncolours + 1);
+  const uint32_t* st = sc.start + long(s) * (visit.n + 1);
   for (int it = 0; it < iterations; ++it) {
-    for (int k = 0; k < ncolours; ++k) {
-      const int col = sb.visit[k];
+    for (int k = 0; k < visit.n; ++k) {
+      const int col = visit.c[k];
       const int e = int(st[col + 1]);
-      for (int i = int(st[col]) + threadIdx.x; i < e; i += kBlock) position_one<kMask>(acc, b, p, sb, int(sc.slot[i]));
+      for (int i = int(st[col]) + threadIdx.x; i < e; i += kBlock) position_one<kMask>(acc, b, p, sb, sc.at(i));
       __syncthreads();
     }
   }
@@ -211,33 +211,33 @@ void launch_position_colour(const DevBodies& b, const DevContacts& c, const SimP
 }
 
 template <bool kMask>
-void position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc, int ncolours,
+void position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit,
                       int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
   if (sc.n_large > 0) {
     if (block == 256)
       hipLaunchKernelGGL((k_position_blocked<256, kLdsBodies, kMask>), dim3(sc.n_large), dim3(256), 0, s_large, b, p,
-                         sb, sc, sc.large_list, ncolours, iterations);
+                         sb, sc, sc.large_list, visit, iterations);
     else if (block == 512)
       hipLaunchKernelGGL((k_position_blocked<512, kLdsBodies, kMask>), dim3(sc.n_large), dim3(512), 0, s_large, b, p,
-                         sb, sc, sc.large_list, ncolours, iterations);
+                         sb, sc, sc.large_list, visit, iterations);
     else
       hipLaunchKernelGGL((k_position_blocked<1024, kLdsBodies, kMask>), dim3(sc.n_large), dim3(1024), 0, s_large, b,
-                         p, sb, sc, sc.large_list, ncolours, iterations);
+                         p, sb, sc, sc.large_list, visit, iterations);
   }
   if (sc.n_small > 0)
     hipLaunchKernelGGL((k_position_blocked<64, kSmallScene, kMask>), dim3(sc.n_small), dim3(64), 0, s_small, b, p, sb,
-                       sc, sc.small_list, ncolours, iterations);
+                       sc, sc.small_list, visit, iterations);
 }
 
 void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
-                             int ncolours, int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
-  if (b.kmask) position_blocked<true>(b, p, sb, sc, ncolours, iterations, block, s_small, s_large);
-  else position_blocked<false>(b, p, sb, sc, ncolours, iterations, block, s_small, s_large);
+                             const VisitOrder& visit, int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
+  if (b.kmask) position_blocked<true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+  else position_blocked<false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
 }
 
-void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, int kv0, int nk, hipStream_t s) {
-  if (b.kmask) hipLaunchKernelGGL(k_position_run<true>, dim3(1), dim3(kRunBlock), 0, s, b, p, sb, kv0, nk);
-  else hipLaunchKernelGGL(k_position_run<false>, dim3(1), dim3(kRunBlock), 0, s, b, p, sb, kv0, nk);
+void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s) {
+  if (b.kmask) hipLaunchKernelGGL(k_position_run<true>, dim3(1), dim3(kRunBlock), 0, s, b, p, sb, run);
+  else hipLaunchKernelGGL(k_position_run<false>, dim3(1), dim3(kRunBlock), 0, s, b, p, sb, run);
 }
 
 }  // namespace nph

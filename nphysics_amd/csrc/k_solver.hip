@@ -58,40 +58,38 @@ __device__ __forceinline__ uint32_t colour_hash(uint32_t x) {
   return x;
 }
 
-__global__ void __launch_bounds__(256) k_degree(DevBodies b, DevContacts c, int M, uint32_t* deg) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M) return;
-  const int2 bb = c.mbody[m];
-  if (b.status[bb.x] == STATUS_DYNAMIC) atomicAdd(&deg[bb.x], 1u);
-  if (b.status[bb.y] == STATUS_DYNAMIC) atomicAdd(&deg[bb.y], 1u);
-}
-
 // Colours persist across steps: a manifold whose body pair was a manifold of the previous solve
-// keeps that colour (marked as coloured in round 0); the others start uncoloured.
-__global__ void __launch_bounds__(256) k_inherit(DevContacts c, int M, DevContacts prev, int prevM,
-                                                const uint32_t* __restrict__ prev_state, uint32_t* state) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= M) return;
-  const int2 key = c.mbody[m];
-  const int j = find_manifold(prev, prevM, key.x, key.y);
-  state[m] = j >= 0 ? (prev_state[j] & 0xffffu) : kUncoloured;
-}
+// keeps that colour (marked as coloured in round 0); the others start uncoloured. Also counts the
+// manifolds of every dynamic body; the count met is the manifold's place in that body's list.
+constexpr uint32_t kNoPlace = 0xffffffffu;  // the static side of a manifold
 
-__global__ void __launch_bounds__(256) k_adjacency(DevBodies b, DevContacts c, int M,
-                                                  const uint32_t* __restrict__ off, uint32_t* fill,
-                                                  int* adj) {
+__global__ void __launch_bounds__(256) k_colour_begin(DevBodies b, DevContacts c, int M, DevContacts prev, int prevM,
+                                                     const uint32_t* __restrict__ prev_state, SolverBufs sb) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= M) return;
   const int2 bb = c.mbody[m];
-  if (b.status[bb.x] == STATUS_DYNAMIC) adj[off[bb.x] + atomicAdd(&fill[bb.x], 1u)] = m;
-  if (b.status[bb.y] == STATUS_DYNAMIC) adj[off[bb.y] + atomicAdd(&fill[bb.y], 1u)] = m;
+  uint2 at = make_uint2(kNoPlace, kNoPlace);
+  if (b.status[bb.x] == STATUS_DYNAMIC) at.x = atomicAdd(&sb.deg[bb.x], 1u);
+  if (b.status[bb.y] == STATUS_DYNAMIC) at.y = atomicAdd(&sb.deg[bb.y], 1u);
+  sb.place[m] = at;
+  const int j = find_manifold(prev, prevM, bb.x, bb.y);
+  sb.state[m] = j >= 0 ? (prev_state[j] & 0xffffu) : kUncoloured;
 }
 
-__global__ void __launch_bounds__(256) k_colour_round(DevBodies b, DevContacts c, int M, uint32_t round,
+__global__ void __launch_bounds__(256) k_adjacency(DevContacts c, int M, SolverBufs sb) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= M) return;
+  const int2 bb = c.mbody[m];
+  const uint2 at = sb.place[m];
+  if (at.x != kNoPlace) sb.adj[sb.adj_off[bb.x] + at.x] = m;
+  if (at.y != kNoPlace) sb.adj[sb.adj_off[bb.y] + at.y] = m;
+}
+
+__global__ void __launch_bounds__(256) k_colour_round(DevContacts c, int M, uint32_t round,
                                                      const uint32_t* __restrict__ off,
                                                      const uint32_t* __restrict__ deg,
-                                                     const int* __restrict__ adj, uint32_t* state,
-                                                     uint32_t* remaining, uint32_t* last_round) {
+                                                     const int* __restrict__ adj, const uint2* __restrict__ place,
+                                                     uint32_t* state, uint32_t* remaining, uint32_t* last_round) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= M) return;
   if (state[m] != kUncoloured) return;
@@ -99,8 +97,9 @@ __global__ void __launch_bounds__(256) k_colour_round(DevBodies b, DevContacts c
   const int2 bb = c.mbody[m];
   const int bs[2] = {bb.x, bb.y};
   bool dyn[2];
-  dyn[0] = b.status[bs[0]] == STATUS_DYNAMIC;
-  dyn[1] = b.status[bs[1]] == STATUS_DYNAMIC;
+  const uint2 at = place[m];
+  dyn[0] = at.x != kNoPlace;
+  dyn[1] = at.y != kNoPlace;
   for (int s = 0; s < 2; ++s) {
     if (!dyn[s]) continue;
     const uint32_t o0 = off[bs[s]], o1 = o0 + deg[bs[s]];
@@ -141,52 +140,121 @@ __global__ void __launch_bounds__(256) k_colour_round(DevBodies b, DevContacts c
   atomicMax(last_round, round);
 }
 
-__global__ void __launch_bounds__(256) k_colour_keys(int M, const uint32_t* __restrict__ state,
-                                                    uint32_t* keys, uint32_t* order, uint32_t* ncol) {
-  __shared__ uint32_t s_max[256];
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t c1 = 0;
-  if (m < M) {
-    const uint32_t c = state[m] & 0xffffu;
-    keys[m] = c;
-    order[m] = uint32_t(m);
-    c1 = c + 1u;
-  }
-  s_max[threadIdx.x] = c1;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) s_max[threadIdx.x] = s_max[threadIdx.x] > s_max[threadIdx.x + off] ? s_max[threadIdx.x] : s_max[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicMax(ncol, s_max[0]);
+// Colour order: a stable counting sort of the manifolds by colour that also adds up their contacts,
+// so that a manifold's slot, its first row record and the classes' bounds come out of one prefix sum over
+// (manifolds per colour and tile, then contacts per colour and tile). k_colour_hist counts per tile of
+// kColourTile manifolds, k_colour_scatter ranks within its tile: lanes of equal colour find each other by
+// ballots, and three ballots more give the contacts of those before. kDigits colours at most (256, or
+// kMaxColours where a readback finds more); a colour beyond, or none yet, counts as the last, and the
+// caller runs it again. The sort by a radix pass (histogram, scan, scatter, two copies back), the class starts, the
+// gather and scan of the counts, the slot records and the fix of empty classes were 14 launches and
+// one readback more: 30 us of a step at 1,233 manifolds, now 13 us.
+constexpr int kColourTile = 2048;
+
+template <int kDigits>
+__device__ __forceinline__ uint32_t colour_digit(uint32_t state) {
+  const uint32_t d = state & 0xffffu;
+  return d < uint32_t(kDigits) ? d : uint32_t(kDigits) - 1u;
 }
 
-__global__ void __launch_bounds__(256) k_colour_starts(DevContacts c, int M,
-                                                      const uint32_t* __restrict__ keys,
-                                                      const uint32_t* __restrict__ order,
-                                                      uint32_t* col_start, uint32_t* mcount_ord) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= M) return;
-  const uint32_t k = keys[s];
-  if (s == 0 || keys[s - 1] != k) col_start[k] = uint32_t(s);
-  if (s == M - 1) col_start[k + 1] = uint32_t(M);
-  mcount_ord[s] = uint32_t(c.mcount[order[s]]);
+template <int kDigits, int kThreads>
+__global__ void __launch_bounds__(kThreads) k_colour_hist(DevContacts c, int M, int ntiles, SolverBufs sb,
+                                                         uint32_t* ncol) {
+  __shared__ uint32_t s_m[kDigits], s_c[kDigits];
+  __shared__ uint32_t s_most;
+  for (int d = threadIdx.x; d < kDigits; d += kThreads) s_m[d] = s_c[d] = 0u;
+  if (threadIdx.x == 0) s_most = 0u;
+  __syncthreads();
+  uint32_t most = 0;
+  for (int k = threadIdx.x; k < kColourTile; k += kThreads) {
+    const int m = int(blockIdx.x) * kColourTile + k;
+    if (m >= M) break;
+    const uint32_t st = sb.state[m];
+    const uint32_t d = colour_digit<kDigits>(st);
+    const uint32_t c1 = (st & 0xffffu) + 1u;
+    most = c1 > most ? c1 : most;
+    atomicAdd(&s_m[d], 1u);
+    atomicAdd(&s_c[d], uint32_t(c.mcount[m]));
+  }
+  atomicMax(&s_most, most);
+  __syncthreads();
+  for (int d = threadIdx.x; d < kDigits; d += kThreads) {
+    sb.hist[long(d) * ntiles + blockIdx.x] = s_m[d];
+    sb.hist[long(kDigits + d) * ntiles + blockIdx.x] = s_c[d];
+  }
+  if (threadIdx.x == 0) atomicMax(ncol, s_most);
 }
 
 // Per slot (colour order): bodies with their dynamic flag in bit 30, first row record, contact
-// count and first contact index, packed into one int4.
-__global__ void __launch_bounds__(256) k_slot_info(DevBodies b, DevContacts c, int M,
-                                                  const uint32_t* __restrict__ order,
-                                                  const uint32_t* __restrict__ soff, int4* sinfo,
-                                                  uint32_t* slot_of) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= M) return;
-  const int m = int(order[s]);
-  slot_of[m] = uint32_t(s);
-  const int2 bb = c.mbody[m];
-  const int d1 = b.status[bb.x] == STATUS_DYNAMIC ? 1 : 0;
-  const int d2 = b.status[bb.y] == STATUS_DYNAMIC ? 1 : 0;
-  sinfo[s] = make_int4(bb.x | (d1 << 30), bb.y | (d2 << 30), int(soff[s]), c.mcount[m] | (c.mfirst[m] << 3));
+// count and first contact index, packed into one int4; per manifold its slot and first row record; per
+// class its first slot and first row record (col_start, class_rec; one more entry ends the last).
+template <int kDigits, int kThreads>
+__global__ void __launch_bounds__(kThreads) k_colour_scatter(DevContacts c, int M, int C, int ntiles, SolverBufs sb) {
+  constexpr int kWaves = kThreads / 64;
+  constexpr int kBits = kDigits == 256 ? 8 : 12;
+  __shared__ uint32_t s_m[kDigits], s_c[kDigits];
+  __shared__ uint32_t s_wave[kWaves][kDigits];  // per wave: manifolds, and their contacts from bit 16 up
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (int d = tid; d < kDigits; d += kThreads) {
+    s_m[d] = sb.offs[long(d) * ntiles + blockIdx.x];
+    s_c[d] = sb.offs[long(kDigits + d) * ntiles + blockIdx.x] - uint32_t(M);
+    if (blockIdx.x == 0) {
+      sb.col_start[d] = s_m[d];
+      sb.class_rec[d] = s_c[d];
+    }
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s_wave[w][d] = 0u;
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    sb.col_start[kDigits] = uint32_t(M);
+    sb.class_rec[kDigits] = uint32_t(C);
+  }
+  __syncthreads();
+  for (int k = 0; k < kColourTile; k += kThreads) {
+    const int m = int(blockIdx.x) * kColourTile + k + tid;
+    if (int(blockIdx.x) * kColourTile + k >= M) break;
+    const bool valid = m < M;
+    const uint32_t d = valid ? colour_digit<kDigits>(sb.state[m]) : 0u;
+    const uint32_t cnt = valid ? uint32_t(c.mcount[m]) : 0u;
+    uint64_t same = __ballot(valid);
+#pragma unroll
+    for (int i = 0; i < kBits; ++i) {
+      const bool bit = (d >> i) & 1u;
+      const uint64_t bb = __ballot(bit);
+      same &= bit ? bb : ~bb;
+    }
+    const uint64_t c0 = __ballot(cnt & 1u), c1 = __ballot(cnt & 2u), c2 = __ballot(cnt & 4u);
+    auto contacts = [&](uint64_t of) {
+      return uint32_t(__popcll(of & c0) + 2 * __popcll(of & c1) + 4 * __popcll(of & c2));
+    };
+    if (valid && (same & below) == 0ull) s_wave[wave][d] = uint32_t(__popcll(same)) | (contacts(same) << 16);
+    __syncthreads();
+    if (valid) {
+      uint32_t before = 0;
+      for (int w = 0; w < wave; ++w) before += s_wave[w][d];
+      const uint32_t slot = s_m[d] + (before & 0xffffu) + uint32_t(__popcll(same & below));
+      const uint32_t r0 = s_c[d] + (before >> 16) + contacts(same & below);
+      const int2 bb = c.mbody[m];
+      const uint2 at = sb.place[m];
+      sb.sinfo[slot] = make_int4(bb.x | (at.x != kNoPlace ? 1 << 30 : 0), bb.y | (at.y != kNoPlace ? 1 << 30 : 0),
+                                 int(r0), int(cnt) | (c.mfirst[m] << 3));
+      sb.ckeys[slot] = d;
+      sb.slot_of[m] = make_uint2(slot, r0);
+    }
+    __syncthreads();
+    for (int i = tid; i < kDigits; i += kThreads) {
+      uint32_t all = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        all += s_wave[w][i];
+        s_wave[w][i] = 0u;
+      }
+      s_m[i] += all & 0xffffu;
+      s_c[i] += all >> 16;
+    }
+    __syncthreads();
+  }
 }
 
 // One fill_constraint_geometry call: body-side jacobian (dir, p x dir), weighted angular part,
@@ -266,7 +334,8 @@ __global__ void __launch_bounds__(256) k_assemble(DevBodies b, DevContacts cur, 
   // the manifold's slot in colour order
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= M) return;
-  const int s = int(sb.slot_of[m]);
+  const uint2 at = sb.slot_of[m];
+  const int s = int(at.x);
   const int2 bb = cur.mbody[m];
   const int b1 = bb.x, b2 = bb.y;
   const bool d1 = b.status[b1] == STATUS_DYNAMIC;
@@ -290,7 +359,7 @@ __global__ void __launch_bounds__(256) k_assemble(DevBodies b, DevContacts cur, 
     }
   }
   const int first = cur.mfirst[m], cnt = cur.mcount[m];
-  const uint32_t r0 = sb.soff[s];
+  const uint32_t r0 = at.y;
   // the position solver's inputs in slot / record order (see k_position.hip)
   const int k1 = b.shape[b1], k2 = b.shape[b2];
   sb.pgeo[2 * long(s)] = f4(xyz(b.dims[b1]), m1);
@@ -356,7 +425,6 @@ __global__ void __launch_bounds__(256) k_assemble(DevBodies b, DevContacts cur, 
     R[2] = f4(p2, rr3[1]);
     R[3] = make_float4(rhs3[0], rhs3[1], rhs3[2], rr3[2]);
     sb.lam[r] = make_float4(lam[0], lam[1], lam[2], has);
-    sb.rec2c[r] = uint32_t(c);
   }
 }
 
@@ -538,14 +606,6 @@ template <bool kMask>
 __device__ __forceinline__ void store_dv(const DevBodies& b, const Manifold<kMask>& m, const Dv& v1, const Dv& v2) {
   if (m.x.d1) b.store_dv(m.x.b1, v1.l, v1.a);
   if (m.x.d2) b.store_dv(m.x.b2, v2.l, v2.a);
-}
-
-// Slot range of the class visited k-th: one load (the host writes the ranges with the visiting
-// order), not a visit -> class start chain.
-__device__ __forceinline__ void colour_range(const SolverBufs& sb, int k, int& first, int& n) {
-  const int2 r = sb.vrange[k];
-  first = r.x;
-  n = r.y;
 }
 
 // Solver velocity increments of the manifold's bodies in HBM (the per-colour kernels) ...
@@ -811,11 +871,10 @@ __global__ void __launch_bounds__(64) k_pgs(DevBodies b, DevContacts c, SolverBu
 // between classes: per body the same updates in the same order as one launch per class, without
 // a launch per class. Each class fits one pass of the workgroup.
 template <bool kWarm, bool kMask>
-__global__ void __launch_bounds__(kRunBlock) k_colour_run(DevBodies b, SolverBufs sb, int kv0, int nk) {
+__global__ void __launch_bounds__(kRunBlock) k_colour_run(DevBodies b, SolverBufs sb, ClassRun run) {
   const GlobalDv acc{b};
-  for (int kv = kv0; kv < kv0 + nk; ++kv) {
-    int first, n;
-    colour_range(sb, kv, first, n);
+  for (int k = 0; k < run.n; ++k) {
+    const int first = run.r[k].x, n = run.r[k].y;
     for (int t = threadIdx.x; t < n; t += kRunBlock) {
       if (kWarm) warm_manifold<kMask>(acc, b, sb, first + t);
       else pgs_manifold<kMask>(acc, b, sb, first + t);
@@ -832,7 +891,7 @@ __global__ void __launch_bounds__(kRunBlock) k_colour_run(DevBodies b, SolverBuf
 // so the results are identical.
 template <int kBlock, int kCap, bool kMask>
 __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBufs sb, SceneBlocks sc,
-                                                         const int* __restrict__ scene_list, int ncolours,
+                                                         const int* __restrict__ scene_list, VisitOrder visit,
                                                          int nsweeps, int warm) {
   __shared__ float4 s_lin[kCap];
   __shared__ float4 s_ang[kCap];
@@ -847,17 +906,17 @@ __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBu
   }
   __syncthreads();
   const LdsDv acc{s_lin, s_ang, sc.local};
-  const uint32_t* st = sc.start + long(s) * (ncolours + 1);
+  const uint32_t* st = sc.start + long(s) * (visit.n + 1);
   for (int pass = warm ? -1 : 0; pass < nsweeps; ++pass) {
-    for (int k = 0; k < ncolours; ++k) {
-      const int col = sb.visit[k];
+    for (int k = 0; k < visit.n; ++k) {
+      const int col = visit.c[k];
       const int s0 = int(st[col]), e = int(st[col + 1]);
       if (pass < 0) {
-        for (int i = s0 + threadIdx.x; i < e; i += kBlock) warm_manifold<kMask>(acc, b, sb, int(sc.slot[i]));
+        for (int i = s0 + threadIdx.x; i < e; i += kBlock) warm_manifold<kMask>(acc, b, sb, sc.at(i));
       } else {
         // both lanes of a manifold are adjacent lanes of one wavefront (kBlock and 2 * s0 are even)
         for (int i = 2 * s0 + threadIdx.x; i < 2 * e; i += kBlock)
-          pgs_manifold_pair<kMask>(acc, b, sb, int(sc.slot[i >> 1]), i & 1);
+          pgs_manifold_pair<kMask>(acc, b, sb, sc.at(i >> 1), i & 1);
       }
       __syncthreads();
     }
@@ -868,50 +927,40 @@ __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBu
   }
 }
 
-// Scene-major slot order for the blocked kernel: key = scene << 12 | colour per slot.
+// Scene-major slot order for the blocked kernel: the slots are in colour order, so a stable sort by scene
+// leaves them in (scene, colour) order.
 __global__ void __launch_bounds__(256) k_scene_keys(DevBodies b, int M, SolverBufs sb, uint32_t* keys,
                                                    uint32_t* slots) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= M) return;
   const int b1 = sb.sinfo[i].x & 0x3fffffff;
-  keys[i] = (uint32_t(b.scene[b1]) << 12) | sb.ckeys[i];
+  keys[i] = uint32_t(b.scene[b1]);
   slots[i] = uint32_t(i);
 }
 
-// start[s][c] = first position of (scene s, colour >= c) in the sorted keys (lower bound).
-__global__ void __launch_bounds__(256) k_scene_starts(const uint32_t* __restrict__ keys, int M, int nscenes,
+// start[s][c] = first position of (scene s, colour >= c) in the sorted slots (lower bound).
+__global__ void __launch_bounds__(256) k_scene_starts(const uint32_t* __restrict__ keys,
+                                                     const uint32_t* __restrict__ slot,
+                                                     const uint32_t* __restrict__ colour, int M, int nscenes,
                                                      int ncolours, uint32_t* start) {
   const long t = long(blockIdx.x) * blockDim.x + threadIdx.x;
   const long total = long(nscenes) * (ncolours + 1);
   if (t >= total) return;
   const int s = int(t / (ncolours + 1)), c = int(t % (ncolours + 1));
-  const uint32_t key = (uint32_t(s) << 12) | uint32_t(c);
   int lo = 0, hi = M;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
-    if (keys[mid] < key) lo = mid + 1;
+    const int ks = int(keys[mid]);
+    if (ks < s || (ks == s && int(colour[slot[mid]]) < c)) lo = mid + 1;
     else hi = mid;
   }
   start[t] = uint32_t(lo);
 }
 
-// Colours left empty (inherited colours can leave gaps) start where the next one does.
-// Also writes the first row record of every class (class_rec[k], class_rec[ncolours] = C),
-// which gives the host the contacts per class.
-__global__ void k_fix_colour_starts(int ncolours, int M, int C, uint32_t* col_start, const uint32_t* __restrict__ soff,
-                                    uint32_t* class_rec) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  col_start[ncolours] = uint32_t(M);
-  class_rec[ncolours] = uint32_t(C);
-  for (int k = ncolours - 1; k >= 0; --k) {
-    if (col_start[k] == 0xffffffffu) col_start[k] = col_start[k + 1];
-    class_rec[k] = col_start[k] < uint32_t(M) ? soff[col_start[k]] : uint32_t(C);
-  }
-}
-
-// Natural-map residual per row; per block (max |phi|, sum phi^2) in double, reduced on the host
-// in block order.
-template <bool kMask>
+// Natural-map residual per row; per block (max |phi|, sum phi^2) in double, written to host memory and
+// reduced there in block order. With kCache the manifold's impulses, which it has in registers, go to
+// the contacts' slots as well (cache_impulses: the warm start of the next step), 16 to 64 contiguous bytes.
+template <bool kMask, bool kCache>
 __global__ void __launch_bounds__(256) k_residual(DevBodies b, DevContacts c, int M, SolverBufs sb) {
   __shared__ double s_max[256];
   __shared__ double s_sum[256];
@@ -926,6 +975,7 @@ __global__ void __launch_bounds__(256) k_residual(DevBodies b, DevContacts c, in
     for (int k = 0; k < 4; ++k) {
       if (k >= m.x.cnt) break;
       const float4 lam = m.c[k].lam;
+      if (kCache) c.imp[m.x.first + k] = lam;
       {
         const Row v = row_of(m, k, 0);
         const float w = row_w(v, v1, v2);
@@ -962,13 +1012,15 @@ __global__ void __launch_bounds__(256) k_residual(DevBodies b, DevContacts c, in
   if (threadIdx.x == 0) {
     sb.red[2 * blockIdx.x] = s_max[0];
     sb.red[2 * blockIdx.x + 1] = s_sum[0];
+    __threadfence_system();
   }
 }
 
-__global__ void __launch_bounds__(256) k_cache(DevContacts c, SolverBufs sb, int C) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= C) return;
-  c.imp[sb.rec2c[r]] = sb.lam[r];
+__global__ void __launch_bounds__(256) k_cache(DevContacts c, int M, SolverBufs sb) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= M) return;
+  const SlotCtx x = slot_ctx(sb, s);
+  for (int k = 0; k < x.cnt; ++k) c.imp[x.first + k] = sb.lam[x.r0 + k];
 }
 
 // ------------------------------------------------------------------ learned warm start
@@ -1071,52 +1123,44 @@ inline unsigned nb(long n) { return unsigned((n + 255) / 256); }
 
 }  // namespace
 
-void launch_colour_prepare(const DevBodies& b, const DevContacts& c, int M, const DevContacts& prev,
-                           int prevM, const uint32_t* prev_state, SolverBufs& sb, hipStream_t s) {
+void launch_colour_begin(const DevBodies& b, const DevContacts& c, int M, const DevContacts& prev, int prevM,
+                         const uint32_t* prev_state, SolverBufs& sb, hipStream_t s) {
   fill_u32(sb.deg, 0u, size_t(b.n), s);
-  fill_u32(sb.adj_fill, 0u, size_t(b.n), s);
-  if (M == 0) return;
-  hipLaunchKernelGGL(k_inherit, dim3(nb(M)), dim3(256), 0, s, c, M, prev, prevM, prev_state, sb.state);
-  hipLaunchKernelGGL(k_degree, dim3(nb(M)), dim3(256), 0, s, b, c, M, sb.deg);
+  hipLaunchKernelGGL(k_colour_begin, dim3(nb(M)), dim3(256), 0, s, b, c, M, prev, prevM, prev_state, sb);
   scan_exclusive_u32(sb.deg, sb.adj_off, b.n, *sb.scan, s);
-  hipLaunchKernelGGL(k_adjacency, dim3(nb(M)), dim3(256), 0, s, b, c, M, sb.adj_off, sb.adj_fill, sb.adj);
+  hipLaunchKernelGGL(k_adjacency, dim3(nb(M)), dim3(256), 0, s, c, M, sb);
 }
 
-void launch_colour_round(const DevBodies& b, const DevContacts& c, int M, int round, SolverBufs& sb,
-                         hipStream_t s) {
-  if (M == 0) return;
-  fill_u32(sb.remaining, 0u, 1, s);
-  hipLaunchKernelGGL(k_colour_round, dim3(nb(M)), dim3(256), 0, s, b, c, M, uint32_t(round), sb.adj_off,
-                     sb.deg, sb.adj, sb.state, sb.remaining, sb.remaining + 1);
-}
-
-void launch_colour_keys(int M, SolverBufs& sb, uint32_t* ncol, hipStream_t s) {
-  fill_u32(ncol, 0u, 1, s);
-  if (M == 0) return;
-  hipLaunchKernelGGL(k_colour_keys, dim3(nb(M)), dim3(256), 0, s, M, sb.state, sb.ckeys, sb.order, ncol);
-}
-
-void launch_colour_order(const DevBodies& b_view_for_slots, const DevContacts& c, int M, int ncolours,
+void launch_colour_round(const DevContacts& c, int M, int round, uint32_t* remaining, uint32_t* last_round,
                          SolverBufs& sb, hipStream_t s) {
-  if (M == 0) return;
-  const int bits = ncolours <= 256 ? 8 : 16;
-  radix_sort_pairs(sb.ckeys, sb.order, sb.ckeys_alt, sb.order_alt, M, bits, sb.tmp, *sb.scan, s);
-  fill_u32(sb.col_start, 0xffffffffu, size_t(ncolours) + 1, s);
-  hipLaunchKernelGGL(k_colour_starts, dim3(nb(M)), dim3(256), 0, s, c, M, sb.ckeys, sb.order, sb.col_start,
-                     sb.mcount_ord);
-  scan_exclusive_u32(sb.mcount_ord, sb.soff, M, *sb.scan, s);
-  hipLaunchKernelGGL(k_slot_info, dim3(nb(M)), dim3(256), 0, s, b_view_for_slots, c, M, sb.order, sb.soff, sb.sinfo,
-                     sb.slot_of);
+  hipLaunchKernelGGL(k_colour_round, dim3(nb(M)), dim3(256), 0, s, c, M, uint32_t(round), sb.adj_off, sb.deg, sb.adj,
+                     sb.place, sb.state, remaining, last_round);
+}
+
+namespace {
+template <int kDigits, int kThreads>
+void colour_order(const DevContacts& c, int M, int C, SolverBufs& sb, uint32_t* ncol, hipStream_t s) {
+  const int ntiles = (M + kColourTile - 1) / kColourTile;
+  hipLaunchKernelGGL((k_colour_hist<kDigits, kThreads>), dim3(ntiles), dim3(kThreads), 0, s, c, M, ntiles, sb, ncol);
+  scan_exclusive_u32(sb.hist, sb.offs, 2 * kDigits * ntiles, *sb.scan, s);
+  hipLaunchKernelGGL((k_colour_scatter<kDigits, kThreads>), dim3(ntiles), dim3(kThreads), 0, s, c, M, C, ntiles, sb);
+}
+}  // namespace
+
+size_t colour_hist_words(int M, int digits) {
+  return 2 * size_t(digits) * size_t((M + kColourTile - 1) / kColourTile);
+}
+
+void launch_colour_order(const DevContacts& c, int M, int C, int digits, SolverBufs& sb, uint32_t* ncol,
+                         hipStream_t s) {
+  if (digits == 256) colour_order<256, 256>(c, M, C, sb, ncol, s);
+  else colour_order<kMaxColours, 64>(c, M, C, sb, ncol, s);
 }
 
 void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContacts& prev, int prevM,
                      int M, const SimParams& p, SolverBufs& sb, const MatTable& mt, hipStream_t s) {
   if (M == 0) return;
   hipLaunchKernelGGL(k_assemble, dim3(nb(M)), dim3(256), 0, s, b, cur, prev, prevM, M, p, sb, mt);
-}
-
-void launch_fix_colour_starts(int ncolours, int M, int C, SolverBufs& sb, uint32_t* class_rec, hipStream_t s) {
-  hipLaunchKernelGGL(k_fix_colour_starts, dim3(1), dim3(1), 0, s, ncolours, M, C, sb.col_start, sb.soff, class_rec);
 }
 
 // One lane per manifold: the cap on a colour launch's grid, one 64-lane workgroup per 64
@@ -1152,26 +1196,32 @@ void launch_pgs_colour(const DevBodies& b, const DevContacts& c, int first, int 
   }
 }
 
-void launch_colour_run(const DevBodies& b, SolverBufs& sb, int kv0, int nk, bool warm, hipStream_t s) {
+void launch_colour_run(const DevBodies& b, SolverBufs& sb, const ClassRun& run, bool warm, hipStream_t s) {
   if (b.kmask) {
-    if (warm) hipLaunchKernelGGL((k_colour_run<true, true>), dim3(1), dim3(kRunBlock), 0, s, b, sb, kv0, nk);
-    else hipLaunchKernelGGL((k_colour_run<false, true>), dim3(1), dim3(kRunBlock), 0, s, b, sb, kv0, nk);
+    if (warm) hipLaunchKernelGGL((k_colour_run<true, true>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
+    else hipLaunchKernelGGL((k_colour_run<false, true>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
     return;
   }
-  if (warm) hipLaunchKernelGGL((k_colour_run<true, false>), dim3(1), dim3(kRunBlock), 0, s, b, sb, kv0, nk);
-  else hipLaunchKernelGGL((k_colour_run<false, false>), dim3(1), dim3(kRunBlock), 0, s, b, sb, kv0, nk);
+  if (warm) hipLaunchKernelGGL((k_colour_run<true, false>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
+  else hipLaunchKernelGGL((k_colour_run<false, false>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
 }
 
 int residual_blocks(int M) { return int(nb(M > 0 ? M : 1)); }
 
-void launch_residual(const DevBodies& b, const DevContacts& c, int M, SolverBufs& sb, hipStream_t s) {
-  if (b.kmask) hipLaunchKernelGGL(k_residual<true>, dim3(nb(M > 0 ? M : 1)), dim3(256), 0, s, b, c, M, sb);
-  else hipLaunchKernelGGL(k_residual<false>, dim3(nb(M > 0 ? M : 1)), dim3(256), 0, s, b, c, M, sb);
+void launch_residual(const DevBodies& b, const DevContacts& c, int M, bool cache, SolverBufs& sb, hipStream_t s) {
+  const dim3 grid(nb(M > 0 ? M : 1));
+  if (b.kmask) {
+    if (cache) hipLaunchKernelGGL((k_residual<true, true>), grid, dim3(256), 0, s, b, c, M, sb);
+    else hipLaunchKernelGGL((k_residual<true, false>), grid, dim3(256), 0, s, b, c, M, sb);
+  } else {
+    if (cache) hipLaunchKernelGGL((k_residual<false, true>), grid, dim3(256), 0, s, b, c, M, sb);
+    else hipLaunchKernelGGL((k_residual<false, false>), grid, dim3(256), 0, s, b, c, M, sb);
+  }
 }
 
-void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int C, hipStream_t s) {
-  if (C == 0) return;
-  hipLaunchKernelGGL(k_cache, dim3(nb(C)), dim3(256), 0, s, c, sb, C);
+void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int M, hipStream_t s) {
+  if (M == 0) return;
+  hipLaunchKernelGGL(k_cache, dim3(nb(M)), dim3(256), 0, s, c, M, sb);
 }
 
 void launch_features(const DevBodies& b, const DevContacts& c, const SimParams& p, int M, SolverBufs& sb, float* X,
@@ -1195,43 +1245,44 @@ void launch_lam_copy(SolverBufs& sb, int C, float4* buf, bool to_buf, hipStream_
   hipLaunchKernelGGL(k_lam_copy, dim3(nb(C)), dim3(256), 0, s, sb, C, buf, to_buf ? 1 : 0);
 }
 
-void launch_scene_order(const DevBodies& b, int M, int nscenes, int ncolours, SolverBufs& sb, SceneBlocks& sc,
-                        hipStream_t s) {
+void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int ncolours, SolverBufs& sb,
+                        SceneBlocks& sc, hipStream_t s) {
   if (M == 0) return;
   hipLaunchKernelGGL(k_scene_keys, dim3(nb(M)), dim3(256), 0, s, b, M, sb, sc.keys, sc.slot);
-  radix_sort_pairs(sc.keys, sc.slot, sc.keys_alt, sc.slot_alt, M, 28, sb.tmp, *sb.scan, s);
+  radix_sort_pairs(sc.keys, sc.slot, sc.keys_alt, sc.slot_alt, M, (scene_bits + 15) / 16 * 16, sb.tmp, *sb.scan, s);
   const long total = long(nscenes) * (ncolours + 1);
-  hipLaunchKernelGGL(k_scene_starts, dim3(nb(total)), dim3(256), 0, s, sc.keys, M, nscenes, ncolours, sc.start);
+  hipLaunchKernelGGL(k_scene_starts, dim3(nb(total)), dim3(256), 0, s, sc.keys, sc.slot, sb.ckeys, M, nscenes,
+                     ncolours, sc.start);
 }
 
 // Two launches: the scenes with more than kSmallScene dynamic bodies (`block` lanes, 64 KB of LDS)
 // on s_large, the others (64-lane workgroups, 8 KB of LDS, many resident per CU) on s_small, so the
 // few large scenes run beside the many small ones.
 template <bool kMask>
-void sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, int ncolours, int nsweeps, bool warm,
-                    int block, hipStream_t s_small, hipStream_t s_large) {
+void sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit, int nsweeps,
+                    bool warm, int block, hipStream_t s_small, hipStream_t s_large) {
   const int w = warm ? 1 : 0;
   if (kMask && block == 1024) block = 512;  // the masked kernel would spill at 1024 lanes (128 VGPRs)
   if (sc.n_large > 0) {
     if (block == 256)
       hipLaunchKernelGGL((k_sweeps_blocked<256, kLdsBodies, kMask>), dim3(sc.n_large), dim3(256), 0, s_large, b, sb,
-                         sc, sc.large_list, ncolours, nsweeps, w);
+                         sc, sc.large_list, visit, nsweeps, w);
     else if (kMask || block == 512)
       hipLaunchKernelGGL((k_sweeps_blocked<512, kLdsBodies, kMask>), dim3(sc.n_large), dim3(512), 0, s_large, b, sb,
-                         sc, sc.large_list, ncolours, nsweeps, w);
+                         sc, sc.large_list, visit, nsweeps, w);
     else
       hipLaunchKernelGGL((k_sweeps_blocked<1024, kLdsBodies, false>), dim3(sc.n_large), dim3(1024), 0, s_large, b,
-                         sb, sc, sc.large_list, ncolours, nsweeps, w);
+                         sb, sc, sc.large_list, visit, nsweeps, w);
   }
   if (sc.n_small > 0)
     hipLaunchKernelGGL((k_sweeps_blocked<64, kSmallScene, kMask>), dim3(sc.n_small), dim3(64), 0, s_small, b, sb, sc,
-                       sc.small_list, ncolours, nsweeps, w);
+                       sc.small_list, visit, nsweeps, w);
 }
 
-void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, int ncolours, int nsweeps,
-                           bool warm, int block, hipStream_t s_small, hipStream_t s_large) {
-  if (b.kmask) sweeps_blocked<true>(b, sb, sc, ncolours, nsweeps, warm, block, s_small, s_large);
-  else sweeps_blocked<false>(b, sb, sc, ncolours, nsweeps, warm, block, s_small, s_large);
+void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit,
+                           int nsweeps, bool warm, int block, hipStream_t s_small, hipStream_t s_large) {
+  if (b.kmask) sweeps_blocked<true>(b, sb, sc, visit, nsweeps, warm, block, s_small, s_large);
+  else sweeps_blocked<false>(b, sb, sc, visit, nsweeps, warm, block, s_small, s_large);
 }
 
 }  // namespace nph

@@ -135,42 +135,40 @@ void launch_gather_contacts(const DevContacts& c, int M, const uint32_t* moff, f
 struct SolverBufs {
   uint32_t* deg;          // [n] dynamic-body degree in the manifold graph
   uint32_t* adj_off;      // [n]
-  uint32_t* adj_fill;     // [n]
   int* adj;               // [2M]
+  uint2* place;           // [M] place of the manifold in its bodies' lists (kNoPlace: a static body)
   uint32_t* state;        // [M] colouring state: 0xffffffff, or round << 16 | colour
-  uint32_t* remaining;    // [2] 0: a manifold left uncoloured by the last round, 1: last round that coloured one
-  uint32_t* ckeys;        // [M] colour keys
-  uint32_t* order;        // [M] manifold ids in colour order
-  uint32_t* ckeys_alt;
-  uint32_t* order_alt;
-  uint32_t* col_start;    // [max colours + 1]
-  uint32_t* mcount_ord;   // [M] contact counts in colour order
-  uint32_t* soff;         // [M] first row record of each slot
+  uint32_t* hist;         // [colour_hist_words] manifolds, then contacts, per colour and tile
+  uint32_t* offs;         // [same] their exclusive sums
+  uint32_t* ckeys;        // [M] colour of each slot
+  uint32_t* col_start;    // [max colours + 1] first slot of each class, and
+  uint32_t* class_rec;    // first row record
   int4* sinfo;            // [M] per slot: body1|dyn1<<30, body2|dyn2<<30, first record, count|first<<3
-  uint32_t* slot_of;      // [M] slot of each manifold (inverse of order)
-  uint32_t* rec2c;        // [C] contact index of each row record
+  uint2* slot_of;         // [M] slot and first row record of each manifold
   float4* rec;            // [kRecFields rec_stride] row records, field f of record r at kRecFields r + f
   float4* lam;            // [rec_stride] impulses of each row record (normal, tangent 1, tangent 2, has cache)
   float4* prec;           // [3 rec_stride] position records: (lp1 | contact kind), (lp2 | shape 1), (ln | shape 2)
   float4* pgeo;           // [2M] per slot: (half extents 1 | margin 1), (half extents 2 | margin 2)
   long rec_stride;        // record capacity (fixed between reallocations)
-  int* visit;             // [max colours] colour classes in visiting order
-  int2* vrange;           // [max colours] (first slot, slots) of the class visited k-th
-  double* red;            // residual partials
+  double* red;            // residual partials, in host memory
   uint32_t* tmp;          // radix scratch
   ScanState* scan;
 };
 constexpr int kMaxColours = 4096;
 constexpr int kRecFields = 4;  // float4 per contact row record
 
-void launch_colour_prepare(const DevBodies& b, const DevContacts& c, int M, const DevContacts& prev,
-                           int prevM, const uint32_t* prev_state, SolverBufs& sb, hipStream_t s);
-void launch_colour_round(const DevBodies& b, const DevContacts& c, int M, int round, SolverBufs& sb,
+// Colours inherited from the previous solve's manifolds, degrees and adjacency (M > 0).
+void launch_colour_begin(const DevBodies& b, const DevContacts& c, int M, const DevContacts& prev, int prevM,
+                         const uint32_t* prev_state, SolverBufs& sb, hipStream_t s);
+// *remaining, zero before, becomes 1 if a manifold stays uncoloured; *last_round the last round that
+// coloured one
+void launch_colour_round(const DevContacts& c, int M, int round, uint32_t* remaining, uint32_t* last_round,
+                         SolverBufs& sb, hipStream_t s);
+// Slots, records and classes in colour order, for up to `digits` colours (256 or kMaxColours); *ncol, zero
+// before, becomes the number of colours.
+size_t colour_hist_words(int M, int digits);
+void launch_colour_order(const DevContacts& c, int M, int C, int digits, SolverBufs& sb, uint32_t* ncol,
                          hipStream_t s);
-void launch_colour_keys(int M, SolverBufs& sb, uint32_t* ncol, hipStream_t s);
-void launch_colour_order(const DevBodies& b, const DevContacts& c, int M, int ncolours, SolverBufs& sb,
-                         hipStream_t s);
-void launch_fix_colour_starts(int ncolours, int M, int C, SolverBufs& sb, uint32_t* class_rec, hipStream_t s);
 int residual_blocks(int M);
 void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContacts& prev,
                      int prevM, int M, const SimParams& p, SolverBufs& sb, const MatTable& mt, hipStream_t s);
@@ -182,22 +180,34 @@ int position_blocks(int max_class);
 // (first, n): the class's slot range, known on the host from the visiting order
 void launch_warmstart_colour(const DevBodies& b, const DevContacts& c, int first, int n, int blocks,
                              SolverBufs& sb, hipStream_t s);
-// Consecutive visited classes kv0 .. kv0 + nk - 1, each of at most kRunBlock manifolds, in one
-// workgroup (warm start or sweep).
+// Consecutive visited classes, each of at most kRunBlock manifolds, as (first slot, slots), in one
+// workgroup (warm start or sweep). Passed by value: no copy to the device stands before the launch.
 constexpr int kRunBlock = 512;
-void launch_colour_run(const DevBodies& b, SolverBufs& sb, int kv0, int nk, bool warm, hipStream_t s);
+constexpr int kRunClasses = 64;
+struct ClassRun {
+  int n;
+  int2 r[kRunClasses];
+};
+void launch_colour_run(const DevBodies& b, SolverBufs& sb, const ClassRun& run, bool warm, hipStream_t s);
 void launch_pgs_colour(const DevBodies& b, const DevContacts& c, int first, int n, int blocks, SolverBufs& sb,
                        hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-void launch_residual(const DevBodies& b, const DevContacts& c, int M, SolverBufs& sb, hipStream_t s);
-void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int C, hipStream_t s);
+// cache: also the impulses to the contacts' slots, as launch_cache_impulses
+void launch_residual(const DevBodies& b, const DevContacts& c, int M, bool cache, SolverBufs& sb, hipStream_t s);
+void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int M, hipStream_t s);
 
 // Scene-blocked sweeps (k_solver.hip): every scene's slots in (scene, colour) order, per scene
 // and colour the first position, and the scene's dynamic bodies (CSR) with each body's rank.
 constexpr int kLdsBodies = 2048;  // dynamic bodies of one scene the blocked kernel keeps in LDS
 constexpr int kSmallScene = 256;  // scenes up to this many dynamic bodies use the small workgroups
+// Visiting order of the colour classes, by value.
+constexpr int kVisitColours = 512;
+struct VisitOrder {
+  int n;
+  uint16_t c[kVisitColours];
+};
 struct SceneBlocks {
-  uint32_t* keys;        // [M] scene << 12 | colour, sorted
-  uint32_t* slot;        // [M] slots in that order
+  uint32_t* keys;        // [M] scene, sorted
+  uint32_t* slot;        // [M] slots in (scene, colour) order; null: the colour order is it (one scene)
   uint32_t* keys_alt;
   uint32_t* slot_alt;
   uint32_t* start;       // [nscenes][ncolours + 1]
@@ -207,17 +217,18 @@ struct SceneBlocks {
   const int* small_list; // scenes with at most kSmallScene dynamic bodies
   const int* large_list; // the other scenes
   int n_small, n_large;
+  __device__ int at(int i) const { return slot ? int(slot[i]) : i; }
 };
-void launch_scene_order(const DevBodies& b, int M, int nscenes, int ncolours, SolverBufs& sb, SceneBlocks& sc,
-                        hipStream_t s);
+void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int ncolours, SolverBufs& sb,
+                        SceneBlocks& sc, hipStream_t s);
 // block: lanes per large scene (256, 512 or 1024); the large scenes go on s_large, the small on s_small
-void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, int ncolours, int nsweeps,
-                           bool warm, int block, hipStream_t s_small, hipStream_t s_large);
+void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit,
+                           int nsweeps, bool warm, int block, hipStream_t s_small, hipStream_t s_large);
 // Scene-blocked position correction: `iterations` passes over the colours in the visiting order,
 // one workgroup per scene with the scene's dynamic poses in LDS (the same corrections in the same
 // order per body as the per-colour launches); streams and block as launch_sweeps_blocked.
 void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
-                             int ncolours, int iterations, int block, hipStream_t s_small, hipStream_t s_large);
+                             const VisitOrder& visit, int iterations, int block, hipStream_t s_small, hipStream_t s_large);
 
 // learned warm start (k_solver.hip): features [C][24] and impulse units ls [C] per row record,
 // the prediction y [C][3] applied as the warm start, post-solve targets t [C][3].
@@ -326,6 +337,6 @@ void launch_ccd_clamp(const DevBodies& b, CcdBufs& c, hipStream_t s);
 // k_position.hip ---------------------------------------------------------------------------
 void launch_position_colour(const DevBodies& b, const DevContacts& c, const SimParams& p, int first, int n,
                             int blocks, SolverBufs& sb, hipStream_t s);
-void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, int kv0, int nk, hipStream_t s);
+void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s);
 
 }  // namespace nph

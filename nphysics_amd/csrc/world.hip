@@ -169,27 +169,26 @@ struct World {
   int sview_M[2] = {0, 0}, sview_C[2] = {0, 0};
   bool sview_compact[2] = {false, false};
   DBuf sv_state2[2];  // colouring state of the manifolds of sview[k]
-  DBuf sv_deg, sv_adj_off, sv_adj_fill, sv_adj, sv_ckeys, sv_order, sv_ckeys_alt,
-      sv_order_alt, sv_col_start, sv_mcount_ord, sv_soff, sv_slot_of, sv_sinfo, sv_rec2c, sv_rec, sv_lam, sv_prec, sv_pgeo, sv_red, sv_tmp;
+  DBuf sv_deg, sv_adj_off, sv_adj, sv_place, sv_hist, sv_ckeys, sv_col_start, sv_slot_of, sv_sinfo, sv_rec, sv_lam,
+      sv_prec, sv_pgeo, sv_tmp;
   int ncolours = 0;
   long rec_stride = 0;
   int colour_rounds = 0;
   static constexpr int kRoundBatch = 4;  // colouring rounds launched between polls
   std::vector<int> colour_visit;  // colour classes in visiting order
   long solve_count = 0;    // solves performed, never reset
-  DBuf sv_visit;           // device copy of colour_visit, then the classes' slot ranges in that order
-  int* h_visit = nullptr;  // pinned staging of the same
+  std::vector<int2> h_range;       // their (first slot, slots), in that order
+  std::vector<int> class_contacts;  // and their contacts
   int solved_M = 0, solved_C = 0;
   double res_inf = 0.0, res_rms = 0.0;
-  double* red_pinned = nullptr;  // deferred residual partials (pinned)
-  size_t red_pinned_cap = 0;
+  double *red_host = nullptr, *red_dev = nullptr;  // residual partials (pinned, device-mapped)
+  size_t red_cap = 0;
   int res_pending_blocks = -1, res_pending_C = 0;
   // solve-to-residual mode (off when res_target <= 0): see nphys_set_residual_target
   double res_target = 0.0;
   int res_max_sweeps = 500, res_check_every = 1, res_norm = NPHYS_RESIDUAL_MAX;
   int last_sweeps = 0;
   int max_class = 0;             // largest colour class of the current solve
-  std::vector<double> red_host;
   // learned warm start: network (FP32 parameters + BF16 images), per-record features, impulse
   // units, predictions and recorded targets; the judge's saved plain solve
   // scene-blocked solve: per-scene dynamic-body lists (host-built at insertion), the per-solve
@@ -248,7 +247,7 @@ struct World {
   static constexpr int kRbClass = 64, kRbFlag = kRbClass + 2 * (kMaxColours + 2) + 64, kRbWords = kRbFlag + 64;
   uint32_t* rb_host = nullptr;
   uint32_t* rb_dev = nullptr;
-  uint32_t rb_seq = 0, class_seq = 0;
+  uint32_t rb_seq = 0;
   // Staging of set_state and get_state (pinned, device-mapped): 52 B per body, grown on first use.
   float *io_host = nullptr, *io_dev = nullptr;
   size_t io_cap = 0;
@@ -264,8 +263,7 @@ struct World {
   int kt_used = 0;
 
   ~World() {
-    if (h_visit) (void)hipHostFree(h_visit);
-    if (red_pinned) (void)hipHostFree(red_pinned);
+    if (red_host) (void)hipHostFree(red_host);
     if (rb_host) (void)hipHostFree(rb_host);
     if (io_host) (void)hipHostFree(io_host);
     for (auto& e : ev)
@@ -313,8 +311,6 @@ struct World {
                         hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(rb_host, 0, kRbWords * sizeof(uint32_t));
     HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&rb_dev), rb_host, 0));
-    HIPCK(hipHostMalloc(reinterpret_cast<void**>(&h_visit), 3 * (kMaxColours + 2) * sizeof(int)));
-    HIPCK(sv_visit.ensure(3 * (kMaxColours + 2) * sizeof(int)));
     for (auto& e : ev) HIPCK(hipEventCreate(&e));
     for (auto& e : tune_ev) HIPCK(hipEventCreate(&e));
     set_params(p);
@@ -1120,27 +1116,39 @@ struct World {
   }
 
   // ------------------------------------------------------------------ solver
-  int ensure_solver(int M, int C) {
+  int ensure_solver(int M, int C, int digits = 256) {
     const size_t nn = size_t(std::max(n, 1));
     const size_t m = size_t(std::max(M, 1)), c = size_t(std::max(C, 1));
-    for (DBuf* b : {&sv_deg, &sv_adj_off, &sv_adj_fill}) HIPCK(b->ensure(nn * 4));
+    for (DBuf* b : {&sv_deg, &sv_adj_off}) HIPCK(b->ensure(nn * 4));
     HIPCK(sv_adj.ensure(2 * m * 4));
-    for (DBuf* b : {&sv_ckeys, &sv_order, &sv_ckeys_alt, &sv_order_alt, &sv_mcount_ord, &sv_soff, &sv_slot_of})
-      HIPCK(b->ensure(m * 4));
+    HIPCK(sv_place.ensure(m * sizeof(uint2)));
+    HIPCK(sv_ckeys.ensure(m * 4));
+    HIPCK(sv_slot_of.ensure(m * sizeof(uint2)));
     HIPCK(sv_state2[cur].ensure(m * 4));
     HIPCK(sv_state2[cur ^ 1].ensure(4));
     HIPCK(sv_col_start.ensure(2 * (kMaxColours + 2) * 4));
+    const size_t hw = colour_hist_words(int(m), digits);
+    HIPCK(sv_hist.ensure(2 * hw * 4));
     HIPCK(sv_sinfo.ensure(m * sizeof(int4)));
-    HIPCK(sv_rec2c.ensure(c * 4));
     HIPCK(sv_rec.ensure(c * kRecFields * sizeof(float4)));
     HIPCK(sv_lam.ensure(c * sizeof(float4)));
     HIPCK(sv_prec.ensure(c * 3 * sizeof(float4)));
     HIPCK(sv_pgeo.ensure(m * 2 * sizeof(float4)));
     rec_stride = long(std::min({sv_rec.bytes / (kRecFields * sizeof(float4)), sv_lam.bytes / sizeof(float4),
                                 sv_prec.bytes / (3 * sizeof(float4))}));
-    HIPCK(sv_red.ensure((size_t(residual_blocks(M)) * 2 + 4) * sizeof(double)));  // + the joints' partial
-    HIPCK(sv_tmp.ensure(radix_temp_words(int(m)) * 4));
-    HIPCK(scan.ensure(std::max({radix_scan_tiles(int(m)), scan_tiles(m), scan_tiles(nn)}), stream));
+    const size_t need = size_t(residual_blocks(M)) * 2 + 4;  // + the joints' partial
+    if (need > red_cap) {
+      HIPCK(hipStreamSynchronize(stream));
+      if (red_host) (void)hipHostFree(red_host);
+      red_host = nullptr;
+      red_cap = 0;
+      const size_t grown = std::max<size_t>(need + need / 2, 1024);
+      HIPCK(hipHostMalloc(reinterpret_cast<void**>(&red_host), grown * sizeof(double),
+                          hipHostMallocMapped | hipHostMallocCoherent));
+      red_cap = grown;
+      HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&red_dev), red_host, 0));
+    }
+    HIPCK(scan.ensure(std::max(scan_tiles(hw), scan_tiles(nn)), stream));
     return NPHYS_OK;
   }
 
@@ -1148,28 +1156,22 @@ struct World {
     SolverBufs v;
     v.deg = sv_deg.as<uint32_t>();
     v.adj_off = sv_adj_off.as<uint32_t>();
-    v.adj_fill = sv_adj_fill.as<uint32_t>();
     v.adj = sv_adj.as<int>();
+    v.place = sv_place.as<uint2>();
     v.state = sv_state2[cur].as<uint32_t>();
-    v.remaining = bp_small.as<uint32_t>() + 32;
+    v.hist = sv_hist.as<uint32_t>();
+    v.offs = v.hist + sv_hist.bytes / 8;
     v.ckeys = sv_ckeys.as<uint32_t>();
-    v.order = sv_order.as<uint32_t>();
-    v.ckeys_alt = sv_ckeys_alt.as<uint32_t>();
-    v.order_alt = sv_order_alt.as<uint32_t>();
     v.col_start = sv_col_start.as<uint32_t>();
-    v.mcount_ord = sv_mcount_ord.as<uint32_t>();
-    v.soff = sv_soff.as<uint32_t>();
+    v.class_rec = v.col_start + (kMaxColours + 2);
     v.sinfo = sv_sinfo.as<int4>();
-    v.slot_of = sv_slot_of.as<uint32_t>();
+    v.slot_of = sv_slot_of.as<uint2>();
     v.rec_stride = rec_stride;
-    v.visit = sv_visit.as<int>();
-    v.vrange = reinterpret_cast<int2*>(sv_visit.as<int>() + (kMaxColours + 2));
-    v.rec2c = sv_rec2c.as<uint32_t>();
     v.rec = sv_rec.as<float4>();
     v.lam = sv_lam.as<float4>();
     v.prec = sv_prec.as<float4>();
     v.pgeo = sv_pgeo.as<float4>();
-    v.red = sv_red.as<double>();
+    v.red = red_dev;
     v.tmp = sv_tmp.as<uint32_t>();
     v.scan = &scan;
     return v;
@@ -1201,61 +1203,86 @@ struct World {
     std::stable_sort(perm.begin(), perm.end(), [&](int a, int b) { return size_bucket(size[a]) < size_bucket(size[b]); });
   }
 
-  int colour(const DevBodies& b, const DevContacts& c, int M, int C, SolverBufs& v) {
+  // Words of bp_small of the colouring: whether each round of a batch left a manifold uncoloured, the
+  // last round that coloured one, the number of colours.
+  static constexpr int kSmRemaining = 32, kSmLastRound = kSmRemaining + kRoundBatch, kSmColours = kSmLastRound + 1;
+
+  // Colouring, slots and assembly of the solve's manifolds, and the class bounds back on the host
+  // (colour_visit, h_range, class_rec, max_class). The rounds run in batches of four: a round after the last one that
+  // colours anything changes nothing, and the device records that last round. A batch, the colour order and the assembly
+  // are enqueued together and read back once; where manifolds stay uncoloured, or there are more than
+  // 256 colours, the rest runs again. `after` enqueues what does not depend on the colouring, before the wait.
+  template <class F>
+  int colour_and_assemble(const DevBodies& b, const DevContacts& c, int M, int C, const SimParams& ps, SolverBufs& v,
+                          F&& after) {
     // colours are inherited from the manifolds of the previous solve
     const int prevM = have_solved ? sview_M[cur ^ 1] : 0;
-    launch_colour_prepare(b, c, M, sview[cur ^ 1], prevM, sv_state2[cur ^ 1].as<uint32_t>(), v, stream);
-    // Rounds in batches of four with one poll per batch: a round after the last one that colours
-    // anything changes nothing, and the device records the last round that did.
-    // The sort keys and colour count are computed after every batch and read back with the poll,
-    // so the usual single batch costs one synchronisation; they are recomputed after a further one.
-    fill_u32(v.remaining + 1, 0u, 1, stream);
-    uint32_t* ncol = bp_small.as<uint32_t>() + 40;
-    for (int round = 1;; round += kRoundBatch) {
-      if (round + kRoundBatch >= 0xffff) return set_err(NPHYS_ERR_STATE, "colouring did not converge");
-      for (int k = 0; k < kRoundBatch; ++k) launch_colour_round(b, c, M, round + k, v, stream);
-      launch_colour_keys(M, v, ncol, stream);
-      const int rc = readback({{v.remaining, 2, 0}, {ncol, 1, 2}});
+    const ContactBufs& pc = cb[cur ^ 1];
+    uint32_t* sm = bp_small.as<uint32_t>();
+    launch_colour_begin(b, c, M, sview[cur ^ 1], prevM, sv_state2[cur ^ 1].as<uint32_t>(), v, stream);
+    int digits = 256;
+    bool rounds = true, waiting = true;
+    for (int round = 1;;) {
+      if (rounds) {
+        if (round + kRoundBatch >= 0xffff) return set_err(NPHYS_ERR_STATE, "colouring did not converge");
+        // the last round's word stays when this is not the first batch
+        fill_u32(sm + kSmRemaining, 0u, round == 1 ? kRoundBatch + 2 : kRoundBatch, stream);
+        if (round > 1) fill_u32(sm + kSmColours, 0u, 1, stream);
+        for (int k = 0; k < kRoundBatch; ++k, ++round)
+          launch_colour_round(c, M, round, sm + kSmRemaining + k, sm + kSmLastRound, v, stream);
+      }
+      launch_colour_order(c, M, C, digits, v, sm + kSmColours, stream);
+      const uint32_t seq = rb_post({{sm + kSmRemaining, kRoundBatch + 2, 0},
+                                    {v.col_start, digits + 1, kRbClass},
+                                    {v.class_rec, digits + 1, kRbClass + kMaxColours + 2}});
+      launch_assemble(b, c, pc.view(), have_solved ? pc.M : 0, M, ps, v, mat_table(), stream);
+      if (waiting) after();
+      waiting = false;
+      const int rc = rb_wait(seq);
       if (rc) return rc;
-      if (rb_host[0] == 0) break;
+      rounds = rb_host[kRoundBatch - 1] != 0;
+      ncolours = int(rb_host[kRoundBatch + 1]);
+      if (rounds) continue;
+      if (ncolours > kMaxColours) return set_err(NPHYS_ERR_STATE, "too many colours");
+      if (ncolours <= digits) break;
+      digits = kMaxColours;
+      const int rc2 = ensure_solver(M, C, digits);
+      if (rc2) return rc2;
+      v = sv_view();
     }
-    ncolours = int(rb_host[2]);
-    colour_rounds = int(rb_host[1]);
-    if (ncolours > kMaxColours) return set_err(NPHYS_ERR_STATE, "too many colours");
-    launch_colour_order(b, c, M, ncolours, v, stream);
-    uint32_t* class_rec = v.col_start + (kMaxColours + 2);
-    launch_fix_colour_starts(ncolours, M, C, v, class_rec, stream);
-    // class offsets (slots and row records) to the host, read after the assembly is enqueued
-    class_seq = rb_post({{v.col_start, ncolours + 1, kRbClass}, {class_rec, ncolours + 1, kRbClass + kMaxColours + 2}});
+    colour_rounds = int(rb_host[kRoundBatch]);
+    // visit order (the SplitMix64 Fisher-Yates shuffle seeded by the solve index), slot ranges in that
+    // order and the largest class
+    const uint32_t* h_colstart = rb_host + kRbClass;
+    const uint32_t* h_rec = h_colstart + kMaxColours + 2;
+    int csize[kMaxColours];
+    for (int k = 0; k < ncolours; ++k) csize[k] = int(h_colstart[k + 1] - h_colstart[k]);
+    colour_visit_order(uint64_t(solve_count), ncolours, csize, colour_visit);
+    max_class = 0;
+    h_range.resize(size_t(ncolours));
+    class_contacts.resize(size_t(ncolours));
+    for (int k = 0; k < ncolours; ++k) {
+      const int col = colour_visit[size_t(k)];
+      h_range[size_t(k)] = int2{int(h_colstart[col]), csize[col]};
+      class_contacts[size_t(k)] = int(h_rec[col + 1] - h_rec[col]);
+      max_class = std::max(max_class, csize[col]);
+    }
     return NPHYS_OK;
   }
 
-  // Visit order of this solve's colour classes (the SplitMix64 Fisher-Yates shuffle seeded by the
-  // solve index, computed on the host) and the largest class (sizes the sweep grids), from the
-  // class offsets read back in colour().
-  int visit_order() {
-    const int rc = rb_wait(class_seq);
-    if (rc) return rc;
-    const uint32_t* h_colstart = rb_host + kRbClass;
-    int csize[kMaxColours];
-    for (int c = 0; c < ncolours; ++c) csize[c] = int(h_colstart[c + 1] - h_colstart[c]);
-    colour_visit_order(uint64_t(solve_count), ncolours, csize, colour_visit);
-    max_class = 0;
-    int* h_range = h_visit + (kMaxColours + 2);
-    for (int k = 0; k < ncolours; ++k) {
-      const int c = colour_visit[k];
-      const int first = int(h_colstart[c]), size = int(h_colstart[c + 1] - h_colstart[c]);
-      max_class = std::max(max_class, size);
-      h_visit[k] = c;
-      h_range[2 * k] = first;
-      h_range[2 * k + 1] = size;
-    }
-    // h_visit is rewritten only by the next solve, after these copies have completed (that solve's
-    // class readback is enqueued after them in stream order)
-    HIPCK(hipMemcpyAsync(sv_visit.p, h_visit, size_t(ncolours) * sizeof(int), hipMemcpyHostToDevice, stream));
-    HIPCK(hipMemcpyAsync(sv_visit.as<int>() + (kMaxColours + 2), h_range, size_t(ncolours) * 2 * sizeof(int),
-                         hipMemcpyHostToDevice, stream));
-    return NPHYS_OK;
+  // The run of small classes that starts with the k-th visited one (at most kRunClasses of them).
+  ClassRun small_run(int k, int ncol) const {
+    ClassRun run;
+    run.n = 0;
+    for (; k < ncol && run.n < kRunClasses && h_range[size_t(k)].y <= kRunBlock; ++k) run.r[run.n++] = h_range[size_t(k)];
+    return run;
+  }
+
+  VisitOrder visit_list() const {
+    VisitOrder v;
+    v.n = ncolours;
+    for (int k = 0; k < ncolours; ++k) v.c[k] = uint16_t(colour_visit[size_t(k)]);
+    return v;
   }
 
   // Warm start (when `warm`) and `nsweeps` coloured SOR-Prox sweeps. With counters enabled the
@@ -1275,7 +1302,7 @@ struct World {
       }
       HIPCK(hipEventRecord(fork_ev, stream));
       HIPCK(hipStreamWaitEvent(stream_large, fork_ev, 0));
-      launch_sweeps_blocked(b, v, sc, ncolours, nsweeps, warm, cur_variant, stream, stream_large);
+      launch_sweeps_blocked(b, v, sc, visit_list(), nsweeps, warm, cur_variant, stream, stream_large);
       HIPCK(hipEventRecord(join_ev, stream_large));
       HIPCK(hipStreamWaitEvent(stream, join_ev, 0));
       if (counters_enabled) {
@@ -1295,32 +1322,28 @@ struct World {
         kt_ev.push_back(e);
       }
     }
-    const int* h_range = h_visit + (kMaxColours + 2);
-    const uint32_t* class_rec = rb_host + kRbClass + kMaxColours + 2;
     auto pass = [&](bool w) {
       for (int k = 0; k < ncolours;) {
-        int e = k;
-        while (e < ncolours && h_range[2 * e + 1] <= kRunBlock) ++e;
-        if (e - k >= 2) {
-          launch_colour_run(b, v, k, e - k, w, stream);
-          k = e;
+        const ClassRun run = small_run(k, ncolours);
+        if (run.n >= 2) {
+          launch_colour_run(b, v, run, w, stream);
+          k += run.n;
           continue;
         }
         // one 64-lane workgroup per 64 manifolds of this class (the grid-stride loop covers the
         // rest above the cap): no idle workgroups for the smaller classes
-        const int cblocks = std::min(sblocks, std::max(1, (h_range[2 * k + 1] + 63) / 64));
+        const int2 r = h_range[size_t(k)];
+        const int cblocks = std::min(sblocks, std::max(1, (r.y + 63) / 64));
         // the sweep kernel runs two lanes per manifold
-        const int pblocks2 = std::min(2 * sblocks, std::max(1, (2 * h_range[2 * k + 1] + 63) / 64));
+        const int pblocks2 = std::min(2 * sblocks, std::max(1, (2 * r.y + 63) / 64));
         if (w) {
-          launch_warmstart_colour(b, cv, h_range[2 * k], h_range[2 * k + 1], cblocks, v, stream);
+          launch_warmstart_colour(b, cv, r.x, r.y, cblocks, v, stream);
         } else if (counters_enabled) {
-          launch_pgs_colour(b, cv, h_range[2 * k], h_range[2 * k + 1], pblocks2, v, stream, kt_ev[kt_used],
-                            kt_ev[kt_used + 1]);
+          launch_pgs_colour(b, cv, r.x, r.y, pblocks2, v, stream, kt_ev[kt_used], kt_ev[kt_used + 1]);
           kt_used += 2;
-          const int c = h_visit[k];
-          counters.sweep_kernel_contacts += int64_t(class_rec[c + 1]) - int64_t(class_rec[c]);
+          counters.sweep_kernel_contacts += class_contacts[size_t(k)];
         } else {
-          launch_pgs_colour(b, cv, h_range[2 * k], h_range[2 * k + 1], pblocks2, v, stream);
+          launch_pgs_colour(b, cv, r.x, r.y, pblocks2, v, stream);
         }
         ++k;
       }
@@ -1340,41 +1363,30 @@ struct World {
     return NPHYS_OK;
   }
 
-  // Residual of the fixed-count mode: the partials are copied into pinned memory without waiting
-  // and reduced after the step's final synchronisation (finish_residual), since nothing in the step
-  // needs them.
-  int residual_deferred(const DevBodies& b, const DevContacts& cv, int M, int C, SolverBufs& v) {
-    launch_residual(b, cv, M, v, stream);
+  // Natural-map residual of the current impulses: the per-block partials go straight to host memory and
+  // are reduced there in block order (max is exact; the sum of squares is the RMS) once the stream
+  // has passed them: residual() waits, while the fixed-count mode's, which nothing in the step
+  // needs, is reduced after the step's last readback (with `cache` the kernel stores the impulses too).
+  void residual_deferred(const DevBodies& b, const DevContacts& cv, int M, int C, bool cache, SolverBufs& v) {
+    launch_residual(b, cv, M, cache, v, stream);
     const int nbk = residual_blocks(M);
     JointBufs jv = joint_view();
     if (nj > 0) launch_joint_residual(b, jv, v.red + 2 * nbk, stream);
-    const size_t need = size_t(nbk) * 2 + (nj > 0 ? 3 : 0);
-    if (need > red_pinned_cap) {
-      HIPCK(hipStreamSynchronize(stream));  // the previous buffer may be the target of a copy
-      if (red_pinned) (void)hipHostFree(red_pinned);
-      red_pinned = nullptr;
-      red_pinned_cap = 0;
-      HIPCK(hipHostMalloc(reinterpret_cast<void**>(&red_pinned), std::max<size_t>(need, 1024) * sizeof(double)));
-      red_pinned_cap = std::max<size_t>(need, 1024);
-    }
-    HIPCK(hipMemcpyAsync(red_pinned, v.red, need * sizeof(double), hipMemcpyDeviceToHost, stream));
     res_pending_blocks = nbk;
     res_pending_C = C;
     res_pending_joints = nj > 0;
-    return NPHYS_OK;
   }
   bool res_pending_joints = false;
 
-  // Reduces a deferred residual; the stream must have passed its copy.
   void finish_residual() {
     if (res_pending_blocks < 0) return;
     double mx = 0.0, ss = 0.0, rows = double(3 * res_pending_C);
     for (int k = 0; k < res_pending_blocks; ++k) {
-      mx = std::max(mx, red_pinned[2 * k]);
-      ss += red_pinned[2 * k + 1];
+      mx = std::max(mx, red_host[2 * k]);
+      ss += red_host[2 * k + 1];
     }
     if (res_pending_joints) {  // the joint rows' partial after the contacts' blocks
-      const double* jp = red_pinned + 2 * res_pending_blocks;
+      const double* jp = red_host + 2 * res_pending_blocks;
       mx = std::max(mx, jp[0]);
       ss += jp[1];
       rows += jp[2];
@@ -1384,39 +1396,20 @@ struct World {
     res_pending_blocks = -1;
   }
 
-  // Natural-map residual of the current impulses: per-block partials reduced on the host in
-  // block order (max is exact; the sum of squares is the RMS).
   int residual(const DevBodies& b, const DevContacts& cv, int M, int C, SolverBufs& v) {
-    launch_residual(b, cv, M, v, stream);
-    const int nbk = residual_blocks(M);
-    JointBufs jv = joint_view();
-    if (nj > 0) launch_joint_residual(b, jv, v.red + 2 * nbk, stream);
-    red_host.resize(size_t(nbk) * 2 + 3);
-    HIPCK(hipMemcpyAsync(red_host.data(), v.red, (size_t(nbk) * 2 + (nj > 0 ? 3 : 0)) * sizeof(double),
-                         hipMemcpyDeviceToHost, stream));
-    HIPCK(hipStreamSynchronize(stream));
-    double mx = 0.0, ss = 0.0, rows = double(3 * C);
-    for (int k = 0; k < nbk; ++k) {
-      mx = std::max(mx, red_host[2 * k]);
-      ss += red_host[2 * k + 1];
-    }
-    if (nj > 0) {
-      mx = std::max(mx, red_host[2 * nbk]);
-      ss += red_host[2 * nbk + 1];
-      rows += red_host[2 * nbk + 2];
-    }
-    res_inf = mx;
-    res_rms = rows > 0.0 ? std::sqrt(ss / rows) : 0.0;
-    return NPHYS_OK;
+    residual_deferred(b, cv, M, C, false, v);
+    const int rc = readback({});
+    finish_residual();
+    return rc;
   }
 
   SceneBlocks sc_view() {
     SceneBlocks v;
     v.keys = sc_keys.as<uint32_t>();
-    v.slot = sc_slot.as<uint32_t>();
+    v.slot = nscenes > 1 ? sc_slot.as<uint32_t>() : nullptr;
     v.keys_alt = sc_keys_alt.as<uint32_t>();
     v.slot_alt = sc_slot_alt.as<uint32_t>();
-    v.start = sc_start.as<uint32_t>();
+    v.start = nscenes > 1 ? sc_start.as<uint32_t>() : sv_col_start.as<uint32_t>();
     v.dyn_start = sc_dyn_start.as<int>();
     v.dyn_list = sc_dyn_list.as<int>();
     v.local = sc_local.as<int>();
@@ -1428,7 +1421,7 @@ struct World {
   }
 
   bool blocked_eligible(int ncol) const {
-    return max_scene_dyn <= kLdsBodies && int64_t(nscenes) * (ncol + 1) <= (int64_t(1) << 24);
+    return max_scene_dyn <= kLdsBodies && ncol <= kVisitColours && int64_t(nscenes) * (ncol + 1) <= (int64_t(1) << 24);
   }
 
   // Variant of this solve's sweeps: forced, or the autotuner's pick, or (while tuning) the next
@@ -1493,7 +1486,8 @@ struct World {
     if (res_target <= 0.0) {
       if ((rc = sweeps(b, cv, v, sblocks, true, prm.max_velocity_iterations))) return rc;
       nsw = prm.max_velocity_iterations;
-      return residual_deferred(b, cv, M, C, v);
+      residual_deferred(b, cv, M, C, true, v);
+      return NPHYS_OK;
     }
     if ((rc = sweeps(b, cv, v, sblocks, true, 0))) return rc;
     int done = 0;
@@ -1603,29 +1597,33 @@ struct World {
     int rc = ensure_solver(M, C);
     if (rc) return rc;
     SolverBufs v = sv_view();
-    if (M > 0) {
-      if ((rc = colour(b, cv, M, C, v))) return rc;
-      launch_assemble(b, cv, pc.view(), prevM, M, sp, v, mat_table(), stream);
-    }
     // the joints' rows (moreau_jean_solver.rs:211-223); the island joints are those neither broken
     // nor removed with an awake dynamic body, decided on the device
     JointBufs jv = joint_view();
-    if (nj > 0) launch_joint_assemble(b, sp, jv, stream);
+    auto joint_rows = [&] {
+      if (nj > 0) launch_joint_assemble(b, sp, jv, stream);
+    };
+    if (M > 0) {
+      if ((rc = colour_and_assemble(b, cv, M, C, sp, v, joint_rows))) return rc;
+    } else {
+      joint_rows();
+    }
     HIPCK(hipEventRecord(ev[EV_ASM], stream));
-    // class sizes (read back while the assembly runs) give the visit order and the sweep grids
-    if (M > 0 && (rc = visit_order())) return rc;
     const int sblocks = sweep_blocks(max_class);
     kt_used = 0;
     choose_variant(M);
     if (tune_pending) HIPCK(hipEventRecord(tune_ev[0], stream));
-    if (cur_variant > 0) {
+    if (cur_variant > 0 && nscenes > 1) {
       HIPCK(sc_keys.ensure(size_t(M) * 4));
       HIPCK(sc_slot.ensure(size_t(M) * 4));
       HIPCK(sc_keys_alt.ensure(size_t(M) * 4));
       HIPCK(sc_slot_alt.ensure(size_t(M) * 4));
       HIPCK(sc_start.ensure(size_t(nscenes) * size_t(ncolours + 1) * 4));
+      HIPCK(sv_tmp.ensure(radix_temp_words(M) * 4));
+      HIPCK(scan.ensure(radix_scan_tiles(M), stream));
+      v.tmp = sv_tmp.as<uint32_t>();
       SceneBlocks sc = sc_view();
-      launch_scene_order(b, M, nscenes, ncolours, v, sc, stream);
+      launch_scene_order(b, M, nscenes, scene_bits, ncolours, v, sc, stream);
     }
     const bool learned = contact_model == NPHYS_CONTACT_MODEL_LEARNED_WARMSTART && C > 0;
     if ((learned || capture) && C > 0) {
@@ -1685,7 +1683,7 @@ struct World {
       samples = C;
     }
     counters.velocity_sweeps += last_sweeps;
-    if (C > 0) launch_cache_impulses(cv, v, C, stream);
+    if (res_target > 0.0) launch_cache_impulses(cv, v, M, stream);  // else with the residual
     if (nj > 0) launch_joint_cache(b, sp, jv, stream);
     HIPCK(hipEventRecord(ev[EV_VEL], stream));
     if (keep_colours && M > 0) {
@@ -1710,7 +1708,7 @@ struct World {
       SceneBlocks sc = sc_view();
       HIPCK(hipEventRecord(fork_ev, stream));
       HIPCK(hipStreamWaitEvent(stream_large, fork_ev, 0));
-      launch_position_blocked(b, ps, v, sc, ncolours, iterations, cur_variant, stream, stream_large);
+      launch_position_blocked(b, ps, v, sc, visit_list(), iterations, cur_variant, stream, stream_large);
       HIPCK(hipEventRecord(join_ev, stream_large));
       HIPCK(hipStreamWaitEvent(stream, join_ev, 0));
       return NPHYS_OK;
@@ -1718,20 +1716,18 @@ struct World {
     const int pblocks = position_blocks(max_class);
     // direct launches, runs of two or more consecutive small classes in one workgroup (as the
     // sweeps); the joints' constraints first in every iteration (nonlinear_sor_prox.rs:33-38)
-    const int* h_range = h_visit + (kMaxColours + 2);
     const int ncol = sview_M[cur] > 0 ? ncolours : 0;
     for (int it = 0; it < iterations; ++it) {
       if (joints) launch_joint_position(b, ps, jv, stream);
       for (int k = 0; k < ncol;) {
-        int e = k;
-        while (e < ncolours && h_range[2 * e + 1] <= kRunBlock) ++e;
-        if (e - k >= 2) {
-          launch_position_run(b, ps, v, k, e - k, stream);
-          k = e;
+        const ClassRun run = small_run(k, ncol);
+        if (run.n >= 2) {
+          launch_position_run(b, ps, v, run, stream);
+          k += run.n;
           continue;
         }
-        launch_position_colour(b, cv, ps, h_range[2 * k], h_range[2 * k + 1],
-                               std::min(pblocks, std::max(1, (h_range[2 * k + 1] + 63) / 64)), v, stream);
+        const int2 r = h_range[size_t(k)];
+        launch_position_colour(b, cv, ps, r.x, r.y, std::min(pblocks, std::max(1, (r.y + 63) / 64)), v, stream);
         ++k;
       }
     }
@@ -1876,10 +1872,7 @@ struct World {
     if (M > 0) {
       if ((rc = ensure_solver(M, C))) return rc;
       v = sv_view();
-      if ((rc = colour(b, cv, M, C, v))) return rc;
-      const ContactBufs& pc = cb[cur ^ 1];
-      launch_assemble(b, cv, pc.view(), have_solved ? pc.M : 0, M, ss, v, mat_table(), stream);
-      if ((rc = visit_order())) return rc;
+      if ((rc = colour_and_assemble(b, cv, M, C, ss, v, [] {}))) return rc;
       sview[cur] = cv;
       sview_M[cur] = M;
       sview_C[cur] = C;

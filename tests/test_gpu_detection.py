@@ -122,3 +122,19 @@ def test_search_by_boxes(nphys, oracle_mod, n, nscenes, groups):
         g.step(1)
         o.step(1)
         _same(g, o, f"{n} bodies, step {k + 1}")
+
+
+@pytest.mark.parametrize("n", [40, 257, 300])
+def test_crowd_steps(nphys, oracle_mod, n):
+    """Steps of a crowd whose bodies all touch each other: n - 1 manifolds per body, so at least as many
+    colours, below and above the 256 that the colour order is built for at first, and classes of a few manifolds."""
+    s = _shuffled(n, n, statics=0.0)
+    s["pos"][:] = np.random.default_rng(n).uniform(-0.02, 0.02, (n, 3))
+    g, o = _worlds(nphys, oracle_mod, s)
+    for k in range(2):
+        g.step(1)
+        o.step(1)
+        gs, os_ = g.get_state(), o.get_state()
+        for key in ("pos", "rot", "linvel", "angvel"):
+            np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
+    assert g.counters()["ncolours"] >= (n - 1 if n < 257 else 257)
