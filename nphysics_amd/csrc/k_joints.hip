@@ -38,7 +38,7 @@ namespace nph {
 
 namespace {
 
-constexpr int kJointBlock = 256;
+constexpr int kJointBlock = 512;
 
 struct JBody {
   f3 com, v, w, el, ea;
@@ -306,8 +306,9 @@ __device__ __forceinline__ void joint_warm_one(const DevBodies& b, const JointBu
   JointCtx c;
   load_ctx(b, j, s, c);
   if (!c.active) return;
-  for (int k = 0; k < c.nrows; ++k)
-    if (c.lam[k] != 0.0f) jrow_add(c, jrow(c, k), c.lam[k]);
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+    if (k < c.nrows && c.lam[k] != 0.0f) jrow_add(c, jrow(c, k), c.lam[k]);
   store_ctx(b, j, s, c, false);
 }
 
@@ -316,7 +317,9 @@ __device__ __forceinline__ void joint_sweep_one(const DevBodies& b, const JointB
   JointCtx c;
   load_ctx(b, j, s, c);
   if (!c.active) return;
-  for (int k = 0; k < c.nrows; ++k) {
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {  // unrolled: an index known late would put the rows in scratch memory
+    if (k >= c.nrows) break;
     const JRow v = jrow(c, k);
     const float w = (jdot6(v.d1, v.a1, c.x1l, c.x1a) + jdot6(v.d2, v.a2, c.x2l, c.x2a)) + c.rhs[k];
     const float lo = -FLT_MAX, hi = FLT_MAX;
