@@ -20,20 +20,20 @@
 // of the contact with the same (body1, body2, feature) key (the ImpulseCache lookup at
 // signorini_coulomb_pyramid_model.rs:104-108).
 //
-// Solve (k_warmstart / k_pgs, all of the manifold's data loaded into registers before its serial
-// chain) restates SORProx (src/solver/sor_prox.rs:19-436): warm start dv += l W J, then per sweep
-// and contact the normal row (projected on l >= 0) and the two friction rows (bounded by mu times
-// the normal impulse just computed, zeroed when it is zero). Manifolds of one colour share no
+// Solve (k_warmstart / k_pgs) restates SORProx (src/solver/sor_prox.rs:19-436): warm start dv += l W J,
+// then per sweep and contact the normal row (projected on l >= 0) and the two friction rows (bounded by
+// mu times the normal impulse just computed, zeroed when it is zero). Manifolds of one colour share no
 // dynamic body, so one launch per colour performs exactly the sequential Gauss-Seidel updates of
-// the colour order. k_pgs gives each manifold two lanes, one per body: each lane forms its body's
-// half of a row's J dv and its body's dv update, and the halves meet by a lane exchange, so the
-// serial chain per row is half as long and twice as many lanes are in flight.
+// the colour order. Every manifold has two adjacent lanes, one per body (PairHalf): a lane loads its
+// body's inverse inertia and velocity increment and every contact up front, forms its body's half of
+// a row's J dv and its body's update, and the halves meet by a register exchange within the quad.
 //
-// Row record (4 contiguous float4 per contact, colour order): 0 n|mu, 1 lever arm p1 of body 1
-// (contact point minus centre of mass, zero for a static body)|r_n, 2 p2|r_t1,
+// Row record (4 contiguous float4 per contact, colour order): 0 n|length of the tangents' seed, 1 lever arm
+// p1 of body 1 (contact point minus centre of mass, zero for a static body)|r_n, 2 p2|r_t1,
 // 3 rhs (n, t1, t2)|r_t2. The impulses live in their own array, one float4 per record (n, t1, t2
-// | 1 if the warm start came from the cache, else 0), so a sweep's impulse writes are contiguous
-// 16-byte runs rather than one dirty line per contact.
+// | mu), so a sweep's impulse writes are contiguous 16-byte runs rather than one dirty line per
+// contact. What the sweeps spend their time on is instructions, one wave per SIMD or two: the seed's
+// length saves them a square root and (a quotient per lane) two of three divisions per contact.
 // Linear jacobians are the row direction d (body 1) and -d (body 2) weighted by the inverse
 // mass; the tangents, the angular jacobians p1 x d and p2 x (-d) and I^-1 J_ang are recomputed
 // in the sweep kernels with the assembly's own expressions, so they carry the same FP32 values.
@@ -303,9 +303,13 @@ __device__ __forceinline__ BodyView load_body(const DevBodies& b, int i) {
   return v;
 }
 
-__device__ __forceinline__ void tangents(f3 n, f3& t1, f3& t2) {
-  f3 a = fabsf(n.x) > fabsf(n.y) ? f3{n.z, 0.0f, -n.x} : f3{0.0f, -n.z, n.y};
-  const float l = sqrtf(dot(a, a));
+// The tangents' seed: a vector orthogonal to n with one zero component, of length l.
+__device__ __forceinline__ f3 tangent_seed(f3 n) {
+  return fabsf(n.x) > fabsf(n.y) ? f3{n.z, 0.0f, -n.x} : f3{0.0f, -n.z, n.y};
+}
+
+__device__ __forceinline__ void tangents(f3 n, float l, f3& t1, f3& t2) {
+  f3 a = tangent_seed(n);
   a = f3{a.x / l, a.y / l, a.z / l};
   t1 = cross(a, n);
   t2 = a;
@@ -390,8 +394,10 @@ __global__ void __launch_bounds__(256) k_assemble(DevBodies b, DevContacts cur, 
       }
     const f3 center1 = add(w1, scale(n, m1));
     const f3 center2 = sub(w2, scale(n, m2));
+    const f3 seed = tangent_seed(n);
+    const float tl = sqrtf(dot(seed, seed));
     f3 t1, t2;
-    tangents(n, t1, t2);
+    tangents(n, tl, t1, t2);
     float rr3[3], rhs3[3];
     float lam[3];
 #pragma unroll
@@ -420,11 +426,12 @@ __global__ void __launch_bounds__(256) k_assemble(DevBodies b, DevContacts cur, 
     lam[1] = imp.y * p.warmstart_coeff;
     lam[2] = imp.z * p.warmstart_coeff;
     float4* R = sb.rec + long(r) * kRecFields;
-    R[0] = f4(n, mu);
+    R[0] = f4(n, tl);
     R[1] = f4(p1, rr3[0]);
     R[2] = f4(p2, rr3[1]);
     R[3] = make_float4(rhs3[0], rhs3[1], rhs3[2], rr3[2]);
-    sb.lam[r] = make_float4(lam[0], lam[1], lam[2], has);
+    sb.lam[r] = make_float4(lam[0], lam[1], lam[2], mu);
+    if (sb.has) sb.has[r] = has;
   }
 }
 
@@ -478,7 +485,7 @@ __device__ __forceinline__ SlotCtx slot_ctx(const SolverBufs& sb, int s) {
 // (tangents(n) and mulv(I^-1, J_ang)), so they carry the same FP32 values.
 struct CRec {
   f3 n;
-  float mu;
+  float tl, mu;
   f3 p1, p2;  // lever arms (zero for a static body)
   float r[3], rhs[3];
   float4 lam;
@@ -492,7 +499,7 @@ __device__ __forceinline__ void load_rec(const SolverBufs& sb, uint32_t r, CRec&
   const float4* p = sb.rec + long(r) * kRecFields;
   const float4 v0 = p[0], v1 = p[1], v2 = p[2], v3 = p[3];
   c.n = xyz(v0);
-  c.mu = v0.w;
+  c.tl = v0.w;
   c.p1 = xyz(v1);
   c.p2 = xyz(v2);
   c.r[0] = v1.w;
@@ -502,6 +509,7 @@ __device__ __forceinline__ void load_rec(const SolverBufs& sb, uint32_t r, CRec&
   c.rhs[1] = v3.y;
   c.rhs[2] = v3.z;
   c.lam = sb.lam[r];
+  c.mu = c.lam.w;
 }
 
 struct Inv {
@@ -555,7 +563,7 @@ __device__ __forceinline__ void load_manifold(const DevBodies& b, const SolverBu
   for (int k = 0; k < 4; ++k)
     if (k < m.x.cnt) {
       load_rec(sb, m.x.r0 + k, m.c[k]);
-      tangents(m.c[k].n, m.t1[k], m.t2[k]);
+      tangents(m.c[k].n, m.c[k].tl, m.t1[k], m.t2[k]);
     }
 }
 
@@ -602,21 +610,11 @@ __device__ __forceinline__ void load_dv(const DevBodies& b, const Manifold<kMask
   if (m.x.d2) b.load_dv(m.x.b2, v2.l, v2.a);
 }
 
-template <bool kMask>
-__device__ __forceinline__ void store_dv(const DevBodies& b, const Manifold<kMask>& m, const Dv& v1, const Dv& v2) {
-  if (m.x.d1) b.store_dv(m.x.b1, v1.l, v1.a);
-  if (m.x.d2) b.store_dv(m.x.b2, v2.l, v2.a);
-}
-
-// Solver velocity increments of the manifold's bodies in HBM (the per-colour kernels) ...
+// Solver velocity increments in HBM (the per-colour kernels) ...
 struct GlobalDv {
   DevBodies b;
-  template <bool kMask>
-  __device__ void load(const Manifold<kMask>& m, Dv& v1, Dv& v2) const { load_dv(b, m, v1, v2); }
-  template <bool kMask>
-  __device__ void store(const Manifold<kMask>& m, const Dv& v1, const Dv& v2) const { store_dv(b, m, v1, v2); }
-  __device__ void load1(int body, Dv& v) const { b.load_dv(body, v.l, v.a); }
-  __device__ void store1(int body, const Dv& v) const { b.store_dv(body, v.l, v.a); }
+  __device__ void load(int body, Dv& v) const { b.load_dv(body, v.l, v.a); }
+  __device__ void store(int body, const Dv& v) const { b.store_dv(body, v.l, v.a); }
 };
 
 // ... or in LDS, indexed by the body's rank among its scene's dynamic bodies (the scene-blocked
@@ -625,135 +623,30 @@ struct LdsDv {
   float4* lin;
   float4* ang;
   const int* local;
-  template <bool kMask>
-  __device__ void load(const Manifold<kMask>& m, Dv& v1, Dv& v2) const {
-    if (m.x.d1) {
-      const int i = local[m.x.b1];
-      v1.l = xyz(lin[i]);
-      v1.a = xyz(ang[i]);
-    }
-    if (m.x.d2) {
-      const int i = local[m.x.b2];
-      v2.l = xyz(lin[i]);
-      v2.a = xyz(ang[i]);
-    }
-  }
-  template <bool kMask>
-  __device__ void store(const Manifold<kMask>& m, const Dv& v1, const Dv& v2) const {
-    if (m.x.d1) {
-      const int i = local[m.x.b1];
-      lin[i] = f4(v1.l, 0.0f);
-      ang[i] = f4(v1.a, 0.0f);
-    }
-    if (m.x.d2) {
-      const int i = local[m.x.b2];
-      lin[i] = f4(v2.l, 0.0f);
-      ang[i] = f4(v2.a, 0.0f);
-    }
-  }
-  __device__ void load1(int body, Dv& v) const {
+  __device__ void load(int body, Dv& v) const {
     const int i = local[body];
     v.l = xyz(lin[i]);
     v.a = xyz(ang[i]);
   }
-  __device__ void store1(int body, const Dv& v) const {
+  __device__ void store(int body, const Dv& v) const {
     const int i = local[body];
     lin[i] = f4(v.l, 0.0f);
     ang[i] = f4(v.a, 0.0f);
   }
 };
 
-// Warm start of one manifold (SORProx::warmstart_set, sor_prox.rs:19-45): dv += l W J for every
-// row with l != 0, normal rows first, then friction rows.
-template <bool kMask, class A>
-__device__ __forceinline__ void warm_manifold(const A& acc, const DevBodies& b, const SolverBufs& sb, int slot) {
-  Manifold<kMask> m;
-  load_manifold(b, sb, slot, m);
-  Dv v1{}, v2{};
-  acc.load(m, v1, v2);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= m.x.cnt) break;
-    if (m.c[k].lam.x != 0.0f) row_add(row_of(m, k, 0), m.c[k].lam.x, m, v1, v2);
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= m.x.cnt) break;
-    if (m.c[k].lam.y != 0.0f) row_add(row_of(m, k, 1), m.c[k].lam.y, m, v1, v2);
-    if (m.c[k].lam.z != 0.0f) row_add(row_of(m, k, 2), m.c[k].lam.z, m, v1, v2);
-  }
-  acc.store(m, v1, v2);
+// The value of the other lane of the pair: a quad permutation (1, 0, 3, 2), one instruction, where a
+// shuffle goes through the LDS crossbar and stands in every row's serial chain. Both lanes of a pair
+// are always active together: they take the same branches, on the same values.
+__device__ __forceinline__ float pair_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));
 }
 
-// One SOR-Prox step of one manifold (sor_prox.rs:159-343), contact by contact: the normal row,
-// projected on l >= 0, then the two friction rows, bounded by mu times that normal impulse and
-// zeroed when it is zero.
-template <bool kMask, class A>
-__device__ __forceinline__ void pgs_manifold(const A& acc, const DevBodies& b, const SolverBufs& sb, int slot) {
-  Manifold<kMask> m;
-  load_manifold(b, sb, slot, m);
-  Dv v1{}, v2{};
-  acc.load(m, v1, v2);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= m.x.cnt) break;
-    {
-      const Row v = row_of(m, k, 0);
-      const float w = row_w(v, v1, v2);
-      const float a = m.c[k].lam.x - v.r * w;
-      const float ni = a > 0.0f ? a : 0.0f;
-      const float dl = ni - m.c[k].lam.x;
-      m.c[k].lam.x = ni;
-      row_add(v, dl, m, v1, v2);
-    }
-    const float mu = m.c[k].mu;
-    const float ln = m.c[k].lam.x;
-#pragma unroll
-    for (int f = 1; f <= 2; ++f) {
-      float li = f == 1 ? m.c[k].lam.y : m.c[k].lam.z;
-      const Row v = row_of(m, k, f);
-      if (ln == 0.0f) {
-        if (li != 0.0f) {
-          row_add(v, -li, m, v1, v2);
-          li = 0.0f;
-        }
-      } else {
-        const float mx = mu * ln;
-        const float mn = -mx;
-        const float w = row_w(v, v1, v2);
-        const float val = li - v.r * w;
-        const float ni = val > mn ? (val < mx ? val : mx) : mn;
-        const float dl = ni - li;
-        li = ni;
-        row_add(v, dl, m, v1, v2);
-      }
-      if (f == 1) m.c[k].lam.y = li;
-      else m.c[k].lam.z = li;
-    }
-  }
-  acc.store(m, v1, v2);
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    if (k < m.x.cnt) sb.lam[m.x.r0 + k] = m.c[k].lam;
-}
-
-// One colour of the warm start / of one sweep: one lane per manifold of the colour visited kv-th.
-template <bool kMask>
-__global__ void __launch_bounds__(64) k_warmstart(DevBodies b, DevContacts c, SolverBufs sb, int first, int n) {
-  const GlobalDv acc{b};
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x)
-    warm_manifold<kMask>(acc, b, sb, first + t);
-}
-
-// One SOR-Prox step of one manifold on two lanes (lane h = 0 body 1, h = 1 body 2), the same
-// arithmetic as pgs_manifold: each lane evaluates its body's dot6 of the row, the two partial sums
-// are exchanged between the lanes (adjacent lanes of one wavefront), both lanes form
-// w = (s1 + s2) + rhs in that order and the same new impulse, and each lane updates its own body.
-// A contact's row data as one lane of the pair needs it: the normal, mu, its body's lever arm,
-// the three r and rhs, the impulses.
+// A contact as one lane of the pair needs it: the normal, the seed's length, its body's lever arm,
+// the three r and rhs, the impulses and mu.
 struct CHalf {
   f3 n, p;
-  float mu;
+  float tl;
   float r[3], rhs[3];
   float4 lam;
 };
@@ -762,7 +655,7 @@ __device__ __forceinline__ void load_half(const SolverBufs& sb, uint32_t r, int 
   const float4* q = sb.rec + long(r) * kRecFields;
   const float4 v0 = q[0], v1 = q[1], v2 = q[2], v3 = q[3];
   c.n = xyz(v0);
-  c.mu = v0.w;
+  c.tl = v0.w;
   c.p = h ? xyz(v2) : xyz(v1);
   c.r[0] = v1.w;
   c.r[1] = v2.w;
@@ -773,112 +666,195 @@ __device__ __forceinline__ void load_half(const SolverBufs& sb, uint32_t r, int 
   c.lam = sb.lam[r];
 }
 
-// One SOR-Prox step of one manifold on two lanes (lane h = 0 body 1, h = 1 body 2), the same
-// arithmetic as pgs_manifold: each lane evaluates its body's dot6 of the row, the two partial sums
-// are exchanged between the lanes (adjacent lanes of one wavefront), both lanes form
-// w = (s1 + s2) + rhs in that order and the same new impulse, and each lane updates its own body.
-template <bool kMask, class A>
-__device__ __forceinline__ void pgs_manifold_pair(const A& acc, const DevBodies& b, const SolverBufs& sb, int slot,
-                                                  int h) {
-  const SlotCtx x = slot_ctx(sb, slot);
-  const int body = h ? x.b2 : x.b1;
-  const bool dyn = h ? x.d2 : x.d1;
-  float im = 0.0f;
-  m33 I{};
-  if (dyn) I = load_inv(b, body, im);
-  f3 ml{1.0f, 1.0f, 1.0f}, ma{1.0f, 1.0f, 1.0f};
-  if (kMask) b.mask(body, ml, ma);
-  Dv v{};
-  if (dyn) acc.load1(body, v);
+// One lane's half of a manifold: its body's inverse mass and inertia (zero for a static body), its
+// jacobian masks, the contacts. Body 2's jacobians are those of body 1's direction negated, so its
+// lane keeps the velocity increment negated instead and both lanes run the same expressions on d:
+// (-d).v = d.(-v) and -(v + a (-w)) = -v + a w, the same roundings (up to the sign of a zero).
+template <bool kMask>
+struct PairHalf {
+  int body, cnt, h;
+  bool dyn;
+  uint32_t r0;
+  float im;
+  m33 I;
+  f3 ml, ma;
   CHalf c[4];
+};
+
+template <bool kMask>
+__device__ __forceinline__ void load_pair(const DevBodies& b, const SolverBufs& sb, const int4& q, int h,
+                                          PairHalf<kMask>& m) {
+  const int w = h ? q.y : q.x;
+  m.h = h;
+  m.body = w & 0x3fffffff;
+  m.dyn = (w >> 30) & 1;
+  m.r0 = uint32_t(q.z);
+  m.cnt = q.w & 7;
+  m.im = 0.0f;
+  m.I = m33{};
+  if (m.dyn) m.I = load_inv(b, m.body, m.im);
+  if (kMask) b.mask(m.body, m.ml, m.ma);
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    if (k < x.cnt) load_half(sb, x.r0 + k, h, c[k]);
-  // body 1 takes d and p1 x d, body 2 -d and p2 x -d (ang1 / ang2), each masked
-  auto half = [&](f3 p, f3 d, f3& d_h, f3& a_h, f3& wa_h) {
-    const f3 dd = h ? neg(d) : d;
-    const f3 a = cross(p, dd);
-    d_h = kMask ? cmul(dd, ml) : dd;
-    a_h = kMask ? cmul(a, ma) : a;
-    wa_h = mulv(I, a_h);
-  };
-  auto w_of = [&](const f3& d_h, const f3& a_h, float rhs) {
-    const float s_h = dot6(d_h, a_h, v);
-    const float s_o = __shfl_xor(s_h, 1);
-    const float s1 = h == 0 ? s_h : s_o;
-    const float s2 = h == 0 ? s_o : s_h;
-    return (s1 + s2) + rhs;
-  };
+    if (k < m.cnt) load_half(sb, m.r0 + k, h, m.c[k]);
+}
+
+__device__ __forceinline__ void flip(Dv& v) {
+  v.l = neg(v.l);
+  v.a = neg(v.a);
+}
+
+template <bool kMask, class A>
+__device__ __forceinline__ void load_pair_dv(const A& acc, const PairHalf<kMask>& m, Dv& v) {
+  if (!m.dyn) return;
+  acc.load(m.body, v);
+  if (m.h) flip(v);
+}
+
+template <bool kMask, class A>
+__device__ __forceinline__ void store_pair_dv(const A& acc, const PairHalf<kMask>& m, Dv& v) {
+  if (!m.dyn) return;
+  if (m.h) flip(v);
+  acc.store(m.body, v);
+}
+
+// The lane's half of the row along d: the jacobian (masked) and its weighted angular part.
+template <bool kMask>
+__device__ __forceinline__ void half_row(const PairHalf<kMask>& m, f3 p, f3 d, f3& dh, f3& ah, f3& wah) {
+  const f3 a = cross(p, d);
+  dh = kMask ? cmul(d, m.ml) : d;
+  ah = kMask ? cmul(a, m.ma) : a;
+  wah = mulv(m.I, ah);
+}
+
+// The tangents of contact c, the seed's quotients one per lane.
+__device__ __forceinline__ void pair_tangents(const CHalf& c, int h, f3& t1, f3& t2) {
+  const bool sel = fabsf(c.n.x) > fabsf(c.n.y);
+  const float a0 = sel ? c.n.z : -c.n.z, a1 = sel ? -c.n.x : c.n.y;
+  const float mine = (h ? a1 : a0) / c.tl, other = pair_swap(mine);
+  const float u = h ? other : mine, v = h ? mine : other;
+  t2 = sel ? f3{u, 0.0f, v} : f3{0.0f, u, v};
+  t1 = cross(t2, c.n);
+}
+
+// Warm start of one manifold (SORProx::warmstart_set, sor_prox.rs:19-45): dv += l W J for every
+// row with l != 0, normal rows first, then friction rows. The lanes need nothing of each other but the
+// quotients of the tangents.
+template <bool kMask>
+__device__ __forceinline__ void pair_warm(const PairHalf<kMask>& m, Dv& v) {
+  f3 dh, ah, wah;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    if (k >= x.cnt) break;
-    {
-      f3 d_h, a_h, wa_h;
-      half(c[k].p, neg(c[k].n), d_h, a_h, wa_h);
-      const float w = w_of(d_h, a_h, c[k].rhs[0]);
-      const float a = c[k].lam.x - c[k].r[0] * w;
-      const float ni = a > 0.0f ? a : 0.0f;
-      const float dl = ni - c[k].lam.x;
-      c[k].lam.x = ni;
-      axpy6(dl, scale(d_h, im), wa_h, v);
-    }
-    const float mu = c[k].mu;
-    const float ln = c[k].lam.x;
-    f3 t[2];
-    tangents(c[k].n, t[0], t[1]);
-#pragma unroll
-    for (int f = 1; f <= 2; ++f) {
-      float li = f == 1 ? c[k].lam.y : c[k].lam.z;
-      f3 d_h, a_h, wa_h;
-      half(c[k].p, t[f - 1], d_h, a_h, wa_h);
-      if (ln == 0.0f) {
-        if (li != 0.0f) {
-          axpy6(-li, scale(d_h, im), wa_h, v);
-          li = 0.0f;
-        }
-      } else {
-        const float mx = mu * ln;
-        const float mn = -mx;
-        const float w = w_of(d_h, a_h, c[k].rhs[f]);
-        const float val = li - c[k].r[f] * w;
-        const float ni = val > mn ? (val < mx ? val : mx) : mn;
-        const float dl = ni - li;
-        li = ni;
-        axpy6(dl, scale(d_h, im), wa_h, v);
-      }
-      if (f == 1) c[k].lam.y = li;
-      else c[k].lam.z = li;
-    }
+    if (k >= m.cnt) break;
+    if (m.c[k].lam.x == 0.0f) continue;
+    half_row(m, m.c[k].p, neg(m.c[k].n), dh, ah, wah);
+    axpy6(m.c[k].lam.x, scale(dh, m.im), wah, v);
   }
-  if (dyn) acc.store1(body, v);
-  if (h == 0) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (k < x.cnt) sb.lam[x.r0 + k] = c[k].lam;
+  for (int k = 0; k < 4; ++k) {
+    if (k >= m.cnt) break;
+    if (m.c[k].lam.y == 0.0f && m.c[k].lam.z == 0.0f) continue;
+    f3 t1, t2;
+    pair_tangents(m.c[k], m.h, t1, t2);
+    if (m.c[k].lam.y != 0.0f) {
+      half_row(m, m.c[k].p, t1, dh, ah, wah);
+      axpy6(m.c[k].lam.y, scale(dh, m.im), wah, v);
+    }
+    if (m.c[k].lam.z != 0.0f) {
+      half_row(m, m.c[k].p, t2, dh, ah, wah);
+      axpy6(m.c[k].lam.z, scale(dh, m.im), wah, v);
+    }
   }
 }
 
-// One colour of one sweep, two lanes per manifold (the grid covers both lanes of every pair in
-// one wavefront: blockDim and the stride are even).
+// One SOR-Prox step of one manifold (sor_prox.rs:159-343), contact by contact: the normal row,
+// projected on l >= 0, then the two friction rows, bounded by mu times that normal impulse and
+// zeroed when it is zero. Both lanes form w = (s1 + s2) + rhs and the same new impulse.
 template <bool kMask>
-__global__ void __launch_bounds__(64) k_pgs(DevBodies b, DevContacts c, SolverBufs sb, int first, int n) {
+__device__ __forceinline__ void pair_sweep(PairHalf<kMask>& m, Dv& v) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (k >= m.cnt) break;
+    CHalf& c = m.c[k];
+    f3 dh, ah, wah;
+    half_row(m, c.p, neg(c.n), dh, ah, wah);
+    {
+      const float s = dot6(dh, ah, v);
+      const float w = (s + pair_swap(s)) + c.rhs[0];
+      const float a = c.lam.x - c.r[0] * w;
+      const float ni = a > 0.0f ? a : 0.0f;
+      const float dl = ni - c.lam.x;
+      c.lam.x = ni;
+      axpy6(dl, scale(dh, m.im), wah, v);
+    }
+    const float ln = c.lam.x;
+    f3 t[2];
+    pair_tangents(c, m.h, t[0], t[1]);
+#pragma unroll
+    for (int f = 1; f <= 2; ++f) {
+      float li = f == 1 ? c.lam.y : c.lam.z;
+      half_row(m, c.p, t[f - 1], dh, ah, wah);
+      if (ln == 0.0f) {
+        if (li != 0.0f) {
+          axpy6(-li, scale(dh, m.im), wah, v);
+          li = 0.0f;
+        }
+      } else {
+        const float mx = c.lam.w * ln;
+        const float mn = -mx;
+        const float s = dot6(dh, ah, v);
+        const float w = (s + pair_swap(s)) + c.rhs[f];
+        const float val = li - c.r[f] * w;
+        const float ni = val > mn ? (val < mx ? val : mx) : mn;
+        const float dl = ni - li;
+        li = ni;
+        axpy6(dl, scale(dh, m.im), wah, v);
+      }
+      if (f == 1) c.lam.y = li;
+      else c.lam.z = li;
+    }
+  }
+}
+
+template <bool kMask>
+__device__ __forceinline__ void store_pair_lam(const SolverBufs& sb, const PairHalf<kMask>& m) {
+  if (m.h) return;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k < m.cnt) sb.lam[m.r0 + k] = m.c[k].lam;
+}
+
+// The warm start or one sweep step of the manifold in `slot`, on this lane's side.
+template <bool kWarm, bool kMask, class A>
+__device__ __forceinline__ void solve_pair(const A& acc, const DevBodies& b, const SolverBufs& sb, int slot, int h) {
+  PairHalf<kMask> m;
+  load_pair(b, sb, sb.sinfo[slot], h, m);
+  Dv v{};
+  load_pair_dv(acc, m, v);
+  if (kWarm) pair_warm(m, v);
+  else pair_sweep(m, v);
+  store_pair_dv(acc, m, v);
+  if (!kWarm) store_pair_lam(sb, m);
+}
+
+// One colour of the warm start or of one sweep (the grid covers both lanes of every pair in one
+// wavefront: blockDim and the stride are even).
+template <bool kWarm, bool kMask>
+__global__ void __launch_bounds__(64) k_pgs(DevBodies b, SolverBufs sb, int first, int n) {
   const GlobalDv acc{b};
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; (t >> 1) < n; t += gridDim.x * blockDim.x)
-    pgs_manifold_pair<kMask>(acc, b, sb, first + (t >> 1), t & 1);
+    solve_pair<kWarm, kMask>(acc, b, sb, first + (t >> 1), t & 1);
 }
 
 // A run of consecutive small colour classes of the visiting order in one workgroup, a barrier
 // between classes: per body the same updates in the same order as one launch per class, without
 // a launch per class. Each class fits one pass of the workgroup.
 template <bool kWarm, bool kMask>
-__global__ void __launch_bounds__(kRunBlock) k_colour_run(DevBodies b, SolverBufs sb, ClassRun run) {
+__global__ void __launch_bounds__(2 * kRunBlock) k_colour_run(DevBodies b, SolverBufs sb, ClassRun run) {
   const GlobalDv acc{b};
   for (int k = 0; k < run.n; ++k) {
-    const int first = run.r[k].x, n = run.r[k].y;
-    for (int t = threadIdx.x; t < n; t += kRunBlock) {
-      if (kWarm) warm_manifold<kMask>(acc, b, sb, first + t);
-      else pgs_manifold<kMask>(acc, b, sb, first + t);
-    }
+    const int t = threadIdx.x;
+    if ((t >> 1) < run.r[k].y) solve_pair<kWarm, kMask>(acc, b, sb, run.r[k].x + (t >> 1), t & 1);
     __syncthreads();
   }
 }
@@ -912,11 +888,12 @@ __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBu
       const int col = visit.c[k];
       const int s0 = int(st[col]), e = int(st[col + 1]);
       if (pass < 0) {
-        for (int i = s0 + threadIdx.x; i < e; i += kBlock) warm_manifold<kMask>(acc, b, sb, sc.at(i));
+        for (int i = 2 * s0 + threadIdx.x; i < 2 * e; i += kBlock)
+          solve_pair<true, kMask>(acc, b, sb, sc.at(i >> 1), i & 1);
       } else {
         // both lanes of a manifold are adjacent lanes of one wavefront (kBlock and 2 * s0 are even)
         for (int i = 2 * s0 + threadIdx.x; i < 2 * e; i += kBlock)
-          pgs_manifold_pair<kMask>(acc, b, sb, sc.at(i >> 1), i & 1);
+          solve_pair<false, kMask>(acc, b, sb, sc.at(i >> 1), i & 1);
       }
       __syncthreads();
     }
@@ -957,6 +934,9 @@ __global__ void __launch_bounds__(256) k_scene_starts(const uint32_t* __restrict
   start[t] = uint32_t(lo);
 }
 
+// What the next step's assembly finds of a solved contact (w >= 0: there is a cached impulse).
+__device__ __forceinline__ float4 cached_impulse(float4 lam) { return make_float4(lam.x, lam.y, lam.z, 0.0f); }
+
 // Natural-map residual per row; per block (max |phi|, sum phi^2) in double, written to host memory and
 // reduced there in block order. With kCache the manifold's impulses, which it has in registers, go to
 // the contacts' slots as well (cache_impulses: the warm start of the next step), 16 to 64 contiguous bytes.
@@ -975,7 +955,7 @@ __global__ void __launch_bounds__(256) k_residual(DevBodies b, DevContacts c, in
     for (int k = 0; k < 4; ++k) {
       if (k >= m.x.cnt) break;
       const float4 lam = m.c[k].lam;
-      if (kCache) c.imp[m.x.first + k] = lam;
+      if (kCache) c.imp[m.x.first + k] = cached_impulse(lam);
       {
         const Row v = row_of(m, k, 0);
         const float w = row_w(v, v1, v2);
@@ -1020,7 +1000,7 @@ __global__ void __launch_bounds__(256) k_cache(DevContacts c, int M, SolverBufs 
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= M) return;
   const SlotCtx x = slot_ctx(sb, s);
-  for (int k = 0; k < x.cnt; ++k) c.imp[x.first + k] = sb.lam[x.r0 + k];
+  for (int k = 0; k < x.cnt; ++k) c.imp[x.first + k] = cached_impulse(sb.lam[x.r0 + k]);
 }
 
 // ------------------------------------------------------------------ learned warm start
@@ -1047,7 +1027,7 @@ __global__ void __launch_bounds__(256) k_features(DevBodies b, DevContacts cur, 
     CRec c;
     load_rec(sb, r, c);
     f3 t1, t2;
-    tangents(c.n, t1, t2);
+    tangents(c.n, c.tl, t1, t2);
     const float depth = cur.contact(x.first + k)[0].w + mm;
     const float lsc = c.r[0] * gdt;
     float* f = X + long(r) * 24;
@@ -1075,7 +1055,7 @@ __global__ void __launch_bounds__(256) k_features(DevBodies b, DevContacts cur, 
     f[20] = e;
     f[21] = gdt;
     f[22] = (x.d1 && x.d2) ? 0.0f : 1.0f;
-    f[23] = c.lam.w;
+    f[23] = sb.has[r];
     ls[r] = lsc;
   }
 }
@@ -1088,9 +1068,9 @@ __global__ void __launch_bounds__(256) k_apply_prediction(SolverBufs sb, int C, 
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= C) return;
   const float s = ls[r];
-  const float mu = sb.rec[long(r) * kRecFields].w;
   float4* L = sb.lam + r;
   const float4 c = *L;
+  const float mu = c.w;
   const float ln = fmaxf(c.x + y[3 * r] * s, 0.0f);
   const float lim = mu * ln;
   const float t1 = fminf(fmaxf(c.y + y[3 * r + 1] * s, -lim), lim);
@@ -1175,35 +1155,31 @@ int sweep_blocks(int max_class) {
 }
 
 // The masked kernel variants run only in worlds where some dynamic body has a kinematic dof.
-void launch_warmstart_colour(const DevBodies& b, const DevContacts& c, int first, int n, int blocks, SolverBufs& sb,
-                             hipStream_t s) {
-  if (b.kmask) hipLaunchKernelGGL(k_warmstart<true>, dim3(blocks), dim3(64), 0, s, b, c, sb, first, n);
-  else hipLaunchKernelGGL(k_warmstart<false>, dim3(blocks), dim3(64), 0, s, b, c, sb, first, n);
+void launch_warmstart_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s) {
+  if (b.kmask) hipLaunchKernelGGL((k_pgs<true, true>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
+  else hipLaunchKernelGGL((k_pgs<true, false>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
 }
 
-void launch_pgs_colour(const DevBodies& b, const DevContacts& c, int first, int n, int blocks, SolverBufs& sb,
-                       hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
+void launch_pgs_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s, hipEvent_t ev0,
+                       hipEvent_t ev1) {
+  // with events, the dispatch packet itself records both, timing the kernel alone
   if (b.kmask) {
-    if (ev0) hipExtLaunchKernelGGL(k_pgs<true>, dim3(blocks), dim3(64), 0, s, ev0, ev1, 0, b, c, sb, first, n);
-    else hipLaunchKernelGGL(k_pgs<true>, dim3(blocks), dim3(64), 0, s, b, c, sb, first, n);
+    if (ev0) hipExtLaunchKernelGGL((k_pgs<false, true>), dim3(blocks), dim3(64), 0, s, ev0, ev1, 0, b, sb, first, n);
+    else hipLaunchKernelGGL((k_pgs<false, true>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
     return;
   }
-  if (ev0) {
-    // the dispatch packet itself records both events, timing the kernel alone
-    hipExtLaunchKernelGGL(k_pgs<false>, dim3(blocks), dim3(64), 0, s, ev0, ev1, 0, b, c, sb, first, n);
-  } else {
-    hipLaunchKernelGGL(k_pgs<false>, dim3(blocks), dim3(64), 0, s, b, c, sb, first, n);
-  }
+  if (ev0) hipExtLaunchKernelGGL((k_pgs<false, false>), dim3(blocks), dim3(64), 0, s, ev0, ev1, 0, b, sb, first, n);
+  else hipLaunchKernelGGL((k_pgs<false, false>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
 }
 
 void launch_colour_run(const DevBodies& b, SolverBufs& sb, const ClassRun& run, bool warm, hipStream_t s) {
   if (b.kmask) {
-    if (warm) hipLaunchKernelGGL((k_colour_run<true, true>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
-    else hipLaunchKernelGGL((k_colour_run<false, true>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
+    if (warm) hipLaunchKernelGGL((k_colour_run<true, true>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
+    else hipLaunchKernelGGL((k_colour_run<false, true>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
     return;
   }
-  if (warm) hipLaunchKernelGGL((k_colour_run<true, false>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
-  else hipLaunchKernelGGL((k_colour_run<false, false>), dim3(1), dim3(kRunBlock), 0, s, b, sb, run);
+  if (warm) hipLaunchKernelGGL((k_colour_run<true, false>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
+  else hipLaunchKernelGGL((k_colour_run<false, false>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
 }
 
 int residual_blocks(int M) { return int(nb(M > 0 ? M : 1)); }

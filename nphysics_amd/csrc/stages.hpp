@@ -146,7 +146,8 @@ struct SolverBufs {
   int4* sinfo;            // [M] per slot: body1|dyn1<<30, body2|dyn2<<30, first record, count|first<<3
   uint2* slot_of;         // [M] slot and first row record of each manifold
   float4* rec;            // [kRecFields rec_stride] row records, field f of record r at kRecFields r + f
-  float4* lam;            // [rec_stride] impulses of each row record (normal, tangent 1, tangent 2, has cache)
+  float4* lam;            // [rec_stride] impulses of each row record (normal, tangent 1, tangent 2) and mu
+  float* has;             // [C] 1 where the warm start came from the cache (null: nobody asks)
   float4* prec;           // [3 rec_stride] position records: (lp1 | contact kind), (lp2 | shape 1), (ln | shape 2)
   float4* pgeo;           // [2M] per slot: (half extents 1 | margin 1), (half extents 2 | margin 2)
   long rec_stride;        // record capacity (fixed between reallocations)
@@ -178,8 +179,7 @@ void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContac
 int sweep_blocks(int max_class);
 int position_blocks(int max_class);
 // (first, n): the class's slot range, known on the host from the visiting order
-void launch_warmstart_colour(const DevBodies& b, const DevContacts& c, int first, int n, int blocks,
-                             SolverBufs& sb, hipStream_t s);
+void launch_warmstart_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s);
 // Consecutive visited classes, each of at most kRunBlock manifolds, as (first slot, slots), in one
 // workgroup (warm start or sweep). Passed by value: no copy to the device stands before the launch.
 constexpr int kRunBlock = 512;
@@ -189,8 +189,8 @@ struct ClassRun {
   int2 r[kRunClasses];
 };
 void launch_colour_run(const DevBodies& b, SolverBufs& sb, const ClassRun& run, bool warm, hipStream_t s);
-void launch_pgs_colour(const DevBodies& b, const DevContacts& c, int first, int n, int blocks, SolverBufs& sb,
-                       hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+void launch_pgs_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s,
+                       hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // cache: also the impulses to the contacts' slots, as launch_cache_impulses
 void launch_residual(const DevBodies& b, const DevContacts& c, int M, bool cache, SolverBufs& sb, hipStream_t s);
 void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int M, hipStream_t s);

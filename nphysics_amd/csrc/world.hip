@@ -170,7 +170,7 @@ struct World {
   bool sview_compact[2] = {false, false};
   DBuf sv_state2[2];  // colouring state of the manifolds of sview[k]
   DBuf sv_deg, sv_adj_off, sv_adj, sv_place, sv_hist, sv_ckeys, sv_col_start, sv_slot_of, sv_sinfo, sv_rec, sv_lam,
-      sv_prec, sv_pgeo, sv_tmp;
+      sv_has, sv_prec, sv_pgeo, sv_tmp;
   int ncolours = 0;
   long rec_stride = 0;
   int colour_rounds = 0;
@@ -1116,6 +1116,9 @@ struct World {
   }
 
   // ------------------------------------------------------------------ solver
+  // Whether this solve computes the network's features, which tell cached impulses from new ones.
+  bool learned_rows() const { return capture || contact_model == NPHYS_CONTACT_MODEL_LEARNED_WARMSTART; }
+
   int ensure_solver(int M, int C, int digits = 256) {
     const size_t nn = size_t(std::max(n, 1));
     const size_t m = size_t(std::max(M, 1)), c = size_t(std::max(C, 1));
@@ -1132,6 +1135,7 @@ struct World {
     HIPCK(sv_sinfo.ensure(m * sizeof(int4)));
     HIPCK(sv_rec.ensure(c * kRecFields * sizeof(float4)));
     HIPCK(sv_lam.ensure(c * sizeof(float4)));
+    if (learned_rows()) HIPCK(sv_has.ensure(c * 4));
     HIPCK(sv_prec.ensure(c * 3 * sizeof(float4)));
     HIPCK(sv_pgeo.ensure(m * 2 * sizeof(float4)));
     rec_stride = long(std::min({sv_rec.bytes / (kRecFields * sizeof(float4)), sv_lam.bytes / sizeof(float4),
@@ -1172,6 +1176,7 @@ struct World {
     v.prec = sv_prec.as<float4>();
     v.pgeo = sv_pgeo.as<float4>();
     v.red = red_dev;
+    v.has = learned_rows() ? sv_has.as<float>() : nullptr;
     v.tmp = sv_tmp.as<uint32_t>();
     v.scan = &scan;
     return v;
@@ -1330,20 +1335,18 @@ struct World {
           k += run.n;
           continue;
         }
-        // one 64-lane workgroup per 64 manifolds of this class (the grid-stride loop covers the
-        // rest above the cap): no idle workgroups for the smaller classes
+        // one 64-lane workgroup per 32 manifolds of this class, two lanes each (the grid-stride loop
+        // covers the rest above the cap): no idle workgroups for the smaller classes
         const int2 r = h_range[size_t(k)];
-        const int cblocks = std::min(sblocks, std::max(1, (r.y + 63) / 64));
-        // the sweep kernel runs two lanes per manifold
         const int pblocks2 = std::min(2 * sblocks, std::max(1, (2 * r.y + 63) / 64));
         if (w) {
-          launch_warmstart_colour(b, cv, r.x, r.y, cblocks, v, stream);
+          launch_warmstart_colour(b, r.x, r.y, pblocks2, v, stream);
         } else if (counters_enabled) {
-          launch_pgs_colour(b, cv, r.x, r.y, pblocks2, v, stream, kt_ev[kt_used], kt_ev[kt_used + 1]);
+          launch_pgs_colour(b, r.x, r.y, pblocks2, v, stream, kt_ev[kt_used], kt_ev[kt_used + 1]);
           kt_used += 2;
           counters.sweep_kernel_contacts += class_contacts[size_t(k)];
         } else {
-          launch_pgs_colour(b, cv, r.x, r.y, pblocks2, v, stream);
+          launch_pgs_colour(b, r.x, r.y, pblocks2, v, stream);
         }
         ++k;
       }
