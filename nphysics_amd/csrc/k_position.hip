@@ -6,11 +6,18 @@
 // margins (src/solver/signorini_model.rs:174-181), rhs = max((-depth + allowed_linear_error) erp,
 // -max_linear_correction); if rhs < 0 move each dynamic body by its weighted jacobian times
 // -rhs / (J M^-1 J^T) (RigidBody::apply_displacement, src/object/rigid_body.rs:371-381),
-// immediately, so later contacts see the corrected poses. One lane per manifold of one colour
-// keeps both poses in registers across the manifold's contacts. Its inputs are laid out by the
-// assembly in colour order: per slot the two bodies' half extents and margins, per contact a
-// 48-byte position record (local points and normal, contact kind, shape kinds), so a manifold
-// reads contiguous runs besides its two bodies' pose and solver blocks.
+// immediately, so later contacts see the corrected poses.
+//
+// A manifold has four adjacent lanes, one per contact (position_lanes). All contacts are evaluated at once;
+// the first that needs a correction is applied and those after it are evaluated again at the poses
+// it leaves, so every contact that moves a body is evaluated at the same poses as one after another,
+// but the rounds are as many as there are corrections plus one, not one per contact, and a wavefront runs the code
+// of each kind of contact once per round. One lane per manifold took 15 us a launch at 1,200 manifolds
+// of cuboids, bound by that chain on a handful of wavefronts: MEASURED_POSITION
+//
+// Its inputs are laid out by the assembly in colour order: per slot the two bodies' half extents and
+// margins, per contact a 48-byte position record (local points and normal, contact kind, shape
+// kinds), so a manifold reads contiguous runs besides its two bodies' pose and solver blocks.
 #include <hip/hip_runtime.h>
 
 #include "np_geometry.hpp"
@@ -57,18 +64,35 @@ struct LdsPose {
   }
 };
 
-template <bool kMask, class A>
-__device__ __forceinline__ void position_one(const A& acc, const DevBodies& b, const SimParams& p,
-                                             const SolverBufs& sb, int slot) {
+// The value of lane `from` of this lane's quad.
+__device__ __forceinline__ float quad_get(float v, int from) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute((int(threadIdx.x & 60u) + from) << 2, __float_as_int(v)));
+}
+__device__ __forceinline__ f3 quad_get(f3 v, int from) {
+  return f3{quad_get(v.x, from), quad_get(v.y, from), quad_get(v.z, from)};
+}
+// The value of the neighbouring lane (0 and 1, 2 and 3 of the quad).
+__device__ __forceinline__ float pair_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));
+}
+
+// One manifold on kLanes lanes: on a quad, whose lane k (threadIdx.x & 3) has contact k, or, with one
+// contact, on one lane. The four lanes stay together: every branch around an exchange is taken on values they share.
+template <int kLanes, bool kMask, class A>
+__device__ __forceinline__ void position_lanes(const A& acc, const DevBodies& b, const SimParams& p,
+                                               const SolverBufs& sb, int slot) {
+  const int k = kLanes == 1 ? 0 : int(threadIdx.x & 3u);
   const int4 q = sb.sinfo[slot];
   const int b1 = q.x & 0x3fffffff, b2 = q.y & 0x3fffffff;
   const bool d1 = (q.x >> 30) & 1;
   const bool d2 = (q.y >> 30) & 1;
   const uint32_t r0 = uint32_t(q.z);
-  const int cnt = q.w & 7;
+  const int cnt = kLanes == 1 ? 1 : q.w & 7;
   const float4 g1 = sb.pgeo[2 * long(slot)], g2 = sb.pgeo[2 * long(slot) + 1];
   const f3 h1 = xyz(g1), h2 = xyz(g2);
   const float m1 = g1.w, m2 = g2.w;
+  const float4* P = sb.prec + 3 * long(r0 + (k < cnt ? k : 0));
+  const float4 pa = P[0], pc = P[1], pe = P[2];
   f3 t1, t2;
   q4 q1, q2;
   acc.load(b1, d1, t1, q1);
@@ -83,91 +107,101 @@ __device__ __forceinline__ void position_one(const A& acc, const DevBodies& b, c
     b.mask(b1, ml1, ma1);
     b.mask(b2, ml2, ma2);
   }
-  // the manifold's kinematics (at most 4 contacts, contiguous position records written by the
-  // assembly in colour order) are loaded up front, independent of the poses
-  int kind[4];
-  f3 lp1[4], lp2[4], ln[4];
-  int k1 = 0, k2 = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k < cnt) {
-      const float4* P = sb.prec + 3 * long(r0 + k);
-      const float4 a = P[0], c = P[1], e = P[2];
-      kind[k] = __float_as_int(a.w);
-      lp1[k] = xyz(a);
-      lp2[k] = xyz(c);
-      ln[k] = xyz(e);
-      k1 = __float_as_int(c.w);
-      k2 = __float_as_int(e.w);
+  const int kind = __float_as_int(pa.w);
+  const int k1 = __float_as_int(pc.w), k2 = __float_as_int(pe.w);
+  const int quad = threadIdx.x & 60;
+  bool moved = false;
+  for (int from = 0; from < cnt;) {
+    bool act = false;
+    f3 l1{0.0f, 0.0f, 0.0f}, a1{0.0f, 0.0f, 0.0f}, l2{0.0f, 0.0f, 0.0f}, a2{0.0f, 0.0f, 0.0f};  // displacements
+    if (k >= from && k < cnt) {
+      const Contact g = reevaluate(kind, xyz(pa), xyz(pc), xyz(pe), k1, h1, t1, q1, k2, h2, t2, q2);
+      const f3 w1 = add(g.w1, scale(g.n, m1));
+      const f3 w2 = sub(g.w2, scale(g.n, m2));
+      const float depth = (g.depth + m1) + m2;
+      const float rhs = fmaxf_((-depth + p.allowed_linear_error) * p.erp, -p.max_linear_correction);
+      if (!(rhs >= 0.0f)) {
+        float inv_r = 0.0f;
+        if (d1) {
+          const f3 dir = neg(g.n);
+          f3 ang = cross(sub(w1, t1), dir);
+          if (kMask) ang = cmul(ang, ma1);
+          l1 = scale(kMask ? cmul(dir, ml1) : dir, im1);
+          a1 = mulv(I1, ang);
+          inv_r = inv_r + (im1 + dot(ang, a1));
+        }
+        if (d2) {
+          const f3 dir = g.n;
+          f3 ang = cross(sub(w2, t2), dir);
+          if (kMask) ang = cmul(ang, ma2);
+          l2 = scale(kMask ? cmul(dir, ml2) : dir, im2);
+          a2 = mulv(I2, ang);
+          inv_r = inv_r + (im2 + dot(ang, a2));
+        }
+        if (inv_r != 0.0f) {
+          act = true;
+          const float r = 1.0f / inv_r;
+          const float impulse = -rhs * r;
+          l1 = scale(l1, impulse);
+          a1 = scale(a1, impulse);
+          l2 = scale(l2, impulse);
+          a2 = scale(a2, impulse);
+        }
+      }
     }
+    if (kLanes == 1) {
+      if (act && d1) apply_displacement(t1, q1, l1, a1);
+      if (act && d2) apply_displacement(t2, q2, l2, a2);
+      moved = act;
+      break;
+    }
+    const uint32_t acts = uint32_t(__ballot(act) >> quad) & 0xfu;
+    if (acts == 0u) break;
+    const int f = __ffs(int(acts)) - 1;
+    // body 1's pose on the even lanes, body 2's on the odd ones, from the displacements of lane f
+    const bool first = (k & 1) == 0;
+    const f3 lf1 = quad_get(l1, f), af1 = quad_get(a1, f), lf2 = quad_get(l2, f), af2 = quad_get(a2, f);
+    f3 t = pick(first, t1, t2);
+    q4 r = pick(first, q1, q2);
+    if (first ? d1 : d2) apply_displacement(t, r, pick(first, lf1, lf2), pick(first, af1, af2));
+    const f3 to{pair_swap(t.x), pair_swap(t.y), pair_swap(t.z)};
+    const q4 ro{pair_swap(r.i), pair_swap(r.j), pair_swap(r.k), pair_swap(r.w)};
+    t1 = pick(first, t, to);
+    q1 = pick(first, r, ro);
+    t2 = pick(first, to, t);
+    q2 = pick(first, ro, r);
+    moved = true;
+    from = f + 1;
   }
-  bool moved1 = false, moved2 = false;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= cnt) break;
-    const Contact g = reevaluate(kind[k], lp1[k], lp2[k], ln[k], k1, h1, t1, q1, k2, h2, t2, q2);
-    const f3 w1 = add(g.w1, scale(g.n, m1));
-    const f3 w2 = sub(g.w2, scale(g.n, m2));
-    const float depth = (g.depth + m1) + m2;
-    const float rhs = fmaxf_((-depth + p.allowed_linear_error) * p.erp, -p.max_linear_correction);
-    if (rhs >= 0.0f) continue;
-    float inv_r = 0.0f;
-    f3 wl1{0.0f, 0.0f, 0.0f}, wa1{0.0f, 0.0f, 0.0f}, wl2{0.0f, 0.0f, 0.0f}, wa2{0.0f, 0.0f, 0.0f};
-    if (d1) {
-      const f3 dir = neg(g.n);
-      f3 ang = cross(sub(w1, t1), dir);
-      if (kMask) ang = cmul(ang, ma1);
-      wl1 = scale(kMask ? cmul(dir, ml1) : dir, im1);
-      wa1 = mulv(I1, ang);
-      inv_r = inv_r + (im1 + dot(ang, wa1));
-    }
-    if (d2) {
-      const f3 dir = g.n;
-      f3 ang = cross(sub(w2, t2), dir);
-      if (kMask) ang = cmul(ang, ma2);
-      wl2 = scale(kMask ? cmul(dir, ml2) : dir, im2);
-      wa2 = mulv(I2, ang);
-      inv_r = inv_r + (im2 + dot(ang, wa2));
-    }
-    if (inv_r == 0.0f) continue;
-    const float r = 1.0f / inv_r;
-    const float impulse = -rhs * r;
-    if (d1) {
-      apply_displacement(t1, q1, scale(wl1, impulse), scale(wa1, impulse));
-      moved1 = true;
-    }
-    if (d2) {
-      apply_displacement(t2, q2, scale(wl2, impulse), scale(wa2, impulse));
-      moved2 = true;
-    }
-  }
-  if (moved1) acc.store(b1, t1, q1);
-  if (moved2) acc.store(b2, t2, q2);
+  if (moved && k == 0 && d1) acc.store(b1, t1, q1);
+  if (moved && k == (kLanes == 1 ? 0 : 1) && d2) acc.store(b2, t2, q2);
 }
 
-template <bool kMask>
+template <int kLanes, bool kMask>
 __global__ void __launch_bounds__(64) k_position(DevBodies b, SimParams p, SolverBufs sb, int first_slot,
                                                 int nslots) {
   const GlobalPose acc{b};
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nslots; t += gridDim.x * blockDim.x)
-    position_one<kMask>(acc, b, p, sb, first_slot + t);
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t / kLanes < nslots; t += gridDim.x * blockDim.x)
+    position_lanes<kLanes, kMask>(acc, b, p, sb, first_slot + t / kLanes);
 }
 
 // Consecutive small classes of the visiting order in one workgroup, a barrier between classes
 // (the same corrections in the same order per body as one launch per class).
-template <bool kMask>
-__global__ void __launch_bounds__(kRunBlock) k_position_run(DevBodies b, SimParams p, SolverBufs sb, ClassRun run) {
+constexpr int kPositionRun = 1024;
+template <int kLanes, bool kMask>
+__global__ void __launch_bounds__(kPositionRun) k_position_run(DevBodies b, SimParams p, SolverBufs sb, ClassRun run) {
   const GlobalPose acc{b};
   for (int k = 0; k < run.n; ++k) {
     const int2 range = run.r[k];
-    for (int t = threadIdx.x; t < range.y; t += kRunBlock) position_one<kMask>(acc, b, p, sb, range.x + t);
+    for (int t = threadIdx.x; t / kLanes < range.y; t += kPositionRun)
+      position_lanes<kLanes, kMask>(acc, b, p, sb, range.x + t / kLanes);
     __syncthreads();
   }
 }
 
 // Scene-blocked position correction: one workgroup per scene, the scene's dynamic poses in LDS,
 // `iterations` passes over the colours in the visiting order with a barrier between colours.
-template <int kBlock, int kCap, bool kMask>
+template <int kBlock, int kCap, int kLanes, bool kMask>
 __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimParams p, SolverBufs sb, SceneBlocks sc,
                                                            const int* __restrict__ scene_list,
                                                            VisitOrder visit, int iterations) {
@@ -186,8 +220,9 @@ __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimPar
   for (int it = 0; it < iterations; ++it) {
     for (int k = 0; k < visit.n; ++k) {
       const int col = visit.c[k];
-      const int e = int(st[col + 1]);
-      for (int i = int(st[col]) + threadIdx.x; i < e; i += kBlock) position_one<kMask>(acc, b, p, sb, sc.at(i));
+      const int s0 = int(st[col]), e = int(st[col + 1]);
+      for (int i = kLanes * s0 + threadIdx.x; i < kLanes * e; i += kBlock)
+        position_lanes<kLanes, kMask>(acc, b, p, sb, sc.at(i / kLanes));
       __syncthreads();
     }
   }
@@ -200,44 +235,68 @@ __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimPar
 
 }  // namespace
 
-// Sized like the sweep grid: from the largest colour class.
-int position_blocks(int max_class) { return sweep_blocks(max_class); }
+namespace {
 
-void launch_position_colour(const DevBodies& b, const DevContacts& c, const SimParams& p, int first, int n,
-                            int blocks, SolverBufs& sb, hipStream_t s) {
-  (void)c;
-  if (b.kmask) hipLaunchKernelGGL(k_position<true>, dim3(blocks), dim3(64), 0, s, b, p, sb, first, n);
-  else hipLaunchKernelGGL(k_position<false>, dim3(blocks), dim3(64), 0, s, b, p, sb, first, n);
+// single: every manifold of the launch has one contact.
+template <bool kMask>
+void position_colour(const DevBodies& b, const SimParams& p, int first, int n, bool single, SolverBufs& sb,
+                     hipStream_t s) {
+  // one 64-lane workgroup per 16 (or 64) manifolds; the grid-stride loop walks what is above the cap
+  const int per = single ? 64 : 16, blocks = n < per * 32768 ? (n + per - 1) / per : 32768;
+  if (single) hipLaunchKernelGGL((k_position<1, kMask>), dim3(blocks), dim3(64), 0, s, b, p, sb, first, n);
+  else hipLaunchKernelGGL((k_position<4, kMask>), dim3(blocks), dim3(64), 0, s, b, p, sb, first, n);
 }
 
 template <bool kMask>
-void position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit,
-                      int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
+void position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, bool single,
+                  hipStream_t s) {
+  if (single) hipLaunchKernelGGL((k_position_run<1, kMask>), dim3(1), dim3(kPositionRun), 0, s, b, p, sb, run);
+  else hipLaunchKernelGGL((k_position_run<4, kMask>), dim3(1), dim3(kPositionRun), 0, s, b, p, sb, run);
+}
+
+template <int kLanes, bool kMask>
+void position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
+                      const VisitOrder& visit, int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
   if (sc.n_large > 0) {
     if (block == 256)
-      hipLaunchKernelGGL((k_position_blocked<256, kLdsBodies, kMask>), dim3(sc.n_large), dim3(256), 0, s_large, b, p,
-                         sb, sc, sc.large_list, visit, iterations);
+      hipLaunchKernelGGL((k_position_blocked<256, kLdsBodies, kLanes, kMask>), dim3(sc.n_large), dim3(256), 0, s_large,
+                         b, p, sb, sc, sc.large_list, visit, iterations);
     else if (block == 512)
-      hipLaunchKernelGGL((k_position_blocked<512, kLdsBodies, kMask>), dim3(sc.n_large), dim3(512), 0, s_large, b, p,
-                         sb, sc, sc.large_list, visit, iterations);
+      hipLaunchKernelGGL((k_position_blocked<512, kLdsBodies, kLanes, kMask>), dim3(sc.n_large), dim3(512), 0, s_large,
+                         b, p, sb, sc, sc.large_list, visit, iterations);
     else
-      hipLaunchKernelGGL((k_position_blocked<1024, kLdsBodies, kMask>), dim3(sc.n_large), dim3(1024), 0, s_large, b,
-                         p, sb, sc, sc.large_list, visit, iterations);
+      hipLaunchKernelGGL((k_position_blocked<1024, kLdsBodies, kLanes, kMask>), dim3(sc.n_large), dim3(1024), 0,
+                         s_large, b, p, sb, sc, sc.large_list, visit, iterations);
   }
   if (sc.n_small > 0)
-    hipLaunchKernelGGL((k_position_blocked<64, kSmallScene, kMask>), dim3(sc.n_small), dim3(64), 0, s_small, b, p, sb,
-                       sc, sc.small_list, visit, iterations);
+    hipLaunchKernelGGL((k_position_blocked<64, kSmallScene, kLanes, kMask>), dim3(sc.n_small), dim3(64), 0, s_small, b,
+                       p, sb, sc, sc.small_list, visit, iterations);
+}
+
+}  // namespace
+
+void launch_position_colour(const DevBodies& b, const SimParams& p, int first, int n, bool single, SolverBufs& sb,
+                            hipStream_t s) {
+  if (b.kmask) position_colour<true>(b, p, first, n, single, sb, s);
+  else position_colour<false>(b, p, first, n, single, sb, s);
 }
 
 void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
-                             const VisitOrder& visit, int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
-  if (b.kmask) position_blocked<true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
-  else position_blocked<false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+                             const VisitOrder& visit, int iterations, bool single, int block, hipStream_t s_small,
+                             hipStream_t s_large) {
+  if (b.kmask) {
+    if (single) position_blocked<1, true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+    else position_blocked<4, true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+  } else {
+    if (single) position_blocked<1, false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+    else position_blocked<4, false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+  }
 }
 
-void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s) {
-  if (b.kmask) hipLaunchKernelGGL(k_position_run<true>, dim3(1), dim3(kRunBlock), 0, s, b, p, sb, run);
-  else hipLaunchKernelGGL(k_position_run<false>, dim3(1), dim3(kRunBlock), 0, s, b, p, sb, run);
+void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, bool single,
+                         hipStream_t s) {
+  if (b.kmask) position_run<true>(b, p, sb, run, single, s);
+  else position_run<false>(b, p, sb, run, single, s);
 }
 
 }  // namespace nph

@@ -422,6 +422,13 @@ NPH_HD int collide_ball_pair(int k1, f3 h1, f3 t1, q4 q1, int k2, f3 h2, f3 t2, 
   return n;
 }
 
+// Selection by value: a conditional between two variables of class type is a choice of address, which
+// puts both in memory.
+NPH_HD f3 pick(bool first, f3 a, f3 b) { return f3{first ? a.x : b.x, first ? a.y : b.y, first ? a.z : b.z}; }
+NPH_HD q4 pick(bool first, q4 a, q4 b) {
+  return q4{first ? a.i : b.i, first ? a.j : b.j, first ? a.k : b.k, first ? a.w : b.w};
+}
+
 // Contact re-evaluation at the current poses (geometric, without margins).
 NPH_HD Contact reevaluate(int kind, f3 lp1, f3 lp2, f3 ln, int k1, f3 h1, f3 t1, q4 q1, int k2,
                           f3 h2, f3 t2, q4 q2) {
@@ -431,38 +438,25 @@ NPH_HD Contact reevaluate(int kind, f3 lp1, f3 lp2, f3 ln, int k1, f3 h1, f3 t1,
   c.lp2 = lp2;
   c.ln = ln;
   c.feature = 0;
-  switch (kind) {
-    case KIN_BALL_BALL:
-      collide_ball_ball(t1, h1.x, t2, h2.x, 0.0f, true, &c);
-      break;
-    case KIN_BALL_BOX:
-      collide_ball_box(t1, h1.x, t2, q2, h2, true, 0.0f, true, &c);
-      break;
-    case KIN_BOX_BALL:
-      collide_ball_box(t2, h2.x, t1, q1, h1, false, 0.0f, true, &c);
-      break;
-    case KIN_PLANE1: {
-      const f3 n = qrot(q1, ln);
-      const f3 a = add(qrot(q1, lp1), t1);
-      const f3 b = add(qrot(q2, lp2), t2);
-      const float depth = dot(sub(a, b), n);
-      c.n = n;
-      c.depth = depth;
-      c.w1 = add(b, scale(n, depth));
-      c.w2 = b;
-      break;
-    }
-    default: {  // KIN_PLANE2
-      const f3 n = qrot(q2, ln);
-      const f3 a = add(qrot(q1, lp1), t1);
-      const f3 b = add(qrot(q2, lp2), t2);
-      const float depth = dot(sub(a, b), n);
-      c.n = n;
-      c.depth = depth;
-      c.w1 = a;
-      c.w2 = sub(a, scale(n, depth));
-      break;
-    }
+  // The two kinds with one ball and the two with a plane share their code, the operands selected: a
+  // wavefront of all kinds runs three blocks instead of five.
+  if (kind == KIN_BALL_BALL) {
+    collide_ball_ball(t1, h1.x, t2, h2.x, 0.0f, true, &c);
+  } else if (kind == KIN_BALL_BOX || kind == KIN_BOX_BALL) {
+    const bool first = kind == KIN_BALL_BOX;
+    collide_ball_box(pick(first, t1, t2), first ? h1.x : h2.x, pick(first, t2, t1), pick(first, q2, q1),
+                     pick(first, h2, h1), first, 0.0f, true, &c);
+  } else {  // KIN_PLANE1, KIN_PLANE2
+    const bool first = kind == KIN_PLANE1;
+    const f3 n = qrot(pick(first, q1, q2), ln);
+    const f3 a = add(qrot(q1, lp1), t1);
+    const f3 b = add(qrot(q2, lp2), t2);
+    const float depth = dot(sub(a, b), n);
+    c.n = n;
+    c.depth = depth;
+    const f3 nd = scale(n, depth);
+    c.w1 = pick(first, add(b, nd), a);
+    c.w2 = pick(first, b, sub(a, nd));
   }
   return c;
 }

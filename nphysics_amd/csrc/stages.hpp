@@ -177,7 +177,6 @@ void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContac
 // launches are independent of per-step sizes (grid = blocks from the largest colour class,
 // grid-stride over the colour).
 int sweep_blocks(int max_class);
-int position_blocks(int max_class);
 // (first, n): the class's slot range, known on the host from the visiting order
 void launch_warmstart_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s);
 // Consecutive visited classes, each of at most kRunBlock manifolds, as (first slot, slots), in one
@@ -228,7 +227,8 @@ void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks
 // one workgroup per scene with the scene's dynamic poses in LDS (the same corrections in the same
 // order per body as the per-colour launches); streams and block as launch_sweeps_blocked.
 void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
-                             const VisitOrder& visit, int iterations, int block, hipStream_t s_small, hipStream_t s_large);
+                             const VisitOrder& visit, int iterations, bool single, int block, hipStream_t s_small,
+                             hipStream_t s_large);
 
 // learned warm start (k_solver.hip): features [C][24] and impulse units ls [C] per row record,
 // the prediction y [C][3] applied as the warm start, post-solve targets t [C][3].
@@ -335,8 +335,10 @@ void launch_ccd_validate(const DevBodies& b, const int2* pairs, CcdBufs& c, int 
 void launch_ccd_clamp(const DevBodies& b, CcdBufs& c, hipStream_t s);
 
 // k_position.hip ---------------------------------------------------------------------------
-void launch_position_colour(const DevBodies& b, const DevContacts& c, const SimParams& p, int first, int n,
-                            int blocks, SolverBufs& sb, hipStream_t s);
-void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s);
+// single: every manifold of the launch has one contact
+void launch_position_colour(const DevBodies& b, const SimParams& p, int first, int n, bool single, SolverBufs& sb,
+                            hipStream_t s);
+void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, bool single,
+                         hipStream_t s);
 
 }  // namespace nph

@@ -1283,6 +1283,13 @@ struct World {
     return run;
   }
 
+  // Whether every manifold of the n classes visited from the k-th on has one contact.
+  bool single_contacts(int k, int n) const {
+    for (int i = k; i < k + n; ++i)
+      if (class_contacts[size_t(i)] != h_range[size_t(i)].y) return false;
+    return true;
+  }
+
   VisitOrder visit_list() const {
     VisitOrder v;
     v.n = ncolours;
@@ -1705,18 +1712,16 @@ struct World {
     DevBodies b = bodies();
     SolverBufs v = sv_view();
     JointBufs jv = joint_view();
-    const DevContacts cv = sview[cur];
     if (cur_variant > 0 && !joints) {
       // scene-blocked, as the sweeps of this solve (worlds without joints)
       SceneBlocks sc = sc_view();
       HIPCK(hipEventRecord(fork_ev, stream));
       HIPCK(hipStreamWaitEvent(stream_large, fork_ev, 0));
-      launch_position_blocked(b, ps, v, sc, visit_list(), iterations, cur_variant, stream, stream_large);
+      launch_position_blocked(b, ps, v, sc, visit_list(), iterations, single_contacts(0, ncolours), cur_variant, stream, stream_large);
       HIPCK(hipEventRecord(join_ev, stream_large));
       HIPCK(hipStreamWaitEvent(stream, join_ev, 0));
       return NPHYS_OK;
     }
-    const int pblocks = position_blocks(max_class);
     // direct launches, runs of two or more consecutive small classes in one workgroup (as the
     // sweeps); the joints' constraints first in every iteration (nonlinear_sor_prox.rs:33-38)
     const int ncol = sview_M[cur] > 0 ? ncolours : 0;
@@ -1725,12 +1730,12 @@ struct World {
       for (int k = 0; k < ncol;) {
         const ClassRun run = small_run(k, ncol);
         if (run.n >= 2) {
-          launch_position_run(b, ps, v, run, stream);
+          launch_position_run(b, ps, v, run, single_contacts(k, run.n), stream);
           k += run.n;
           continue;
         }
         const int2 r = h_range[size_t(k)];
-        launch_position_colour(b, cv, ps, r.x, r.y, std::min(pblocks, std::max(1, (r.y + 63) / 64)), v, stream);
+        launch_position_colour(b, ps, r.x, r.y, single_contacts(k, 1), v, stream);
         ++k;
       }
     }
