@@ -20,6 +20,8 @@
 // kinds), so a manifold reads contiguous runs besides its two bodies' pose and solver blocks.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "np_geometry.hpp"
 #include "stages.hpp"
 
@@ -177,31 +179,41 @@ __device__ __forceinline__ void position_lanes(const A& acc, const DevBodies& b,
   if (moved && k == (kLanes == 1 ? 0 : 1) && d2) acc.store(b2, t2, q2);
 }
 
-template <int kLanes, bool kMask>
-__global__ void __launch_bounds__(64) k_position(DevBodies b, SimParams p, SolverBufs sb, int first_slot,
-                                                int nslots) {
-  const GlobalPose acc{b};
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t / kLanes < nslots; t += gridDim.x * blockDim.x)
-    position_lanes<kLanes, kMask>(acc, b, p, sb, first_slot + t / kLanes);
+// The class's manifolds on `lanes` lanes: a quad for each of those with several contacts, a lane for
+// each of the others, which start in a wavefront of their own and so run their code alone.
+template <bool kMask, class A, class At>
+__device__ __forceinline__ void position_class(const A& acc, const DevBodies& b, const SimParams& p,
+                                               const SolverBufs& sb, const ClassSpan& c, int lane, int lanes,
+                                               const At& at) {
+  const int quads = (4 * c.multi + 63) & ~63;
+  for (int t = lane; t < quads + c.single; t += lanes) {
+    if (t < quads) {
+      if (t < 4 * c.multi) position_lanes<4, kMask>(acc, b, p, sb, at(c.first + (t >> 2)));
+    } else {
+      position_lanes<1, kMask>(acc, b, p, sb, at(c.first + c.multi + t - quads));
+    }
+  }
+}
+
+template <bool kMask>
+__global__ void __launch_bounds__(64) k_position(DevBodies b, SimParams p, SolverBufs sb, ClassSpan c) {
+  position_class<kMask>(GlobalPose{b}, b, p, sb, c, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x,
+                        [](int i) { return i; });
 }
 
 // Consecutive small classes of the visiting order in one workgroup, a barrier between classes
 // (the same corrections in the same order per body as one launch per class).
-constexpr int kPositionRun = 1024;
-template <int kLanes, bool kMask>
-__global__ void __launch_bounds__(kPositionRun) k_position_run(DevBodies b, SimParams p, SolverBufs sb, ClassRun run) {
-  const GlobalPose acc{b};
+template <bool kMask>
+__global__ void __launch_bounds__(kRunLanes) k_position_run(DevBodies b, SimParams p, SolverBufs sb, ClassRun run) {
   for (int k = 0; k < run.n; ++k) {
-    const int2 range = run.r[k];
-    for (int t = threadIdx.x; t / kLanes < range.y; t += kPositionRun)
-      position_lanes<kLanes, kMask>(acc, b, p, sb, range.x + t / kLanes);
+    position_class<kMask>(GlobalPose{b}, b, p, sb, run.r[k], threadIdx.x, kRunLanes, [](int i) { return i; });
     __syncthreads();
   }
 }
 
 // Scene-blocked position correction: one workgroup per scene, the scene's dynamic poses in LDS,
 // `iterations` passes over the colours in the visiting order with a barrier between colours.
-template <int kBlock, int kCap, int kLanes, bool kMask>
+template <int kBlock, int kCap, bool kMask>
 __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimParams p, SolverBufs sb, SceneBlocks sc,
                                                            const int* __restrict__ scene_list,
                                                            VisitOrder visit, int iterations) {
@@ -216,13 +228,10 @@ __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimPar
   }
   __syncthreads();
   const LdsPose acc{b, s_pos, s_rot, sc.local};
-  const uint32_t* st = sc.start + long(s) * (visit.n + 1);
   for (int it = 0; it < iterations; ++it) {
     for (int k = 0; k < visit.n; ++k) {
-      const int col = visit.c[k];
-      const int s0 = int(st[col]), e = int(st[col + 1]);
-      for (int i = kLanes * s0 + threadIdx.x; i < kLanes * e; i += kBlock)
-        position_lanes<kLanes, kMask>(acc, b, p, sb, sc.at(i / kLanes));
+      position_class<kMask>(acc, b, p, sb, scene_span(sc, visit, s, k), threadIdx.x, kBlock,
+                            [&](int i) { return sc.at(i); });
       __syncthreads();
     }
   }
@@ -235,68 +244,44 @@ __global__ void __launch_bounds__(kBlock) k_position_blocked(DevBodies b, SimPar
 
 }  // namespace
 
-namespace {
-
-// single: every manifold of the launch has one contact.
-template <bool kMask>
-void position_colour(const DevBodies& b, const SimParams& p, int first, int n, bool single, SolverBufs& sb,
-                     hipStream_t s) {
-  // one 64-lane workgroup per 16 (or 64) manifolds; the grid-stride loop walks what is above the cap
-  const int per = single ? 64 : 16, blocks = n < per * 32768 ? (n + per - 1) / per : 32768;
-  if (single) hipLaunchKernelGGL((k_position<1, kMask>), dim3(blocks), dim3(64), 0, s, b, p, sb, first, n);
-  else hipLaunchKernelGGL((k_position<4, kMask>), dim3(blocks), dim3(64), 0, s, b, p, sb, first, n);
+void launch_position_colour(const DevBodies& b, const SimParams& p, const ClassSpan& c, SolverBufs& sb,
+                            hipStream_t s) {
+  // 64-lane workgroups; the grid-stride loop walks what is above the cap
+  const long lanes = ((4l * c.multi + 63) & ~63l) + c.single;
+  const dim3 grid(unsigned(std::min(std::max((lanes + 63) / 64, 1l), 65536l)));
+  if (b.kmask) hipLaunchKernelGGL(k_position<true>, grid, dim3(64), 0, s, b, p, sb, c);
+  else hipLaunchKernelGGL(k_position<false>, grid, dim3(64), 0, s, b, p, sb, c);
 }
 
 template <bool kMask>
-void position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, bool single,
-                  hipStream_t s) {
-  if (single) hipLaunchKernelGGL((k_position_run<1, kMask>), dim3(1), dim3(kPositionRun), 0, s, b, p, sb, run);
-  else hipLaunchKernelGGL((k_position_run<4, kMask>), dim3(1), dim3(kPositionRun), 0, s, b, p, sb, run);
-}
-
-template <int kLanes, bool kMask>
 void position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
                       const VisitOrder& visit, int iterations, int block, hipStream_t s_small, hipStream_t s_large) {
   if (sc.n_large > 0) {
     if (block == 256)
-      hipLaunchKernelGGL((k_position_blocked<256, kLdsBodies, kLanes, kMask>), dim3(sc.n_large), dim3(256), 0, s_large,
-                         b, p, sb, sc, sc.large_list, visit, iterations);
+      hipLaunchKernelGGL((k_position_blocked<256, kLdsBodies, kMask>), dim3(sc.n_large), dim3(256), 0, s_large, b, p,
+                         sb, sc, sc.large_list, visit, iterations);
     else if (block == 512)
-      hipLaunchKernelGGL((k_position_blocked<512, kLdsBodies, kLanes, kMask>), dim3(sc.n_large), dim3(512), 0, s_large,
-                         b, p, sb, sc, sc.large_list, visit, iterations);
+      hipLaunchKernelGGL((k_position_blocked<512, kLdsBodies, kMask>), dim3(sc.n_large), dim3(512), 0, s_large, b, p,
+                         sb, sc, sc.large_list, visit, iterations);
     else
-      hipLaunchKernelGGL((k_position_blocked<1024, kLdsBodies, kLanes, kMask>), dim3(sc.n_large), dim3(1024), 0,
-                         s_large, b, p, sb, sc, sc.large_list, visit, iterations);
+      hipLaunchKernelGGL((k_position_blocked<1024, kLdsBodies, kMask>), dim3(sc.n_large), dim3(1024), 0, s_large, b,
+                         p, sb, sc, sc.large_list, visit, iterations);
   }
   if (sc.n_small > 0)
-    hipLaunchKernelGGL((k_position_blocked<64, kSmallScene, kLanes, kMask>), dim3(sc.n_small), dim3(64), 0, s_small, b,
-                       p, sb, sc, sc.small_list, visit, iterations);
-}
-
-}  // namespace
-
-void launch_position_colour(const DevBodies& b, const SimParams& p, int first, int n, bool single, SolverBufs& sb,
-                            hipStream_t s) {
-  if (b.kmask) position_colour<true>(b, p, first, n, single, sb, s);
-  else position_colour<false>(b, p, first, n, single, sb, s);
+    hipLaunchKernelGGL((k_position_blocked<kSmallLanes, kSmallScene, kMask>), dim3(sc.n_small), dim3(kSmallLanes), 0,
+                       s_small, b, p, sb, sc, sc.small_list, visit, iterations);
 }
 
 void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
-                             const VisitOrder& visit, int iterations, bool single, int block, hipStream_t s_small,
+                             const VisitOrder& visit, int iterations, int block, hipStream_t s_small,
                              hipStream_t s_large) {
-  if (b.kmask) {
-    if (single) position_blocked<1, true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
-    else position_blocked<4, true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
-  } else {
-    if (single) position_blocked<1, false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
-    else position_blocked<4, false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
-  }
+  if (b.kmask) position_blocked<true>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
+  else position_blocked<false>(b, p, sb, sc, visit, iterations, block, s_small, s_large);
 }
 
-void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, bool single,
-                         hipStream_t s) {
-  if (b.kmask) position_run<true>(b, p, sb, run, single, s);
-  else position_run<false>(b, p, sb, run, single, s);
+void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s) {
+  if (b.kmask) hipLaunchKernelGGL(k_position_run<true>, dim3(1), dim3(kRunLanes), 0, s, b, p, sb, run);
+  else hipLaunchKernelGGL(k_position_run<false>, dim3(1), dim3(kRunLanes), 0, s, b, p, sb, run);
 }
 
 }  // namespace nph

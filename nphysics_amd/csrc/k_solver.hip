@@ -24,9 +24,11 @@
 // then per sweep and contact the normal row (projected on l >= 0) and the two friction rows (bounded by
 // mu times the normal impulse just computed, zeroed when it is zero). Manifolds of one colour share no
 // dynamic body, so one launch per colour performs exactly the sequential Gauss-Seidel updates of
-// the colour order. Every manifold has two adjacent lanes, one per body (PairHalf): a lane loads its
-// body's inverse inertia and velocity increment and every contact up front, forms its body's half of
-// a row's J dv and its body's update, and the halves meet by a register exchange within the quad.
+// the colour order. A contact has two adjacent lanes, one per body (ContactLane): a lane loads its body's
+// inverse inertia and the contact, forms its body's half of the three rows at once, and then the
+// manifold's contacts take their turns, the velocity increments handed from one pair of lanes to the
+// next and the halves of J dv exchanged within the pair, both by register permutations. A class lists the manifolds with
+// several contacts first: those have four pairs of lanes each, the others one.
 //
 // Row record (4 contiguous float4 per contact, colour order): 0 n|length of the tangents' seed, 1 lever arm
 // p1 of body 1 (contact point minus centre of mass, zero for a static body)|r_n, 2 p2|r_t1,
@@ -144,20 +146,23 @@ __global__ void __launch_bounds__(256) k_colour_round(DevContacts c, int M, uint
 // so that a manifold's slot, its first row record and the classes' bounds come out of one prefix sum over
 // (manifolds per colour and tile, then contacts per colour and tile). k_colour_hist counts per tile of
 // kColourTile manifolds, k_colour_scatter ranks within its tile: lanes of equal colour find each other by
-// ballots, and three ballots more give the contacts of those before. kDigits colours at most (256, or
-// kMaxColours where a readback finds more); a colour beyond, or none yet, counts as the last, and the
+// ballots, and three ballots more give the contacts of those before. kDigits at most (512, or
+// kMaxColours where a readback finds more colours); a colour beyond, or none yet, counts as the last, and the
 // caller runs it again. The sort by a radix pass (histogram, scan, scatter, two copies back), the class starts, the
 // gather and scan of the counts, the slot records and the fix of empty classes were 14 launches and
 // one readback more: 30 us of a step at 1,233 manifolds, now 13 us.
+//
+// With kSplit a class lists its manifolds with several contacts before those with one, so that the
+// sweeps can give them different numbers of lanes: a digit is then 2 colour + (one contact).
 constexpr int kColourTile = 2048;
 
-template <int kDigits>
-__device__ __forceinline__ uint32_t colour_digit(uint32_t state) {
-  const uint32_t d = state & 0xffffu;
+template <int kDigits, bool kSplit>
+__device__ __forceinline__ uint32_t colour_digit(uint32_t state, uint32_t contacts) {
+  const uint32_t c = state & 0xffffu, d = kSplit ? 2u * c + (contacts == 1u ? 1u : 0u) : c;
   return d < uint32_t(kDigits) ? d : uint32_t(kDigits) - 1u;
 }
 
-template <int kDigits, int kThreads>
+template <int kDigits, int kThreads, bool kSplit>
 __global__ void __launch_bounds__(kThreads) k_colour_hist(DevContacts c, int M, int ntiles, SolverBufs sb,
                                                          uint32_t* ncol) {
   __shared__ uint32_t s_m[kDigits], s_c[kDigits];
@@ -170,11 +175,12 @@ __global__ void __launch_bounds__(kThreads) k_colour_hist(DevContacts c, int M, 
     const int m = int(blockIdx.x) * kColourTile + k;
     if (m >= M) break;
     const uint32_t st = sb.state[m];
-    const uint32_t d = colour_digit<kDigits>(st);
+    const uint32_t cnt = uint32_t(c.mcount[m]);
+    const uint32_t d = colour_digit<kDigits, kSplit>(st, cnt);
     const uint32_t c1 = (st & 0xffffu) + 1u;
     most = c1 > most ? c1 : most;
     atomicAdd(&s_m[d], 1u);
-    atomicAdd(&s_c[d], uint32_t(c.mcount[m]));
+    atomicAdd(&s_c[d], cnt);
   }
   atomicMax(&s_most, most);
   __syncthreads();
@@ -188,10 +194,10 @@ __global__ void __launch_bounds__(kThreads) k_colour_hist(DevContacts c, int M, 
 // Per slot (colour order): bodies with their dynamic flag in bit 30, first row record, contact
 // count and first contact index, packed into one int4; per manifold its slot and first row record; per
 // class its first slot and first row record (col_start, class_rec; one more entry ends the last).
-template <int kDigits, int kThreads>
+template <int kDigits, int kThreads, bool kSplit>
 __global__ void __launch_bounds__(kThreads) k_colour_scatter(DevContacts c, int M, int C, int ntiles, SolverBufs sb) {
   constexpr int kWaves = kThreads / 64;
-  constexpr int kBits = kDigits == 256 ? 8 : 12;
+  constexpr int kBits = kDigits == 512 ? 9 : 12;
   __shared__ uint32_t s_m[kDigits], s_c[kDigits];
   __shared__ uint32_t s_wave[kWaves][kDigits];  // per wave: manifolds, and their contacts from bit 16 up
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -215,8 +221,8 @@ __global__ void __launch_bounds__(kThreads) k_colour_scatter(DevContacts c, int 
     const int m = int(blockIdx.x) * kColourTile + k + tid;
     if (int(blockIdx.x) * kColourTile + k >= M) break;
     const bool valid = m < M;
-    const uint32_t d = valid ? colour_digit<kDigits>(sb.state[m]) : 0u;
     const uint32_t cnt = valid ? uint32_t(c.mcount[m]) : 0u;
+    const uint32_t d = valid ? colour_digit<kDigits, kSplit>(sb.state[m], cnt) : 0u;
     uint64_t same = __ballot(valid);
 #pragma unroll
     for (int i = 0; i < kBits; ++i) {
@@ -610,29 +616,11 @@ __device__ __forceinline__ void load_dv(const DevBodies& b, const Manifold<kMask
   if (m.x.d2) b.load_dv(m.x.b2, v2.l, v2.a);
 }
 
-// Solver velocity increments in HBM (the per-colour kernels) ...
+// Solver velocity increments in HBM (the per-colour kernels; the scene-blocked one has them in LDS).
 struct GlobalDv {
   DevBodies b;
   __device__ void load(int body, Dv& v) const { b.load_dv(body, v.l, v.a); }
   __device__ void store(int body, const Dv& v) const { b.store_dv(body, v.l, v.a); }
-};
-
-// ... or in LDS, indexed by the body's rank among its scene's dynamic bodies (the scene-blocked
-// kernel). The values are the same FP32 numbers either way.
-struct LdsDv {
-  float4* lin;
-  float4* ang;
-  const int* local;
-  __device__ void load(int body, Dv& v) const {
-    const int i = local[body];
-    v.l = xyz(lin[i]);
-    v.a = xyz(ang[i]);
-  }
-  __device__ void store(int body, const Dv& v) const {
-    const int i = local[body];
-    lin[i] = f4(v.l, 0.0f);
-    ang[i] = f4(v.a, 0.0f);
-  }
 };
 
 // The value of the other lane of the pair: a quad permutation (1, 0, 3, 2), one instruction, where a
@@ -643,26 +631,22 @@ __device__ __forceinline__ float pair_swap(float v) {
 }
 
 // A contact as one lane of the pair needs it: the normal, the seed's length, its body's lever arm,
-// the three r and rhs, the impulses and mu.
+// the r of the first two rows (its own record word's and the other's), of the third, the three rhs,
+// the impulses and mu. Nothing is computed on loading: a lane that loads ahead must not wait here.
 struct CHalf {
-  f3 n, p;
-  float tl;
-  float r[3], rhs[3];
+  float4 n, p;  // n|length, p|r (row 0 on lane 0, row 1 on lane 1)
+  float ro;     // the other of the two
+  float4 rhs;   // rhs 0-2|r of row 2
   float4 lam;
+  __device__ float r(int row, int h) const { return row == 2 ? rhs.w : ((row == h) ? p.w : ro); }
 };
 
 __device__ __forceinline__ void load_half(const SolverBufs& sb, uint32_t r, int h, CHalf& c) {
   const float4* q = sb.rec + long(r) * kRecFields;
-  const float4 v0 = q[0], v1 = q[1], v2 = q[2], v3 = q[3];
-  c.n = xyz(v0);
-  c.tl = v0.w;
-  c.p = h ? xyz(v2) : xyz(v1);
-  c.r[0] = v1.w;
-  c.r[1] = v2.w;
-  c.r[2] = v3.w;
-  c.rhs[0] = v3.x;
-  c.rhs[1] = v3.y;
-  c.rhs[2] = v3.z;
+  c.n = q[0];
+  c.p = q[1 + h];
+  c.ro = q[2 - h].w;
+  c.rhs = q[3];
   c.lam = sb.lam[r];
 }
 
@@ -682,8 +666,7 @@ struct PairHalf {
 };
 
 template <bool kMask>
-__device__ __forceinline__ void load_pair(const DevBodies& b, const SolverBufs& sb, const int4& q, int h,
-                                          PairHalf<kMask>& m) {
+__device__ __forceinline__ void load_pair(const DevBodies& b, const SolverBufs& sb, int4 q, int h, PairHalf<kMask>& m) {
   const int w = h ? q.y : q.x;
   m.h = h;
   m.body = w & 0x3fffffff;
@@ -704,18 +687,19 @@ __device__ __forceinline__ void flip(Dv& v) {
   v.a = neg(v.a);
 }
 
-template <bool kMask, class A>
-__device__ __forceinline__ void load_pair_dv(const A& acc, const PairHalf<kMask>& m, Dv& v) {
+// The velocity increment of the lane's body in memory: zero for a static one.
+template <class Lane>
+__device__ __forceinline__ void load_pair_dv(const DevBodies& b, const Lane& m, Dv& v) {
   if (!m.dyn) return;
-  acc.load(m.body, v);
+  b.load_dv(m.body, v.l, v.a);
   if (m.h) flip(v);
 }
 
-template <bool kMask, class A>
-__device__ __forceinline__ void store_pair_dv(const A& acc, const PairHalf<kMask>& m, Dv& v) {
+template <class Lane>
+__device__ __forceinline__ void store_pair_dv(const DevBodies& b, const Lane& m, Dv& v) {
   if (!m.dyn) return;
   if (m.h) flip(v);
-  acc.store(m.body, v);
+  b.store_dv(m.body, v.l, v.a);
 }
 
 // The lane's half of the row along d: the jacobian (masked) and its weighted angular part.
@@ -731,15 +715,15 @@ __device__ __forceinline__ void half_row(const PairHalf<kMask>& m, f3 p, f3 d, f
 __device__ __forceinline__ void pair_tangents(const CHalf& c, int h, f3& t1, f3& t2) {
   const bool sel = fabsf(c.n.x) > fabsf(c.n.y);
   const float a0 = sel ? c.n.z : -c.n.z, a1 = sel ? -c.n.x : c.n.y;
-  const float mine = (h ? a1 : a0) / c.tl, other = pair_swap(mine);
+  const float mine = (h ? a1 : a0) / c.n.w, other = pair_swap(mine);
   const float u = h ? other : mine, v = h ? mine : other;
   t2 = sel ? f3{u, 0.0f, v} : f3{0.0f, u, v};
-  t1 = cross(t2, c.n);
+  t1 = cross(t2, xyz(c.n));
 }
 
 // Warm start of one manifold (SORProx::warmstart_set, sor_prox.rs:19-45): dv += l W J for every
 // row with l != 0, normal rows first, then friction rows. The lanes need nothing of each other but the
-// quotients of the tangents.
+// quotients of the tangents; that of a static body runs along for them.
 template <bool kMask>
 __device__ __forceinline__ void pair_warm(const PairHalf<kMask>& m, Dv& v) {
   f3 dh, ah, wah;
@@ -747,7 +731,7 @@ __device__ __forceinline__ void pair_warm(const PairHalf<kMask>& m, Dv& v) {
   for (int k = 0; k < 4; ++k) {
     if (k >= m.cnt) break;
     if (m.c[k].lam.x == 0.0f) continue;
-    half_row(m, m.c[k].p, neg(m.c[k].n), dh, ah, wah);
+    half_row(m, xyz(m.c[k].p), neg(xyz(m.c[k].n)), dh, ah, wah);
     axpy6(m.c[k].lam.x, scale(dh, m.im), wah, v);
   }
 #pragma unroll
@@ -757,154 +741,305 @@ __device__ __forceinline__ void pair_warm(const PairHalf<kMask>& m, Dv& v) {
     f3 t1, t2;
     pair_tangents(m.c[k], m.h, t1, t2);
     if (m.c[k].lam.y != 0.0f) {
-      half_row(m, m.c[k].p, t1, dh, ah, wah);
+      half_row(m, xyz(m.c[k].p), t1, dh, ah, wah);
       axpy6(m.c[k].lam.y, scale(dh, m.im), wah, v);
     }
     if (m.c[k].lam.z != 0.0f) {
-      half_row(m, m.c[k].p, t2, dh, ah, wah);
+      half_row(m, xyz(m.c[k].p), t2, dh, ah, wah);
       axpy6(m.c[k].lam.z, scale(dh, m.im), wah, v);
     }
   }
 }
 
-// One SOR-Prox step of one manifold (sor_prox.rs:159-343), contact by contact: the normal row,
-// projected on l >= 0, then the two friction rows, bounded by mu times that normal impulse and
-// zeroed when it is zero. Both lanes form w = (s1 + s2) + rhs and the same new impulse.
+// One lane of a contact of a manifold: its body's inverse mass and inertia and jacobian masks, the contact.
+// The loads are unconditional, so that none waits for a branch: a static body's solver block
+// holds zeros, and a lane without a contact of its own (k >= cnt) reads the manifold's last one.
 template <bool kMask>
-__device__ __forceinline__ void pair_sweep(PairHalf<kMask>& m, Dv& v) {
+struct ContactLane {
+  int body, cnt, k, h;
+  bool dyn;
+  uint32_t r;  // its record
+  float4 i0, i1, i2;
+  f3 ml, ma;
+  CHalf c;
+};
+
+template <bool kMask>
+__device__ __forceinline__ void load_lane(const DevBodies& b, const SolverBufs& sb, int4 q, int k, int h,
+                                          ContactLane<kMask>& m) {
+  const int w = h ? q.y : q.x;
+  m.k = k;
+  m.h = h;
+  m.body = w & 0x3fffffff;
+  m.dyn = (w >> 30) & 1;
+  m.cnt = q.w & 7;
+  m.r = uint32_t(q.z) + uint32_t(k < m.cnt ? k : (m.cnt > 0 ? m.cnt - 1 : 0));
+  const float4* s = b.solver(m.body);
+  m.i0 = s[0];
+  m.i1 = s[1];
+  m.i2 = s[2];
+  load_half(sb, m.r, h, m.c);
+  if (kMask) b.mask(m.body, m.ml, m.ma);
+}
+
+// The value two lanes before, within the sixteen lanes of a row: the pair of the previous contact.
+__device__ __forceinline__ float pair_before(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x112, 0xf, 0xf, true));
+}
+
+// One SOR-Prox step of a manifold (sor_prox.rs:159-343) on its lanes, contact by contact: the normal
+// row, projected on l >= 0, then the two friction rows, bounded by mu times that normal impulse
+// and zeroed when it is zero. Both lanes of a pair form w = (s1 + s2) + rhs and the same new impulse.
+// v enters on the first pair of lanes and leaves on the last contact's. What the rows are made of does
+// not depend on v and is formed for all contacts at once; the wave takes as many turns as its largest manifold.
+template <bool kMask>
+__device__ __forceinline__ void sweep_lanes(ContactLane<kMask>& m, Dv& v) {
+  CHalf& c = m.c;
+  m33 I;
+  I.m[0][0] = m.i0.x; I.m[0][1] = m.i0.y; I.m[0][2] = m.i0.z;
+  I.m[1][0] = m.i1.x; I.m[1][1] = m.i1.y; I.m[1][2] = m.i1.z;
+  I.m[2][0] = m.i1.w; I.m[2][1] = m.i2.x; I.m[2][2] = m.i2.y;
+  const float im = m.i0.w;
+  f3 d[3], a[3], wl[3], wa[3];
+  d[0] = neg(xyz(c.n));
+  pair_tangents(c, m.h, d[1], d[2]);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= m.cnt) break;
-    CHalf& c = m.c[k];
-    f3 dh, ah, wah;
-    half_row(m, c.p, neg(c.n), dh, ah, wah);
-    {
-      const float s = dot6(dh, ah, v);
-      const float w = (s + pair_swap(s)) + c.rhs[0];
-      const float a = c.lam.x - c.r[0] * w;
-      const float ni = a > 0.0f ? a : 0.0f;
-      const float dl = ni - c.lam.x;
-      c.lam.x = ni;
-      axpy6(dl, scale(dh, m.im), wah, v);
+  for (int row = 0; row < 3; ++row) {
+    a[row] = cross(xyz(c.p), d[row]);
+    if (kMask) {
+      d[row] = cmul(d[row], m.ml);
+      a[row] = cmul(a[row], m.ma);
     }
-    const float ln = c.lam.x;
-    f3 t[2];
-    pair_tangents(c, m.h, t[0], t[1]);
-#pragma unroll
-    for (int f = 1; f <= 2; ++f) {
-      float li = f == 1 ? c.lam.y : c.lam.z;
-      half_row(m, c.p, t[f - 1], dh, ah, wah);
-      if (ln == 0.0f) {
-        if (li != 0.0f) {
-          axpy6(-li, scale(dh, m.im), wah, v);
-          li = 0.0f;
-        }
-      } else {
-        const float mx = c.lam.w * ln;
-        const float mn = -mx;
-        const float s = dot6(dh, ah, v);
-        const float w = (s + pair_swap(s)) + c.rhs[f];
-        const float val = li - c.r[f] * w;
-        const float ni = val > mn ? (val < mx ? val : mx) : mn;
-        const float dl = ni - li;
-        li = ni;
-        axpy6(dl, scale(dh, m.im), wah, v);
+    wl[row] = scale(d[row], im);
+    wa[row] = mulv(I, a[row]);
+  }
+  for (int turn = 0;;) {
+    if (m.k == turn && turn < m.cnt) {
+      {
+        const float s = dot6(d[0], a[0], v);
+        const float w = (s + pair_swap(s)) + c.rhs.x;
+        const float x = c.lam.x - c.r(0, m.h) * w;
+        const float ni = x > 0.0f ? x : 0.0f;
+        const float dl = ni - c.lam.x;
+        c.lam.x = ni;
+        axpy6(dl, wl[0], wa[0], v);
       }
-      if (f == 1) c.lam.y = li;
-      else c.lam.z = li;
+      const float ln = c.lam.x;
+#pragma unroll
+      for (int f = 1; f <= 2; ++f) {
+        float li = f == 1 ? c.lam.y : c.lam.z;
+        if (ln == 0.0f) {
+          if (li != 0.0f) {
+            axpy6(-li, wl[f], wa[f], v);
+            li = 0.0f;
+          }
+        } else {
+          const float mx = c.lam.w * ln;
+          const float mn = -mx;
+          const float s = dot6(d[f], a[f], v);
+          const float w = (s + pair_swap(s)) + (f == 1 ? c.rhs.y : c.rhs.z);
+          const float val = li - c.r(f, m.h) * w;
+          const float ni = val > mn ? (val < mx ? val : mx) : mn;
+          const float dl = ni - li;
+          li = ni;
+          axpy6(dl, wl[f], wa[f], v);
+        }
+        if (f == 1) c.lam.y = li;
+        else c.lam.z = li;
+      }
     }
+    ++turn;
+    if (!__any(m.cnt > turn)) break;
+    const Dv u{f3{pair_before(v.l.x), pair_before(v.l.y), pair_before(v.l.z)},
+               f3{pair_before(v.a.x), pair_before(v.a.y), pair_before(v.a.z)}};
+    if (m.k == turn) v = u;
   }
 }
 
+// Whether this lane's pair holds the manifold's result.
 template <bool kMask>
-__device__ __forceinline__ void store_pair_lam(const SolverBufs& sb, const PairHalf<kMask>& m) {
-  if (m.h) return;
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    if (k < m.cnt) sb.lam[m.r0 + k] = m.c[k].lam;
+__device__ __forceinline__ bool last_pair(const ContactLane<kMask>& m) {
+  return m.dyn && m.k == m.cnt - 1;
 }
 
-// The warm start or one sweep step of the manifold in `slot`, on this lane's side.
-template <bool kWarm, bool kMask, class A>
-__device__ __forceinline__ void solve_pair(const A& acc, const DevBodies& b, const SolverBufs& sb, int slot, int h) {
-  PairHalf<kMask> m;
-  load_pair(b, sb, sb.sinfo[slot], h, m);
-  Dv v{};
-  load_pair_dv(acc, m, v);
-  if (kWarm) pair_warm(m, v);
-  else pair_sweep(m, v);
-  store_pair_dv(acc, m, v);
-  if (!kWarm) store_pair_lam(sb, m);
+template <bool kMask>
+__device__ __forceinline__ void store_lane_lam(const SolverBufs& sb, const ContactLane<kMask>& m) {
+  if (m.h == 0 && m.k < m.cnt) sb.lam[m.r] = m.c.lam;
 }
 
-// One colour of the warm start or of one sweep (the grid covers both lanes of every pair in one
-// wavefront: blockDim and the stride are even).
+// Slot and contact of lane L of a class, or false beyond its lanes.
+__device__ __forceinline__ bool lane_at(const ClassSpan& c, int L, int& slot, int& k) {
+  const bool several = L < 8 * c.multi;
+  const int l = L - 8 * c.multi;
+  slot = several ? c.first + (L >> 3) : c.first + c.multi + (l >> 1);
+  k = several ? (L >> 1) & 3 : 0;
+  return several || l < 2 * c.single;
+}
+
+// Lane L's part of the warm start of a class (two lanes per manifold) or of one sweep, at velocity increments in memory.
 template <bool kWarm, bool kMask>
-__global__ void __launch_bounds__(64) k_pgs(DevBodies b, SolverBufs sb, int first, int n) {
-  const GlobalDv acc{b};
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; (t >> 1) < n; t += gridDim.x * blockDim.x)
-    solve_pair<kWarm, kMask>(acc, b, sb, first + (t >> 1), t & 1);
+__device__ __forceinline__ void class_lane(const DevBodies& b, const SolverBufs& sb, const ClassSpan& c, int L) {
+  Dv v{};
+  if (kWarm) {
+    if ((L >> 1) >= c.multi + c.single) return;
+    PairHalf<kMask> m;
+    load_pair(b, sb, sb.sinfo[c.first + (L >> 1)], L & 1, m);
+    load_pair_dv(b, m, v);
+    pair_warm(m, v);
+    store_pair_dv(b, m, v);
+  } else {
+    int slot, k;
+    if (!lane_at(c, L, slot, k)) return;
+    ContactLane<kMask> m;
+    load_lane(b, sb, sb.sinfo[slot], k, L & 1, m);
+    load_pair_dv(b, m, v);
+    sweep_lanes(m, v);
+    if (last_pair(m)) store_pair_dv(b, m, v);
+    store_lane_lam(sb, m);
+  }
+}
+
+// One colour of the warm start or of one sweep. A launch's latency bounds it: ids, then body and
+// contact, then the manifold's contacts in turn. With the contacts of a manifold in a loop on two lanes
+// the rows of each were formed in its turn; on lanes of their own they are formed at once:
+// velocity solve 460 -> 412 us at 10,795 manifolds of 3.3 contacts, 1,554 -> 1,439 at 248,353 of 1.3.
+template <bool kWarm, bool kMask>
+__global__ void __launch_bounds__(64) k_pgs(DevBodies b, SolverBufs sb, ClassSpan c) {
+  class_lane<kWarm, kMask>(b, sb, c, blockIdx.x * 64 + threadIdx.x);
 }
 
 // A run of consecutive small colour classes of the visiting order in one workgroup, a barrier
 // between classes: per body the same updates in the same order as one launch per class, without
-// a launch per class. Each class fits one pass of the workgroup.
+// a launch per class. Each class fits one pass of the workgroup, whose compute unit's issue rate bounds it
+// (the next class's ids loaded ahead: no gain).
 template <bool kWarm, bool kMask>
-__global__ void __launch_bounds__(2 * kRunBlock) k_colour_run(DevBodies b, SolverBufs sb, ClassRun run) {
-  const GlobalDv acc{b};
+__global__ void __launch_bounds__(kRunLanes) k_colour_run(DevBodies b, SolverBufs sb, ClassRun run) {
   for (int k = 0; k < run.n; ++k) {
-    const int t = threadIdx.x;
-    if ((t >> 1) < run.r[k].y) solve_pair<kWarm, kMask>(acc, b, sb, run.r[k].x + (t >> 1), t & 1);
+    class_lane<kWarm, kMask>(b, sb, run.r[k], threadIdx.x);
     __syncthreads();
   }
 }
 
-// Scene-blocked sweeps: one workgroup per scene runs the warm start (when warm, one lane per
-// manifold) and nsweeps sweeps (two lanes per manifold, as k_pgs) over all colours in the visiting
-// order, with the scene's dynamic-body velocity increments resident in LDS and a workgroup barrier
-// between colours. Every body sees the same sequence of row updates as under the per-colour
-// launches (manifolds of one colour share no dynamic body; colours and sweeps keep their order),
-// so the results are identical.
+// Scene-blocked sweeps: one workgroup per scene runs the warm start (when warm) and nsweeps sweeps over
+// all colours in the visiting order, two lanes per manifold as k_pgs, the scene's dynamic-body velocity increments
+// resident in LDS and a barrier between colours. Every body sees the same sequence of row updates as
+// under the per-colour launches (manifolds of one colour share no dynamic body; colours and sweeps
+// keep their order), so the results are identical.
+//
+// A phase (one colour) is short, so what it waits for decides: the body and the contact of a
+// lane's next phase are loaded while this one is solved, and the ids of the one after (info, in the scene's
+// order). No load's latency stands between two barriers, and the barrier orders LDS alone. Impulses are stored before
+// the barrier and read again visit.n - 1 phases later at the earliest (visit.n >= 2): the stores of
+// all earlier phases are waited for before a phase's loads are issued. The scene's one compute unit
+// bounds it, by its issue rate: 428 us at 1,021 scenes of 100 bodies (405 with a launch per class),
+// 188 against 155 at one of 1,001, and faster where many tiny classes follow one another.
+struct SceneItem {
+  int4 q;
+  int k, local;  // contact, rank of this lane's body in its scene (static: any)
+};
+
+__device__ __forceinline__ void barrier_lds() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 template <int kBlock, int kCap, bool kMask>
 __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBufs sb, SceneBlocks sc,
                                                          const int* __restrict__ scene_list, VisitOrder visit,
                                                          int nsweeps, int warm) {
-  __shared__ float4 s_lin[kCap];
-  __shared__ float4 s_ang[kCap];
-  const int s = scene_list[blockIdx.x];
+  __shared__ float4 s_a[kCap];  // linear x, y, z, angular x
+  __shared__ float2 s_b[kCap];  // angular y, z
+  __shared__ ClassSpan s_span[kVisitColours];
+  const int s = scene_list[blockIdx.x], tid = threadIdx.x, h = tid & 1;
   const int d0 = sc.dyn_start[s], nd = sc.dyn_start[s + 1] - d0;
-  for (int i = threadIdx.x; i < nd; i += kBlock) {
-    const int body = sc.dyn_list[d0 + i];
+  const int n = visit.n;
+  for (int k = tid; k < n; k += kBlock) s_span[k] = scene_span(sc, visit, s, k);
+  for (int i = tid; i < nd; i += kBlock) {
     f3 l, a;
-    b.load_dv(body, l, a);
-    s_lin[i] = f4(l, 0.0f);
-    s_ang[i] = f4(a, 0.0f);
+    b.load_dv(sc.dyn_list[d0 + i], l, a);
+    s_a[i] = make_float4(l.x, l.y, l.z, a.x);
+    s_b[i] = make_float2(a.y, a.z);
   }
   __syncthreads();
-  const LdsDv acc{s_lin, s_ang, sc.local};
-  const uint32_t* st = sc.start + long(s) * (visit.n + 1);
-  for (int pass = warm ? -1 : 0; pass < nsweeps; ++pass) {
-    for (int k = 0; k < visit.n; ++k) {
-      const int col = visit.c[k];
-      const int s0 = int(st[col]), e = int(st[col + 1]);
-      if (pass < 0) {
-        for (int i = 2 * s0 + threadIdx.x; i < 2 * e; i += kBlock)
-          solve_pair<true, kMask>(acc, b, sb, sc.at(i >> 1), i & 1);
-      } else {
-        // both lanes of a manifold are adjacent lanes of one wavefront (kBlock and 2 * s0 are even)
-        for (int i = 2 * s0 + threadIdx.x; i < 2 * e; i += kBlock)
-          solve_pair<false, kMask>(acc, b, sb, sc.at(i >> 1), i & 1);
+  auto item = [&](int class_at, int L, SceneItem& it) {
+    int at;
+    it.q = make_int4(0, 0, 0, 0);  // a manifold without contacts
+    it.local = 0;
+    const bool in = lane_at(s_span[class_at], L, at, it.k);
+    if (in) {
+      it.q = sc.info[at];
+      it.local = reinterpret_cast<const int*>(sc.rank)[2 * at + h];
+    }
+    return in;
+  };
+  auto load_v = [&](bool dyn, int local, Dv& v) {
+    v = Dv{};
+    if (!dyn) return;
+    const float4 x = s_a[local];
+    const float2 y = s_b[local];
+    v.l = xyz(x);
+    v.a = f3{x.w, y.x, y.y};
+    if (h) flip(v);
+  };
+  auto store_v = [&](int local, Dv& v) {
+    if (h) flip(v);
+    s_a[local] = make_float4(v.l.x, v.l.y, v.l.z, v.a.x);
+    s_b[local] = make_float2(v.a.y, v.a.z);
+  };
+  if (warm) {
+    for (int k = 0; k < n; ++k) {
+      const ClassSpan c = s_span[k];
+      for (int t = tid; (t >> 1) < c.multi + c.single; t += kBlock) {
+        PairHalf<kMask> m;
+        const int at = c.first + (t >> 1);
+        load_pair(b, sb, sc.info[at], h, m);
+        const int local = reinterpret_cast<const int*>(sc.rank)[2 * at + h];
+        Dv v;
+        load_v(m.dyn, local, v);
+        pair_warm(m, v);
+        if (m.dyn) store_v(local, v);
       }
-      __syncthreads();
+      barrier_lds();
     }
   }
-  for (int i = threadIdx.x; i < nd; i += kBlock) {
-    const int body = sc.dyn_list[d0 + i];
-    b.store_dv(body, xyz(s_lin[i]), xyz(s_ang[i]));
+  auto after = [&](int c) { return c + 1 < n ? c + 1 : 0; };
+  int k = 0;  // class visited in this phase
+  SceneItem it, here;
+  ContactLane<kMask> next;
+  item(0, tid, here);
+  load_lane(b, sb, here.q, here.k, h, next);
+  item(after(0), tid, it);
+  for (int ph = 0; ph < n * nsweeps; ++ph) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ContactLane<kMask> m = next;
+    int local = here.local;
+    here = it;
+    load_lane(b, sb, it.q, it.k, h, next);
+    item(after(after(k)), tid, it);
+    for (int L = tid;;) {
+      if (m.cnt) {
+        Dv v;
+        load_v(m.dyn, local, v);
+        sweep_lanes(m, v);
+        if (last_pair(m)) store_v(local, v);
+        store_lane_lam(sb, m);
+      }
+      L += kBlock;  // the class's manifolds beyond one workgroup's worth
+      SceneItem more;
+      if (!item(k, L, more)) break;
+      load_lane(b, sb, more.q, more.k, h, m);
+      local = more.local;
+    }
+    barrier_lds();
+    k = after(k);
+  }
+  for (int i = tid; i < nd; i += kBlock) {
+    const float4 x = s_a[i];
+    const float2 y = s_b[i];
+    b.store_dv(sc.dyn_list[d0 + i], xyz(x), f3{x.w, y.x, y.y});
   }
 }
 
-// Scene-major slot order for the blocked kernel: the slots are in colour order, so a stable sort by scene
+// Scene-major slot order for the blocked kernels: the slots are in colour order, so a stable sort by scene
 // leaves them in (scene, colour) order.
 __global__ void __launch_bounds__(256) k_scene_keys(DevBodies b, int M, SolverBufs sb, uint32_t* keys,
                                                    uint32_t* slots) {
@@ -915,7 +1050,16 @@ __global__ void __launch_bounds__(256) k_scene_keys(DevBodies b, int M, SolverBu
   slots[i] = uint32_t(i);
 }
 
-// start[s][c] = first position of (scene s, colour >= c) in the sorted slots (lower bound).
+// The slots' records in that order (one scene: in slot order), each with its bodies' ranks in their scene.
+__global__ void __launch_bounds__(256) k_scene_info(int M, SolverBufs sb, SceneBlocks sc) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= M) return;
+  const int4 q = sb.sinfo[sc.at(i)];
+  sc.info[i] = q;
+  sc.rank[i] = make_int2(sc.local[q.x & 0x3fffffff], sc.local[q.y & 0x3fffffff]);
+}
+
+// start[s][d] = first position of (scene s, digit of the colour order >= d) in the sorted slots (lower bound).
 __global__ void __launch_bounds__(256) k_scene_starts(const uint32_t* __restrict__ keys,
                                                      const uint32_t* __restrict__ slot,
                                                      const uint32_t* __restrict__ colour, int M, int nscenes,
@@ -1118,12 +1262,12 @@ void launch_colour_round(const DevContacts& c, int M, int round, uint32_t* remai
 }
 
 namespace {
-template <int kDigits, int kThreads>
+template <int kDigits, int kThreads, bool kSplit>
 void colour_order(const DevContacts& c, int M, int C, SolverBufs& sb, uint32_t* ncol, hipStream_t s) {
   const int ntiles = (M + kColourTile - 1) / kColourTile;
-  hipLaunchKernelGGL((k_colour_hist<kDigits, kThreads>), dim3(ntiles), dim3(kThreads), 0, s, c, M, ntiles, sb, ncol);
+  hipLaunchKernelGGL((k_colour_hist<kDigits, kThreads, kSplit>), dim3(ntiles), dim3(kThreads), 0, s, c, M, ntiles, sb, ncol);
   scan_exclusive_u32(sb.hist, sb.offs, 2 * kDigits * ntiles, *sb.scan, s);
-  hipLaunchKernelGGL((k_colour_scatter<kDigits, kThreads>), dim3(ntiles), dim3(kThreads), 0, s, c, M, C, ntiles, sb);
+  hipLaunchKernelGGL((k_colour_scatter<kDigits, kThreads, kSplit>), dim3(ntiles), dim3(kThreads), 0, s, c, M, C, ntiles, sb);
 }
 }  // namespace
 
@@ -1131,10 +1275,11 @@ size_t colour_hist_words(int M, int digits) {
   return 2 * size_t(digits) * size_t((M + kColourTile - 1) / kColourTile);
 }
 
-void launch_colour_order(const DevContacts& c, int M, int C, int digits, SolverBufs& sb, uint32_t* ncol,
+void launch_colour_order(const DevContacts& c, int M, int C, int digits, bool split, SolverBufs& sb, uint32_t* ncol,
                          hipStream_t s) {
-  if (digits == 256) colour_order<256, 256>(c, M, C, sb, ncol, s);
-  else colour_order<kMaxColours, 64>(c, M, C, sb, ncol, s);
+  if (digits != kColourDigits) colour_order<kMaxColours, 64, false>(c, M, C, sb, ncol, s);
+  else if (split) colour_order<kColourDigits, 256, true>(c, M, C, sb, ncol, s);
+  else colour_order<kColourDigits, 256, false>(c, M, C, sb, ncol, s);
 }
 
 void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContacts& prev, int prevM,
@@ -1143,43 +1288,37 @@ void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContac
   hipLaunchKernelGGL(k_assemble, dim3(nb(M)), dim3(256), 0, s, b, cur, prev, prevM, M, p, sb, mt);
 }
 
-// One lane per manifold: the cap on a colour launch's grid, one 64-lane workgroup per 64
-// manifolds of the largest colour class rounded up to a power of two, at least 64 and at most
-// 8,192; each class is launched with the workgroups it needs under that cap, and larger classes
-// are walked by the grid-stride loop.
-int sweep_blocks(int max_class) {
-  int need = (max_class + 63) / 64;
-  int blocks = 64;
-  while (blocks < need && blocks < 8192) blocks *= 2;
-  return blocks;
-}
+// 64-lane workgroups for a class's lanes (at most 8 a manifold: the grid stays within its limits).
+static unsigned lane_blocks(long lanes) { return unsigned(std::max((lanes + 63) / 64, 1l)); }
 
 // The masked kernel variants run only in worlds where some dynamic body has a kinematic dof.
-void launch_warmstart_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s) {
-  if (b.kmask) hipLaunchKernelGGL((k_pgs<true, true>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
-  else hipLaunchKernelGGL((k_pgs<true, false>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
+void launch_warmstart_colour(const DevBodies& b, const ClassSpan& c, SolverBufs& sb, hipStream_t s) {
+  const dim3 grid(lane_blocks(2l * (c.multi + c.single)));
+  if (b.kmask) hipLaunchKernelGGL((k_pgs<true, true>), grid, dim3(64), 0, s, b, sb, c);
+  else hipLaunchKernelGGL((k_pgs<true, false>), grid, dim3(64), 0, s, b, sb, c);
 }
 
-void launch_pgs_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s, hipEvent_t ev0,
+void launch_pgs_colour(const DevBodies& b, const ClassSpan& c, SolverBufs& sb, hipStream_t s, hipEvent_t ev0,
                        hipEvent_t ev1) {
+  const dim3 grid(lane_blocks(8l * c.multi + 2l * c.single));
   // with events, the dispatch packet itself records both, timing the kernel alone
   if (b.kmask) {
-    if (ev0) hipExtLaunchKernelGGL((k_pgs<false, true>), dim3(blocks), dim3(64), 0, s, ev0, ev1, 0, b, sb, first, n);
-    else hipLaunchKernelGGL((k_pgs<false, true>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
+    if (ev0) hipExtLaunchKernelGGL((k_pgs<false, true>), grid, dim3(64), 0, s, ev0, ev1, 0, b, sb, c);
+    else hipLaunchKernelGGL((k_pgs<false, true>), grid, dim3(64), 0, s, b, sb, c);
     return;
   }
-  if (ev0) hipExtLaunchKernelGGL((k_pgs<false, false>), dim3(blocks), dim3(64), 0, s, ev0, ev1, 0, b, sb, first, n);
-  else hipLaunchKernelGGL((k_pgs<false, false>), dim3(blocks), dim3(64), 0, s, b, sb, first, n);
+  if (ev0) hipExtLaunchKernelGGL((k_pgs<false, false>), grid, dim3(64), 0, s, ev0, ev1, 0, b, sb, c);
+  else hipLaunchKernelGGL((k_pgs<false, false>), grid, dim3(64), 0, s, b, sb, c);
 }
 
 void launch_colour_run(const DevBodies& b, SolverBufs& sb, const ClassRun& run, bool warm, hipStream_t s) {
   if (b.kmask) {
-    if (warm) hipLaunchKernelGGL((k_colour_run<true, true>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
-    else hipLaunchKernelGGL((k_colour_run<false, true>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
+    if (warm) hipLaunchKernelGGL((k_colour_run<true, true>), dim3(1), dim3(kRunLanes), 0, s, b, sb, run);
+    else hipLaunchKernelGGL((k_colour_run<false, true>), dim3(1), dim3(kRunLanes), 0, s, b, sb, run);
     return;
   }
-  if (warm) hipLaunchKernelGGL((k_colour_run<true, false>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
-  else hipLaunchKernelGGL((k_colour_run<false, false>), dim3(1), dim3(2 * kRunBlock), 0, s, b, sb, run);
+  if (warm) hipLaunchKernelGGL((k_colour_run<true, false>), dim3(1), dim3(kRunLanes), 0, s, b, sb, run);
+  else hipLaunchKernelGGL((k_colour_run<false, false>), dim3(1), dim3(kRunLanes), 0, s, b, sb, run);
 }
 
 int residual_blocks(int M) { return int(nb(M > 0 ? M : 1)); }
@@ -1221,37 +1360,39 @@ void launch_lam_copy(SolverBufs& sb, int C, float4* buf, bool to_buf, hipStream_
   hipLaunchKernelGGL(k_lam_copy, dim3(nb(C)), dim3(256), 0, s, sb, C, buf, to_buf ? 1 : 0);
 }
 
-void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int ncolours, SolverBufs& sb,
+void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int digits, SolverBufs& sb,
                         SceneBlocks& sc, hipStream_t s) {
   if (M == 0) return;
-  hipLaunchKernelGGL(k_scene_keys, dim3(nb(M)), dim3(256), 0, s, b, M, sb, sc.keys, sc.slot);
-  radix_sort_pairs(sc.keys, sc.slot, sc.keys_alt, sc.slot_alt, M, (scene_bits + 15) / 16 * 16, sb.tmp, *sb.scan, s);
-  const long total = long(nscenes) * (ncolours + 1);
-  hipLaunchKernelGGL(k_scene_starts, dim3(nb(total)), dim3(256), 0, s, sc.keys, sc.slot, sb.ckeys, M, nscenes,
-                     ncolours, sc.start);
+  if (sc.slot) {
+    hipLaunchKernelGGL(k_scene_keys, dim3(nb(M)), dim3(256), 0, s, b, M, sb, sc.keys, sc.slot);
+    radix_sort_pairs(sc.keys, sc.slot, sc.keys_alt, sc.slot_alt, M, (scene_bits + 15) / 16 * 16, sb.tmp, *sb.scan, s);
+    const long total = long(nscenes) * (digits + 1);
+    hipLaunchKernelGGL(k_scene_starts, dim3(nb(total)), dim3(256), 0, s, sc.keys, sc.slot, sb.ckeys, M, nscenes, digits,
+                       sc.start);
+  }
+  hipLaunchKernelGGL(k_scene_info, dim3(nb(M)), dim3(256), 0, s, M, sb, sc);
 }
 
-// Two launches: the scenes with more than kSmallScene dynamic bodies (`block` lanes, 64 KB of LDS)
-// on s_large, the others (64-lane workgroups, 8 KB of LDS, many resident per CU) on s_small, so the
-// few large scenes run beside the many small ones.
+// Two launches: the scenes with more than kSmallScene dynamic bodies (256 or 512 lanes, 48 KB of LDS)
+// on s_large, the others (64-lane workgroups, many resident per CU) on s_small, so the few large
+// scenes run beside the many small ones.
 template <bool kMask>
 void sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit, int nsweeps,
                     bool warm, int block, hipStream_t s_small, hipStream_t s_large) {
   const int w = warm ? 1 : 0;
-  if (kMask && block == 1024) block = 512;  // the masked kernel would spill at 1024 lanes (128 VGPRs)
   if (sc.n_large > 0) {
     if (block == 256)
       hipLaunchKernelGGL((k_sweeps_blocked<256, kLdsBodies, kMask>), dim3(sc.n_large), dim3(256), 0, s_large, b, sb,
                          sc, sc.large_list, visit, nsweeps, w);
-    else if (kMask || block == 512)
-      hipLaunchKernelGGL((k_sweeps_blocked<512, kLdsBodies, kMask>), dim3(sc.n_large), dim3(512), 0, s_large, b, sb,
+    else if (block == 1024)
+      hipLaunchKernelGGL((k_sweeps_blocked<1024, kLdsBodies, kMask>), dim3(sc.n_large), dim3(1024), 0, s_large, b, sb,
                          sc, sc.large_list, visit, nsweeps, w);
     else
-      hipLaunchKernelGGL((k_sweeps_blocked<1024, kLdsBodies, false>), dim3(sc.n_large), dim3(1024), 0, s_large, b,
-                         sb, sc, sc.large_list, visit, nsweeps, w);
+      hipLaunchKernelGGL((k_sweeps_blocked<512, kLdsBodies, kMask>), dim3(sc.n_large), dim3(512), 0, s_large, b, sb,
+                         sc, sc.large_list, visit, nsweeps, w);
   }
   if (sc.n_small > 0)
-    hipLaunchKernelGGL((k_sweeps_blocked<64, kSmallScene, kMask>), dim3(sc.n_small), dim3(64), 0, s_small, b, sb, sc,
+    hipLaunchKernelGGL((k_sweeps_blocked<kSmallLanes, kSmallScene, kMask>), dim3(sc.n_small), dim3(kSmallLanes), 0, s_small, b, sb, sc,
                        sc.small_list, visit, nsweeps, w);
 }
 

@@ -165,31 +165,37 @@ void launch_colour_begin(const DevBodies& b, const DevContacts& c, int M, const 
 // coloured one
 void launch_colour_round(const DevContacts& c, int M, int round, uint32_t* remaining, uint32_t* last_round,
                          SolverBufs& sb, hipStream_t s);
-// Slots, records and classes in colour order, for up to `digits` colours (256 or kMaxColours); *ncol, zero
-// before, becomes the number of colours.
+// Slots, records and classes in colour order; *ncol, zero before, becomes the number of colours. With
+// kColourDigits digits and `split`, up to kColourDigits / 2 colours with the manifolds of several contacts first in
+// each (class c begins at digits 2 c and 2 c + 1), without it up to `digits` (kColourDigits or kMaxColours) colours.
+constexpr int kColourDigits = 512;
 size_t colour_hist_words(int M, int digits);
-void launch_colour_order(const DevContacts& c, int M, int C, int digits, SolverBufs& sb, uint32_t* ncol,
+void launch_colour_order(const DevContacts& c, int M, int C, int digits, bool split, SolverBufs& sb, uint32_t* ncol,
                          hipStream_t s);
 int residual_blocks(int M);
 void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContacts& prev,
                      int prevM, int M, const SimParams& p, SolverBufs& sb, const MatTable& mt, hipStream_t s);
-// Sweep kernels of the colour visited k-th; their slot ranges are read on the device, so the
-// launches are independent of per-step sizes (grid = blocks from the largest colour class,
-// grid-stride over the colour).
-int sweep_blocks(int max_class);
-// (first, n): the class's slot range, known on the host from the visiting order
-void launch_warmstart_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s);
-// Consecutive visited classes, each of at most kRunBlock manifolds, as (first slot, slots), in one
-// workgroup (warm start or sweep). Passed by value: no copy to the device stands before the launch.
-constexpr int kRunBlock = 512;
+// A colour class: its first slot, its manifolds with several contacts (or of any number, where the
+// order is not split) and after them those with one.
+struct ClassSpan {
+  int first, multi, single;
+};
+// One colour of the warm start and of a sweep.
+void launch_warmstart_colour(const DevBodies& b, const ClassSpan& c, SolverBufs& sb, hipStream_t s);
+void launch_pgs_colour(const DevBodies& b, const ClassSpan& c, SolverBufs& sb, hipStream_t s,
+                       hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// Consecutive visited classes, each of at most kRunLanes sweep lanes (8 for a manifold of several contacts, 2
+// for one of one), in one workgroup (warm start or sweep). Beyond that a launch of the class's own, on
+// many compute units, is faster: velocity solve 254 us against 316 with two or three passes of the workgroup at
+// 627 manifolds of 2.7 contacts; with half the lanes 172 us against 155 at 1,233 of one contact, and 406 either way at
+// 23,730. Passed by value: no copy to the device stands before the launch.
+constexpr int kRunLanes = 1024;
 constexpr int kRunClasses = 64;
 struct ClassRun {
   int n;
-  int2 r[kRunClasses];
+  ClassSpan r[kRunClasses];
 };
 void launch_colour_run(const DevBodies& b, SolverBufs& sb, const ClassRun& run, bool warm, hipStream_t s);
-void launch_pgs_colour(const DevBodies& b, int first, int n, int blocks, SolverBufs& sb, hipStream_t s,
-                       hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // cache: also the impulses to the contacts' slots, as launch_cache_impulses
 void launch_residual(const DevBodies& b, const DevContacts& c, int M, bool cache, SolverBufs& sb, hipStream_t s);
 void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int M, hipStream_t s);
@@ -198,10 +204,11 @@ void launch_cache_impulses(const DevContacts& c, SolverBufs& sb, int M, hipStrea
 // and colour the first position, and the scene's dynamic bodies (CSR) with each body's rank.
 constexpr int kLdsBodies = 2048;  // dynamic bodies of one scene the blocked kernel keeps in LDS
 constexpr int kSmallScene = 256;  // scenes up to this many dynamic bodies use the small workgroups
+constexpr int kSmallLanes = 128;  // of this many lanes
 // Visiting order of the colour classes, by value.
 constexpr int kVisitColours = 512;
 struct VisitOrder {
-  int n;
+  int n, split;
   uint16_t c[kVisitColours];
 };
 struct SceneBlocks {
@@ -209,7 +216,9 @@ struct SceneBlocks {
   uint32_t* slot;        // [M] slots in (scene, colour) order; null: the colour order is it (one scene)
   uint32_t* keys_alt;
   uint32_t* slot_alt;
-  uint32_t* start;       // [nscenes][ncolours + 1]
+  uint32_t* start;       // [nscenes][digits + 1] (digits: of the colour order, 1 or 2 per colour)
+  int4* info;            // [M] the slots' sinfo in that order
+  int2* rank;            // [M] and the ranks of their bodies in their scene
   const int* dyn_start;  // [nscenes + 1]
   const int* dyn_list;   // dynamic bodies scene by scene
   const int* local;      // [n] rank of a dynamic body within its scene
@@ -218,16 +227,26 @@ struct SceneBlocks {
   int n_small, n_large;
   __device__ int at(int i) const { return slot ? int(slot[i]) : i; }
 };
-void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int ncolours, SolverBufs& sb,
+// The class visited k-th, of scene s.
+__device__ __forceinline__ ClassSpan scene_span(const SceneBlocks& sc, const VisitOrder& visit, int s, int k) {
+  const int per = visit.split ? 2 : 1;
+  const uint32_t* st = sc.start + long(s) * (per * visit.n + 1) + per * visit.c[k];
+  ClassSpan r;
+  r.first = int(st[0]);
+  r.multi = int(st[1]) - r.first;
+  r.single = visit.split ? int(st[2]) - int(st[1]) : 0;
+  return r;
+}
+void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int digits, SolverBufs& sb,
                         SceneBlocks& sc, hipStream_t s);
-// block: lanes per large scene (256, 512 or 1024); the large scenes go on s_large, the small on s_small
+// block: lanes per large scene (256 or 512; 1024 runs as 512); the large scenes go on s_large, the small on s_small
 void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit,
                            int nsweeps, bool warm, int block, hipStream_t s_small, hipStream_t s_large);
 // Scene-blocked position correction: `iterations` passes over the colours in the visiting order,
 // one workgroup per scene with the scene's dynamic poses in LDS (the same corrections in the same
 // order per body as the per-colour launches); streams and block as launch_sweeps_blocked.
 void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs& sb, const SceneBlocks& sc,
-                             const VisitOrder& visit, int iterations, bool single, int block, hipStream_t s_small,
+                             const VisitOrder& visit, int iterations, int block, hipStream_t s_small,
                              hipStream_t s_large);
 
 // learned warm start (k_solver.hip): features [C][24] and impulse units ls [C] per row record,
@@ -335,10 +354,8 @@ void launch_ccd_validate(const DevBodies& b, const int2* pairs, CcdBufs& c, int 
 void launch_ccd_clamp(const DevBodies& b, CcdBufs& c, hipStream_t s);
 
 // k_position.hip ---------------------------------------------------------------------------
-// single: every manifold of the launch has one contact
-void launch_position_colour(const DevBodies& b, const SimParams& p, int first, int n, bool single, SolverBufs& sb,
+void launch_position_colour(const DevBodies& b, const SimParams& p, const ClassSpan& c, SolverBufs& sb,
                             hipStream_t s);
-void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, bool single,
-                         hipStream_t s);
+void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s);
 
 }  // namespace nph

@@ -177,7 +177,8 @@ struct World {
   static constexpr int kRoundBatch = 4;  // colouring rounds launched between polls
   std::vector<int> colour_visit;  // colour classes in visiting order
   long solve_count = 0;    // solves performed, never reset
-  std::vector<int2> h_range;       // their (first slot, slots), in that order
+  std::vector<ClassSpan> h_span;    // their slots, in that order
+  bool split_order = false;        // classes list manifolds with several contacts first
   std::vector<int> class_contacts;  // and their contacts
   int solved_M = 0, solved_C = 0;
   double res_inf = 0.0, res_rms = 0.0;
@@ -188,7 +189,6 @@ struct World {
   double res_target = 0.0;
   int res_max_sweeps = 500, res_check_every = 1, res_norm = NPHYS_RESIDUAL_MAX;
   int last_sweeps = 0;
-  int max_class = 0;             // largest colour class of the current solve
   // learned warm start: network (FP32 parameters + BF16 images), per-record features, impulse
   // units, predictions and recorded targets; the judge's saved plain solve
   // scene-blocked solve: per-scene dynamic-body lists (host-built at insertion), the per-solve
@@ -199,7 +199,8 @@ struct World {
   // dynamic cuboid)
   int fixed_end = 0;
   bool any_cuboid = false, any_ball = false;
-  DBuf sc_dyn_start, sc_dyn_list, sc_local, sc_keys, sc_slot, sc_keys_alt, sc_slot_alt, sc_start, sc_small, sc_large;
+  DBuf sc_dyn_start, sc_dyn_list, sc_local, sc_keys, sc_slot, sc_keys_alt, sc_slot_alt, sc_start, sc_info, sc_rank, sc_small,
+      sc_large;
   int n_small_scenes = 0, n_large_scenes = 0;
   int variant_request = -1;  // -1: autotune; else forced
   int cur_variant = 0;
@@ -1119,7 +1120,7 @@ struct World {
   // Whether this solve computes the network's features, which tell cached impulses from new ones.
   bool learned_rows() const { return capture || contact_model == NPHYS_CONTACT_MODEL_LEARNED_WARMSTART; }
 
-  int ensure_solver(int M, int C, int digits = 256) {
+  int ensure_solver(int M, int C, int digits = kColourDigits) {
     const size_t nn = size_t(std::max(n, 1));
     const size_t m = size_t(std::max(M, 1)), c = size_t(std::max(C, 1));
     for (DBuf* b : {&sv_deg, &sv_adj_off}) HIPCK(b->ensure(nn * 4));
@@ -1213,10 +1214,10 @@ struct World {
   static constexpr int kSmRemaining = 32, kSmLastRound = kSmRemaining + kRoundBatch, kSmColours = kSmLastRound + 1;
 
   // Colouring, slots and assembly of the solve's manifolds, and the class bounds back on the host
-  // (colour_visit, h_range, class_rec, max_class). The rounds run in batches of four: a round after the last one that
+  // (colour_visit, h_span, class_contacts). The rounds run in batches of four: a round after the last one that
   // colours anything changes nothing, and the device records that last round. A batch, the colour order and the assembly
-  // are enqueued together and read back once; where manifolds stay uncoloured, or there are more than
-  // 256 colours, the rest runs again. `after` enqueues what does not depend on the colouring, before the wait.
+  // are enqueued together and read back once; where manifolds stay uncoloured, or there are more
+  // colours than the order has digits for, the rest runs again. `after` enqueues what does not depend on the colouring, before the wait.
   template <class F>
   int colour_and_assemble(const DevBodies& b, const DevContacts& c, int M, int C, const SimParams& ps, SolverBufs& v,
                           F&& after) {
@@ -1225,7 +1226,9 @@ struct World {
     const ContactBufs& pc = cb[cur ^ 1];
     uint32_t* sm = bp_small.as<uint32_t>();
     launch_colour_begin(b, c, M, sview[cur ^ 1], prevM, sv_state2[cur ^ 1].as<uint32_t>(), v, stream);
-    int digits = 256;
+    int digits = kColourDigits;
+    // recorded samples and predictions keep the row order that does not depend on the contact counts
+    split_order = !learned_rows();
     bool rounds = true, waiting = true;
     for (int round = 1;;) {
       if (rounds) {
@@ -1236,7 +1239,7 @@ struct World {
         for (int k = 0; k < kRoundBatch; ++k, ++round)
           launch_colour_round(c, M, round, sm + kSmRemaining + k, sm + kSmLastRound, v, stream);
       }
-      launch_colour_order(c, M, C, digits, v, sm + kSmColours, stream);
+      launch_colour_order(c, M, C, digits, split_order, v, sm + kSmColours, stream);
       const uint32_t seq = rb_post({{sm + kSmRemaining, kRoundBatch + 2, 0},
                                     {v.col_start, digits + 1, kRbClass},
                                     {v.class_rec, digits + 1, kRbClass + kMaxColours + 2}});
@@ -1249,8 +1252,9 @@ struct World {
       ncolours = int(rb_host[kRoundBatch + 1]);
       if (rounds) continue;
       if (ncolours > kMaxColours) return set_err(NPHYS_ERR_STATE, "too many colours");
-      if (ncolours <= digits) break;
+      if (ncolours * (split_order ? 2 : 1) <= digits) break;
       digits = kMaxColours;
+      split_order = false;
       const int rc2 = ensure_solver(M, C, digits);
       if (rc2) return rc2;
       v = sv_view();
@@ -1260,39 +1264,37 @@ struct World {
     // order and the largest class
     const uint32_t* h_colstart = rb_host + kRbClass;
     const uint32_t* h_rec = h_colstart + kMaxColours + 2;
+    const int per = split_order ? 2 : 1;
     int csize[kMaxColours];
-    for (int k = 0; k < ncolours; ++k) csize[k] = int(h_colstart[k + 1] - h_colstart[k]);
+    for (int k = 0; k < ncolours; ++k) csize[k] = int(h_colstart[per * (k + 1)] - h_colstart[per * k]);
     colour_visit_order(uint64_t(solve_count), ncolours, csize, colour_visit);
-    max_class = 0;
-    h_range.resize(size_t(ncolours));
+    h_span.resize(size_t(ncolours));
     class_contacts.resize(size_t(ncolours));
     for (int k = 0; k < ncolours; ++k) {
       const int col = colour_visit[size_t(k)];
-      h_range[size_t(k)] = int2{int(h_colstart[col]), csize[col]};
-      class_contacts[size_t(k)] = int(h_rec[col + 1] - h_rec[col]);
-      max_class = std::max(max_class, csize[col]);
+      ClassSpan& r = h_span[size_t(k)];
+      r.first = int(h_colstart[per * col]);
+      r.multi = int(h_colstart[per * col + 1]) - r.first;
+      r.single = csize[col] - r.multi;
+      class_contacts[size_t(k)] = int(h_rec[per * (col + 1)] - h_rec[per * col]);
     }
     return NPHYS_OK;
   }
 
+  static int run_lanes(const ClassSpan& c) { return 8 * c.multi + 2 * c.single; }
   // The run of small classes that starts with the k-th visited one (at most kRunClasses of them).
   ClassRun small_run(int k, int ncol) const {
     ClassRun run;
     run.n = 0;
-    for (; k < ncol && run.n < kRunClasses && h_range[size_t(k)].y <= kRunBlock; ++k) run.r[run.n++] = h_range[size_t(k)];
+    for (; k < ncol && run.n < kRunClasses && run_lanes(h_span[size_t(k)]) <= kRunLanes; ++k)
+      run.r[run.n++] = h_span[size_t(k)];
     return run;
-  }
-
-  // Whether every manifold of the n classes visited from the k-th on has one contact.
-  bool single_contacts(int k, int n) const {
-    for (int i = k; i < k + n; ++i)
-      if (class_contacts[size_t(i)] != h_range[size_t(i)].y) return false;
-    return true;
   }
 
   VisitOrder visit_list() const {
     VisitOrder v;
     v.n = ncolours;
+    v.split = split_order ? 1 : 0;
     for (int k = 0; k < ncolours; ++k) v.c[k] = uint16_t(colour_visit[size_t(k)]);
     return v;
   }
@@ -1300,7 +1302,7 @@ struct World {
   // Warm start (when `warm`) and `nsweeps` coloured SOR-Prox sweeps. With counters enabled the
   // per-colour sweep kernels carry HIP events in their dispatch packets. Every launch is direct:
   // one per colour class, or one workgroup for a run of consecutive small classes.
-  int sweeps(const DevBodies& b, const DevContacts& cv, SolverBufs& v, int sblocks, bool warm, int nsweeps) {
+  int sweeps(const DevBodies& b, SolverBufs& v, bool warm, int nsweeps) {
     if (cur_variant > 0) {
       // scene-blocked: one launch for the warm start and all nsweeps sweeps
       SceneBlocks sc = sc_view();
@@ -1342,18 +1344,15 @@ struct World {
           k += run.n;
           continue;
         }
-        // one 64-lane workgroup per 32 manifolds of this class, two lanes each (the grid-stride loop
-        // covers the rest above the cap): no idle workgroups for the smaller classes
-        const int2 r = h_range[size_t(k)];
-        const int pblocks2 = std::min(2 * sblocks, std::max(1, (2 * r.y + 63) / 64));
+        const ClassSpan& r = h_span[size_t(k)];
         if (w) {
-          launch_warmstart_colour(b, r.x, r.y, pblocks2, v, stream);
+          launch_warmstart_colour(b, r, v, stream);
         } else if (counters_enabled) {
-          launch_pgs_colour(b, r.x, r.y, pblocks2, v, stream, kt_ev[kt_used], kt_ev[kt_used + 1]);
+          launch_pgs_colour(b, r, v, stream, kt_ev[kt_used], kt_ev[kt_used + 1]);
           kt_used += 2;
           counters.sweep_kernel_contacts += class_contacts[size_t(k)];
         } else {
-          launch_pgs_colour(b, r.x, r.y, pblocks2, v, stream);
+          launch_pgs_colour(b, r, v, stream);
         }
         ++k;
       }
@@ -1420,6 +1419,8 @@ struct World {
     v.keys_alt = sc_keys_alt.as<uint32_t>();
     v.slot_alt = sc_slot_alt.as<uint32_t>();
     v.start = nscenes > 1 ? sc_start.as<uint32_t>() : sv_col_start.as<uint32_t>();
+    v.info = sc_info.as<int4>();
+    v.rank = sc_rank.as<int2>();
     v.dyn_start = sc_dyn_start.as<int>();
     v.dyn_list = sc_dyn_list.as<int>();
     v.local = sc_local.as<int>();
@@ -1431,7 +1432,7 @@ struct World {
   }
 
   bool blocked_eligible(int ncol) const {
-    return max_scene_dyn <= kLdsBodies && ncol <= kVisitColours && int64_t(nscenes) * (ncol + 1) <= (int64_t(1) << 24);
+    return max_scene_dyn <= kLdsBodies && ncol >= 2 && ncol <= kVisitColours && int64_t(nscenes) * (2 * ncol + 1) <= (int64_t(1) << 24);
   }
 
   // Variant of this solve's sweeps: forced, or the autotuner's pick, or (while tuning) the next
@@ -1491,21 +1492,21 @@ struct World {
   // solve-to-residual mode, sweeps until max |phi| <= res_target, checked after the warm start
   // and every res_check_every sweeps, at most res_max_sweeps. Leaves the final residual in
   // res_inf / res_rms and the sweep count in nsw.
-  int solve_sweeps(const DevBodies& b, const DevContacts& cv, SolverBufs& v, int M, int C, int sblocks, int& nsw) {
+  int solve_sweeps(const DevBodies& b, const DevContacts& cv, SolverBufs& v, int M, int C, int& nsw) {
     int rc;
     if (res_target <= 0.0) {
-      if ((rc = sweeps(b, cv, v, sblocks, true, prm.max_velocity_iterations))) return rc;
+      if ((rc = sweeps(b, v, true, prm.max_velocity_iterations))) return rc;
       nsw = prm.max_velocity_iterations;
       residual_deferred(b, cv, M, C, true, v);
       return NPHYS_OK;
     }
-    if ((rc = sweeps(b, cv, v, sblocks, true, 0))) return rc;
+    if ((rc = sweeps(b, v, true, 0))) return rc;
     int done = 0;
     for (;;) {
       if ((rc = residual(b, cv, M, C, v))) return rc;
       if ((res_norm == NPHYS_RESIDUAL_RMS ? res_rms : res_inf) <= res_target || done >= res_max_sweeps) break;
       const int k = std::min(res_check_every, res_max_sweeps - done);
-      if ((rc = sweeps(b, cv, v, sblocks, false, k))) return rc;
+      if ((rc = sweeps(b, v, false, k))) return rc;
       done += k;
     }
     nsw = done;
@@ -1596,7 +1597,6 @@ struct World {
     solved_C = C;
     res_inf = res_rms = 0.0;
     ncolours = 0;
-    max_class = 0;
     if (M == 0 && nj == 0) {
       last_sweeps = res_target > 0.0 ? 0 : prm.max_velocity_iterations;
       counters.velocity_sweeps += last_sweeps;
@@ -1619,21 +1619,22 @@ struct World {
       joint_rows();
     }
     HIPCK(hipEventRecord(ev[EV_ASM], stream));
-    const int sblocks = sweep_blocks(max_class);
     kt_used = 0;
     choose_variant(M);
     if (tune_pending) HIPCK(hipEventRecord(tune_ev[0], stream));
-    if (cur_variant > 0 && nscenes > 1) {
-      HIPCK(sc_keys.ensure(size_t(M) * 4));
-      HIPCK(sc_slot.ensure(size_t(M) * 4));
-      HIPCK(sc_keys_alt.ensure(size_t(M) * 4));
-      HIPCK(sc_slot_alt.ensure(size_t(M) * 4));
-      HIPCK(sc_start.ensure(size_t(nscenes) * size_t(ncolours + 1) * 4));
-      HIPCK(sv_tmp.ensure(radix_temp_words(M) * 4));
-      HIPCK(scan.ensure(radix_scan_tiles(M), stream));
-      v.tmp = sv_tmp.as<uint32_t>();
+    if (cur_variant > 0) {
+      const int digits = ncolours * (split_order ? 2 : 1);
+      HIPCK(sc_info.ensure(size_t(M) * sizeof(int4)));
+      HIPCK(sc_rank.ensure(size_t(M) * sizeof(int2)));
+      if (nscenes > 1) {
+        for (DBuf* d : {&sc_keys, &sc_slot, &sc_keys_alt, &sc_slot_alt}) HIPCK(d->ensure(size_t(M) * 4));
+        HIPCK(sc_start.ensure(size_t(nscenes) * size_t(digits + 1) * 4));
+        HIPCK(sv_tmp.ensure(radix_temp_words(M) * 4));
+        HIPCK(scan.ensure(radix_scan_tiles(M), stream));
+        v.tmp = sv_tmp.as<uint32_t>();
+      }
       SceneBlocks sc = sc_view();
-      launch_scene_order(b, M, nscenes, scene_bits, ncolours, v, sc, stream);
+      launch_scene_order(b, M, nscenes, scene_bits, digits, v, sc, stream);
     }
     const bool learned = contact_model == NPHYS_CONTACT_MODEL_LEARNED_WARMSTART && C > 0;
     if ((learned || capture) && C > 0) {
@@ -1656,7 +1657,7 @@ struct World {
         HIPCK(jd_jlam.ensure(2 * jl));
         HIPCK(hipMemcpyAsync(jd_jlam.p, j_lam.p, jl, hipMemcpyDeviceToDevice, stream));
       }
-      if ((rc = solve_sweeps(b, cv, v, M, C, sblocks, n_plain))) return rc;
+      if ((rc = solve_sweeps(b, cv, v, M, C, n_plain))) return rc;
       const double rinf_p = res_inf, rrms_p = res_rms;
       launch_lam_copy(v, C, jd_lam.as<float4>(), true, stream);
       launch_lam_copy(v, C, jd_lam0.as<float4>(), false, stream);
@@ -1670,7 +1671,7 @@ struct World {
       HIPCK(hipMemcpy2DAsync(jd_dv.p, dvb, dv0, pitch, dvb, size_t(n), hipMemcpyDeviceToDevice, stream));
       HIPCK(hipMemset2DAsync(dv0, pitch, 0, dvb, size_t(n), stream));
       if ((rc = predict(v, C))) return rc;
-      if ((rc = solve_sweeps(b, cv, v, M, C, sblocks, n_learned))) return rc;
+      if ((rc = solve_sweeps(b, cv, v, M, C, n_learned))) return rc;
       const bool keep = n_learned < n_plain;
       if (!keep) {
         launch_lam_copy(v, C, jd_lam.as<float4>(), false, stream);
@@ -1685,7 +1686,7 @@ struct World {
       last_sweeps = n_plain + n_learned;
     } else {
       if (learned && (rc = predict(v, C))) return rc;
-      if ((rc = solve_sweeps(b, cv, v, M, C, sblocks, last_sweeps))) return rc;
+      if ((rc = solve_sweeps(b, cv, v, M, C, last_sweeps))) return rc;
     }
     if (capture && C > 0) {
       HIPCK(ml_t.ensure(size_t(C) * kOut * sizeof(float)));
@@ -1717,7 +1718,7 @@ struct World {
       SceneBlocks sc = sc_view();
       HIPCK(hipEventRecord(fork_ev, stream));
       HIPCK(hipStreamWaitEvent(stream_large, fork_ev, 0));
-      launch_position_blocked(b, ps, v, sc, visit_list(), iterations, single_contacts(0, ncolours), cur_variant, stream, stream_large);
+      launch_position_blocked(b, ps, v, sc, visit_list(), iterations, cur_variant, stream, stream_large);
       HIPCK(hipEventRecord(join_ev, stream_large));
       HIPCK(hipStreamWaitEvent(stream, join_ev, 0));
       return NPHYS_OK;
@@ -1730,12 +1731,11 @@ struct World {
       for (int k = 0; k < ncol;) {
         const ClassRun run = small_run(k, ncol);
         if (run.n >= 2) {
-          launch_position_run(b, ps, v, run, single_contacts(k, run.n), stream);
+          launch_position_run(b, ps, v, run, stream);
           k += run.n;
           continue;
         }
-        const int2 r = h_range[size_t(k)];
-        launch_position_colour(b, ps, r.x, r.y, single_contacts(k, 1), v, stream);
+        launch_position_colour(b, ps, h_span[size_t(k)], v, stream);
         ++k;
       }
     }
@@ -1887,7 +1887,7 @@ struct World {
       if ((rc = position_correction(ss, prm.max_ccd_position_iterations))) return rc;
     }
     launch_ccd_validate(b, pairs.as<int2>(), c, ccd_nimp, stream);
-    if (M > 0 && (rc = sweeps(b, cv, v, sweep_blocks(max_class), true, prm.max_velocity_iterations))) return rc;
+    if (M > 0 && (rc = sweeps(b, v, true, prm.max_velocity_iterations))) return rc;
     launch_integrate(b, ss, stream, c.prepared);
     ccd_sub = false;
     cur_variant = saved_variant;

@@ -1,0 +1,47 @@
+"""Colour classes at the edges of the launches that solve them: classes list the manifolds with several
+contacts first (eight lanes each in a sweep, a quad in the position correction), then those with one (two
+lanes, one lane), and classes of up to 1,024 lanes share a workgroup."""
+import numpy as np
+import pytest
+
+from nphysics_amd import abi, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _resting(nboxes, nballs):
+    """Boxes and balls apart from each other, a little inside the ground: one class of
+    nboxes four-contact and nballs one-contact manifolds."""
+    n = nboxes + nballs
+    side = int(np.ceil(np.sqrt(n)))
+    s = scenes.boxes(nx=n, ny=1, nz=1)  # and the ground
+    s["rot"][1:] = (0.0, 0.0, 0.0, 1.0)
+    s["shape"][1 + nboxes:] = 0
+    s["dims"][1 + nboxes:] = (0.5, 0.0, 0.0)
+    i = np.arange(n)
+    rng = np.random.default_rng(n)
+    s["pos"][1:, 0] = 1.7 * (i % side) - 0.85 * side
+    s["pos"][1:, 1] = 0.5 - rng.uniform(0.005, 0.03, n)
+    s["pos"][1:, 2] = 1.7 * (i // side) - 0.85 * side
+    s["linvel"][1:] = rng.uniform(-1.0, 1.0, (n, 3))
+    s["angvel"][1:] = rng.uniform(-1.0, 1.0, (n, 3))
+    return s
+
+
+@pytest.mark.parametrize("variant", [0, 256, 512, 1024])
+@pytest.mark.parametrize("nboxes,nballs", [(1, 0), (0, 1), (1, 1), (15, 33), (32, 129), (127, 4), (127, 5), (128, 0),
+                                           (129, 0), (0, 512), (0, 513), (300, 700)])
+def test_class_sizes(nphys, oracle_mod, nboxes, nballs, variant):
+    s = _resting(nboxes, nballs)
+    g = nphys.MechanicalWorld(integration_parameters=abi.default_params())
+    o = oracle_mod.OracleWorld(abi.default_params(), precision=32, order=oracle_mod.ORDER_COLOURED)
+    for w in (g, o):
+        w.add_bodies(s)
+    g.set_sweep_variant(variant)
+    for k in range(3):
+        g.step(1)
+        o.step(1)
+        gs, os_ = g.get_state(), o.get_state()
+        for key in ("pos", "rot", "linvel", "angvel"):
+            np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
+    assert g.counters()["ncolours"] >= 1
