@@ -3,14 +3,18 @@
 //
 // Restates MechanicalWorld::predict_next_impacts and the island traversal of solve_ccd
 // (src/world/mechanical_world.rs:400-557, 630-861) with TOIEntry::try_from_colliders (:946-1022):
-//   * k_ccd_first_pass, one lane per broad-phase pair with a CCD-enabled side: the pair gets a CCD
-//     slot and its time of impact up to the step's end (conservative advancement, np_geometry.hpp);
-//     impacts within the window go to the queue, later ones lower the earliest-later time;
-//   * k_ccd_events, one workgroup: wave 0 pops the earliest impact (ties by pair index) from an
-//     indexed 64-ary heap, confirms pairs of two frozen bodies only at the later freeze time, and
-//     freezes the two bodies (their keys: a static collider shares its static body's); then every
-//     lane re-sweeps the CCD slots of the two bodies' dynamic colliders with the frozen bodies held
-//     at their freeze poses, and wave 0 replaces, removes or adds those slots' entries;
+//   * k_ccd_first_pass: every broad-phase pair with a CCD-enabled side gets a CCD slot and its time
+//     of impact up to the step's end (conservative advancement, np_geometry.hpp); impacts within
+//     the window become the slots' keys, later ones lower the earliest-later time;
+//   * k_ccd_events, one workgroup, takes the earliest impact (ties by pair index) again and again,
+//     confirms pairs of two frozen bodies only at the later freeze time, and freezes the two bodies
+//     (their keys: a static collider shares its static body's); then the CCD slots of the frozen
+//     bodies' dynamic colliders are re-swept with the frozen bodies held at their freeze poses;
+//   * k_ccd_foresee, on the whole chip, does those re-sweeps beforehand: a body not frozen yet will freeze
+//     at its earliest key unless an event before changes that, so the times of impact of its slots
+//     with it held there are recorded with the freeze time they hold for. An event takes the
+//     recorded times where the freeze time is the one that came true and computes the others itself; after
+//     kEventMisses events with such others it stops for k_ccd_foresee to look again from there;
 //   * the island of a substep grows in rounds: the dynamic bodies of every pair touching a
 //     traversed collider are moved to their impact time (k_ccd_touch, k_ccd_prepare; the dynamics
 //     update of the substep, no gravity, forces cleared), those pairs' manifolds are computed by
@@ -18,9 +22,11 @@
 //     traversed from the next round (k_ccd_grow, k_ccd_merge);
 //   * k_ccd_validate (validate_advancement of the impacting bodies) and k_ccd_clamp (bodies still
 //     predicted to impact go back to the start of their motion, rigid_body.rs:530-537).
-// The queue is serial by nature; it holds the few impacts of a step, while the time-of-impact
-// queries (the arithmetic) run one per lane.
+// The queue is serial by nature; what an event does is a few hundred instructions, while the
+// time-of-impact queries (the arithmetic) have sixteen lanes each, over all compute units.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "kernels.hpp"
 #include "np_geometry.hpp"
@@ -30,7 +36,9 @@ namespace nph {
 
 namespace {
 
-constexpr int kEventBlock = 512;  // eight waves: one freeze re-sweeps a few hundred swept-AABB pairs in one round
+constexpr int kEventBlock = 512;
+// Events with times not foreseen, some 10 us each, before the next round (2 to 16: within 2% of each other).
+constexpr int kEventMisses = 4;
 
 __device__ __forceinline__ unsigned long long toi_key(float toi, int pair) {
   return (static_cast<unsigned long long>(__float_as_uint(toi)) << 32) | static_cast<unsigned long long>(uint32_t(pair));
@@ -61,109 +69,223 @@ __device__ __forceinline__ CcdMotion part_motion(const DevBodies& b, int i, floa
   return m;
 }
 
+// ---- time of impact on sixteen lanes ----
+// Sixteen lanes (one DPP row) share a query, all with the same arguments: lanes 0-7 move body 1 and lanes 8-15 body 2, each
+// lane measures one of the 15 axes of the cuboid / cuboid separation, and the largest is found by
+// three permutation steps. The same expressions as time_of_impact's and toi_separation's, in the same order,
+// so the same bits; a single lane takes some 1,000 instructions per iterate, these some 350.
+constexpr int kToiLanes = 16;
+
+template <int Ctrl>
+__device__ __forceinline__ float row_perm(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), Ctrl, 0xf, 0xf, true));
+}
+template <int Ctrl>
+__device__ __forceinline__ void max_axis_step(float& s, int& r) {
+  const float os = row_perm<Ctrl>(s);
+  const int orr = __builtin_amdgcn_mov_dpp(r, Ctrl, 0xf, 0xf, true);
+  const bool other = os > s || (os == s && orr < r);
+  s = other ? os : s;
+  r = other ? orr : r;
+}
+constexpr int kQuadXor1 = 0xb1, kQuadXor2 = 0x4e, kHalfMirror = 0x141, kMirror = 0x140;
+
+// toi_separation of two cuboids whose axes are the columns of RA and RB; r: the lane's place in its row.
+__device__ __forceinline__ float boxes_separation(f3 h1, const m33& RA, f3 h2, const m33& RB, f3 d, int r, f3& n) {
+  f3 a[3], b[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    a[i] = mcol(RA, i);
+    b[i] = mcol(RB, i);
+  }
+  // lanes 0-2: the faces of A, 3-5: of B, 6-14: the edge axes, in toi_separation's order
+  const int e = r < 6 ? 0 : r - 6;
+  const int i = r < 3 ? r : (r < 6 ? 0 : (e * 11) >> 5);  // e / 3 for e < 10
+  const int j = r < 6 ? (r < 3 ? 0 : r - 3) : e - 3 * i;
+  const f3 ai = pick(i == 0, a[0], pick(i == 1, a[1], a[2])), bj = pick(j == 0, b[0], pick(j == 1, b[1], b[2]));
+  const f3 c = cross(ai, bj);
+  const f3 L = pick(r < 3, ai, pick(r < 6, bj, c));
+  float l = 1.0f, s = -INFINITY;
+  const float l2 = dot(c, c);
+  if (r >= 6) l = sqrtf(l2);
+  const float pa = (h1.x * fabsf(dot(a[0], L)) + h1.y * fabsf(dot(a[1], L))) + h1.z * fabsf(dot(a[2], L));
+  const float pb = (h2.x * fabsf(dot(b[0], L)) + h2.y * fabsf(dot(b[1], L))) + h2.z * fabsf(dot(b[2], L));
+  const float ra = r < 3 ? comp(h1, i) : pa, rb = (r >= 3 && r < 6) ? comp(h2, j) : pb;
+  if (r < 6 || (r < 15 && !(l2 < 1e-6f))) {
+    const float m = (fabsf(dot(d, L)) - (ra + rb)) / l;
+    s = m > s ? m : s;  // never a NaN
+  }
+  int best = r;
+  max_axis_step<kQuadXor1>(s, best);
+  max_axis_step<kQuadXor2>(s, best);
+  max_axis_step<kHalfMirror>(s, best);
+  max_axis_step<kMirror>(s, best);
+  f3 axis{__shfl(L.x, best, kToiLanes), __shfl(L.y, best, kToiLanes), __shfl(L.z, best, kToiLanes)};
+  const float scale = __shfl(l, best, kToiLanes);
+  if (scale != 1.0f) axis = f3{axis.x / scale, axis.y / scale, axis.z / scale};
+  n = dot(d, axis) < 0.0f ? neg(axis) : axis;
+  return s;
+}
+
 // TOIEntry::try_from_colliders for bodies i, j with freeze times f1, f2 (< 0: not frozen): the
 // global time of impact up to end_time.
 __device__ bool pair_toi(const DevBodies& b, const CcdBufs& c, int i, int j, float f1, float f2, float end_time,
-                         float target, int on_penetration, float* out) {
+                         float target, int on_penetration, int r, float* out) {
+  const bool second = r >= kToiLanes / 2;
   const float bt1 = c.body_time[i], bt2 = c.body_time[j];
   const float time1 = f1 >= 0.0f ? f1 : bt1;
   const float time2 = f2 >= 0.0f ? f2 : bt2;
   const float start = time1 > time2 ? time1 : time2;
-  const float o1 = time1 - start, o2 = time2 - start;
-  CcdMotion m1 = part_motion(b, i, o1), m2 = part_motion(b, j, o2);
-  if (f1 >= 0.0f) {
-    m1.at((f1 + o1) - bt1, m1.t0p, m1.q0);
-    m1.kind = MOTION_STATIC;
+  const float o = (second ? time2 : time1) - start;
+  const float f = second ? f2 : f1;
+  CcdMotion m = part_motion(b, second ? j : i, o);
+  if (f >= 0.0f) {
+    m.at((f + o) - (second ? bt2 : bt1), m.t0p, m.q0);
+    m.kind = MOTION_STATIC;
   }
-  if (f2 >= 0.0f) {
-    m2.at((f2 + o2) - bt2, m2.t0p, m2.q0);
-    m2.kind = MOTION_STATIC;
+  const int k1 = b.shape[i], k2 = b.shape[j];
+  const f3 h1 = xyz(b.dims[i]), h2 = xyz(b.dims[j]);
+  const float max_toi = end_time - start;
+  // velocities as time_of_impact takes them; both bodies' in every lane
+  const f3 z{0.0f, 0.0f, 0.0f};
+  const f3 v = m.kind == MOTION_STATIC ? z : m.v;
+  const f3 w = m.kind == MOTION_ROTATING ? m.w : z;
+  const float reach = sqrtf(dot(w, w)) * (second ? rotation_reach(k2, h2) : rotation_reach(k1, h1));
+  const float reach_o = row_perm<kMirror>(reach);
+  const float spin = second ? reach_o + reach : reach + reach_o;
+  const f3 vo{row_perm<kMirror>(v.x), row_perm<kMirror>(v.y), row_perm<kMirror>(v.z)};
+  const f3 dv = second ? sub(v, vo) : sub(vo, v);
+  float tau = 0.0f;
+  int status = TOI_OUT_OF_ITERATIONS;
+  for (int it = 0; it < kToiMaxIterations; ++it) {
+    f3 p, n;
+    q4 q;
+    m.at(tau, p, q);
+    const f3 po{row_perm<kMirror>(p.x), row_perm<kMirror>(p.y), row_perm<kMirror>(p.z)};
+    const f3 p1 = pick(second, po, p), p2 = pick(second, p, po);
+    float d;
+    if (k1 == SHAPE_BALL || k2 == SHAPE_BALL) {
+      const q4 qo{row_perm<kMirror>(q.i), row_perm<kMirror>(q.j), row_perm<kMirror>(q.k), row_perm<kMirror>(q.w)};
+      d = toi_separation(k1, h1, p1, second ? qo : q, k2, h2, p2, second ? q : qo, n);
+    } else {
+      const m33 R = qmat(q);
+      m33 R1, R2;
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+          const float ro = row_perm<kMirror>(R.m[x][y]);
+          R1.m[x][y] = second ? ro : R.m[x][y];
+          R2.m[x][y] = second ? R.m[x][y] : ro;
+        }
+      d = boxes_separation(h1, R1, h2, R2, sub(p2, p1), r, n);
+    }
+    if (it == 0 && d < 0.0f) {
+      status = TOI_PENETRATING;
+      break;
+    }
+    if (d <= target + kToiTolerance) {
+      status = TOI_CONVERGED;
+      break;
+    }
+    const float a = spin - dot(dv, n);
+    if (!(a > 0.0f)) return false;
+    tau = tau + (d - target) / a;
+    if (tau > max_toi) return false;
   }
-  float toi = 0.0f;
-  int status = 0;
-  if (!time_of_impact(b.shape[i], xyz(b.dims[i]), m1, b.shape[j], xyz(b.dims[j]), m2, end_time - start, target, &toi,
-                      &status))
-    return false;
   if (!on_penetration && status == TOI_PENETRATING) return false;
-  *out = start + toi;
+  *out = start + tau;
   return true;
 }
 
-__global__ void k_ccd_reset(uint32_t* ctl) {
-  const int t = threadIdx.x;
-  if (t < kCcdWords) ctl[t] = t == kCcdMinAfter ? 0x7f800000u : 0u;  // +inf
+__global__ void __launch_bounds__(256) k_ccd_begin(int n, CcdBufs c) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < kCcdWords) c.ctl[i] = i == kCcdMinAfter ? 0x7f800000u : 0u;  // +inf
+  if (i >= n) return;
+  c.frozen[i] = -1.0f;
+  c.deg[i] = 0u;
+  c.fill[i] = 0u;
 }
 
-__global__ void __launch_bounds__(128) k_ccd_first_pass(DevBodies b, const int2* __restrict__ pairs, int npairs,
+constexpr unsigned long long kNoKey = ~0ull;
+constexpr int kFirstPairs = 64;  // pairs of one workgroup of the first pass
+
+// Wave 0 gives the CCD pairs of the workgroup's 64 their slots, then its sixteen rows of lanes take those in turn.
+__global__ void __launch_bounds__(256) k_ccd_first_pass(DevBodies b, const int2* __restrict__ pairs, int npairs,
                                                         CcdBufs c, float end_time, float dt0, float target,
                                                         int on_penetration) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= npairs) return;
-  const int2 pr = pairs[p];
-  if (!((b.ccd[pr.x] | b.ccd[pr.y]) & 1)) return;
-  const uint32_t slot = atomicAdd(&c.ctl[kCcdSlots], 1u);
-  c.slot_pair[slot] = p;
-  c.slot_bodies[slot] = int4{pr.x, pr.y, b.ccd_key[pr.x] | (b.status[pr.x] != STATUS_DYNAMIC ? kSlotStatic : 0),
-                             b.ccd_key[pr.y] | (b.status[pr.y] != STATUS_DYNAMIC ? kSlotStatic : 0)};
-  c.pos[slot] = -1;
-  float toi;
-  if (!pair_toi(b, c, pr.x, pr.y, -1.0f, -1.0f, dt0, target, on_penetration, &toi)) return;
-  if (toi > end_time) {
-    atomicMin(&c.ctl[kCcdMinAfter], __float_as_uint(toi));  // toi > 0: the bits order as the values
-  } else {
-    atomicOr(&c.ctl[kCcdAnyIn], 1u);
-    const uint32_t e = atomicAdd(&c.ctl[kCcdEntries], 1u);
-    if (int(e) < c.cap) c.heap[e] = ToiEntry{toi_key(toi, p), int(slot)};
-    else atomicOr(&c.ctl[kCcdOverflow], 1u);
+  __shared__ int s_pair[kFirstPairs];
+  __shared__ int2 s_body[kFirstPairs];
+  __shared__ uint32_t s_first;
+  __shared__ int s_n;
+  const int t = threadIdx.x;
+  if (t < 64) {
+    const int p = blockIdx.x * kFirstPairs + t;
+    const int2 pr = p < npairs ? pairs[p] : int2{0, 0};
+    const bool on = p < npairs && ((b.ccd[pr.x] | b.ccd[pr.y]) & 1);
+    const unsigned long long m = __ballot(on);
+    const int at = __popcll(m & ((1ull << t) - 1ull));
+    uint32_t first = 0;
+    if (t == 0) {
+      if (m) first = atomicAdd(&c.ctl[kCcdSlots], uint32_t(__popcll(m)));
+      s_first = first;
+      s_n = __popcll(m);
+    }
+    first = uint32_t(__builtin_amdgcn_readfirstlane(int(first)));
+    if (on) {
+      s_pair[at] = p;
+      s_body[at] = pr;
+      const uint32_t slot = first + uint32_t(at);
+      const bool st1 = b.status[pr.x] != STATUS_DYNAMIC, st2 = b.status[pr.y] != STATUS_DYNAMIC;
+      c.slot_pair[slot] = p;
+      c.slot_bodies[slot] =
+          int4{pr.x, pr.y, b.ccd_key[pr.x] | (st1 ? kSlotStatic : 0), b.ccd_key[pr.y] | (st2 ? kSlotStatic : 0)};
+      c.seen_at[2 * slot] = c.seen_at[2 * slot + 1] = -1.0f;
+      if (!st1) atomicAdd(&c.deg[pr.x], 1u);
+      if (!st2) atomicAdd(&c.deg[pr.y], 1u);
+    }
+  }
+  __syncthreads();
+  const int r = t & (kToiLanes - 1);
+  for (int k = t / kToiLanes; k < s_n; k += 256 / kToiLanes) {
+    const int2 pr = s_body[k];
+    unsigned long long key = kNoKey;
+    float toi;
+    if (pair_toi(b, c, pr.x, pr.y, -1.0f, -1.0f, dt0, target, on_penetration, r, &toi)) {
+      if (!(toi > end_time)) key = toi_key(toi, s_pair[k]);
+      else if (r == 0) atomicMin(&c.ctl[kCcdMinAfter], __float_as_uint(toi));  // toi > 0: the bits order as the values
+    }
+    if (r == 0) {
+      c.key[s_first + uint32_t(k)] = key;
+      if (key != kNoKey) c.ctl[kCcdAnyIn] = 1u;
+    }
   }
 }
 
 // The CCD slots of every dynamic body (adjacency in slot order is not needed: the re-sweep's
-// results go into the queue, whose order is by key).
-__global__ void __launch_bounds__(256) k_ccd_degree(int npairs, CcdBufs c) {
-  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= npairs || slot >= int(c.ctl[kCcdSlots])) return;
-  const int4 sb = c.slot_bodies[slot];
-  if (!(sb.z & kSlotStatic)) atomicAdd(&c.deg[sb.x], 1u);
-  if (!(sb.w & kSlotStatic)) atomicAdd(&c.deg[sb.y], 1u);
-}
-
+// results go into the queue, whose order is by key), and the bodies that have any.
 __global__ void __launch_bounds__(256) k_ccd_fill(int npairs, CcdBufs c) {
   const int slot = blockIdx.x * blockDim.x + threadIdx.x;
   if (slot >= npairs || slot >= int(c.ctl[kCcdSlots])) return;
   const int4 sb = c.slot_bodies[slot];
-  if (!(sb.z & kSlotStatic)) c.adj[c.off[sb.x] + atomicAdd(&c.fill[sb.x], 1u)] = slot;
-  if (!(sb.w & kSlotStatic)) c.adj[c.off[sb.y] + atomicAdd(&c.fill[sb.y], 1u)] = slot;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if ((h ? sb.w : sb.z) & kSlotStatic) continue;
+    const int i = h ? sb.y : sb.x;
+    const uint32_t k = atomicAdd(&c.fill[i], 1u);
+    c.adj[c.off[i] + k] = slot;
+    if (k == 0u) c.bodies[atomicAdd(&c.ctl[kCcdBodies], 1u)] = i;
+  }
 }
 
-// ---- the impact queue: an indexed 64-ary heap, its top three levels in LDS, operated by wave 0 ----
-// Each CCD slot holds at most one entry (its latest time of impact), so a re-sweep replaces or
-// removes it in place instead of leaving a superseded entry behind: the pop sequence of the valid
-// entries is the reference's, without popping stale ones. A node's 64 children are compared across
-// the wave in one step; nodes 0..4160 (levels 0-2) live in LDS and deeper ones in HBM, so a node's
-// children are all in one of the two. Keys are unique (they hold the pair index): the order is
-// total. pos[slot] (HBM) is the node of each slot's entry, -1 when it has none.
-constexpr int kHeapD = 64;
-constexpr int kTop = 1 + kHeapD + kHeapD * kHeapD;  // 4,161 nodes, 12 B each in LDS
-constexpr unsigned long long kNoKey = ~0ull;
-
-struct Queue {
-  unsigned long long* lk;  // LDS keys, nodes < kTop
-  int* ls;                 // LDS slots
-  ToiEntry* g;             // HBM entries, nodes >= kTop
-  int* pos;
-  __device__ unsigned long long key(int i) const { return i < kTop ? lk[i] : g[i].key; }
-  __device__ int slot(int i) const { return i < kTop ? ls[i] : g[i].slot; }
-  __device__ void set(int i, unsigned long long k, int s) const {  // one lane
-    if (i < kTop) {
-      lk[i] = k;
-      ls[i] = s;
-    } else {
-      g[i] = ToiEntry{k, s};
-    }
-    pos[s] = i;
-  }
-};
+// ---- the impact queue ----
+// Each CCD slot holds at most one key (its latest time of impact, kNoKey for none), so a re-sweep
+// replaces it in place: no superseded entries to pop. The slots are cut into groups of 64 (more where
+// that gives over kGroups) whose smallest keys live in LDS: the earliest of all is found by one wave among
+// those, a key that falls is one LDS atomic, and only a group whose smallest key rose is
+// searched again. Keys are unique (they hold the pair index): the order is total. It takes the place of an indexed 64-ary
+// heap, whose updates one wave did one by one: see k_ccd_events.
+constexpr int kGroups = kCcdGroups;
 
 // Smallest value across the wave, in every lane: DPP steps within quads, half rows and rows, then
 // row broadcasts; lane 63 ends with the minimum.
@@ -182,83 +304,91 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
   return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
 }
 
-// The smallest of the wave's 64 keys (uniform) and the lane holding it: the time bits first, then
-// the pair index among the lanes with that time.
-__device__ __forceinline__ int wave_argmin(unsigned long long k, unsigned long long& mk) {
+// The smallest of the wave's 64 keys (uniform): the time bits first, then the pair index among the
+// lanes with that time.
+__device__ __forceinline__ unsigned long long wave_min(unsigned long long k) {
   const uint32_t hi = uint32_t(k >> 32), lo = uint32_t(k & 0xffffffffull);
   const uint32_t mh = wave_min_u32(hi);
   const uint32_t ml = wave_min_u32(hi == mh ? lo : 0xffffffffu);
-  mk = (static_cast<unsigned long long>(mh) << 32) | ml;
-  return __ffsll(static_cast<long long>(__ballot(hi == mh && lo == ml))) - 1;
+  return (static_cast<unsigned long long>(mh) << 32) | ml;
 }
 
-// Every lane of wave 0 runs the queue operations with the same values (lane 0 writes); a lane may
-// track one slot's node (tslot, tnode), kept current as entries move.
-__device__ void sift_down(const Queue& q, int n, int k, unsigned long long ek, int es, int lane, int tslot,
-                          int& tnode) {
-  for (;;) {
-    const int c0 = kHeapD * k + 1;
-    if (c0 >= n) break;
-    const int ch = c0 + lane;
-    unsigned long long ck = kNoKey;
-    int cs = -1;
-    if (ch < n) {
-      ck = q.key(ch);
-      cs = q.slot(ch);
+// The smallest key of slots [first, last) (uniform) but for slot `but`.
+__device__ __forceinline__ unsigned long long range_min(const unsigned long long* key, int first, int last, int but,
+                                                        int lane) {
+  unsigned long long m = kNoKey;
+  for (int k = first + lane; k < last; k += 64) {
+    const unsigned long long x = key[k];
+    m = (k != but && x < m) ? x : m;
+  }
+  return wave_min(m);
+}
+
+// The times of impact that freezing a body at its earliest key would ask for, recorded per slot and side
+// with that freeze time: a row of lanes per slot, a workgroup per body.
+__global__ void __launch_bounds__(256) k_ccd_foresee(DevBodies b, CcdBufs c, float end_time, float target,
+                                                     int on_penetration) {
+  if (c.ctl[kCcdState] == kQueueDone || c.ctl[kCcdAnyIn] == 0u) return;
+  const int t = threadIdx.x, lane = t & 63, r = t & (kToiLanes - 1);
+  const int nb = int(c.ctl[kCcdBodies]);
+  for (int at = blockIdx.x; at < nb; at += gridDim.x) {
+    const int x = c.bodies[at];
+    if (c.frozen[b.ccd_key[x]] >= 0.0f) continue;
+    const int first = int(c.off[x]), n = int(c.deg[x]);
+    unsigned long long m = kNoKey;
+    for (int k = lane; k < n; k += 64) {
+      const unsigned long long key = c.key[c.adj[first + k]];
+      m = key < m ? key : m;
     }
-    unsigned long long mk;
-    const int wl = wave_argmin(ck, mk);
-    if (!(mk < ek)) break;
-    const int bs = __builtin_amdgcn_readlane(cs, wl);
-    if (lane == 0) q.set(k, mk, bs);
-    if (tslot == bs) tnode = k;
-    k = c0 + wl;
+    m = wave_min(m);
+    if (m == kNoKey) continue;
+    const float f = key_toi(m);
+    for (int k = t / kToiLanes; k < n; k += 256 / kToiLanes) {
+      const int slot = c.adj[first + k];
+      const int4 sb = c.slot_bodies[slot];
+      const int h = sb.x == x ? 0 : 1;
+      const int other = h ? sb.z : sb.w;
+      if ((other & kSlotStatic) || c.frozen[other] >= 0.0f || c.seen_at[2 * slot + h] == f) continue;
+      float toi;
+      const bool hit = pair_toi(b, c, sb.x, sb.y, h ? -1.0f : f, h ? f : -1.0f, end_time, target, on_penetration, r, &toi);
+      if (r == 0) {
+        c.seen_key[2 * slot + h] = hit ? toi_key(toi, c.slot_pair[slot]) : kNoKey;
+        c.seen_at[2 * slot + h] = f;
+      }
+    }
   }
-  if (lane == 0) q.set(k, ek, es);
-  if (tslot == es) tnode = k;
 }
 
-__device__ void sift_up(const Queue& q, int k, unsigned long long ek, int es, int lane, int tslot, int& tnode) {
-  while (k > 0) {
-    const int par = (k - 1) / kHeapD;
-    const unsigned long long pk = q.key(par);
-    if (!(ek < pk)) break;
-    const int ps = q.slot(par);
-    if (lane == 0) q.set(k, pk, ps);
-    if (tslot == ps) tnode = k;
-    k = par;
-  }
-  if (lane == 0) q.set(k, ek, es);
-  if (tslot == es) tnode = k;
-}
-
-// The entry at node p takes key (ek, es): up or down as the key decreased or grew.
-__device__ void place(const Queue& q, int n, int p, unsigned long long ek, int es, int lane, int tslot, int& tnode) {
-  if (ek < q.key(p)) sift_up(q, p, ek, es, lane, tslot, tnode);
-  else sift_down(q, n, p, ek, es, lane, tslot, tnode);
-}
-
-// Freeze times held in LDS for up to this many body keys (the rest of the 160 KB beside the queue).
+// Freeze times held in LDS for up to this many body keys (the rest of the 160 KB beside the groups).
 constexpr int kFzCap = 27648;
 
-// predict_next_impacts' event loop (mechanical_world.rs:453-557) in one workgroup; with LdsFrozen
-// the freeze times live in LDS for the loop and are written back at its end.
+// predict_next_impacts' event loop (mechanical_world.rs:453-557) in one workgroup, from where the last
+// launch left it to the end of the window or the kEventMisses-th event with times not foreseen; with LdsFrozen
+// the freeze times live in LDS meanwhile. What bounds it is the chain of events. With every re-sweep
+// made in it, one query per lane, and a heap updated entry by entry, an event took 30-60 us (15-38 of re-sweep, the
+// rest pops of keys that no longer counted and updates): 18.9 ms a step at 343 cuboids, 280 impacts and 9,000 pairs.
+// Now some 25 events share a round of 30 us of k_ccd_foresee and 90 us here: 6.1 ms, with the substep.
 template <bool LdsFrozen>
 __global__ void __launch_bounds__(kEventBlock) k_ccd_events(DevBodies b, CcdBufs c, float end_time, float dt0,
                                                             float target, int on_penetration) {
-  __shared__ unsigned long long s_hk[kTop];
-  __shared__ int s_hs[kTop];
+  __shared__ unsigned long long s_min[kGroups];
   __shared__ float s_fz[LdsFrozen ? kFzCap : 1];
-  __shared__ int s_go, s_i, s_j, s_nstage, s_hsize, s_nimp;
+  __shared__ uint32_t s_bits[kGroups / 32];
+  __shared__ uint16_t s_dirty[kGroups];
+  __shared__ int s_go, s_i, s_j, s_fresh, s_nmiss, s_ndirty, s_nimp;
   float* const fz = LdsFrozen ? s_fz : c.frozen;
   constexpr int kKey = kSlotStatic - 1;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int nent = int(c.ctl[kCcdEntries]);
-  const Queue q{s_hk, s_hs, c.heap, c.pos};
-  if (t == 0) {
-    const bool any = c.ctl[kCcdAnyIn] != 0u;
+  const uint32_t state = c.ctl[kCcdState];
+  if (state == kQueueDone) return;
+  const int ns = int(c.ctl[kCcdSlots]);
+  int sh = 6;
+  while (((ns - 1) >> sh) >= kGroups) ++sh;
+  const int ng = (ns + (1 << sh) - 1) >> sh;
+  if (state == kQueueNew) {
     // min_overstep (mechanical_world.rs:412-451): the step's end lowered to the earliest impact
     // after the window, or the window's end when an impact lies within it
+    const bool any = c.ctl[kCcdAnyIn] != 0u;
     float min_over = dt0;
     const float after = __uint_as_float(c.ctl[kCcdMinAfter]);
     if (after < min_over) min_over = after;
@@ -266,167 +396,160 @@ __global__ void __launch_bounds__(kEventBlock) k_ccd_events(DevBodies b, CcdBufs
     int kind = PREDICT_IMPACTS;
     if (min_over == dt0 && !any) kind = PREDICT_NONE;
     else if (min_over > end_time) kind = PREDICT_AFTER_END;
-    c.ctl[kCcdKind] = uint32_t(kind);
-    c.ctl[kCcdMinOver] = __float_as_uint(min_over);
-    s_go = (kind == PREDICT_IMPACTS && c.ctl[kCcdOverflow] == 0u) ? 1 : 0;
-    s_hsize = nent;
-    s_nimp = 0;
+    __syncthreads();
+    if (t == 0) {
+      c.ctl[kCcdKind] = uint32_t(kind);
+      c.ctl[kCcdMinOver] = __float_as_uint(min_over);
+      if (kind != PREDICT_IMPACTS) c.ctl[kCcdState] = kQueueDone;
+    }
+    if (kind != PREDICT_IMPACTS) return;
   }
-  __syncthreads();
-  if (!s_go) {
-    if (t == 0) c.ctl[kCcdImpacts] = 0u;
-    return;
-  }
-  // ---- the first pass's entries into a heap: the LDS levels copied in, then the internal nodes
-  // sifted down level by level from the deepest (the subtrees of one level are disjoint: one wave
-  // per node), then every entry's node recorded
-  for (int k = t; k < nent && k < kTop; k += kEventBlock) {
-    s_hk[k] = c.heap[k].key;
-    s_hs[k] = c.heap[k].slot;
+  for (int g = wave; g < ng; g += kEventBlock / 64) {
+    const unsigned long long m =
+        state == kQueueNew ? range_min(c.key, g << sh, min((g + 1) << sh, ns), -1, lane) : c.group[g];
+    if (lane == 0) s_min[g] = m;
   }
   if (LdsFrozen)
     for (int k = t; k < b.n; k += kEventBlock) s_fz[k] = c.frozen[k];
-  __syncthreads();
-  if (nent > 1) {
-    const int last = (nent - 2) / kHeapD;  // the last internal node
-    int first = 0, width = 1;
-    while (first + width <= last) {  // the first node of the deepest internal level
-      first += width;
-      width *= kHeapD;
-    }
-    for (;;) {
-      const int end = first + width - 1 < last ? first + width - 1 : last;
-      int none = -1;
-      for (int k = first + wave; k <= end; k += kEventBlock / 64) sift_down(q, nent, k, q.key(k), q.slot(k), lane, -1, none);
-      __syncthreads();
-      if (first == 0) break;
-      width /= kHeapD;
-      first -= width;
-    }
+  for (int k = t; k < kGroups / 32; k += kEventBlock) s_bits[k] = 0u;
+  if (t == 0) {
+    s_nimp = state == kQueueNew ? 0 : int(c.ctl[kCcdImpacts]);
+    s_nmiss = s_ndirty = 0;
   }
-  for (int k = t; k < nent; k += kEventBlock) c.pos[q.slot(k)] = k;
   __syncthreads();
+  // The slot's key, and its group's smallest: lowered at once, or noted to be searched again.
+  auto set_key = [&](int slot, unsigned long long k) {
+    const unsigned long long old = c.key[slot];
+    if (k == old) return;
+    c.key[slot] = k;
+    const int g = slot >> sh;
+    if (k < old) {
+      atomicMin(&s_min[g], k);
+    } else if (s_min[g] == old) {
+      const uint32_t bit = 1u << (g & 31);
+      if (!(atomicOr(&s_bits[g >> 5], bit) & bit)) s_dirty[atomicAdd(&s_ndirty, 1)] = uint16_t(g);
+    }
+  };
+  int late = 0;  // events with times not foreseen
   for (;;) {
-    // ---- pop to the next impact that freezes a body
+    // ---- wave 0 takes the earliest keys up to the next impact that freezes a body
     if (t < 64) {
-      int n = s_hsize, nimp = s_nimp, found = 0, none = -1;
-      while (n > 0) {
+      int nimp = s_nimp, go = 0;
+      for (;;) {
+        unsigned long long mine = kNoKey;
+        int mg = 0;
+        for (int g = lane; g < ng; g += 64) {
+          const unsigned long long x = s_min[g];
+          if (x < mine) {
+            mine = x;
+            mg = g;
+          }
+        }
+        const unsigned long long ek = wave_min(mine);
+        if (ek == kNoKey) break;
         if (nimp >= c.cap) {  // the impact list is full: reported as an overflow
           if (lane == 0) c.ctl[kCcdOverflow] = 1u;
           break;
         }
-        const unsigned long long ek = s_hk[0];
-        const int es = s_hs[0];
-        --n;
-        if (n > 0) sift_down(q, n, 0, q.key(n), q.slot(n), lane, -1, none);
-        int d = 0;  // 0 next entry, 1 freeze
+        const int g = __builtin_amdgcn_readlane(mg, __ffsll(static_cast<long long>(__ballot(mine == ek))) - 1);
+        int es = 0;
+        unsigned long long rest = kNoKey;
+        for (int k = (g << sh) + lane; k - lane < min((g + 1) << sh, ns); k += 64) {
+          const unsigned long long x = k < ns ? c.key[k] : kNoKey;
+          const unsigned long long hit = __ballot(x == ek);
+          if (hit) es = k - lane + __ffsll(static_cast<long long>(hit)) - 1;
+          rest = (x != ek && x < rest) ? x : rest;
+        }
+        const int4 sb = c.slot_bodies[es];
+        rest = wave_min(rest);
         if (lane == 0) {
-          c.pos[es] = -1;
-          const float toi = key_toi(ek);
-          const int4 sb = c.slot_bodies[es];
-          const int ki = sb.z & kKey, kj = sb.w & kKey;
-          const float t1 = fz[ki], t2 = fz[kj];
-          if (t1 >= 0.0f && t2 >= 0.0f) {
-            if (toi == (t1 > t2 ? t1 : t2)) c.impacts[nimp++] = ek;
-          } else {
-            if (t1 < 0.0f) fz[ki] = toi;
-            if (t2 < 0.0f) fz[kj] = toi;
-            c.impacts[nimp++] = ek;
-            s_i = sb.x;
-            s_j = sb.y;
-            d = 1;
+          s_min[g] = rest;
+          c.key[es] = kNoKey;
+        }
+        const float toi = key_toi(ek);
+        const int ki = sb.z & kKey, kj = sb.w & kKey;
+        const float t1 = fz[ki], t2 = fz[kj];
+        if (t1 >= 0.0f && t2 >= 0.0f) {
+          if (toi == (t1 > t2 ? t1 : t2)) {
+            if (lane == 0) c.impacts[nimp] = ek;
+            ++nimp;
           }
+          continue;
         }
-        d = __shfl(d, 0);
-        nimp = __shfl(nimp, 0);
-        if (d) {
-          found = 1;
-          break;
+        if (lane == 0) {
+          if (t1 < 0.0f) fz[ki] = toi;
+          if (t2 < 0.0f) fz[kj] = toi;
+          c.impacts[nimp] = ek;
+          s_i = sb.x;
+          s_j = sb.y;
+          s_fresh = (t1 < 0.0f ? 1 : 0) | (t2 < 0.0f ? 2 : 0);
         }
+        ++nimp;
+        go = 1;
+        break;
       }
       if (lane == 0) {
-        s_hsize = n;
         s_nimp = nimp;
-        s_go = found;
-        s_nstage = 0;
+        s_go = go;
       }
     }
     __syncthreads();
     if (!s_go) break;
-    // ---- re-sweep the CCD slots of the two bodies' dynamic colliders (mechanical_world.rs:503-551);
-    // the event's own pair is in both lists and skipped there (both bodies are frozen). A slot's
-    // entry is replaced by its new time, or removed when there is none.
-    const int si = s_i, sj = s_j;
-    const int ni = int(c.deg[si]), nj = int(c.deg[sj]);  // 0 for a body that is not dynamic
+    // ---- re-sweep the CCD slots of the bodies' dynamic colliders (mechanical_world.rs:503-551); a body
+    // frozen before has its slots' times already. A slot whose key no longer counts, its two bodies
+    // being frozen at other times, is emptied; the event's own is empty.
+    const int si = s_i, sj = s_j, fresh = s_fresh;
+    const int ni = (fresh & 1) ? int(c.deg[si]) : 0;  // deg: 0 for a body that is not dynamic
+    const int nj = (fresh & 2) ? int(c.deg[sj]) : 0;
     for (int k = t; k < ni + nj; k += kEventBlock) {
       const int slot = k < ni ? c.adj[c.off[si] + k] : c.adj[c.off[sj] + (k - ni)];
       const int4 sb = c.slot_bodies[slot];
-      const int p = c.slot_pair[slot];
-      const int had = c.pos[slot];
       const float fa = fz[sb.z & kKey], fb = fz[sb.w & kKey];
-      if ((fa >= 0.0f || (sb.z & kSlotStatic)) && (fb >= 0.0f || (sb.w & kSlotStatic))) continue;
-      float toi;
-      const bool hit = pair_toi(b, c, sb.x, sb.y, fa, fb, end_time, target, on_penetration, &toi);
-      if (hit || had >= 0) {
-        const int st = atomicAdd(&s_nstage, 1);
-        c.stage[st] = ToiEntry{hit ? toi_key(toi, p) : kNoKey, slot};
+      if (fa >= 0.0f && fb >= 0.0f) {
+        const unsigned long long old = c.key[slot];
+        if (old != kNoKey && key_toi(old) != (fa > fb ? fa : fb)) set_key(slot, kNoKey);
+        continue;
       }
+      if ((sb.z | sb.w) & kSlotStatic) continue;  // as it was: the static side moves no more than before
+      const int h = fa >= 0.0f ? 0 : 1;
+      if (c.seen_at[2 * slot + h] == (h ? fb : fa)) set_key(slot, c.seen_key[2 * slot + h]);
+      else c.stage[atomicAdd(&s_nmiss, 1)] = slot;
     }
     __syncthreads();
-    // ---- the re-sweep's results into the queue, 64 at a time: each lane loads one entry and its
-    // slot's node, and keeps the node current while the entries before it move
-    if (t < 64) {
-      int n = s_hsize, ovf = 0;
-      const int ns = s_nstage;
-      for (int base = 0; base < ns && !ovf; base += 64) {
-        const int cnt = ns - base < 64 ? ns - base : 64;
-        unsigned long long mkey = kNoKey;
-        int tslot = -1, tnode = -1;
-        if (lane < cnt) {
-          const ToiEntry u = c.stage[base + lane];
-          mkey = u.key;
-          tslot = u.slot;
-          tnode = c.pos[u.slot];
-        }
-        for (int k = 0; k < cnt; ++k) {
-          const uint32_t khi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(mkey >> 32)), k));
-          const uint32_t klo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(mkey & 0xffffffffull)), k));
-          const unsigned long long uk = (static_cast<unsigned long long>(khi) << 32) | klo;
-          const int us = __builtin_amdgcn_readlane(tslot, k);
-          const int p = __builtin_amdgcn_readlane(tnode, k);
-          if (lane == k) tslot = -1;  // this lane's slot is handled now
-          if (uk == kNoKey) {  // removed: the last entry takes its node (a removal always has one)
-            if (p >= 0) {
-              --n;
-              if (p < n) place(q, n, p, q.key(n), q.slot(n), lane, tslot, tnode);
-              if (lane == 0) c.pos[us] = -1;
-            }
-          } else if (p >= 0) {
-            place(q, n, p, uk, us, lane, tslot, tnode);
-          } else if (n < c.cap) {
-            sift_up(q, n, uk, us, lane, tslot, tnode);
-            ++n;
-          } else {  // the queue is full: reported as an overflow
-            if (lane == 0) c.ctl[kCcdOverflow] = 1u;
-            ovf = 1;
-            break;
-          }
-        }
+    const int nmiss = s_nmiss;
+    if (nmiss) {
+      const int r = t & (kToiLanes - 1);
+      for (int k = t / kToiLanes; k < nmiss; k += kEventBlock / kToiLanes) {
+        const int slot = c.stage[k];
+        const int4 sb = c.slot_bodies[slot];
+        float toi;
+        const bool hit = pair_toi(b, c, sb.x, sb.y, fz[sb.z & kKey], fz[sb.w & kKey], end_time, target, on_penetration,
+                                  r, &toi);
+        if (r == 0) set_key(slot, hit ? toi_key(toi, c.slot_pair[slot]) : kNoKey);
       }
+      ++late;
+      __syncthreads();
+    }
+    const int nd = s_ndirty;
+    for (int k = wave; k < nd; k += kEventBlock / 64) {
+      const int g = s_dirty[k];
+      const unsigned long long m = range_min(c.key, g << sh, min((g + 1) << sh, ns), -1, lane);
       if (lane == 0) {
-        s_hsize = n;
-        if (ovf) s_go = 0;
+        s_min[g] = m;
+        s_bits[g >> 5] = 0u;
       }
     }
     __syncthreads();
-    if (!s_go) break;
+    if (t == 0) s_nmiss = s_ndirty = 0;
+    if (late >= kEventMisses) break;
   }
-  if (LdsFrozen) {
-    __syncthreads();
+  __syncthreads();
+  if (LdsFrozen)
     for (int k = t; k < b.n; k += kEventBlock) c.frozen[k] = s_fz[k];
-  }
+  for (int g = t; g < ng; g += kEventBlock) c.group[g] = s_min[g];
   if (t == 0) {
     const int nimp = s_nimp;
+    c.ctl[kCcdState] = s_go ? kQueueOpen : kQueueDone;
     c.ctl[kCcdImpacts] = uint32_t(nimp);
     c.ctl[kCcdLastToi] = nimp > 0 ? uint32_t(c.impacts[nimp - 1] >> 32) : 0u;
   }
@@ -537,19 +660,20 @@ int blocks_of(int n, int bs) { return (n + bs - 1) / bs; }
 
 }  // namespace
 
-void launch_ccd_predict(const DevBodies& b, const int2* pairs, int npairs, CcdBufs& c, float end_time, float dt0,
-                        float target, int on_penetration, hipStream_t s) {
-  hipLaunchKernelGGL(k_ccd_reset, dim3(1), dim3(64), 0, s, c.ctl);
-  fill_u32(reinterpret_cast<uint32_t*>(c.frozen), 0xbf800000u, size_t(b.n), s);  // -1
-  fill_u32(c.deg, 0u, size_t(b.n), s);
-  fill_u32(c.fill, 0u, size_t(b.n), s);
-  if (npairs > 0) {
-    hipLaunchKernelGGL(k_ccd_first_pass, dim3(blocks_of(npairs, 128)), dim3(128), 0, s, b, pairs, npairs, c,
-                       end_time, dt0, target, on_penetration);
-    hipLaunchKernelGGL(k_ccd_degree, dim3(blocks_of(npairs, 256)), dim3(256), 0, s, npairs, c);
-    scan_exclusive_u32(c.deg, c.off, b.n, *c.scan, s);
-    hipLaunchKernelGGL(k_ccd_fill, dim3(blocks_of(npairs, 256)), dim3(256), 0, s, npairs, c);
-  }
+void launch_ccd_first(const DevBodies& b, const int2* pairs, int npairs, CcdBufs& c, float end_time, float dt0,
+                      float target, int on_penetration, hipStream_t s) {
+  hipLaunchKernelGGL(k_ccd_begin, dim3(blocks_of(std::max(b.n, int(kCcdWords)), 256)), dim3(256), 0, s, b.n, c);
+  if (npairs <= 0) return;
+  hipLaunchKernelGGL(k_ccd_first_pass, dim3(blocks_of(npairs, kFirstPairs)), dim3(256), 0, s, b, pairs, npairs, c,
+                     end_time, dt0, target, on_penetration);
+  scan_exclusive_u32(c.deg, c.off, b.n, *c.scan, s);
+  hipLaunchKernelGGL(k_ccd_fill, dim3(blocks_of(npairs, 256)), dim3(256), 0, s, npairs, c);
+}
+
+void launch_ccd_events(const DevBodies& b, CcdBufs& c, float end_time, float dt0, float target, int on_penetration,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(k_ccd_foresee, dim3(std::min(std::max(b.n, 1), 4096)), dim3(256), 0, s, b, c, end_time, target,
+                     on_penetration);
   if (b.n <= kFzCap)
     hipLaunchKernelGGL(k_ccd_events<true>, dim3(1), dim3(kEventBlock), 0, s, b, c, end_time, dt0, target,
                        on_penetration);

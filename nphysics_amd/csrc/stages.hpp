@@ -299,21 +299,19 @@ void launch_joint_residual(const DevBodies& b, JointBufs& j, double* out, hipStr
 void launch_joint_union(const DevBodies& b, const JointBufs& j, int* parent, uint32_t* touch, hipStream_t s);
 
 // k_ccd.hip --------------------------------------------------------------------------------
-// A queued time of impact: key = time bits << 32 | pair index (times are >= 0, so keys order by
-// time, then pair) and the pair's CCD slot.
-struct ToiEntry {
-  unsigned long long key;
-  int slot;
-};
 struct CcdBufs {
   float* body_time;        // [n] time each body's motion starts from (SubstepState::body_times)
   float* frozen;           // [n] per body key: freeze time, < 0 when not frozen
   int* slot_pair;          // [P] pair index of each CCD slot (pairs with a CCD-enabled side)
   int4* slot_bodies;       // [P] the slot's two bodies and their keys; a key | kSlotStatic when its
                            // body is not dynamic
-  int* pos;                // [P] node of each slot's entry in the queue, -1 when it has none
-  ToiEntry* heap;          // [cap] first-pass entries, then the queue's nodes below its LDS levels
-  ToiEntry* stage;         // [P] entries of one re-sweep
+  // times of impact: key = time bits << 32 | pair index (times are >= 0, so keys order by time, then pair)
+  unsigned long long* key;       // [P] each slot's queued one, all ones for none
+  unsigned long long* seen_key;  // [2P] per slot and side: with that side's body frozen at seen_at
+  float* seen_at;                // [2P] (< 0: not known)
+  unsigned long long* group;     // [kCcdGroups] smallest keys of groups of slots, between two launches of the queue
+  int* stage;              // [P] slots of one re-sweep to be computed
+  int* bodies;             // [n] the dynamic bodies with CCD slots
   unsigned long long* impacts;  // [cap] keys of the confirmed impacts, in order
   uint32_t* ctl;           // control words kCcd*
   int cap;
@@ -334,15 +332,21 @@ struct CcdBufs {
   int* adj;                // [2P] the slots of each dynamic body, at off
 };
 enum : int {
-  kCcdSlots = 0, kCcdEntries = 1, kCcdAnyIn = 2, kCcdMinAfter = 3, kCcdKind = 4, kCcdImpacts = 5,
-  kCcdLastToi = 6, kCcdOverflow = 7, kCcdMinOver = 8, kCcdList = 9, kCcdWords = 16
+  kCcdSlots = 0, kCcdBodies = 1, kCcdAnyIn = 2, kCcdMinAfter = 3, kCcdKind = 4, kCcdImpacts = 5,
+  kCcdLastToi = 6, kCcdOverflow = 7, kCcdMinOver = 8, kCcdList = 9, kCcdState = 10,
+  kCcdWords = 16
 };
+enum : uint32_t { kQueueNew = 0, kQueueOpen = 1, kQueueDone = 2 };
 enum : int { PREDICT_NONE = 0, PREDICT_AFTER_END = 1, PREDICT_IMPACTS = 2 };
+constexpr int kCcdGroups = 4096;
 constexpr int kSlotStatic = 1 << 30;  // body counts stay below 2^30
-// predict_next_impacts up to end_time: control words reset, freeze times cleared, every CCD pair's
-// time of impact, then the queue in one workgroup (kind, impacts, last impact time in ctl)
-void launch_ccd_predict(const DevBodies& b, const int2* pairs, int npairs, CcdBufs& c, float end_time, float dt0,
-                        float target, int on_penetration, hipStream_t s);
+// predict_next_impacts up to end_time: control words reset, freeze times cleared and every CCD pair's
+// time of impact; then rounds of the queue until ctl[kCcdState] is kQueueDone (kind, impacts and last impact time
+// in ctl). A round gets further by one event at least.
+void launch_ccd_first(const DevBodies& b, const int2* pairs, int npairs, CcdBufs& c, float end_time, float dt0,
+                      float target, int on_penetration, hipStream_t s);
+void launch_ccd_events(const DevBodies& b, CcdBufs& c, float end_time, float dt0, float target, int on_penetration,
+                       hipStream_t s);
 void launch_ccd_seed(const DevBodies& b, const int2* pairs, CcdBufs& c, int nimp, hipStream_t s);
 void launch_ccd_touch(const DevBodies& b, const int2* pairs, int npairs, CcdBufs& c, hipStream_t s);
 void launch_ccd_prepare(const DevBodies& b, CcdBufs& c, float dt_sub, float last_toi, hipStream_t s);

@@ -234,9 +234,9 @@ struct World {
   bool any_ccd = false;
   std::vector<int> h_ccd, h_ccd_key;
   std::map<std::pair<int, int>, int> static_owner;  // (scene, static body index) -> first collider
-  DBuf ccd_flags, ccd_keys, ccd_rot, ccd_time, ccd_frozen, ccd_slot, ccd_heap, ccd_stage, ccd_imp, ccd_ctl,
+  DBuf ccd_flags, ccd_keys, ccd_rot, ccd_time, ccd_frozen, ccd_slot, ccd_queue, ccd_seen, ccd_seen_at, ccd_group, ccd_stage, ccd_imp, ccd_ctl,
       ccd_in, ccd_new, ccd_prep, ccd_prepared, ccd_eval, ccd_kept, ccd_cand, ccd_cpos, ccd_list, ccd_lpair,
-      ccd_deg, ccd_off, ccd_fill, ccd_adj, ccd_pos, ccd_sbodies;
+      ccd_deg, ccd_off, ccd_fill, ccd_adj, ccd_bodies, ccd_sbodies;
   ContactBufs ccd_cb;
   int ccd_cap = 0, ccd_nimp = 0;
   float ccd_last_toi = 0.0f, ccd_min_over = 0.0f;
@@ -1747,20 +1747,20 @@ struct World {
   int ensure_ccd() {
     if (n >= kSlotStatic) return set_err(NPHYS_ERR_CAPACITY, "CCD supports fewer than 2^30 bodies");
     const size_t nn = size_t(std::max(n, 1)), P = size_t(std::max(npairs, 1));
-    for (DBuf* b : {&ccd_time, &ccd_frozen, &ccd_in, &ccd_new, &ccd_prep, &ccd_prepared, &ccd_deg, &ccd_off, &ccd_fill})
+    for (DBuf* b : {&ccd_time, &ccd_frozen, &ccd_in, &ccd_new, &ccd_prep, &ccd_prepared, &ccd_deg, &ccd_off, &ccd_fill, &ccd_bodies})
       HIPCK(b->ensure(nn * 4));
     HIPCK(ccd_adj.ensure(2 * P * 4));
-    for (DBuf* b : {&ccd_slot, &ccd_pos, &ccd_eval, &ccd_kept, &ccd_cand, &ccd_cpos, &ccd_lpair})
+    for (DBuf* b : {&ccd_slot, &ccd_stage, &ccd_eval, &ccd_kept, &ccd_cand, &ccd_cpos, &ccd_lpair})
       HIPCK(b->ensure(P * 4));
     HIPCK(ccd_list.ensure(P * sizeof(int2)));
     HIPCK(ccd_sbodies.ensure(P * sizeof(int4)));
-    HIPCK(ccd_stage.ensure(P * sizeof(ToiEntry)));
-    // the queue holds at most one entry per CCD slot (at most P); the impact list takes 3P + 4096
-    // confirmed impacts (a full list is an error, never a silent loss)
-    const size_t cap = 3 * P + 4096;
-    HIPCK(ccd_heap.ensure(cap * sizeof(ToiEntry)));
-    HIPCK(ccd_imp.ensure(cap * sizeof(unsigned long long)));
-    ccd_cap = int(std::min<size_t>(ccd_heap.bytes / sizeof(ToiEntry), ccd_imp.bytes / sizeof(unsigned long long)));
+    HIPCK(ccd_queue.ensure(P * 8));
+    HIPCK(ccd_seen.ensure(2 * P * 8));
+    HIPCK(ccd_seen_at.ensure(2 * P * 4));
+    HIPCK(ccd_group.ensure(kCcdGroups * 8));
+    // the impact list takes 3P + 4096 confirmed impacts (a full list is an error, never a silent loss)
+    HIPCK(ccd_imp.ensure((3 * P + 4096) * 8));
+    ccd_cap = int(std::min<size_t>(ccd_imp.bytes / 8, size_t(INT_MAX)));
     HIPCK(ccd_ctl.ensure(kCcdWords * 4));
     HIPCK(scan.ensure(std::max(scan_tiles(P), scan_tiles(nn)), stream));
     return NPHYS_OK;
@@ -1772,9 +1772,12 @@ struct World {
     c.frozen = ccd_frozen.as<float>();
     c.slot_pair = ccd_slot.as<int>();
     c.slot_bodies = ccd_sbodies.as<int4>();
-    c.pos = ccd_pos.as<int>();
-    c.heap = ccd_heap.as<ToiEntry>();
-    c.stage = ccd_stage.as<ToiEntry>();
+    c.key = ccd_queue.as<unsigned long long>();
+    c.seen_key = ccd_seen.as<unsigned long long>();
+    c.seen_at = ccd_seen_at.as<float>();
+    c.group = ccd_group.as<unsigned long long>();
+    c.stage = ccd_stage.as<int>();
+    c.bodies = ccd_bodies.as<int>();
     c.impacts = ccd_imp.as<unsigned long long>();
     c.ctl = ccd_ctl.as<uint32_t>();
     c.cap = ccd_cap;
@@ -1817,11 +1820,17 @@ struct World {
   // impact time and min_overstep.
   int ccd_predict(float end_time, float dt0, int* kind) {
     CcdBufs c = ccd_view();
-    launch_ccd_predict(bodies(), pairs.as<int2>(), npairs, c, end_time, dt0, sp.allowed_linear_error,
-                       prm.ccd_on_penetration_enabled, stream);
-    const int rc = readback({{c.ctl, kCcdWords, 0}});
-    if (rc) return rc;
-    if (rb_host[kCcdOverflow]) return set_err(NPHYS_ERR_CAPACITY, "CCD impact queue overflow");
+    const DevBodies b = bodies();
+    const float target = sp.allowed_linear_error;
+    const int on_pen = prm.ccd_on_penetration_enabled;
+    launch_ccd_first(b, pairs.as<int2>(), npairs, c, end_time, dt0, target, on_pen, stream);
+    for (int rounds = 1;; rounds = 4) {  // no impacts, or few: one round ends it
+      for (int k = 0; k < rounds; ++k) launch_ccd_events(b, c, end_time, dt0, target, on_pen, stream);
+      const int rc = readback({{c.ctl, kCcdWords, 0}});
+      if (rc) return rc;
+      if (rb_host[kCcdOverflow]) return set_err(NPHYS_ERR_CAPACITY, "CCD impact queue overflow");
+      if (rb_host[kCcdState] == kQueueDone) break;
+    }
     *kind = int(rb_host[kCcdKind]);
     ccd_nimp = *kind == PREDICT_IMPACTS ? int(rb_host[kCcdImpacts]) : 0;
     uint32_t u = rb_host[kCcdLastToi];
