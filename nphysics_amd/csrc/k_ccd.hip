@@ -555,6 +555,12 @@ __global__ void __launch_bounds__(kEventBlock) k_ccd_events(DevBodies b, CcdBufs
   }
 }
 
+__global__ void __launch_bounds__(256) k_ccd_island(int n, int P, CcdBufs c) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) c.in_t[i] = c.new_t[i] = c.prep[i] = c.prepared[i] = 0u;
+  if (i < P) c.evaluated[i] = c.kept[i] = 0u;
+}
+
 __global__ void __launch_bounds__(256) k_ccd_seed(DevBodies b, const int2* __restrict__ pairs, CcdBufs c, int nimp) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= nimp) return;
@@ -680,6 +686,10 @@ void launch_ccd_events(const DevBodies& b, CcdBufs& c, float end_time, float dt0
   else
     hipLaunchKernelGGL(k_ccd_events<false>, dim3(1), dim3(kEventBlock), 0, s, b, c, end_time, dt0, target,
                        on_penetration);
+}
+
+void launch_ccd_island(int n, int P, CcdBufs& c, hipStream_t s) {
+  hipLaunchKernelGGL(k_ccd_island, dim3(blocks_of(std::max(n, P), 256)), dim3(256), 0, s, n, P, c);
 }
 
 void launch_ccd_seed(const DevBodies& b, const int2* pairs, CcdBufs& c, int nimp, hipStream_t s) {

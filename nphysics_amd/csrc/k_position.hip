@@ -206,7 +206,7 @@ __global__ void __launch_bounds__(64) k_position(DevBodies b, SimParams p, Solve
 template <bool kMask>
 __global__ void __launch_bounds__(kRunLanes) k_position_run(DevBodies b, SimParams p, SolverBufs sb, ClassRun run) {
   for (int k = 0; k < run.n; ++k) {
-    position_class<kMask>(GlobalPose{b}, b, p, sb, run.r[k], threadIdx.x, kRunLanes, [](int i) { return i; });
+    position_class<kMask>(GlobalPose{b}, b, p, sb, run.r[k], threadIdx.x, blockDim.x, [](int i) { return i; });
     __syncthreads();
   }
 }
@@ -280,8 +280,12 @@ void launch_position_blocked(const DevBodies& b, const SimParams& p, SolverBufs&
 }
 
 void launch_position_run(const DevBodies& b, const SimParams& p, SolverBufs& sb, const ClassRun& run, hipStream_t s) {
-  if (b.kmask) hipLaunchKernelGGL(k_position_run<true>, dim3(1), dim3(kRunLanes), 0, s, b, p, sb, run);
-  else hipLaunchKernelGGL(k_position_run<false>, dim3(1), dim3(kRunLanes), 0, s, b, p, sb, run);
+  // as many lanes as the largest class takes: fewer waves meet at each barrier
+  int lanes = 64;
+  for (int k = 0; k < run.n; ++k) lanes = std::max(lanes, ((4 * run.r[k].multi + 63) & ~63) + run.r[k].single);
+  const dim3 block(unsigned(std::min((lanes + 63) & ~63, kRunLanes)));
+  if (b.kmask) hipLaunchKernelGGL(k_position_run<true>, dim3(1), block, 0, s, b, p, sb, run);
+  else hipLaunchKernelGGL(k_position_run<false>, dim3(1), block, 0, s, b, p, sb, run);
 }
 
 }  // namespace nph

@@ -347,6 +347,8 @@ void launch_ccd_first(const DevBodies& b, const int2* pairs, int npairs, CcdBufs
                       float target, int on_penetration, hipStream_t s);
 void launch_ccd_events(const DevBodies& b, CcdBufs& c, float end_time, float dt0, float target, int on_penetration,
                        hipStream_t s);
+// in_t, new_t, prep and prepared of n, evaluated and kept of P cleared
+void launch_ccd_island(int n, int P, CcdBufs& c, hipStream_t s);
 void launch_ccd_seed(const DevBodies& b, const int2* pairs, CcdBufs& c, int nimp, hipStream_t s);
 void launch_ccd_touch(const DevBodies& b, const int2* pairs, int npairs, CcdBufs& c, hipStream_t s);
 void launch_ccd_prepare(const DevBodies& b, CcdBufs& c, float dt_sub, float last_toi, hipStream_t s);

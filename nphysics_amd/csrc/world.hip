@@ -174,7 +174,10 @@ struct World {
   int ncolours = 0;
   long rec_stride = 0;
   int colour_rounds = 0;
-  static constexpr int kRoundBatch = 4;  // colouring rounds launched between polls
+  // colouring rounds enqueued before the host looks: what the last solve took (a step's, a CCD substep's) and one
+  // more, within these bounds
+  static constexpr int kMinRounds = 4, kMaxRounds = 32;
+  int round_batch[2] = {kMinRounds, kMinRounds};
   std::vector<int> colour_visit;  // colour classes in visiting order
   long solve_count = 0;    // solves performed, never reset
   std::vector<ClassSpan> h_span;    // their slots, in that order
@@ -1094,8 +1097,9 @@ struct World {
     return NPHYS_OK;
   }
 
-  // The narrow phase of `np` pairs (in pair order; their number also at *count_dev) into `out`.
-  int narrow_phase_of(const int2* list, int np, uint32_t* count_dev, ContactBufs& out) {
+  // The narrow phase of `np` pairs (in pair order; their number also at *count_dev) into `out`. Without
+  // `totals`, the host does not wait for its contact and manifold counts.
+  int narrow_phase_of(const int2* list, int np, uint32_t* count_dev, ContactBufs& out, bool totals = true) {
     NarrowPhaseBufs v{};
     const int rc0 = ensure_narrow(np, &out, v);
     if (rc0) return rc0;
@@ -1103,6 +1107,7 @@ struct World {
     fill_u32(v.totals, 0u, 4, stream);
     launch_narrow_bins(bodies(), list, v, out.view(), stream);
     launch_narrow_phase(bodies(), list, v, out.view(), stream);
+    if (!totals) return NPHYS_OK;
     const int rc = readback({{v.totals, 2, 0}});
     if (rc) return rc;
     out.C = int(rb_host[0]);
@@ -1209,12 +1214,12 @@ struct World {
     std::stable_sort(perm.begin(), perm.end(), [&](int a, int b) { return size_bucket(size[a]) < size_bucket(size[b]); });
   }
 
-  // Words of bp_small of the colouring: whether each round of a batch left a manifold uncoloured, the
-  // last round that coloured one, the number of colours.
-  static constexpr int kSmRemaining = 32, kSmLastRound = kSmRemaining + kRoundBatch, kSmColours = kSmLastRound + 1;
+  // Words of bp_small of the colouring: whether a round of a batch but the last, and the last one, left a
+  // manifold uncoloured, the number of colours, the last round that coloured one.
+  static constexpr int kSmRemaining = 32, kSmColours = kSmRemaining + 2, kSmLastRound = kSmColours + 1, kSmColouring = 4;
 
   // Colouring, slots and assembly of the solve's manifolds, and the class bounds back on the host
-  // (colour_visit, h_span, class_contacts). The rounds run in batches of four: a round after the last one that
+  // (colour_visit, h_span, class_contacts). The rounds run in batches: a round after the last one that
   // colours anything changes nothing, and the device records that last round. A batch, the colour order and the assembly
   // are enqueued together and read back once; where manifolds stay uncoloured, or there are more
   // colours than the order has digits for, the rest runs again. `after` enqueues what does not depend on the colouring, before the wait.
@@ -1230,17 +1235,17 @@ struct World {
     // recorded samples and predictions keep the row order that does not depend on the contact counts
     split_order = !learned_rows();
     bool rounds = true, waiting = true;
+    int& batch = round_batch[ccd_sub ? 1 : 0];
     for (int round = 1;;) {
       if (rounds) {
-        if (round + kRoundBatch >= 0xffff) return set_err(NPHYS_ERR_STATE, "colouring did not converge");
+        if (round + batch >= 0xffff) return set_err(NPHYS_ERR_STATE, "colouring did not converge");
         // the last round's word stays when this is not the first batch
-        fill_u32(sm + kSmRemaining, 0u, round == 1 ? kRoundBatch + 2 : kRoundBatch, stream);
-        if (round > 1) fill_u32(sm + kSmColours, 0u, 1, stream);
-        for (int k = 0; k < kRoundBatch; ++k, ++round)
-          launch_colour_round(c, M, round, sm + kSmRemaining + k, sm + kSmLastRound, v, stream);
+        fill_u32(sm + kSmRemaining, 0u, round == 1 ? kSmColouring : kSmColouring - 1, stream);
+        for (int k = 0; k < batch; ++k, ++round)
+          launch_colour_round(c, M, round, sm + kSmRemaining + (k == batch - 1 ? 1 : 0), sm + kSmLastRound, v, stream);
       }
       launch_colour_order(c, M, C, digits, split_order, v, sm + kSmColours, stream);
-      const uint32_t seq = rb_post({{sm + kSmRemaining, kRoundBatch + 2, 0},
+      const uint32_t seq = rb_post({{sm + kSmRemaining, kSmColouring, 0},
                                     {v.col_start, digits + 1, kRbClass},
                                     {v.class_rec, digits + 1, kRbClass + kMaxColours + 2}});
       launch_assemble(b, c, pc.view(), have_solved ? pc.M : 0, M, ps, v, mat_table(), stream);
@@ -1248,8 +1253,8 @@ struct World {
       waiting = false;
       const int rc = rb_wait(seq);
       if (rc) return rc;
-      rounds = rb_host[kRoundBatch - 1] != 0;
-      ncolours = int(rb_host[kRoundBatch + 1]);
+      rounds = rb_host[1] != 0;
+      ncolours = int(rb_host[kSmColours - kSmRemaining]);
       if (rounds) continue;
       if (ncolours > kMaxColours) return set_err(NPHYS_ERR_STATE, "too many colours");
       if (ncolours * (split_order ? 2 : 1) <= digits) break;
@@ -1259,7 +1264,8 @@ struct World {
       if (rc2) return rc2;
       v = sv_view();
     }
-    colour_rounds = int(rb_host[kRoundBatch]);
+    colour_rounds = int(rb_host[kSmLastRound - kSmRemaining]);
+    batch = std::min(std::max(colour_rounds + 1, kMinRounds), kMaxRounds);
     // visit order (the SplitMix64 Fisher-Yates shuffle seeded by the solve index), slot ranges in that
     // order and the largest class
     const uint32_t* h_colstart = rb_host + kRbClass;
@@ -1852,9 +1858,7 @@ struct World {
     const float dt_sub = dt0 - last_toi;
     const DevBodies b = bodies();
     CcdBufs c = ccd_view();
-    const size_t nn = size_t(n), P = size_t(std::max(npairs, 1));
-    for (uint32_t* a : {c.in_t, c.new_t, c.prep, c.prepared}) fill_u32(a, 0u, nn, stream);
-    for (uint32_t* a : {c.evaluated, c.kept}) fill_u32(a, 0u, P, stream);
+    launch_ccd_island(n, std::max(npairs, 1), c, stream);
     launch_ccd_seed(b, pairs.as<int2>(), c, ccd_nimp, stream);
     for (;;) {  // island rounds
       launch_ccd_touch(b, pairs.as<int2>(), npairs, c, stream);
@@ -1863,7 +1867,7 @@ struct World {
       if ((rc = readback({{c.ctl + kCcdList, 1, 0}}))) return rc;
       const int nl = int(rb_host[0]);
       if (nl == 0) break;
-      if ((rc = narrow_phase_of(c.list, nl, c.ctl + kCcdList, ccd_cb))) return rc;
+      if ((rc = narrow_phase_of(c.list, nl, c.ctl + kCcdList, ccd_cb, false))) return rc;
       launch_ccd_grow(b, c, nl, np_count.as<uint32_t>(), stream);
       launch_ccd_merge(n, c, stream);
     }
