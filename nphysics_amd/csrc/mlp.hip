@@ -2,7 +2,7 @@
 //
 // The network and its training have no reference counterpart: the reference warm-starts only
 // from the impulse cache (signorini_coulomb_pyramid_model.rs:104-108). Training runs on the GPU:
-// the dataset lives in HBM, each mini-batch is one forward pass with stores, one backward pass,
+// the dataset lives in HBM, each mini-batch is one forward and backward pass,
 // a weight-gradient reduction and an Adam update, all on the trainer's stream.
 #include <hip/hip_runtime.h>
 
@@ -22,7 +22,7 @@ struct nphys_mlp {
   hipStream_t stream = nullptr;
   DBuf params, mom1, mom2, grad, img;
   DBuf X, T, perm, losses;
-  DBuf A0, Z1, Z2, H1, H2, Y, D3, D2, D1, loss_part, gpart, fx, fy;
+  DBuf A0, H1, H2, D3, D2, D1, loss_part, gpart, fx, fy, ft, floss;
   long n = 0;          // dataset rows
   int bcap = 0;        // batch capacity of the buffers
   long adam_t = 0;     // Adam steps taken
@@ -38,8 +38,7 @@ struct nphys_mlp {
     if (B <= bcap) return hipSuccess;
     const size_t b = size_t(B);
     hipError_t e;
-    if ((e = A0.ensure(b * kK1 * 2)) || (e = Z1.ensure(b * kHid * 4)) || (e = Z2.ensure(b * kHid * 4)) ||
-        (e = H1.ensure(b * kHid * 2)) || (e = H2.ensure(b * kHid * 2)) || (e = Y.ensure(b * kOut * 4)) ||
+    if ((e = A0.ensure(b * kK1 * 2)) || (e = H1.ensure(b * kHid * 2)) || (e = H2.ensure(b * kHid * 2)) ||
         (e = D3.ensure(b * kK1 * 2)) || (e = D2.ensure(b * kHid * 2)) || (e = D1.ensure(b * kHid * 2)) ||
         (e = loss_part.ensure(size_t(1024) * 8)) ||
         (e = gpart.ensure(size_t(mlp_grad_blocks(B)) * kNumTrained * 4)))
@@ -55,11 +54,8 @@ struct nphys_mlp {
     b.T = Td;
     b.idx = idx;
     b.A0 = A0.as<uint16_t>();
-    b.Z1 = Z1.as<float>();
-    b.Z2 = Z2.as<float>();
     b.H1 = H1.as<uint16_t>();
     b.H2 = H2.as<uint16_t>();
-    b.Y = Y.as<float>();
     b.D3 = D3.as<uint16_t>();
     b.D2 = D2.as<uint16_t>();
     b.D1 = D1.as<uint16_t>();
@@ -96,21 +92,16 @@ void init_params(uint64_t seed, std::vector<float>& p) {
 }
 
 // Scratch of nphys_mlp_gradients_noalloc: the training-pass buffers of one batch of at most
-// kNoAllocMaxRows rows (what ensure_batch allocates for nphys_mlp_gradients) and the identity row
-// index, carved out of one file-scope device array at 256-byte aligned offsets (about 9.9 MB; every
-// device the library runs on holds its copy until the process ends). Every byte a call reads is
+// kNoAllocMaxRows rows (what ensure_batch allocates for nphys_mlp_gradients), carved out of
+// one file-scope device array at 256-byte aligned offsets (about 6.0 MB; every device the library runs on holds its copy until the process ends). Every byte a call reads is
 // written earlier in the same call, so nothing needs clearing between calls.
 constexpr int64_t kNoAllocMaxRows = 4096;
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 constexpr size_t kR = size_t(kNoAllocMaxRows);
-constexpr size_t kScrIdx = 0;
-constexpr size_t kScrA0 = align256(kScrIdx + kR * 4);
-constexpr size_t kScrZ1 = align256(kScrA0 + kR * kK1 * 2);
-constexpr size_t kScrZ2 = align256(kScrZ1 + kR * kHid * 4);
-constexpr size_t kScrH1 = align256(kScrZ2 + kR * kHid * 4);
+constexpr size_t kScrA0 = 0;
+constexpr size_t kScrH1 = align256(kScrA0 + kR * kK1 * 2);
 constexpr size_t kScrH2 = align256(kScrH1 + kR * kHid * 2);
-constexpr size_t kScrY = align256(kScrH2 + kR * kHid * 2);
-constexpr size_t kScrD3 = align256(kScrY + kR * kOut * 4);
+constexpr size_t kScrD3 = align256(kScrH2 + kR * kHid * 2);
 constexpr size_t kScrD2 = align256(kScrD3 + kR * kK1 * 2);
 constexpr size_t kScrD1 = align256(kScrD2 + kR * kHid * 2);
 constexpr size_t kScrLoss = align256(kScrD1 + kR * kHid * 2);
@@ -142,11 +133,6 @@ int scratch_on_current_device(unsigned char** out) {
   }
   *out = static_cast<unsigned char*>(g_scratch_ptr[dev]);
   return NPHYS_OK;
-}
-
-__global__ void k_mlp_iota(int* __restrict__ idx, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) idx[i] = i;
 }
 
 }  // namespace
@@ -311,22 +297,15 @@ int nphys_mlp_gradients(nphys_mlp* m, const float* X, const float* T, int64_t n,
   const int B = int(n);
   HIPCK(m->ensure_batch(((B + 63) / 64) * 64));
   HIPCK(m->fx.ensure(size_t(n) * kFeat * 4));
-  HIPCK(m->fy.ensure(std::max(size_t(n) * kOut * 4, size_t(n) * 4)));
-  DBuf tt, id;
-  HIPCK(tt.ensure(size_t(n) * kOut * 4));
-  HIPCK(id.ensure(size_t(n) * 4));
-  std::vector<int> iota(static_cast<size_t>(n));
-  for (int i = 0; i < B; ++i) iota[size_t(i)] = i;
-  DBuf dl;
-  HIPCK(dl.ensure(8));
+  HIPCK(m->ft.ensure(size_t(n) * kOut * 4));
+  HIPCK(m->floss.ensure(8));
   HIPCK(hipMemcpyAsync(m->fx.p, X, size_t(n) * kFeat * 4, hipMemcpyHostToDevice, m->stream));
-  HIPCK(hipMemcpyAsync(tt.p, T, size_t(n) * kOut * 4, hipMemcpyHostToDevice, m->stream));
-  HIPCK(hipMemcpyAsync(id.p, iota.data(), size_t(n) * 4, hipMemcpyHostToDevice, m->stream));
-  MlpBatch b = m->batch(B, m->fx.as<float>(), tt.as<float>(), id.as<int>());
-  mlp_batch_gradients(m->dev(), b, m->grad.as<float>(), dl.as<double>(), m->stream);
+  HIPCK(hipMemcpyAsync(m->ft.p, T, size_t(n) * kOut * 4, hipMemcpyHostToDevice, m->stream));
+  MlpBatch b = m->batch(B, m->fx.as<float>(), m->ft.as<float>(), nullptr);
+  mlp_batch_gradients(m->dev(), b, m->grad.as<float>(), m->floss.as<double>(), m->stream);
   HIPCK(hipGetLastError());
   HIPCK(hipMemcpyAsync(grad, m->grad.p, kNumTrained * 4, hipMemcpyDeviceToHost, m->stream));
-  HIPCK(hipMemcpyAsync(loss, dl.p, 8, hipMemcpyDeviceToHost, m->stream));
+  HIPCK(hipMemcpyAsync(loss, m->floss.p, 8, hipMemcpyDeviceToHost, m->stream));
   HIPCK(hipStreamSynchronize(m->stream));
   return NPHYS_OK;
 }
@@ -344,20 +323,15 @@ int nphys_mlp_gradients_noalloc(nphys_mlp* m, const float* X, const float* T, in
   b.B = int(n);
   b.X = X;
   b.T = T;
-  b.idx = reinterpret_cast<const int*>(base + kScrIdx);
+  b.idx = nullptr;
   b.A0 = reinterpret_cast<uint16_t*>(base + kScrA0);
-  b.Z1 = reinterpret_cast<float*>(base + kScrZ1);
-  b.Z2 = reinterpret_cast<float*>(base + kScrZ2);
   b.H1 = reinterpret_cast<uint16_t*>(base + kScrH1);
   b.H2 = reinterpret_cast<uint16_t*>(base + kScrH2);
-  b.Y = reinterpret_cast<float*>(base + kScrY);
   b.D3 = reinterpret_cast<uint16_t*>(base + kScrD3);
   b.D2 = reinterpret_cast<uint16_t*>(base + kScrD2);
   b.D1 = reinterpret_cast<uint16_t*>(base + kScrD1);
   b.loss_part = reinterpret_cast<double*>(base + kScrLoss);
   b.gpart = reinterpret_cast<float*>(base + kScrGpart);
-  hipLaunchKernelGGL(k_mlp_iota, dim3((b.B + 255) / 256), dim3(256), 0, s, reinterpret_cast<int*>(base + kScrIdx),
-                     b.B);
   mlp_batch_gradients(m->dev(), b, grad, loss, s);
   HIPCK(hipGetLastError());
   if (!stream) HIPCK(hipStreamSynchronize(s));

@@ -54,13 +54,10 @@ struct MlpBatch {
   int B;
   const float* X;        // [n][24] dataset features
   const float* T;        // [n][3] dataset targets (impulse units)
-  const int* idx;        // [B] dataset rows of this batch
+  const int* idx;        // [B] dataset rows of this batch, or null for rows 0 .. B - 1
   uint16_t* A0;          // [B][32] normalised inputs, bf16
-  float* Z1;             // [B][128] pre-activations
-  float* Z2;
   uint16_t* H1;          // [B][128] activations, bf16
   uint16_t* H2;
-  float* Y;              // [B][3] outputs (normalised units)
   uint16_t* D3;          // [B][32] dL/dY, bf16 (k padded)
   uint16_t* D2;          // [B][128] dL/dZ2, bf16
   uint16_t* D1;          // [B][128] dL/dZ1, bf16
@@ -72,7 +69,7 @@ struct MlpBatch {
 void mlp_pack_images(const float* params, uint16_t* img, hipStream_t s);
 // Inference: out[r][3] = network(features[r]) in impulse units.
 void mlp_infer(const MlpDev& m, const float* X, int n, float* out, hipStream_t s);
-// One training pass over a batch: forward with stores, loss and backward, weight gradients
+// One training pass over a batch: forward, loss and backward, weight gradients
 // reduced into grad[kNumTrained] (mean over the batch), loss (mean) into *loss.
 int mlp_grad_blocks(int B);
 void mlp_batch_gradients(const MlpDev& m, MlpBatch& b, float* grad, double* loss, hipStream_t s);
