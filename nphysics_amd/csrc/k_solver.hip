@@ -205,35 +205,17 @@ __global__ void __launch_bounds__(kThreads) k_colour_hist(DevContacts c, int M, 
   if (threadIdx.x == 0) atomicMax(ncol, s_most);
 }
 
-// Per slot (colour order): bodies with their dynamic flag in bit 30, first row record, contact
-// count and first contact index, packed into one int4; per manifold its slot and first row record; per
-// class its first slot and first row record (col_start, class_rec; one more entry ends the last).
+// The manifolds of the tile at `base` into their slots; s_m, s_c: the digits' first slots and records in this tile.
 template <int kDigits, int kThreads, bool kSplit>
-__global__ void __launch_bounds__(kThreads) k_colour_scatter(DevContacts c, int M, int C, int ntiles, SolverBufs sb) {
+__device__ void scatter_tile(const DevContacts& c, int M, int base, const SolverBufs& sb, uint32_t* s_m, uint32_t* s_c,
+                             uint32_t (*s_wave)[kDigits]) {
   constexpr int kWaves = kThreads / 64;
   constexpr int kBits = kDigits == 512 ? 9 : 12;
-  __shared__ uint32_t s_m[kDigits], s_c[kDigits];
-  __shared__ uint32_t s_wave[kWaves][kDigits];  // per wave: manifolds, and their contacts from bit 16 up
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const uint64_t below = (1ull << lane) - 1ull;
-  for (int d = tid; d < kDigits; d += kThreads) {
-    s_m[d] = sb.offs[long(d) * ntiles + blockIdx.x];
-    s_c[d] = sb.offs[long(kDigits + d) * ntiles + blockIdx.x] - uint32_t(M);
-    if (blockIdx.x == 0) {
-      sb.col_start[d] = s_m[d];
-      sb.class_rec[d] = s_c[d];
-    }
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) s_wave[w][d] = 0u;
-  }
-  if (blockIdx.x == 0 && tid == 0) {
-    sb.col_start[kDigits] = uint32_t(M);
-    sb.class_rec[kDigits] = uint32_t(C);
-  }
-  __syncthreads();
   for (int k = 0; k < kColourTile; k += kThreads) {
-    const int m = int(blockIdx.x) * kColourTile + k + tid;
-    if (int(blockIdx.x) * kColourTile + k >= M) break;
+    const int m = base + k + tid;
+    if (base + k >= M) break;
     const bool valid = m < M;
     const uint32_t cnt = valid ? uint32_t(c.mcount[m]) : 0u;
     const uint32_t d = valid ? colour_digit<kDigits, kSplit>(sb.state[m], cnt) : 0u;
@@ -275,6 +257,223 @@ __global__ void __launch_bounds__(kThreads) k_colour_scatter(DevContacts c, int 
     }
     __syncthreads();
   }
+}
+
+// Per slot (colour order): bodies with their dynamic flag in bit 30, first row record, contact
+// count and first contact index, packed into one int4; per manifold its slot and first row record; per
+// class its first slot and first row record (col_start, class_rec; one more entry ends the last).
+template <int kDigits, int kThreads, bool kSplit>
+__global__ void __launch_bounds__(kThreads) k_colour_scatter(DevContacts c, int M, int C, int ntiles, SolverBufs sb) {
+  constexpr int kWaves = kThreads / 64;
+  __shared__ uint32_t s_m[kDigits], s_c[kDigits];
+  __shared__ uint32_t s_wave[kWaves][kDigits];  // per wave: manifolds, and their contacts from bit 16 up
+  const int tid = threadIdx.x;
+  for (int d = tid; d < kDigits; d += kThreads) {
+    s_m[d] = sb.offs[long(d) * ntiles + blockIdx.x];
+    s_c[d] = sb.offs[long(kDigits + d) * ntiles + blockIdx.x] - uint32_t(M);
+    if (blockIdx.x == 0) {
+      sb.col_start[d] = s_m[d];
+      sb.class_rec[d] = s_c[d];
+    }
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s_wave[w][d] = 0u;
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    sb.col_start[kDigits] = uint32_t(M);
+    sb.class_rec[kDigits] = uint32_t(C);
+  }
+  __syncthreads();
+  scatter_tile<kDigits, kThreads, kSplit>(c, M, int(blockIdx.x) * kColourTile, sb, s_m, s_c, s_wave);
+}
+
+// ---- colouring and colour order of a small world in one workgroup ----
+// Degrees, adjacency, rounds and order with the graph in LDS: the same states, colours and slots as the
+// kernels above give, whose thirteen dependent launches of 2 to 8 us each a world of this size spends its time on:
+// assembly stage 64 -> 45 us at 1,233 manifolds, 59 -> 39 at 320. Its one lane per manifold reads its
+// neighbours one after another, so with a body of more than kSmallDegree manifolds it leaves the rounds to
+// k_colour_round: in a cloud where all bodies touch, every round of some 60 to 200 waits for the longest list (24
+// bodies: 689 us here, 731 there; 45: 3,096 and 1,726).
+constexpr int kSmallThreads = 1024;
+constexpr uint32_t kSmallDegree = 24;
+
+// Exclusive sum over the workgroup's threads (uses s_tot, and ends on a barrier).
+__device__ __forceinline__ uint32_t block_exclusive(uint32_t v, uint32_t* s_tot) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) s_tot[wave] = x;
+  __syncthreads();
+  uint32_t before = 0;
+  for (int w = 0; w < wave; ++w) before += s_tot[w];
+  __syncthreads();
+  return before + x - v;
+}
+
+template <bool kSplit>
+__global__ void __launch_bounds__(kSmallThreads) k_colour_small(DevBodies b, DevContacts c, int M, int C, DevContacts prev,
+                                                              int prevM, const uint32_t* __restrict__ prev_state,
+                                                              SolverBufs sb, uint32_t* words) {
+  constexpr int kEach = kSmallManifolds / kSmallThreads;
+  constexpr int kBodies = kSmallColourBodies / kSmallThreads;
+  __shared__ uint32_t s_state[kSmallManifolds];
+  __shared__ uint32_t s_deg[kSmallColourBodies], s_off[kSmallColourBodies];
+  __shared__ uint16_t s_adj[2 * kSmallManifolds];
+  __shared__ uint32_t s_m[kColourDigits], s_c[kColourDigits];
+  __shared__ uint32_t s_wave[kSmallThreads / 64][kColourDigits];
+  __shared__ uint32_t s_tot[kSmallThreads / 64];
+  __shared__ uint32_t s_left[2], s_last, s_most, s_crowd;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < kSmallColourBodies; i += kSmallThreads) s_deg[i] = 0u;
+  if (tid == 0) s_left[0] = s_left[1] = s_last = s_most = s_crowd = 0u;
+  __syncthreads();
+  int2 bb[kEach];
+  uint2 at[kEach];
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    const int m = tid + kSmallThreads * e;
+    bb[e] = make_int2(0, 0);
+    at[e] = make_uint2(kNoPlace, kNoPlace);
+    if (m >= M) continue;
+    bb[e] = c.mbody[m];
+    if (b.status[bb[e].x] == STATUS_DYNAMIC) at[e].x = atomicAdd(&s_deg[bb[e].x], 1u);
+    if (b.status[bb[e].y] == STATUS_DYNAMIC) at[e].y = atomicAdd(&s_deg[bb[e].y], 1u);
+    sb.place[m] = at[e];
+    const int j = find_manifold(prev, prevM, bb[e].x, bb[e].y);
+    s_state[m] = j >= 0 ? (prev_state[j] & 0xffffu) : kUncoloured;
+  }
+  __syncthreads();
+  {
+    uint32_t sum = 0, most = 0;
+    for (int i = 0; i < kBodies; ++i) {
+      const uint32_t d = s_deg[tid * kBodies + i];
+      sum += d;
+      most = d > most ? d : most;
+    }
+    if (most > kSmallDegree) s_crowd = 1u;
+    uint32_t off = block_exclusive(sum, s_tot);
+    for (int i = 0; i < kBodies; ++i) {
+      s_off[tid * kBodies + i] = off;
+      off += s_deg[tid * kBodies + i];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    const int m = tid + kSmallThreads * e;
+    if (at[e].x != kNoPlace) s_adj[s_off[bb[e].x] + at[e].x] = uint16_t(m);
+    if (at[e].y != kNoPlace) s_adj[s_off[bb[e].y] + at[e].y] = uint16_t(m);
+  }
+  __syncthreads();
+  const bool crowd = s_crowd != 0u;
+  if (crowd) {  // the graph for k_colour_round
+    for (int i = tid; i < b.n; i += kSmallThreads) {
+      sb.deg[i] = s_deg[i];
+      sb.adj_off[i] = s_off[i];
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const int m = tid + kSmallThreads * e;
+      if (at[e].x != kNoPlace) sb.adj[s_off[bb[e].x] + at[e].x] = m;
+      if (at[e].y != kNoPlace) sb.adj[s_off[bb[e].y] + at[e].y] = m;
+    }
+  }
+  // the rounds of k_colour_round; the first manifold in priority is coloured in each, so M rounds end it
+  for (uint32_t round = 1; !crowd && round <= uint32_t(M); ++round) {
+    uint32_t* left = &s_left[round & 1u];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const int m = tid + kSmallThreads * e;
+      if (m >= M || s_state[m] != kUncoloured) continue;
+      const uint32_t pm = colour_hash(uint32_t(m));
+      const uint32_t n1 = at[e].x != kNoPlace ? s_deg[bb[e].x] : 0u, n2 = at[e].y != kNoPlace ? s_deg[bb[e].y] : 0u;
+      const uint32_t o1 = s_off[bb[e].x], o2 = s_off[bb[e].y];
+      const uint32_t n = n1 + n2;
+      bool wait = false;
+      uint64_t mask = 0;  // colours 0-63 of the neighbours coloured before this round
+      for (uint32_t k = 0; k < n && !wait; ++k) {
+        const int o = int(s_adj[k < n1 ? o1 + k : o2 + (k - n1)]);
+        if (o == m) continue;
+        const uint32_t so = s_state[o];
+        if (so == kUncoloured || (so >> 16) == round) {
+          const uint32_t po = colour_hash(uint32_t(o));
+          wait = po > pm || (po == pm && o > m);
+        } else {
+          const uint32_t cc = so & 0xffffu;
+          if (cc < 64u) mask |= 1ull << cc;
+        }
+      }
+      if (wait) {
+        *left = 1u;
+        continue;
+      }
+      uint32_t colour = 0;
+      for (uint32_t base = 0;; base += 64) {
+        if (base > 0u) {
+          mask = 0;
+          for (uint32_t k = 0; k < n; ++k) {
+            const int o = int(s_adj[k < n1 ? o1 + k : o2 + (k - n1)]);
+            if (o == m) continue;
+            const uint32_t so = s_state[o];
+            if (so == kUncoloured || (so >> 16) == round) continue;
+            const uint32_t cc = so & 0xffffu;
+            if (cc >= base && cc < base + 64) mask |= 1ull << (cc - base);
+          }
+        }
+        if (mask != ~0ull) {
+          colour = base + uint32_t(__ffsll((long long)(~mask))) - 1u;
+          break;
+        }
+      }
+      s_state[m] = (round << 16) | colour;
+      s_last = round;  // every writer of a round stores the same
+    }
+    __syncthreads();
+    const bool more = *left != 0u;
+    if (tid == 0) s_left[(round & 1u) ^ 1u] = 0u;
+    __syncthreads();
+    if (!more) break;
+  }
+  // the order
+  for (int d = tid; d < kColourDigits; d += kSmallThreads) {
+    s_m[d] = s_c[d] = 0u;
+    for (int w = 0; w < kSmallThreads / 64; ++w) s_wave[w][d] = 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    const int m = tid + kSmallThreads * e;
+    if (m >= M) continue;
+    const uint32_t st = s_state[m], cnt = uint32_t(c.mcount[m]);
+    sb.state[m] = st;
+    const uint32_t d = colour_digit<kColourDigits, kSplit>(st, cnt);
+    atomicAdd(&s_m[d], 1u);
+    atomicAdd(&s_c[d], cnt);
+    atomicMax(&s_most, (st & 0xffffu) + 1u);
+  }
+  __syncthreads();
+  const uint32_t vm = tid < kColourDigits ? s_m[tid] : 0u, vc = tid < kColourDigits ? s_c[tid] : 0u;
+  const uint32_t em = block_exclusive(vm, s_tot), ec = block_exclusive(vc, s_tot);
+  if (tid < kColourDigits) {
+    s_m[tid] = em;
+    s_c[tid] = ec;
+    sb.col_start[tid] = em;
+    sb.class_rec[tid] = ec;
+  }
+  if (tid == 0) {
+    sb.col_start[kColourDigits] = uint32_t(M);
+    sb.class_rec[kColourDigits] = uint32_t(C);
+    words[0] = 0u;
+    words[1] = crowd ? 1u : 0u;
+    words[2] = s_most;
+    words[3] = s_last;
+  }
+  __syncthreads();  // also sb.state and sb.place, which the tiles read again
+  for (int base = 0; base < M; base += kColourTile)
+    scatter_tile<kColourDigits, kSmallThreads, kSplit>(c, M, base, sb, s_m, s_c, s_wave);
 }
 
 // One fill_constraint_geometry call: body-side jacobian (dir, p x dir), weighted angular part,
@@ -1267,6 +1466,16 @@ void launch_colour_begin(const DevBodies& b, const DevContacts& c, int M, const 
   hipLaunchKernelGGL(k_colour_begin, dim3(nb(M)), dim3(256), 0, s, b, c, M, prev, prevM, prev_state, sb);
   scan_exclusive_u32(sb.deg, sb.adj_off, b.n, *sb.scan, s);
   hipLaunchKernelGGL(k_adjacency, dim3(nb(M)), dim3(256), 0, s, c, M, sb);
+}
+
+void launch_colour_small(const DevBodies& b, const DevContacts& c, int M, int C, const DevContacts& prev, int prevM,
+                         const uint32_t* prev_state, bool split, SolverBufs& sb, uint32_t* words, hipStream_t s) {
+  if (split)
+    hipLaunchKernelGGL(k_colour_small<true>, dim3(1), dim3(kSmallThreads), 0, s, b, c, M, C, prev, prevM, prev_state, sb,
+                       words);
+  else
+    hipLaunchKernelGGL(k_colour_small<false>, dim3(1), dim3(kSmallThreads), 0, s, b, c, M, C, prev, prevM, prev_state, sb,
+                       words);
 }
 
 void launch_colour_round(const DevContacts& c, int M, int round, uint32_t* remaining, uint32_t* last_round,

@@ -172,6 +172,13 @@ constexpr int kColourDigits = 512;
 size_t colour_hist_words(int M, int digits);
 void launch_colour_order(const DevContacts& c, int M, int C, int digits, bool split, SolverBufs& sb, uint32_t* ncol,
                          hipStream_t s);
+// All of the above in one launch, for 0 < M <= kSmallManifolds and b.n <= kSmallColourBodies: words[0] becomes 0, words[1]
+// too but where a body has too many manifolds for it, which leaves the rounds to launch_colour_round, words[2] the number of colours and words[3] the last round that coloured a manifold. The order is of
+// kColourDigits digits, as launch_colour_order's, and where the colours are more it has to be made again.
+constexpr int kSmallManifolds = 2048;
+constexpr int kSmallColourBodies = 4096;
+void launch_colour_small(const DevBodies& b, const DevContacts& c, int M, int C, const DevContacts& prev, int prevM,
+                         const uint32_t* prev_state, bool split, SolverBufs& sb, uint32_t* words, hipStream_t s);
 int residual_blocks(int M);
 void launch_assemble(const DevBodies& b, const DevContacts& cur, const DevContacts& prev,
                      int prevM, int M, const SimParams& p, SolverBufs& sb, const MatTable& mt, hipStream_t s);

@@ -178,6 +178,9 @@ struct World {
   // more, within these bounds
   static constexpr int kMinRounds = 4, kMaxRounds = 32;
   int round_batch[2] = {kMinRounds, kMinRounds};
+  // solves left for which a world too crowded for k_colour_small goes by it
+  static constexpr int kCrowdedSolves = 16;
+  int crowded[2] = {0, 0};
   std::vector<int> colour_visit;  // colour classes in visiting order
   long solve_count = 0;    // solves performed, never reset
   std::vector<ClassSpan> h_span;    // their slots, in that order
@@ -1230,11 +1233,18 @@ struct World {
     const int prevM = have_solved ? sview_M[cur ^ 1] : 0;
     const ContactBufs& pc = cb[cur ^ 1];
     uint32_t* sm = bp_small.as<uint32_t>();
-    launch_colour_begin(b, c, M, sview[cur ^ 1], prevM, sv_state2[cur ^ 1].as<uint32_t>(), v, stream);
+    const uint32_t* prev_state = sv_state2[cur ^ 1].as<uint32_t>();
     int digits = kColourDigits;
     // recorded samples and predictions keep the row order that does not depend on the contact counts
     split_order = !learned_rows();
-    bool rounds = true, waiting = true;
+    // one workgroup while its lanes have two manifolds each at most (as many as its LDS holds with the bodies, and a
+    // world whose launches cost more than they do), and not soon after one that was too crowded for it
+    int& wait_small = crowded[ccd_sub ? 1 : 0];
+    const bool small = M <= kSmallManifolds && n <= kSmallColourBodies && wait_small == 0;
+    if (wait_small > 0) --wait_small;
+    if (small) launch_colour_small(b, c, M, C, sview[cur ^ 1], prevM, prev_state, split_order, v, sm + kSmRemaining, stream);
+    else launch_colour_begin(b, c, M, sview[cur ^ 1], prevM, prev_state, v, stream);
+    bool rounds = !small, ordered = small, waiting = true;
     int& batch = round_batch[ccd_sub ? 1 : 0];
     for (int round = 1;;) {
       if (rounds) {
@@ -1244,7 +1254,8 @@ struct World {
         for (int k = 0; k < batch; ++k, ++round)
           launch_colour_round(c, M, round, sm + kSmRemaining + (k == batch - 1 ? 1 : 0), sm + kSmLastRound, v, stream);
       }
-      launch_colour_order(c, M, C, digits, split_order, v, sm + kSmColours, stream);
+      if (!ordered) launch_colour_order(c, M, C, digits, split_order, v, sm + kSmColours, stream);
+      ordered = false;
       const uint32_t seq = rb_post({{sm + kSmRemaining, kSmColouring, 0},
                                     {v.col_start, digits + 1, kRbClass},
                                     {v.class_rec, digits + 1, kRbClass + kMaxColours + 2}});
@@ -1254,6 +1265,7 @@ struct World {
       const int rc = rb_wait(seq);
       if (rc) return rc;
       rounds = rb_host[1] != 0;
+      if (small && rounds && round == 1) wait_small = kCrowdedSolves;
       ncolours = int(rb_host[kSmColours - kSmRemaining]);
       if (rounds) continue;
       if (ncolours > kMaxColours) return set_err(NPHYS_ERR_STATE, "too many colours");
@@ -1265,7 +1277,7 @@ struct World {
       v = sv_view();
     }
     colour_rounds = int(rb_host[kSmLastRound - kSmRemaining]);
-    batch = std::min(std::max(colour_rounds + 1, kMinRounds), kMaxRounds);
+    if (colour_rounds > 0 || !small) batch = std::min(std::max(colour_rounds + 1, kMinRounds), kMaxRounds);
     // visit order (the SplitMix64 Fisher-Yates shuffle seeded by the solve index), slot ranges in that
     // order and the largest class
     const uint32_t* h_colstart = rb_host + kRbClass;

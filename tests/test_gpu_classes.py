@@ -45,3 +45,35 @@ def test_class_sizes(nphys, oracle_mod, nboxes, nballs, variant):
         for key in ("pos", "rot", "linvel", "angvel"):
             np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
     assert g.counters()["ncolours"] >= 1
+
+
+def _same_steps(nphys, oracle_mod, s, steps):
+    g = nphys.MechanicalWorld(integration_parameters=abi.default_params())
+    o = oracle_mod.OracleWorld(abi.default_params(), precision=32, order=oracle_mod.ORDER_COLOURED)
+    for w in (g, o):
+        w.add_bodies(s)
+    for k in range(steps):
+        g.step(1)
+        o.step(1)
+        gs, os_ = g.get_state(), o.get_state()
+        for key in ("pos", "rot", "linvel", "angvel"):
+            np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
+    return g.counters()
+
+
+@pytest.mark.parametrize("nballs,above", [(1023, 0), (1024, 0), (1025, 0), (2047, 0), (2048, 0), (2049, 0), (100, 3995),
+                                          (100, 3996)])
+def test_colouring_edges(nphys, oracle_mod, nballs, above):
+    """Up to 2,048 manifolds among 4,096 bodies one workgroup colours and orders them: the last sizes it takes
+    and the first it does not, with `above` bodies that touch nothing."""
+    s = _resting(0, nballs + above)
+    s["pos"][1 + nballs:, 1] += 20.0
+    _same_steps(nphys, oracle_mod, s, 2)
+
+
+@pytest.mark.parametrize("grid", [(6, 6, 6), (9, 8, 9), (9, 9, 9), (10, 9, 9), (12, 9, 9)])
+def test_colouring_of_stacks(nphys, oracle_mod, grid):
+    """Cuboids inside their neighbours: some 600 to 2,700 manifolds of several colours, on both sides of the
+    2,048 that one workgroup colours."""
+    nx, ny, nz = grid
+    _same_steps(nphys, oracle_mod, scenes.boxes(nx=nx, ny=ny, nz=nz, spacing=0.995), 3)
