@@ -159,6 +159,36 @@ __global__ void __launch_bounds__(256) k_gather_contacts(DevContacts c, int M, c
   }
 }
 
+// The contacts as the arrays that a caller reads, four lanes per manifold, written straight to host memory
+// (neighbouring lanes, neighbouring places). What bounds it is that link: 56 bytes a contact. Copying bodies and counts to the host
+// for their prefix sum, that back, and the 48-byte records then took
+// 328 us a call at 10,007 cuboids; this, with the copy out of the staging buffer, 87.
+__global__ void __launch_bounds__(256) k_contacts_out(DevContacts c, int M, const uint32_t* __restrict__ moff, uint32_t cap,
+                                                     ContactRows out, uint32_t* counted) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int m = t >> 2, k = t & 3;
+  if (m >= M) return;
+  const int cnt = c.mcount[m];
+  if (m == M - 1 && k == 0) *counted = moff[m] + uint32_t(cnt);
+  const uint32_t i = moff[m] + uint32_t(k);
+  if (k >= cnt || i >= cap) return;
+  const float4* r = c.contact(c.mfirst[m] + k);
+  const float4 r0 = r[0], r1 = r[1], r2 = r[2];
+  const int2 bb = c.mbody[m];
+  if (out.row[0]) reinterpret_cast<int2*>(out.row[0])[i] = bb;
+  if (out.row[1]) out.row[1][i] = r1.w;
+  const float3 v[3] = {make_float3(r0.x, r0.y, r0.z), make_float3(r1.x, r1.y, r1.z), make_float3(r2.x, r2.y, r2.z)};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    if (!out.row[2 + a]) continue;
+    float* o = out.row[2 + a] + 3 * long(i);
+    o[0] = v[a].x;
+    o[1] = v[a].y;
+    o[2] = v[a].z;
+  }
+  if (out.row[5]) out.row[5][i] = r0.w;
+}
+
 }  // namespace
 
 size_t manifold_tiles(int npairs) { return (size_t(npairs) + kManifoldTile - 1) / kManifoldTile; }
@@ -183,6 +213,11 @@ void launch_gather_contacts(const DevContacts& c, int M, const uint32_t* moff, f
   if (M <= 0) return;
   hipLaunchKernelGGL(k_gather_contacts, dim3(unsigned((M + 255) / 256)), dim3(256), 0, s, c, M, moff, dense,
                      dense_imp);
+}
+
+void launch_contacts_out(const DevContacts& c, int M, const uint32_t* moff, uint32_t cap, const ContactRows& out,
+                         uint32_t* counted, hipStream_t s) {
+  hipLaunchKernelGGL(k_contacts_out, dim3(unsigned((4l * M + 255) / 256)), dim3(256), 0, s, c, M, moff, cap, out, counted);
 }
 
 }  // namespace nph

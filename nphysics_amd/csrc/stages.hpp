@@ -125,6 +125,15 @@ struct NarrowPhaseBufs {
 void launch_narrow_bins(const DevBodies& b, const int2* pairs, NarrowPhaseBufs& np, DevContacts out, hipStream_t s);
 size_t manifold_tiles(int npairs);  // tiles of the scan state that the narrow phase takes
 void launch_narrow_phase(const DevBodies& b, const int2* pairs, NarrowPhaseBufs& np, DevContacts out, hipStream_t s);
+// Contact arrays by row: bodies, feature (as bits), world1, world2, normal, depth (null: not wanted).
+struct ContactRows {
+  static constexpr int kRows = 6;
+  static constexpr int kWidth[kRows] = {2, 1, 3, 3, 3, 1};
+  float* row[kRows];
+};
+// Contact k of manifold m to place moff[m] + k of the rows (at most `cap` places); their number to *counted.
+void launch_contacts_out(const DevContacts& c, int M, const uint32_t* moff, uint32_t cap, const ContactRows& out,
+                         uint32_t* counted, hipStream_t s);
 // Contacts of all manifolds in manifold order, gathered from their slots into dense records
 // (kContactFields float4 each) and impulses (dense_imp may be null); moff = exclusive scan of the
 // manifolds' counts.

@@ -781,19 +781,25 @@ struct World {
     return NPHYS_OK;
   }
 
+  // At least `need` bytes of the staging buffer.
+  int io_room(size_t need) {
+    if (need <= io_cap) return NPHYS_OK;
+    HIPCK(hipStreamSynchronize(stream));
+    if (io_host) (void)hipHostFree(io_host);
+    io_host = nullptr;
+    io_cap = 0;
+    HIPCK(hipHostMalloc(reinterpret_cast<void**>(&io_host), need, hipHostMallocMapped | hipHostMallocCoherent));
+    io_cap = need;
+    HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&io_dev), io_host, 0));
+    return NPHYS_OK;
+  }
+
   // Where the four packed state arrays stand in the pinned staging buffer (grown to fit, at 16-byte
   // aligned starts): as the host and as the device address them.
   int state_rows(const bool (&want)[4], StateRows& host, StateRows& dev) {
-    const size_t pad = (size_t(n) + 3) & ~size_t(3), need = pad * 13 * sizeof(float);
-    if (need > io_cap) {
-      HIPCK(hipStreamSynchronize(stream));
-      if (io_host) (void)hipHostFree(io_host);
-      io_host = nullptr;
-      io_cap = 0;
-      HIPCK(hipHostMalloc(reinterpret_cast<void**>(&io_host), need, hipHostMallocMapped | hipHostMallocCoherent));
-      io_cap = need;
-      HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&io_dev), io_host, 0));
-    }
+    const size_t pad = (size_t(n) + 3) & ~size_t(3);
+    const int rc = io_room(pad * 13 * sizeof(float));
+    if (rc) return rc;
     const size_t off[4] = {0, pad * 3, pad * 7, pad * 10};
     for (int a = 0; a < 4; ++a) {
       host.row[a] = want[a] ? io_host + off[a] : nullptr;
@@ -1040,6 +1046,44 @@ struct World {
       }
       return NPHYS_OK;
     }
+  }
+
+  int pairs_out(int32_t* out) {
+    const size_t bytes = size_t(npairs) * sizeof(int2);
+    int rc = io_room(bytes);
+    if (rc) return rc;
+    HIPCK(hipMemcpyAsync(io_host, pairs.p, bytes, hipMemcpyDeviceToHost, stream));
+    HIPCK(hipStreamSynchronize(stream));
+    std::memcpy(out, io_host, bytes);
+    return NPHYS_OK;
+  }
+
+  // The contacts of `c` in manifold order into `out` (arrays may be null): their places by a prefix sum, the
+  // arrays written by the device in the staging buffer.
+  int contacts_out(ContactBufs& c, const ContactRows& out) {
+    const int M = c.M;
+    const size_t C = size_t(c.C), pad = (C + 3) & ~size_t(3);
+    HIPCK(rd_moff.ensure(size_t(std::max(M, 1)) * 4));
+    HIPCK(scan.ensure(scan_tiles(size_t(std::max(M, 1))), stream));
+    int rc = io_room((pad * 13 + 4) * sizeof(float));
+    if (rc) return rc;
+    ContactRows dev, host;
+    size_t off = 4;  // the first word: the contacts counted
+    for (int a = 0; a < ContactRows::kRows; ++a) {
+      host.row[a] = io_host + off;
+      dev.row[a] = out.row[a] ? io_dev + off : nullptr;
+      off += pad * ContactRows::kWidth[a];
+    }
+    const DevContacts v = c.view();
+    scan_exclusive_u32(reinterpret_cast<const uint32_t*>(v.mcount), rd_moff.as<uint32_t>(), M, scan, stream);
+    launch_contacts_out(v, M, rd_moff.as<uint32_t>(), uint32_t(C), dev, reinterpret_cast<uint32_t*>(io_dev), stream);
+    if ((rc = readback({}))) return rc;
+    uint32_t counted;
+    std::memcpy(&counted, io_host, 4);
+    if (counted != uint32_t(C)) return set_err(NPHYS_ERR_STATE, "contact count mismatch");
+    for (int a = 0; a < ContactRows::kRows; ++a)
+      if (out.row[a]) std::memcpy(out.row[a], host.row[a], C * size_t(ContactRows::kWidth[a]) * sizeof(float));
+    return NPHYS_OK;
   }
 
   // The contacts of `c` in manifold order (dense records and, when imp is given, impulses), with
@@ -2369,9 +2413,7 @@ int nphys_read_pairs(nphys_world* w, int32_t* pairs, int64_t cap) {
   if (!w || (!pairs && w->w.npairs)) return set_err(NPHYS_ERR_INVALID, "null argument");
   if (cap < w->w.npairs) return set_err(NPHYS_ERR_CAPACITY, "pair buffer too small");
   if (w->w.npairs == 0) return NPHYS_OK;
-  if (hipMemcpy(pairs, w->w.pairs.p, size_t(w->w.npairs) * sizeof(int2), hipMemcpyDeviceToHost) != hipSuccess)
-    return set_err(NPHYS_ERR_HIP, "pair copy failed");
-  return NPHYS_OK;
+  return w->w.pairs_out(pairs);
 }
 
 int nphys_num_contacts(nphys_world* w, int64_t* n) {
@@ -2386,23 +2428,8 @@ int nphys_read_contacts(nphys_world* w, int32_t* bodies, uint32_t* feature, floa
   nph::ContactBufs& c = w->w.cb[w->w.cur];
   if (cap < c.C) return set_err(NPHYS_ERR_CAPACITY, "contact buffer too small");
   if (c.C == 0) return NPHYS_OK;
-  std::vector<int2> mb;
-  std::vector<int> mc;
-  std::vector<float4> rec;
-  int rc = w->w.gather_contacts(c, mb, mc, rec, nullptr);
-  if (rc) return rc;
-  long i = 0;
-  for (size_t m = 0; m < mb.size(); ++m)
-    for (int k = 0; k < mc[m]; ++k, ++i) {
-      const float4* r = &rec[size_t(i) * nph::kContactFields];
-      if (bodies) { bodies[2 * i] = mb[m].x; bodies[2 * i + 1] = mb[m].y; }
-      if (feature) feature[i] = nph::bits_of(r[1].w);
-      if (world1) { world1[3 * i] = r[0].x; world1[3 * i + 1] = r[0].y; world1[3 * i + 2] = r[0].z; }
-      if (world2) { world2[3 * i] = r[1].x; world2[3 * i + 1] = r[1].y; world2[3 * i + 2] = r[1].z; }
-      if (normal) { normal[3 * i] = r[2].x; normal[3 * i + 1] = r[2].y; normal[3 * i + 2] = r[2].z; }
-      if (depth) depth[i] = r[0].w;
-    }
-  return NPHYS_OK;
+  return w->w.contacts_out(c, nph::ContactRows{{reinterpret_cast<float*>(bodies), reinterpret_cast<float*>(feature),
+                                                world1, world2, normal, depth}});
 }
 
 int nphys_num_manifolds(nphys_world* w, int64_t* n) {
