@@ -771,7 +771,7 @@ def main():
         "stage_rooflines": stage_rooflines(c, args.steps, C, M, n_dyn, c["npairs"], iters,
                                            params.max_position_iterations),
         "roofline": {
-            "kernel": "k_pgs (one colour class of one SOR-Prox sweep, classes of more than 512 manifolds; "
+            "kernel": "k_pgs (one colour class of one SOR-Prox sweep, classes of more than 1,024 lanes; "
                       "average over every k_pgs launch of the timing region)",
             "bound": "hbm",
             "achieved": achieved,
@@ -873,7 +873,7 @@ def stage_rooflines(c, steps, C, M, N, P, sweeps, pos_iters):
     impulse cache add to its time); the broad phase counts a full pass (the incremental update
     moves less)."""
     rows = {
-        "velocity_resolution": (sweeps * (168 * C + 76 * N), "k_warmstart + k_pgs sweeps: (168 C + 76 N) per sweep"),
+        "velocity_resolution": (sweeps * (168 * C + 76 * N), "k_pgs sweeps: (168 C + 76 N) per sweep"),
         "position_resolution": (pos_iters * (48 * C + 84 * N), "k_position: (48 C + 84 N) per iteration"),
         "assembly": (224 * C + 104 * N, "colouring + k_assemble: 224 C + 104 N"),
         "narrow_phase": (100 * P + 48 * C, "narrow phase: 100 P + 48 C"),

@@ -378,8 +378,8 @@ int nphys_set_residual_target(nphys_world* w, double target, int32_t max_sweeps,
  * pass over all manifolds of the colour; 256, 512, 1024: per solve one launch for the warm start
  * and sweeps and one for the position passes, one workgroup per scene (the scene's velocity
  * increments, then its poses, in LDS; that many lanes for a scene of more than 256 dynamic bodies,
- * 64 for the others, which run beside them on a second stream). Scene-blocked only when every
- * scene has at most 2048 dynamic bodies and the world has no joints; otherwise 0 is used.
+ * 128 for the others, which run beside them on a second stream). Scene-blocked only when every
+ * scene has at most 2048 dynamic bodies, the world has no joints and a solve 2 to 512 colours; otherwise 0 is used.
  * -1 (default): an autotuner times every eligible variant over the first steps and keeps the
  * fastest. All variants give bit-identical results. No reference counterpart (the reference has
  * one sequential loop). */

@@ -1,4 +1,4 @@
-// nphysics_amd/csrc/k_broadphase.hip -- broad phase: loose AABBs, Morton LBVH, pair emission.
+// nphysics_amd/csrc/k_broadphase.hip -- broad phase: loose AABBs, search by boxes in Morton order, pair emission.
 //
 // Replaces ncollide's DBVTBroadPhase behind GeometricalWorld::perform_broad_phase
 // (src/world/geometrical_world.rs:60, 285-312) and its DefaultCollisionFilter (:926-971):

@@ -20,7 +20,7 @@
 // of the contact with the same (body1, body2, feature) key (the ImpulseCache lookup at
 // signorini_coulomb_pyramid_model.rs:104-108).
 //
-// Solve (k_warmstart / k_pgs) restates SORProx (src/solver/sor_prox.rs:19-436): warm start dv += l W J,
+// Solve (k_pgs) restates SORProx (src/solver/sor_prox.rs:19-436): warm start dv += l W J,
 // then per sweep and contact the normal row (projected on l >= 0) and the two friction rows (bounded by
 // mu times the normal impulse just computed, zeroed when it is zero). Manifolds of one colour share no
 // dynamic body, so one launch per colour performs exactly the sequential Gauss-Seidel updates of
@@ -828,13 +828,6 @@ __device__ __forceinline__ void load_dv(const DevBodies& b, const Manifold<kMask
   if (m.x.d1) b.load_dv(m.x.b1, v1.l, v1.a);
   if (m.x.d2) b.load_dv(m.x.b2, v2.l, v2.a);
 }
-
-// Solver velocity increments in HBM (the per-colour kernels; the scene-blocked one has them in LDS).
-struct GlobalDv {
-  DevBodies b;
-  __device__ void load(int body, Dv& v) const { b.load_dv(body, v.l, v.a); }
-  __device__ void store(int body, const Dv& v) const { b.store_dv(body, v.l, v.a); }
-};
 
 // The value of the other lane of the pair: a quad permutation (1, 0, 3, 2), one instruction, where a
 // shuffle goes through the LDS crossbar and stands in every row's serial chain. Both lanes of a pair
