@@ -245,7 +245,7 @@ __device__ __forceinline__ bool overlap(const aabb& a, const aabb& c) {
 // loose-AABB passes are on the device, so no readback stands between the passes and the search.
 __device__ __forceinline__ bool search_incremental(const BroadPhaseBufs& bp, const SearchRun& r, int n) {
   const uint32_t all = bp.changed[0] + bp.changed[2], fixed = bp.changed[1] + bp.changed[3];
-  return r.may_increment && fixed == 0u && r.dirty_before + long(all) <= long(kept_limit(n));
+  return r.may_increment && fixed == 0u && all <= uint32_t(kept_limit(n));
 }
 
 // ---- search by boxes -----------------------------------------------------------------------------

@@ -79,8 +79,7 @@ inline size_t search_boxes(size_t n) { return (n + 63) / 64 + (n + 4095) / 4096;
 // The order of the colliders (by scene and Morton code), sorted anew.
 void launch_order(const DevBodies& b, BroadPhaseBufs& bp, hipStream_t s);
 // A pair search: directly, with the end of the last non-dynamic collider, or by boxes over the order;
-// the segment capacity, and whether segments may be kept (loose AABBs replaced before this step's
-// passes since the last search: dirty_before).
+// the segment capacity, and whether segments may be kept.
 // Segments are kept while at most this many of n bodies are dirty: every clean body tests them all,
 // which at 1,024 costs as much as a search of its own.
 __host__ __device__ inline int kept_limit(int n) { return n / 8 < 1024 ? n / 8 : 1024; }
@@ -90,7 +89,6 @@ struct SearchRun {
   int fixed_end;
   int cap;
   int may_increment;
-  long dirty_before;
 };
 void launch_search(const DevBodies& b, BroadPhaseBufs& bp, const SearchRun& r, hipStream_t s);
 // Where the compaction leaves the pairs: their number, the narrow phase's lists (cuboid-cuboid pairs

@@ -140,20 +140,22 @@ struct World {
   // broad phase
   DBuf bp_dirty, bp_list;
   // The segments of the last search stand; searches by the present order (sorted anew every
-  // kOrderAge-th, and when the bodies were added or moved by the caller); the loose-AABB replacements (all,
-  // of non-dynamic bodies) since the last search.
+  // kOrderAge-th, and when the bodies were added or moved by the caller).
   bool segments_valid = false;
   bool incremental_bp = true;
   static constexpr int kOrderAge = 16;
   int order_age = kOrderAge;
-  int64_t dirty_pending = 0, dirty_static_pending = 0;
   DBuf bp_small, keys, vals, keys_alt, vals_alt, leaf_mn, leaf_mx, box_mn, box_mx, box_top, cand, cand_count, pairs,
       bp_tmp;
   int cap = 32;
   int npairs = 0;
   bool pairs_dirty = true;
+  // Pairs a narrow phase takes: a manifold's first slot is packed in 28 bits of the solver's slot record.
+  static constexpr int kMostPairs = (1 << 28) / kPairSlots - 1;
+  int most_pairs = kMostPairs;
   bool moved = true;
-  bool recollide = false;  // collision groups changed: the next step starts with collision detection
+  // the next step starts with collision detection: collision groups changed, or the last detection failed
+  bool recollide = false;
 
   // narrow phase
   DBuf np_count, np_perm;
@@ -962,11 +964,26 @@ struct World {
   static constexpr int kSmStats = 16, kSmTotals = 24, kSmBoxes = 26, kSmBalls = 27, kSmListCount = 28, kSmPairs = 29;
 
   // GeometricalWorld::sync_colliders (the loose-AABB passes of `passes`), perform_broad_phase and,
-  // when `narrow`, perform_narrow_phase into cb[cur]. Everything is enqueued with room for an eighth
-  // more pairs than last time and read back once at the end; if the pairs or a body's segment did not
-  // fit, buffers grow and the launches after the loose passes run again. *changed: loose AABBs replaced.
-  // bp_done and np_done, when given, are recorded after the two phases.
+  // when `narrow`, perform_narrow_phase into cb[cur]. *changed: loose AABBs replaced. bp_done and np_done, when
+  // given, are recorded after the two phases. Where it fails there are no manifolds, and no pairs unless their
+  // list is complete (too many of them for the narrow phase); the next step begins with another detection.
   int detect(int passes, bool narrow, int64_t* changed, hipEvent_t bp_done = nullptr, hipEvent_t np_done = nullptr) {
+    bool listed = false;
+    const int rc = find_pairs(passes, narrow, changed, bp_done, np_done, listed);
+    segments_valid = listed;
+    pairs_dirty = !listed;
+    if (!listed) npairs = 0;
+    if (rc) {
+      cb[cur].C = cb[cur].M = 0;
+      recollide = true;
+    }
+    return rc;
+  }
+
+  // Everything is enqueued with room for an eighth more pairs than last time and read back once at the end;
+  // if the pairs or a body's segment did not fit, buffers grow and the launches after the loose passes
+  // run again. npairs is the new list's length from when it is stored (`listed`).
+  int find_pairs(int passes, bool narrow, int64_t* changed, hipEvent_t bp_done, hipEvent_t np_done, bool& listed) {
     int rc = ensure_bp();
     if (rc) return rc;
     const DevBodies b = bodies();
@@ -980,17 +997,13 @@ struct World {
       launch_order(b, v, stream);
       order_age = 0;
     }
-    bool may = segments_valid && incremental_bp && !pairs_dirty && dirty_static_pending == 0;
-    const long dirty_before = long(dirty_pending);
-    bool first = true;
-    for (int room = npairs + npairs / 8 + 1024;;) {
-      // a manifold's first slot is packed in 28 bits of the solver's slot record
-      constexpr int kMostPairs = ((1 << 28) / kPairSlots) - 1;
-      if (npairs > kMostPairs) return set_err(NPHYS_ERR_CAPACITY, "too many broad-phase pairs");
-      room = std::min(room, kMostPairs);
+    bool may = segments_valid && incremental_bp && !pairs_dirty;
+    bool manifolds = narrow;
+    for (int64_t want = int64_t(npairs) + npairs / 8 + 1024;;) {
+      const int room = int(std::min<int64_t>(want, manifolds ? most_pairs : INT_MAX));
       ContactBufs& out = cb[cur];
       NarrowPhaseBufs np{};
-      if ((rc = ensure_narrow(room, narrow ? &out : nullptr, np))) return rc;
+      if ((rc = ensure_narrow(room, manifolds ? &out : nullptr, np))) return rc;
       HIPCK(pairs.ensure(size_t(room) * sizeof(int2)));
       v = bp_view();
       SearchRun r{};
@@ -998,28 +1011,22 @@ struct World {
       r.fixed_end = fixed_end;
       r.cap = cap;
       r.may_increment = may ? 1 : 0;
-      r.dirty_before = dirty_before;
       launch_search(b, v, r, stream);
       PairOut po;
       po.npairs = sm + kSmPairs;
       po.nbox = np.nbox;
       po.nball = np.nball;
       po.perm = np.perm;
-      po.bfirst = narrow ? out.bfirst.as<int>() : nullptr;
+      po.bfirst = manifolds ? out.bfirst.as<int>() : nullptr;
       po.pair_cap = room;
       launch_compact_pairs(b, v, cap, direct, po, stream);
       if (bp_done) HIPCK(hipEventRecord(bp_done, stream));
-      if (narrow) launch_narrow_phase(b, pairs.as<int2>(), np, out.view(), stream);
+      if (manifolds) launch_narrow_phase(b, pairs.as<int2>(), np, out.view(), stream);
       if (np_done) HIPCK(hipEventRecord(np_done, stream));
       if ((rc = readback({{sm, kSmPairs + 1, 0}}))) return rc;
-      if (first) {
-        dirty_pending += int64_t(h[0]) + h[2];
-        dirty_static_pending += int64_t(h[1]) + h[3];
-        *changed = int64_t(h[0]) + h[2];
-        first = false;
-      }
+      *changed = int64_t(h[0]) + h[2];
       // the device's rule (search_incremental), for the counters
-      const bool incremental = may && dirty_static_pending == 0 && dirty_pending <= kept_limit(n);
+      const bool incremental = may && h[1] + h[3] == 0 && *changed <= kept_limit(n);
       if (int(h[kSmStats]) > cap) {
         // a segment took more partners than it has room for: all search again, with larger segments
         if (incremental) ++counters.incremental_overflows;
@@ -1029,21 +1036,22 @@ struct World {
         fill_u32(sm + kSmStats, 0u, kSmListCount - kSmStats, stream);
         continue;
       }
-      npairs = int(h[kSmPairs]);
-      if (npairs > room) {
-        room = npairs + npairs / 8;
+      const uint32_t found = h[kSmPairs];
+      if (found > uint32_t(room)) {
+        if (found > uint32_t(INT_MAX)) return set_err(NPHYS_ERR_CAPACITY, "too many broad-phase pairs");
+        manifolds = manifolds && int(found) <= most_pairs;  // else the pair list alone
+        want = int64_t(found) + found / 8;
         // the segments stand, and as the dirty flags are cleared an incremental search keeps them
         fill_u32(sm + kSmStats, 0u, kSmListCount - kSmStats, stream);
         continue;
       }
+      npairs = int(found);
+      listed = true;
       if (incremental && *changed != 0) ++counters.incremental_pair_updates;
-      dirty_pending = dirty_static_pending = 0;
-      segments_valid = true;
-      pairs_dirty = false;
-      if (narrow) {
-        out.C = int(h[kSmTotals]);
-        out.M = int(h[kSmTotals + 1]);
-      }
+      if (!narrow) return NPHYS_OK;
+      if (!manifolds) return set_err(NPHYS_ERR_CAPACITY, "too many broad-phase pairs");
+      out.C = int(h[kSmTotals]);
+      out.M = int(h[kSmTotals + 1]);
       return NPHYS_OK;
     }
   }
@@ -1147,6 +1155,7 @@ struct World {
   // The narrow phase of `np` pairs (in pair order; their number also at *count_dev) into `out`. Without
   // `totals`, the host does not wait for its contact and manifold counts.
   int narrow_phase_of(const int2* list, int np, uint32_t* count_dev, ContactBufs& out, bool totals = true) {
+    if (np > most_pairs) return set_err(NPHYS_ERR_CAPACITY, "too many broad-phase pairs");
     NarrowPhaseBufs v{};
     const int rc0 = ensure_narrow(np, &out, v);
     if (rc0) return rc0;
@@ -2388,6 +2397,14 @@ int nphys_set_sweep_variant(nphys_world* w, int32_t variant) {
   w->w.variant_request = variant;
   w->w.tune_cands.clear();
   w->w.tuned = false;
+  return NPHYS_OK;
+}
+
+// For the tests, and so not in the header: a smaller limit than kMostPairs for this world (at least 1: no
+// launch of the narrow phase is for fewer pairs).
+int nphys_test_most_pairs(nphys_world* w, int32_t pairs) {
+  if (!w || pairs < 1 || pairs > nph::World::kMostPairs) return set_err(NPHYS_ERR_INVALID, "bad argument");
+  w->w.most_pairs = pairs;
   return NPHYS_OK;
 }
 
