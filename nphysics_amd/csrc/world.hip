@@ -1202,18 +1202,6 @@ struct World {
     HIPCK(sv_pgeo.ensure(m * 2 * sizeof(float4)));
     rec_stride = long(std::min({sv_rec.bytes / (kRecFields * sizeof(float4)), sv_lam.bytes / sizeof(float4),
                                 sv_prec.bytes / (3 * sizeof(float4))}));
-    const size_t need = size_t(residual_blocks(M)) * 2 + 4;  // + the joints' partial
-    if (need > red_cap) {
-      HIPCK(hipStreamSynchronize(stream));
-      if (red_host) (void)hipHostFree(red_host);
-      red_host = nullptr;
-      red_cap = 0;
-      const size_t grown = std::max<size_t>(need + need / 2, 1024);
-      HIPCK(hipHostMalloc(reinterpret_cast<void**>(&red_host), grown * sizeof(double),
-                          hipHostMallocMapped | hipHostMallocCoherent));
-      red_cap = grown;
-      HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&red_dev), red_host, 0));
-    }
     HIPCK(scan.ensure(std::max(scan_tiles(hw), scan_tiles(nn)), stream));
     return NPHYS_OK;
   }
@@ -1446,15 +1434,30 @@ struct World {
   // Natural-map residual of the current impulses: the per-block partials go straight to host memory and
   // are reduced there in block order (max is exact; the sum of squares is the RMS) once the stream
   // has passed them: residual() waits, while the fixed-count mode's, which nothing in the step
-  // needs, is reduced after the step's last readback (with `cache` the kernel stores the impulses too).
-  void residual_deferred(const DevBodies& b, const DevContacts& cv, int M, int C, bool cache, SolverBufs& v) {
-    launch_residual(b, cv, M, cache, v, stream);
+  // needs, is reduced after the step's last readback (with `cache` the kernel stores the impulses too). The
+  // buffer grows here alone: a CCD substep, which solves in between, has no residual.
+  int residual_deferred(const DevBodies& b, const DevContacts& cv, int M, int C, bool cache, SolverBufs& v) {
     const int nbk = residual_blocks(M);
+    const size_t need = size_t(nbk) * 2 + 4;  // + the joints' partial
+    if (need > red_cap) {
+      HIPCK(hipStreamSynchronize(stream));
+      if (red_host) (void)hipHostFree(red_host);
+      red_host = nullptr;
+      red_cap = 0;
+      const size_t grown = std::max<size_t>(need + need / 2, 1024);
+      HIPCK(hipHostMalloc(reinterpret_cast<void**>(&red_host), grown * sizeof(double),
+                          hipHostMallocMapped | hipHostMallocCoherent));
+      red_cap = grown;
+      HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&red_dev), red_host, 0));
+    }
+    v.red = red_dev;
+    launch_residual(b, cv, M, cache, v, stream);
     JointBufs jv = joint_view();
     if (nj > 0) launch_joint_residual(b, jv, v.red + 2 * nbk, stream);
     res_pending_blocks = nbk;
     res_pending_C = C;
     res_pending_joints = nj > 0;
+    return NPHYS_OK;
   }
   bool res_pending_joints = false;
 
@@ -1477,10 +1480,10 @@ struct World {
   }
 
   int residual(const DevBodies& b, const DevContacts& cv, int M, int C, SolverBufs& v) {
-    residual_deferred(b, cv, M, C, false, v);
-    const int rc = readback({});
+    int rc = residual_deferred(b, cv, M, C, false, v);
+    if (rc || (rc = readback({}))) return rc;
     finish_residual();
-    return rc;
+    return NPHYS_OK;
   }
 
   SceneBlocks sc_view() {
@@ -1568,8 +1571,7 @@ struct World {
     if (res_target <= 0.0) {
       if ((rc = sweeps(b, v, true, prm.max_velocity_iterations))) return rc;
       nsw = prm.max_velocity_iterations;
-      residual_deferred(b, cv, M, C, true, v);
-      return NPHYS_OK;
+      return residual_deferred(b, cv, M, C, true, v);
     }
     if ((rc = sweeps(b, v, true, 0))) return rc;
     int done = 0;
@@ -1667,6 +1669,7 @@ struct World {
     solved_M = M;
     solved_C = C;
     res_inf = res_rms = 0.0;
+    res_pending_blocks = -1;  // of a step that failed after its solve
     ncolours = 0;
     if (M == 0 && nj == 0) {
       last_sweeps = res_target > 0.0 ? 0 : prm.max_velocity_iterations;

@@ -141,3 +141,33 @@ def test_ccd_rejects_sleeping_bodies(nphys):
     g.add_bodies(s)
     with pytest.raises(Exception):
         g.step(1)
+
+
+def test_residual_of_a_step_with_a_larger_substep(nphys):
+    """The step's residual is that of its solve, also where a CCD substep after it solves far more manifolds
+    (131,044, in 512 workgroups of a residual; the first buffer holds 510): the same as without the CCD phase."""
+    side = 362
+    n = side * side
+    pile = scenes.boxes(nx=3, ny=3, nz=3, spacing=0.995)  # cuboids inside their neighbours, in motion
+    pile["linvel"][1:] = np.random.default_rng(3).uniform(-1.0, 1.0, (27, 3))
+    pile["ccd_enabled"] = np.zeros(len(pile["shape"]), np.int32)
+    rain = scenes._empty(n)
+    rain["dims"][:, 0] = 0.2
+    i = np.arange(n)
+    rain["pos"][:] = np.stack([100.0 + 0.6 * (i % side), np.full(n, 0.7), 100.0 + 0.6 * (i // side)], 1)
+    rain["linvel"][:, 1] = -60.0
+    rain["ccd_enabled"] = np.ones(n, np.int32)
+    floor = scenes.ground(half_extents=(500.0, 0.5, 500.0))
+    floor["ccd_enabled"] = np.zeros(len(floor["shape"]), np.int32)
+    got = []
+    for substeps in (0, 1):
+        p = abi.default_params(max_velocity_iterations=1, max_ccd_substeps=substeps)
+        w = nphys.MechanicalWorld(integration_parameters=p)
+        w.add_bodies(scenes.concat(floor, pile, rain))
+        w.step(1)
+        got.append(w.residual())
+        c = w.counters()
+        assert c["ccd_substeps"] == substeps and (c["ccd_impacts"] >= n) == (substeps == 1)
+        assert 0 < c["nmanifolds"] < 1000
+        w.close()
+    assert got[0] == got[1] and got[0][0] > 0.0
