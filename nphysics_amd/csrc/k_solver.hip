@@ -1127,7 +1127,7 @@ __global__ void __launch_bounds__(kRunLanes) k_colour_run(DevBodies b, SolverBuf
 }
 
 // Scene-blocked sweeps: one workgroup per scene runs the warm start (when warm) and nsweeps sweeps over
-// all colours in the visiting order, two lanes per manifold as k_pgs, the scene's dynamic-body velocity increments
+// all colours in the visiting order, on the lanes that k_pgs gives a class, the scene's dynamic-body velocity increments
 // resident in LDS and a barrier between colours. Every body sees the same sequence of row updates as
 // under the per-colour launches (manifolds of one colour share no dynamic body; colours and sweeps
 // keep their order), so the results are identical.
@@ -1136,7 +1136,9 @@ __global__ void __launch_bounds__(kRunLanes) k_colour_run(DevBodies b, SolverBuf
 // lane's next phase are loaded while this one is solved, and the ids of the one after (info, in the scene's
 // order). No load's latency stands between two barriers, and the barrier orders LDS alone. Impulses are stored before
 // the barrier and read again visit.n - 1 phases later at the earliest (visit.n >= 2): the stores of
-// all earlier phases are waited for before a phase's loads are issued. The scene's one compute unit
+// all earlier phases are waited for before a phase's loads are issued. With 1,024 lanes (128 registers each) a second
+// contact in flight would spill, and four waves per SIMD cover its loads: sweeps 493 -> 426 us in a pile of 1,900
+// without it, 608 -> 461 with jacobian masks (512 lanes: 557 and 593). The scene's one compute unit
 // bounds it, by its issue rate: 428 us at 1,021 scenes of 100 bodies (405 with a launch per class),
 // 188 against 155 at one of 1,001, and faster where many tiny classes follow one another.
 struct SceneItem {
@@ -1155,6 +1157,7 @@ __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBu
   __shared__ float4 s_a[kCap];  // linear x, y, z, angular x
   __shared__ float2 s_b[kCap];  // angular y, z
   __shared__ ClassSpan s_span[kVisitColours];
+  constexpr bool kAhead = kBlock <= 512;
   const int s = scene_list[blockIdx.x], tid = threadIdx.x, h = tid & 1;
   const int d0 = sc.dyn_start[s], nd = sc.dyn_start[s + 1] - d0;
   const int n = visit.n;
@@ -1212,14 +1215,16 @@ __global__ void __launch_bounds__(kBlock) k_sweeps_blocked(DevBodies b, SolverBu
   SceneItem it, here;
   ContactLane<kMask> next;
   item(0, tid, here);
-  load_lane(b, sb, here.q, here.k, h, next);
+  if (kAhead) load_lane(b, sb, here.q, here.k, h, next);
   item(after(0), tid, it);
   for (int ph = 0; ph < n * nsweeps; ++ph) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    ContactLane<kMask> m = next;
+    ContactLane<kMask> m;
+    if (kAhead) m = next;
+    else load_lane(b, sb, here.q, here.k, h, m);
     int local = here.local;
     here = it;
-    load_lane(b, sb, it.q, it.k, h, next);
+    if (kAhead) load_lane(b, sb, it.q, it.k, h, next);
     item(after(after(k)), tid, it);
     for (int L = tid;;) {
       if (m.cnt) {
@@ -1603,8 +1608,8 @@ void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, 
   hipLaunchKernelGGL(k_scene_info, dim3(nb(M)), dim3(256), 0, s, M, sb, sc);
 }
 
-// Two launches: the scenes with more than kSmallScene dynamic bodies (256 or 512 lanes, 48 KB of LDS)
-// on s_large, the others (64-lane workgroups, many resident per CU) on s_small, so the few large
+// Two launches: the scenes with more than kSmallScene dynamic bodies (256, 512 or 1,024 lanes, 54 KB of LDS)
+// on s_large, the others (128-lane workgroups, many resident per CU) on s_small, so the few large
 // scenes run beside the many small ones.
 template <bool kMask>
 void sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit, int nsweeps,

@@ -253,7 +253,7 @@ __device__ __forceinline__ ClassSpan scene_span(const SceneBlocks& sc, const Vis
 }
 void launch_scene_order(const DevBodies& b, int M, int nscenes, int scene_bits, int digits, SolverBufs& sb,
                         SceneBlocks& sc, hipStream_t s);
-// block: lanes per large scene (256 or 512; 1024 runs as 512); the large scenes go on s_large, the small on s_small
+// block: lanes per large scene (256, 512 or 1024); the large scenes go on s_large, the small on s_small
 void launch_sweeps_blocked(const DevBodies& b, SolverBufs& sb, const SceneBlocks& sc, const VisitOrder& visit,
                            int nsweeps, bool warm, int block, hipStream_t s_small, hipStream_t s_large);
 // Scene-blocked position correction: `iterations` passes over the colours in the visiting order,
