@@ -138,3 +138,46 @@ def test_crowd_steps(nphys, oracle_mod, n):
         for key in ("pos", "rot", "linvel", "angvel"):
             np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
     assert g.counters()["ncolours"] >= (n - 1 if n < 257 else 257)
+
+
+def _sliding(n, ccd):
+    """Balls and cuboids on a ground without friction, a third of them sliding at 1 mm a step: their loose AABBs,
+    10 mm wider, are replaced every tenth step or so, and from the thirtieth step on bodies come near each other."""
+    s = scenes.boxes(nx=n, ny=1, nz=1)
+    i = np.arange(n)
+    side = int(np.ceil(np.sqrt(n)))
+    ball = i % 2 == 0
+    s["rot"][1:] = (0.0, 0.0, 0.0, 1.0)
+    s["shape"][1:] = np.where(ball, 0, 1)
+    s["dims"][1:] = np.where(ball[:, None], [0.5, 0.0, 0.0], [0.4, 0.5, 0.5])
+    s["pos"][1:] = np.stack([1.3 * (i % side) - 0.65 * side, np.full(n, 0.519), 1.07 * (i // side) - 0.535 * side], 1)
+    s["dims"][0] = (3.0 * side, 0.5, 3.0 * side)
+    s["friction"][:] = 0.0
+    s["linvel"][1:] = s["angvel"][1:] = 0.0
+    s["linvel"][1:, 2] = np.where(np.random.default_rng(n).random(n) < 0.3, 0.06, 0.0)
+    if ccd:
+        s["ccd_enabled"] = (np.arange(n + 1) % 10 == 5).astype(np.int32)
+    return s
+
+
+@pytest.mark.parametrize("ccd", [False, True])
+@pytest.mark.parametrize("n", [65, 700, 2100])
+def test_calm_steps(nphys, oracle_mod, n, ccd):
+    """Most detections replace no loose AABB and keep the pairs and their lists by kind; those that follow
+    and do replace some begin as if they did not."""
+    s = _sliding(n, ccd)
+    g = nphys.MechanicalWorld(integration_parameters=abi.default_params())
+    o = oracle_mod.OracleWorld(abi.default_params(), precision=32, order=oracle_mod.ORDER_COLOURED)
+    for w in (g, o):
+        w.add_bodies(s)
+    steps = ""
+    for k in range(40):
+        before = g.counters()["pair_rebuilds"]
+        for w in (g, o):
+            w.step(1)
+        steps += "x" if g.counters()["pair_rebuilds"] > before else "."
+        _same(g, o, f"step {k + 1}")
+        gs, os_ = g.get_state(), o.get_state()
+        for key in ("pos", "rot", "linvel", "angvel"):
+            np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
+    assert steps.count("......") >= 3 and steps.count("...x") >= 3, steps
