@@ -47,6 +47,29 @@ def test_class_sizes(nphys, oracle_mod, nboxes, nballs, variant):
     assert g.counters()["ncolours"] >= 1
 
 
+@pytest.mark.parametrize("crowd", [256, 300])
+def test_many_colours_in_many_scenes(nphys, oracle_mod, crowd):
+    """As many scenes as there can be, all but one of them empty, and in that one a crowd of as many colours as
+    bodies: the blocked launches hold a class's place for each."""
+    s = scenes._empty(crowd)
+    s["dims"][:, 0] = 0.3
+    s["pos"][:] = np.random.default_rng(crowd).uniform(-0.02, 0.02, (crowd, 3))
+    s["scene"] = np.full(crowd, 32767, np.int32)
+    g = nphys.MechanicalWorld(integration_parameters=abi.default_params())
+    o = oracle_mod.OracleWorld(abi.default_params(), precision=32, order=oracle_mod.ORDER_COLOURED)
+    for w in (g, o):
+        w.add_bodies(s)
+    g.set_sweep_variant(256)
+    for k in range(2):
+        for w in (g, o):
+            w.step(1)
+        gs, os_ = g.get_state(), o.get_state()
+        for key in ("pos", "rot", "linvel", "angvel"):
+            np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
+    assert crowd - 1 <= g.counters()["ncolours"] <= 511
+    assert g.counters()["sweep_variant"] == 256
+
+
 def _same_steps(nphys, oracle_mod, s, steps):
     g = nphys.MechanicalWorld(integration_parameters=abi.default_params())
     o = oracle_mod.OracleWorld(abi.default_params(), precision=32, order=oracle_mod.ORDER_COLOURED)
