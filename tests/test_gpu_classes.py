@@ -9,9 +9,12 @@ from nphysics_amd import abi, scenes
 pytestmark = pytest.mark.gpu
 
 
-def _resting(nboxes, nballs):
+def _resting(nboxes, nballs, chain=False):
     """Boxes and balls apart from each other, a little inside the ground: one class of
-    nboxes four-contact and nballs one-contact manifolds."""
+    nboxes four-contact and nballs one-contact manifolds. chain: the last ball in a row with two more above the
+    ground instead (with nballs 0, three balls more), which gives the class one of their two manifolds and a second class the other."""
+    if chain:
+        nballs = max(nballs - 1, 0) + 3
     n = nboxes + nballs
     side = int(np.ceil(np.sqrt(n)))
     s = scenes.boxes(nx=n, ny=1, nz=1)  # and the ground
@@ -25,6 +28,9 @@ def _resting(nboxes, nballs):
     s["pos"][1:, 2] = 1.7 * (i // side) - 0.85 * side
     s["linvel"][1:] = rng.uniform(-1.0, 1.0, (n, 3))
     s["angvel"][1:] = rng.uniform(-1.0, 1.0, (n, 3))
+    if chain:
+        s["pos"][-3:] = [(0.99 * k, 20.0, 0.0) for k in range(3)]
+        s["linvel"][-3:] = 0.0
     return s
 
 
@@ -32,7 +38,7 @@ def _resting(nboxes, nballs):
 @pytest.mark.parametrize("nboxes,nballs", [(1, 0), (0, 1), (1, 1), (15, 33), (32, 129), (127, 4), (127, 5), (128, 0),
                                            (129, 0), (0, 512), (0, 513), (300, 700)])
 def test_class_sizes(nphys, oracle_mod, nboxes, nballs, variant):
-    s = _resting(nboxes, nballs)
+    s = _resting(nboxes, nballs, chain=variant > 0)  # the blocked variants are for two colours and more
     g = nphys.MechanicalWorld(integration_parameters=abi.default_params())
     o = oracle_mod.OracleWorld(abi.default_params(), precision=32, order=oracle_mod.ORDER_COLOURED)
     for w in (g, o):
@@ -44,7 +50,8 @@ def test_class_sizes(nphys, oracle_mod, nboxes, nballs, variant):
         gs, os_ = g.get_state(), o.get_state()
         for key in ("pos", "rot", "linvel", "angvel"):
             np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
-    assert g.counters()["ncolours"] >= 1
+        assert g.counters()["ncolours"] == (2 if variant else 1)
+        assert g.counters()["sweep_variant"] == variant
 
 
 @pytest.mark.parametrize("crowd", [256, 300])
