@@ -788,16 +788,18 @@ struct World {
     return NPHYS_OK;
   }
 
-  // At least `need` bytes of the staging buffer.
+  // At least `need` bytes of the staging buffer, which grows by half at least: contacts and pairs read at every
+  // frame of a filling scene would else pin a new buffer at each.
   int io_room(size_t need) {
     if (need <= io_cap) return NPHYS_OK;
+    need = std::max(need, io_cap + io_cap / 2);
     HIPCK(hipStreamSynchronize(stream));
     if (io_host) (void)hipHostFree(io_host);
     io_host = nullptr;
     io_cap = 0;
     HIPCK(hipHostMalloc(reinterpret_cast<void**>(&io_host), need, hipHostMallocMapped | hipHostMallocCoherent));
-    io_cap = need;
     HIPCK(hipHostGetDevicePointer(reinterpret_cast<void**>(&io_dev), io_host, 0));
+    io_cap = need;
     return NPHYS_OK;
   }
 
