@@ -1940,13 +1940,19 @@ struct World {
     const DevBodies b = bodies();
     const float target = sp.allowed_linear_error;
     const int on_pen = prm.ccd_on_penetration_enabled;
+    (void)hipGetLastError();  // an earlier call's
     launch_ccd_first(b, pairs.as<int2>(), npairs, c, end_time, dt0, target, on_pen, stream);
-    for (int rounds = 1;; rounds = 4) {  // no impacts, or few: one round ends it
+    // The first batch is one round, which ends it where there are no impacts or few. Every round but the last
+    // freezes a body at least, so n + 1 of them end it; a launch that was refused would leave the queue as it is.
+    int64_t done = 0;
+    for (int rounds = 1;; rounds = 4) {
       for (int k = 0; k < rounds; ++k) launch_ccd_events(b, c, end_time, dt0, target, on_pen, stream);
+      HIPCK(hipGetLastError());
       const int rc = readback({{c.ctl, kCcdWords, 0}});
       if (rc) return rc;
       if (rb_host[kCcdOverflow]) return set_err(NPHYS_ERR_CAPACITY, "CCD impact queue overflow");
       if (rb_host[kCcdState] == kQueueDone) break;
+      if ((done += rounds) > n) return set_err(NPHYS_ERR_STATE, "CCD impact queue did not end");
     }
     *kind = int(rb_host[kCcdKind]);
     ccd_nimp = *kind == PREDICT_IMPACTS ? int(rb_host[kCcdImpacts]) : 0;
