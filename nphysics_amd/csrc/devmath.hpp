@@ -23,7 +23,6 @@ struct f3 {
   float x, y, z;
 };
 
-NPH_HD f3 mk3(float x, float y, float z) { return f3{x, y, z}; }
 NPH_HD f3 add(f3 a, f3 b) { return f3{a.x + b.x, a.y + b.y, a.z + b.z}; }
 NPH_HD f3 sub(f3 a, f3 b) { return f3{a.x - b.x, a.y - b.y, a.z - b.z}; }
 NPH_HD f3 neg(f3 a) { return f3{-a.x, -a.y, -a.z}; }
@@ -260,10 +259,6 @@ NPH_HD aabb merged(aabb a, aabb b) { return aabb{vmin(a.mn, b.mn), vmax(a.mx, b.
 NPH_HD bool contains(aabb a, aabb b) {
   return a.mn.x <= b.mn.x && a.mn.y <= b.mn.y && a.mn.z <= b.mn.z && a.mx.x >= b.mx.x &&
          a.mx.y >= b.mx.y && a.mx.z >= b.mx.z;
-}
-NPH_HD bool intersects(aabb a, aabb b) {
-  return a.mn.x <= b.mx.x && a.mn.y <= b.mx.y && a.mn.z <= b.mx.z && a.mx.x >= b.mn.x &&
-         a.mx.y >= b.mn.y && a.mx.z >= b.mn.z;
 }
 
 enum : int { SHAPE_BALL = 0, SHAPE_CUBOID = 1 };

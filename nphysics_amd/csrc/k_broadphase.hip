@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(64) k_top(BroadPhaseBufs bp, int nbox) {
   }
 }
 
-// All six comparisons evaluated (intersects() stops at the first that fails: a branch each).
+// All six comparisons evaluated (with && it would stop at the first that fails: a branch each).
 __device__ __forceinline__ bool overlap(const aabb& a, const aabb& c) {
   return (a.mn.x <= c.mx.x) & (c.mn.x <= a.mx.x) & (a.mn.y <= c.mx.y) & (c.mn.y <= a.mx.y) & (a.mn.z <= c.mx.z) &
          (c.mn.z <= a.mx.z);

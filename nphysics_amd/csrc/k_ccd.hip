@@ -72,8 +72,8 @@ __device__ __forceinline__ CcdMotion part_motion(const DevBodies& b, int i, floa
 // ---- time of impact on sixteen lanes ----
 // Sixteen lanes (one DPP row) share a query, all with the same arguments: lanes 0-7 move body 1 and lanes 8-15 body 2, each
 // lane measures one of the 15 axes of the cuboid / cuboid separation, and the largest is found by
-// three permutation steps. The same expressions as time_of_impact's and toi_separation's, in the same order,
-// so the same bits; a single lane takes some 1,000 instructions per iterate, these some 350.
+// four permutation steps. The expressions of the scalar form (of toi_separation for the axes), in its order, so the
+// same bits; a single lane takes some 1,000 instructions per iterate, these some 350.
 constexpr int kToiLanes = 16;
 
 template <int Ctrl>
@@ -146,7 +146,7 @@ __device__ bool pair_toi(const DevBodies& b, const CcdBufs& c, int i, int j, flo
   const int k1 = b.shape[i], k2 = b.shape[j];
   const f3 h1 = xyz(b.dims[i]), h2 = xyz(b.dims[j]);
   const float max_toi = end_time - start;
-  // velocities as time_of_impact takes them; both bodies' in every lane
+  // what turns and moves: both bodies' velocities in every lane
   const f3 z{0.0f, 0.0f, 0.0f};
   const f3 v = m.kind == MOTION_STATIC ? z : m.v;
   const f3 w = m.kind == MOTION_ROTATING ? m.w : z;
@@ -313,14 +313,10 @@ __device__ __forceinline__ unsigned long long wave_min(unsigned long long k) {
   return (static_cast<unsigned long long>(mh) << 32) | ml;
 }
 
-// The smallest key of slots [first, last) (uniform) but for slot `but`.
-__device__ __forceinline__ unsigned long long range_min(const unsigned long long* key, int first, int last, int but,
-                                                        int lane) {
+// The smallest key of slots [first, last) (uniform).
+__device__ __forceinline__ unsigned long long range_min(const unsigned long long* key, int first, int last, int lane) {
   unsigned long long m = kNoKey;
-  for (int k = first + lane; k < last; k += 64) {
-    const unsigned long long x = key[k];
-    m = (k != but && x < m) ? x : m;
-  }
+  for (int k = first + lane; k < last; k += 64) m = key[k] < m ? key[k] : m;
   return wave_min(m);
 }
 
@@ -406,7 +402,7 @@ __global__ void __launch_bounds__(kEventBlock) k_ccd_events(DevBodies b, CcdBufs
   }
   for (int g = wave; g < ng; g += kEventBlock / 64) {
     const unsigned long long m =
-        state == kQueueNew ? range_min(c.key, g << sh, min((g + 1) << sh, ns), -1, lane) : c.group[g];
+        state == kQueueNew ? range_min(c.key, g << sh, min((g + 1) << sh, ns), lane) : c.group[g];
     if (lane == 0) s_min[g] = m;
   }
   if (LdsFrozen)
@@ -533,7 +529,7 @@ __global__ void __launch_bounds__(kEventBlock) k_ccd_events(DevBodies b, CcdBufs
     const int nd = s_ndirty;
     for (int k = wave; k < nd; k += kEventBlock / 64) {
       const int g = s_dirty[k];
-      const unsigned long long m = range_min(c.key, g << sh, min((g + 1) << sh, ns), -1, lane);
+      const unsigned long long m = range_min(c.key, g << sh, min((g + 1) << sh, ns), lane);
       if (lane == 0) {
         s_min[g] = m;
         s_bits[g >> 5] = 0u;

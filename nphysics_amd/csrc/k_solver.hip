@@ -8,7 +8,7 @@
 // seen as "this round" whichever value the load returns; the result is independent of timing.
 // Colours persist across steps: manifolds whose body pair was solved in the previous step keep
 // their colour and only new manifolds run the rounds, so at rest colouring costs one pass.
-// Manifolds are then sorted by colour (stable radix sort) and row records laid out in that order.
+// Manifolds are then put in colour order by a stable counting sort and row records laid out in that order.
 //
 // Assembly (k_assemble, one lane per manifold) restates SignoriniCoulombPyramidModel::constraints
 // (src/solver/signorini_coulomb_pyramid_model.rs:56-224), SignoriniModel::build_velocity_constraint
@@ -685,7 +685,7 @@ struct SlotCtx {
   uint32_t r0;
 };
 
-// One 16-byte load gives everything a lane needs about its manifold (see k_slot_info).
+// One 16-byte load gives everything a lane needs about its manifold (see k_colour_scatter).
 __device__ __forceinline__ SlotCtx slot_ctx(const SolverBufs& sb, int s) {
   const int4 q = sb.sinfo[s];
   SlotCtx x;
@@ -731,11 +731,6 @@ __device__ __forceinline__ void load_rec(const SolverBufs& sb, uint32_t r, CRec&
   c.mu = c.lam.w;
 }
 
-struct Inv {
-  m33 m;
-  float im;
-};
-
 // Jacobian masks of a manifold's two bodies (only the masked kernel variants carry them).
 template <bool kMask>
 struct Masks {
@@ -761,22 +756,15 @@ struct Masks<true> {
 template <bool kMask>
 struct Manifold {
   SlotCtx x;
-  Inv i1, i2;
   CRec c[4];
   f3 t1[4], t2[4];
   Masks<kMask> mk;
 };
 
-// Everything a lane needs for its manifold, loaded up front: the loads are independent of the
-// Gauss-Seidel chain, so they are all in flight together.
+// A whole manifold on one lane (the residual), loaded up front: all loads are in flight together.
 template <bool kMask>
 __device__ __forceinline__ void load_manifold(const DevBodies& b, const SolverBufs& sb, int s, Manifold<kMask>& m) {
   m.x = slot_ctx(sb, s);
-  m.i1.im = m.i2.im = 0.0f;
-  m.i1.m = m33{};
-  m.i2.m = m33{};
-  if (m.x.d1) m.i1.m = load_inv(b, m.x.b1, m.i1.im);
-  if (m.x.d2) m.i2.m = load_inv(b, m.x.b2, m.i2.im);
   m.mk.load(b, m.x);
 #pragma unroll
   for (int k = 0; k < 4; ++k)
@@ -786,14 +774,13 @@ __device__ __forceinline__ void load_manifold(const DevBodies& b, const SolverBu
     }
 }
 
-// Row `row` (0 normal, 1 and 2 friction) of contact k: w = J dv + rhs and the dv update. Both
-// bodies' terms are always evaluated, a static body having zero inverse mass and inertia and a
-// zero dv: its terms are then exact zeros, so w and every dv component equal those of the
+// Row `row` (0 normal, 1 and 2 friction) of contact k, for w = J dv + rhs. Both bodies' terms are always
+// evaluated, a static body having a zero dv: its terms are then exact zeros, so w equals the
 // one-body expression (up to the sign of a zero), and a wavefront mixing ground and body-body
 // manifolds runs one code path. The masked variant multiplies each body's jacobian by its mask,
 // as k_assemble's fill_geom does.
 struct Row {
-  f3 d1, d2, a1, a2, wa1, wa2;
+  f3 d1, d2, a1, a2;
   float r, rhs;
 };
 
@@ -808,19 +795,11 @@ __device__ __forceinline__ Row row_of(const Manifold<kMask>& m, int k, int row) 
   v.a2 = m.mk.a2(ang2(c, d));
   v.r = c.r[row];
   v.rhs = c.rhs[row];
-  v.wa1 = mulv(m.i1.m, v.a1);
-  v.wa2 = mulv(m.i2.m, v.a2);
   return v;
 }
 
 __device__ __forceinline__ float row_w(const Row& v, const Dv& x1, const Dv& x2) {
   return (dot6(v.d1, v.a1, x1) + dot6(v.d2, v.a2, x2)) + v.rhs;
-}
-
-template <bool kMask>
-__device__ __forceinline__ void row_add(const Row& v, float alpha, const Manifold<kMask>& m, Dv& x1, Dv& x2) {
-  axpy6(alpha, scale(v.d1, m.i1.im), v.wa1, x1);
-  axpy6(alpha, scale(v.d2, m.i2.im), v.wa2, x2);
 }
 
 template <bool kMask>

@@ -49,7 +49,7 @@ struct MlpDev {
   const float* params;   // [kNumParams] FP32 (biases and normalisation are read from here)
 };
 
-// Training-time buffers of one batch of B rows (B a multiple of 64).
+// Training-time buffers of one batch of B rows.
 struct MlpBatch {
   int B;
   const float* X;        // [n][24] dataset features

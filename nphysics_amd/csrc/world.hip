@@ -690,7 +690,7 @@ struct World {
                     &ccd_flags, &ccd_keys})
       HIPCK(b->ensure(size_t(n1) * 4));
     HIPCK(ccd_rot.ensure(size_t(n1) * f4b));
-    // scene bits above the Morton code: the BVH keeps every scene in its own key range
+    // scene bits above the Morton code: the order keeps every scene in its own key range
     int max_scene = 0;
     for (int sc : h_scene) max_scene = std::max(max_scene, sc);
     scene_bits = 0;

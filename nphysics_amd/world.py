@@ -314,7 +314,7 @@ class MechanicalWorld:
         _check(self._L.nphys_set_sweep_variant(self._h, variant))
 
     def set_incremental_pairs(self, on=True):
-        """Incremental pair-set updates (default) or a full tree build on every change."""
+        """Incremental pair-set updates (default) or a search of every body on every change."""
         _check(self._L.nphys_set_incremental_pairs(self._h, 1 if on else 0))
 
     def set_warmstart_judge(self, on=True):
