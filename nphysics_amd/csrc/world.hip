@@ -1006,7 +1006,7 @@ struct World {
     // and only where the readback tells of a replaced AABB is everything searched. Broad phase at rest
     // 137 -> 16 us at 262,144 balls and 67 -> 14 at 99,996 (with a readback before every search, as there was once,
     // 22 at rest, and the search waits for it otherwise).
-    const bool stand = calm[narrow ? 1 : 0] == kCalm && segments_valid && !pairs_dirty && !(passes & LOOSE_STATIC) &&
+    const bool stand = calm[narrow ? 1 : 0] == kCalm && segments_valid && !pairs_dirty &&
                        (!narrow || (list_room > 0 && npairs <= most_pairs));
     fill_u32(sm, 0u, stand ? kSmBoxes : kSmPairs + 1, stream);
     launch_loose_update(b, passes, v, stream);

@@ -181,3 +181,23 @@ def test_calm_steps(nphys, oracle_mod, n, ccd):
         for key in ("pos", "rot", "linvel", "angvel"):
             np.testing.assert_array_equal(gs[key], np.asarray(os_[key]).astype(np.float32), err_msg=f"{key}, step {k + 1}")
     assert steps.count("......") >= 3 and steps.count("...x") >= 3, steps
+
+
+@pytest.mark.parametrize("n", [65, 2100])
+def test_calm_queries(nphys, oracle_mod, n):
+    """Collision queries that move the bodies by less than their margins, and then one that moves static ones
+    (alone) further: after the calm ones it begins as one of them."""
+    s = _shuffled(n, n, statics=0.3)
+    g, o = _worlds(nphys, oracle_mod, s)
+    rng = np.random.default_rng(n)
+    static = s["status"] == 1
+    pos = s["pos"].copy()
+    for far in (0.0, 0.0, 0.0, 0.0, 0.3, 0.0, 0.0, 0.0, 0.0):
+        query = pos + rng.uniform(-2e-4, 2e-4, (n, 3)).astype(np.float32)
+        if far:
+            pos[static] += rng.uniform(-far, far, (int(static.sum()), 3)).astype(np.float32)
+            query[static] = pos[static]
+        for w in (g, o):
+            w.set_state(pos=query)
+            w.collide()
+        _same(g, o, f"far {far}")
