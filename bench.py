@@ -174,7 +174,7 @@ def learned_section(fresh, net_params, train, iters, targets, steps, max_sweeps)
             if ci["warmstart_inference_time"] > 0:
                 tf = MLP_FLOP_PER_ROW * ci["warmstart_inference_rows"] / ci["warmstart_inference_time"] / 1e12
                 r["inference_roofline"] = {
-                    "kernel": "k_mlp_fwd (fused 3-layer BF16 MFMA inference, one row per contact)",
+                    "kernel": "k_mlp_pass<false> (fused 3-layer BF16 MFMA inference, one row per contact)",
                     "bound": "mfma", "achieved": tf, "peak": BF16_DENSE_TFLOPS, "unit": "TFLOP/s",
                     "frac": tf / BF16_DENSE_TFLOPS, "rows": ci["warmstart_inference_rows"],
                     "us": 1e6 * ci["warmstart_inference_time"], "flop_per_row": MLP_FLOP_PER_ROW}
